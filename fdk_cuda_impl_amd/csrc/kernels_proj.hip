@@ -413,81 +413,88 @@ joseph_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy
     finish_joseph(proj, i, nu, nv, u, v, pix, lo <= hi, acc, r.L, accumulate);
 }
 
+// The copy kernels write every entry of their copy, the zero guards among
+// them: no zero fill before them (a second pass over the copy; without it one
+// OS-SART sweep of 10 subsets at 128 x 128 x 100 x 120 views went from 5.66 to
+// 5.32 ms, a SART sweep at 64 x 60 x 48 x 40 views from 2.09 to 1.92 ms).
+//
 // paired separable copy, X-main: [x][row y + guard][column z + guard];
-// blockIdx.z is the row, 32 x 32 (x, z) tiles of the two source rows
+// blockIdx.z is the row, 32 x 32 (x, column) tiles of the two source rows
 // through LDS
 __global__ void pair_zfast_x_kernel(const float* __restrict__ in, float2* __restrict__ out,
     int nx, int ny, int nz)
 {
     __shared__ float tile[2][32][33];
     const int r = blockIdx.z;
-    const int x0 = blockIdx.x * 32, z0 = blockIdx.y * 32;
+    const int x0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
     const size_t rows = size_t(ny) + 2 * kJosephGuard - 1, cols = size_t(nz) + 2 * kJosephGuard;
     for (int k = threadIdx.y; k < 32; k += 8) {
-        const int z = z0 + k, x = x0 + threadIdx.x;
+        const int z = e0 + k - kJosephGuard, x = x0 + threadIdx.x;
+        const bool in_xz = x < nx && z >= 0 && z < nz;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int y = r + h - kJosephGuard;
-            tile[h][k][threadIdx.x] = x < nx && z < nz && y >= 0 && y < ny ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
+            tile[h][k][threadIdx.x] = in_xz && y >= 0 && y < ny ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
         }
     }
     __syncthreads();
     for (int k = threadIdx.y; k < 32; k += 8) {
-        const int x = x0 + k, z = z0 + threadIdx.x;
-        if (x < nx && z < nz)
-            out[(size_t(x) * rows + r) * cols + z + kJosephGuard] = make_float2(tile[0][threadIdx.x][k], tile[1][threadIdx.x][k]);
+        const int x = x0 + k, e = e0 + threadIdx.x;
+        if (x < nx && e < int(cols))
+            out[(size_t(x) * rows + r) * cols + e] = make_float2(tile[0][threadIdx.x][k], tile[1][threadIdx.x][k]);
     }
 }
 
 // paired separable copy, Y-main: [y][row x + guard][column z + guard];
-// blockIdx.z is y, 32 x 32 (row, z) tiles (33 source columns of x) through
-// LDS
+// blockIdx.z is y, 32 x 32 (row, column) tiles (33 source columns of x)
+// through LDS
 __global__ void pair_zfast_y_kernel(const float* __restrict__ in, float2* __restrict__ out,
     int nx, int ny, int nz)
 {
     __shared__ float tile[32][34];
     const int y = blockIdx.z;
-    const int r0 = blockIdx.x * 32, z0 = blockIdx.y * 32;
+    const int r0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
     const int rows = nx + 2 * kJosephGuard - 1;
     const size_t cols = size_t(nz) + 2 * kJosephGuard;
     for (int k = threadIdx.y; k < 32; k += 8) {
-        const int z = z0 + k;
+        const int z = e0 + k - kJosephGuard;
         for (int t = threadIdx.x; t < 33; t += 32) {
             const int x = r0 + t - kJosephGuard;
-            tile[k][t] = z < nz && x >= 0 && x < nx ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
+            tile[k][t] = z >= 0 && z < nz && x >= 0 && x < nx ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
         }
     }
     __syncthreads();
     for (int k = threadIdx.y; k < 32; k += 8) {
-        const int r = r0 + k, z = z0 + threadIdx.x;
-        if (r < rows && z < nz)
-            out[(size_t(y) * rows + r) * cols + z + kJosephGuard] = make_float2(tile[threadIdx.x][k], tile[threadIdx.x][k + 1]);
+        const int r = r0 + k, e = e0 + threadIdx.x;
+        if (r < rows && e < int(cols))
+            out[(size_t(y) * rows + r) * cols + e] = make_float2(tile[threadIdx.x][k], tile[threadIdx.x][k + 1]);
     }
 }
 
 // paired slab copy, X-main: [x][row z + guard][column y + guard];
-// blockIdx.z is the row, 32 x 32 (x, y) tiles of the two source planes
+// blockIdx.z is the row, 32 x 32 (x, column) tiles of the two source planes
 // through LDS
 __global__ void pair_slab_x_kernel(const float* __restrict__ in, float2* __restrict__ out,
     int nx, int ny, int nz)
 {
     __shared__ float tile[2][32][33];
     const int r = blockIdx.z;
-    const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
+    const int x0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
     const size_t rows = size_t(nz) + 2 * kJosephGuard - 1, cols = size_t(ny) + 2 * kJosephGuard;
     for (int k = threadIdx.y; k < 32; k += 8) {
-        const int y = y0 + k, x = x0 + threadIdx.x;
+        const int y = e0 + k - kJosephGuard, x = x0 + threadIdx.x;
+        const bool in_xy = x < nx && y >= 0 && y < ny;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int z = r + h - kJosephGuard;
-            tile[h][k][threadIdx.x] = x < nx && y < ny && z >= 0 && z < nz ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
+            tile[h][k][threadIdx.x] = in_xy && z >= 0 && z < nz ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
         }
     }
     __syncthreads();
     for (int k = threadIdx.y; k < 32; k += 8) {
-        const int x = x0 + k, y = y0 + threadIdx.x;
-        if (x < nx && y < ny)
-            out[(size_t(x) * rows + r) * cols + y + kJosephGuard] = make_float2(tile[0][threadIdx.x][k], tile[1][threadIdx.x][k]);
+        const int x = x0 + k, e = e0 + threadIdx.x;
+        if (x < nx && e < int(cols))
+            out[(size_t(x) * rows + r) * cols + e] = make_float2(tile[0][threadIdx.x][k], tile[1][threadIdx.x][k]);
     }
 }
 
@@ -496,14 +503,15 @@ __global__ void pair_slab_x_kernel(const float* __restrict__ in, float2* __restr
 __global__ void pair_slab_y_kernel(const float* __restrict__ in, float2* __restrict__ out,
     int nx, int ny, int nz)
 {
-    const int x = blockIdx.x * 256 + threadIdx.x;
+    const int e = blockIdx.x * 256 + threadIdx.x;
     const int y = blockIdx.y, r = blockIdx.z;
-    if (x >= nx) return;
     const size_t rows = size_t(nz) + 2 * kJosephGuard - 1, cols = size_t(nx) + 2 * kJosephGuard;
-    const int z = r - kJosephGuard;
-    const float a = z >= 0 && z < nz ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
-    const float b = z + 1 >= 0 && z + 1 < nz ? in[(size_t(z + 1) * ny + y) * nx + x] : 0.f;
-    out[(size_t(y) * rows + r) * cols + x + kJosephGuard] = make_float2(a, b);
+    if (e >= int(cols)) return;
+    const int x = e - kJosephGuard, z = r - kJosephGuard;
+    const bool in_x = x >= 0 && x < nx;
+    const float a = in_x && z >= 0 && z < nz ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
+    const float b = in_x && z + 1 >= 0 && z + 1 < nz ? in[(size_t(z + 1) * ny + y) * nx + x] : 0.f;
+    out[(size_t(y) * rows + r) * cols + e] = make_float2(a, b);
 }
 
 // [z][y][x] -> [z][x][y]
@@ -1293,21 +1301,19 @@ size_t joseph_pair_size(int nx, int ny, int nz, bool x_main, bool slab)
 void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, bool slab,
     hipStream_t s)
 {
-    // the guard columns stay zero from the fill; every row is written
-    launch_fill(out, 0.f, joseph_pair_size(nx, ny, nz, x_main, slab), s);
     float2* o = reinterpret_cast<float2*>(out);
     const int g = 2 * kJosephGuard;
     if (!slab && x_main) {
-        dim3 block(32, 8), grid((nx + 31) / 32, (nz + 31) / 32, ny + g - 1);
+        dim3 block(32, 8), grid((nx + 31) / 32, (nz + g + 31) / 32, ny + g - 1);
         hipLaunchKernelGGL(pair_zfast_x_kernel, grid, block, 0, s, in, o, nx, ny, nz);
     } else if (!slab) {
-        dim3 block(32, 8), grid((nx + g - 1 + 31) / 32, (nz + 31) / 32, ny);
+        dim3 block(32, 8), grid((nx + g - 1 + 31) / 32, (nz + g + 31) / 32, ny);
         hipLaunchKernelGGL(pair_zfast_y_kernel, grid, block, 0, s, in, o, nx, ny, nz);
     } else if (x_main) {
-        dim3 block(32, 8), grid((nx + 31) / 32, (ny + 31) / 32, nz + g - 1);
+        dim3 block(32, 8), grid((nx + 31) / 32, (ny + g + 31) / 32, nz + g - 1);
         hipLaunchKernelGGL(pair_slab_x_kernel, grid, block, 0, s, in, o, nx, ny, nz);
     } else {
-        dim3 block(256), grid((nx + 255) / 256, ny, nz + g - 1);
+        dim3 block(256), grid((nx + g + 255) / 256, ny, nz + g - 1);
         hipLaunchKernelGGL(pair_slab_y_kernel, grid, block, 0, s, in, o, nx, ny, nz);
     }
     YK_HIP(hipGetLastError());

@@ -89,6 +89,7 @@ struct yk_projector {
     void project(int kind, const float* d_volume, float* d_proj, int first, int count, int accumulate);
     void backproject(int kind, const float* d_proj, float* d_volume, int first, int count, int accumulate);
     double dot(const float* a, const float* b, size_t n);
+    bool siddon_copies(yk_projector& w, const float* d_volume);
 
     yk_ctx* ctx;
     int nu, nv, n_views;
@@ -114,8 +115,9 @@ struct yk_projector {
     // on one stream can share them.
     yk_projector* scratch_owner = nullptr;
     yk::DeviceArray<float> d_vol_t;
-    yk::DeviceArray<float> d_vol_zx;   // Z-fastest volume copies of the separable Joseph projection
+    yk::DeviceArray<float> d_vol_zx;   // paired volume copies of the Joseph and Siddon projections
     yk::DeviceArray<float> d_vol_zy;
+    yk::DeviceArray<int> d_flag;       // one word: see siddon_value_check_kernel
     yk::DeviceArray<double> d_partials;
     yk::DeviceArray<yk::OpBpViewDev> d_opviews;  // operator-form FDK backprojection records
     std::vector<double> op_scale;      // per first view: vx vy vz / (du dv)

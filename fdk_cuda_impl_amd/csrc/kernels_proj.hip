@@ -20,6 +20,8 @@
 // off), so <A x, y> = <x, A^T y> up to summation order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "yk_internal.hpp"
 
 namespace yk {
@@ -867,64 +869,240 @@ __device__ __forceinline__ void siddon_ray_geom(const SiddonViewDev& sv, int u, 
     }
 }
 
-// Siddon projection of any view set: one lane per ray, an exact Amanatides-
-// Woo walk through the [z][y][x] volume, clipped to t in [0, 1] and to the
-// volume box.  Plane crossings are recomputed from integer indices as
-// (plane - src) * (1 / ray), the values the transposes rebuild, and the ray
-// sum adds the segments in walk order.
-__global__ void __launch_bounds__(256)
-siddon_fp_kernel(const float* __restrict__ vol, float* __restrict__ proj,
-    const SiddonViewDev* __restrict__ views, VolumeGeom g, int nu, int nv, int count, int accumulate)
+// Exact Amanatides-Woo walk of one ray through the [z][y][x] volume, clipped
+// to t in [0, 1] and to the volume box.  Plane crossings are recomputed from
+// integer indices as (plane - src) * (1 / ray), and the ray sum adds the
+// segments in walk order.
+__device__ __forceinline__ float siddon_walk(const float* __restrict__ vol, const SiddonViewDev& sv, const VolumeGeom& g,
+    int u, int v)
 {
-    // a workgroup is an 8 x 4 pixel tile of eight consecutive views: their
-    // rays nearly coincide, so the scattered voxel reads of the walk share
-    // cache lines in the CU's L1 (the walk is bound by those reads): 822 ->
-    // 389 ms at 512^3 x 720 against a 16 x 16 tile of one view; a 4 x 4 tile
-    // of sixteen views measured 409 ms
-    const int u = blockIdx.x * 8 + (threadIdx.x & 7);
-    const int v = blockIdx.y * 4 + ((threadIdx.x >> 3) & 3);
-    const int i = int(blockIdx.z) * 8 + int(threadIdx.x >> 5);
-    if (u >= nu || v >= nv || i >= count) return;
-    const SiddonViewDev sv = views[i];
     float src[3], ray[3];
     siddon_ray_geom(sv, u, v, src, ray);
     const Box b = volume_box(g);
     const int dims[3] = { g.nx, g.ny, g.nz };
     const float vox[3] = { g.vx, g.vy, g.vz };
     float t0, t1, acc = 0.f;
-    if (clip_ray(src, ray, b.lo, b.hi, t0, t1)) {
-        const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
-        int idx[3], step[3];
-        float tn[3], rcp[3];
-        bool valid[3];
-        for (int k = 0; k < 3; ++k) {
-            const float e = src[k] + t0 * ray[k];
-            idx[k] = min(dims[k] - 1, max(0, int(floorf((e - b.lo[k]) / vox[k]))));
-            step[k] = ray[k] >= 0.f ? 1 : -1;
-            valid[k] = fabsf(ray[k]) > 1e-8f;
-            rcp[k] = valid[k] ? 1.f / ray[k] : 0.f;
-            const float plane = b.lo[k] + float(idx[k] + (step[k] > 0 ? 1 : 0)) * vox[k];
-            tn[k] = valid[k] ? (plane - src[k]) * rcp[k] : 3.0e38f;
-        }
-        float t = t0;
-        const int max_steps = g.nx + g.ny + g.nz + 3;
-        for (int n = 0; n < max_steps && t < t1; ++n) {
-            const float tnext = fminf(fminf(tn[0], tn[1]), fminf(tn[2], t1));
-            acc += vol[((size_t)idx[2] * g.ny + idx[1]) * g.nx + idx[0]] * (tnext - t);
-            t = tnext;
-            int k;
-            if (tn[0] <= tn[1] && tn[0] <= tn[2]) k = 0;
-            else if (tn[1] <= tn[2]) k = 1;
-            else k = 2;
-            idx[k] += step[k];
-            if (idx[k] < 0 || idx[k] >= dims[k]) break;
-            const float plane = b.lo[k] + float(idx[k] + (step[k] > 0 ? 1 : 0)) * vox[k];
-            tn[k] = (plane - src[k]) * rcp[k];
-        }
-        acc *= len;
+    if (!clip_ray(src, ray, b.lo, b.hi, t0, t1)) return 0.f;
+    const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
+    int idx[3], step[3];
+    float tn[3], rcp[3];
+    bool valid[3];
+    for (int k = 0; k < 3; ++k) {
+        const float e = src[k] + t0 * ray[k];
+        idx[k] = min(dims[k] - 1, max(0, int(floorf((e - b.lo[k]) / vox[k]))));
+        step[k] = ray[k] >= 0.f ? 1 : -1;
+        valid[k] = fabsf(ray[k]) > 1e-8f;
+        rcp[k] = valid[k] ? 1.f / ray[k] : 0.f;
+        const float plane = b.lo[k] + float(idx[k] + (step[k] > 0 ? 1 : 0)) * vox[k];
+        tn[k] = valid[k] ? (plane - src[k]) * rcp[k] : 3.0e38f;
     }
+    float t = t0;
+    const int max_steps = g.nx + g.ny + g.nz + 3;
+    for (int n = 0; n < max_steps && t < t1; ++n) {
+        const float tnext = fminf(fminf(tn[0], tn[1]), fminf(tn[2], t1));
+        acc += vol[((size_t)idx[2] * g.ny + idx[1]) * g.nx + idx[0]] * (tnext - t);
+        t = tnext;
+        int k;
+        if (tn[0] <= tn[1] && tn[0] <= tn[2]) k = 0;
+        else if (tn[1] <= tn[2]) k = 1;
+        else k = 2;
+        idx[k] += step[k];
+        if (idx[k] < 0 || idx[k] >= dims[k]) break;
+        const float plane = b.lo[k] + float(idx[k] + (step[k] > 0 ? 1 : 0)) * vox[k];
+        tn[k] = (plane - src[k]) * rcp[k];
+    }
+    return acc * len;
+}
+
+// Siddon projection by the walk, one lane per ray.  It serves the calls whose
+// rays are too few to pay for the volume copies of siddon_fp_slab_kernel.
+__global__ void __launch_bounds__(256)
+siddon_fp_kernel(const float* __restrict__ vol, float* __restrict__ proj,
+    const SiddonViewDev* __restrict__ views, VolumeGeom g, int nu, int nv, int count, int accumulate)
+{
+    // a workgroup is an 8 x 4 pixel tile of eight consecutive views: their
+    // rays nearly coincide, so the scattered voxel reads of the walk share
+    // cache lines in the CU's L1
+    const int u = blockIdx.x * 8 + (threadIdx.x & 7);
+    const int v = blockIdx.y * 4 + ((threadIdx.x >> 3) & 3);
+    const int i = int(blockIdx.z) * 8 + int(threadIdx.x >> 5);
+    if (u >= nu || v >= nv || i >= count) return;
+    const float acc = siddon_walk(vol, views[i], g, u, v);
     float* dst = proj + ((size_t)i * nv + v) * nu + u;
     *dst = accumulate ? *dst + acc : acc;
+}
+
+// A volume whose values the slab projection's differences of taps cannot
+// carry (infinities, NaN, values near the type's ends): *flag is raised and
+// the projection walks instead, which reads only the voxels a ray crosses.
+constexpr float kSiddonLargest = 1e37f;
+__global__ void __launch_bounds__(256)
+siddon_value_check_kernel(const float* __restrict__ vol, size_t n, int* __restrict__ flag)
+{
+    bool bad = false;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
+        bad = bad || !(fabsf(vol[i]) <= kSiddonLargest);
+    if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
+}
+
+__global__ void clear_flag_kernel(int* __restrict__ flag) { *flag = 0; }
+
+// One minor axis of a ray in cell coordinates (cell j spans [j, j + 1)) over
+// the slabs of its main axis: in slab c it runs from low to low + |slope|,
+// low = slope (c - n0 / 2) + base, so at |slope| <= 1 it crosses at most one
+// plane, and the part of the slab it spends past it is
+// clamp((fract(low) + |slope| - 1) / |slope|).
+struct SiddonMinor {
+    float slope, base;  // of low
+    float inv, off;     // 1 / |slope|, (|slope| - 1) / |slope|
+};
+
+__device__ __forceinline__ SiddonMinor siddon_minor(double at_mid, double slope)
+{
+    SiddonMinor m;
+    m.slope = float(slope);
+    m.base = float(at_mid + fmin(slope, 0.0));
+    const float a = fabsf(m.slope);
+    m.inv = a > 1e-30f ? 1.f / a : 1e30f;
+    m.off = fminf(a * m.inv, 1.f) - m.inv;
+    return m;
+}
+
+// slabs in which the axis can lie inside [0, n), with a slab of margin
+__device__ __forceinline__ void siddon_slab_range(const SiddonMinor& m, float half0, int n, float& lo, float& hi)
+{
+    const float a = fabsf(m.slope);
+    if (a > 1e-12f) {
+        const float r = 1.f / m.slope;
+        const float t0 = (-a - m.base) * r + half0, t1 = (float(n) - m.base) * r + half0;
+        lo = fmaxf(lo, fminf(t0, t1) - 1.f);
+        hi = fminf(hi, fmaxf(t0, t1) + 1.f);
+    } else if (m.base < -1.f || m.base > float(n)) {
+        hi = -1.f;
+    }
+}
+
+// Siddon projection over slabs: a ray whose main axis (the largest |ray /
+// voxel| of X and Y, per ray) advances one slab at a time crosses at most one
+// plane of either minor axis inside it, so the up to three voxels it visits
+// lie in one 2 x 2 block of taps and their segments follow from two clamped
+// fractions: h1, h2 (the parts of the slab past the crossing of either axis)
+// and the part past both.  With the paired slab copies of the Joseph
+// projection a slab is one 16-byte load, where the walk took a dependent
+// 4-byte gather and ~50 instructions for each of ~1.5 voxels.
+// Bound: one 16-cycle gather and ~75 VALU cycles (on four SIMDs) a slab, both
+// about 18 cycles a wave on each CU.  256^3 x 360 views of 512 x 384, copies
+// included: 27.7 ms by the walk -> 10.5 ms here (10.8 with a tilted detector);
+// 240 x 231 x 190 x 240 views of 480 x 360, tilted: 12.4 -> 6.0 ms.
+// The ray is set up in FP64 about the middle of the volume, so positions carry
+// ~1e-5 voxel of rounding.  Rays that the slab form does not cover (steepest
+// along Z, or the source or the pixel inside the main-axis extent, where t in
+// [0, 1] can clip) walk, as do all rays of a flagged volume.
+__global__ void __launch_bounds__(512)
+siddon_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy, const float* __restrict__ vol,
+    const int* __restrict__ flag, float* __restrict__ proj, const SiddonViewDev* __restrict__ views, VolumeGeom g,
+    int nu, int nv, int count, int accumulate)
+{
+    // eight waves: one 64-ray row segment of eight consecutive views, as in
+    // joseph_fp_slab_kernel
+    const int u = blockIdx.x * 64 + threadIdx.x;
+    const int v = blockIdx.y;
+    const int i = blockIdx.z * 8 + threadIdx.y;
+    if (i >= count) return;  // whole wave
+    const bool pix = u < nu;
+    const SiddonViewDev sv = views[i];
+    double S[3], R[3], len2 = 0.0;
+    const double lo[3] = { double(g.ox) - 0.5 * double(g.vx), double(g.oy) - 0.5 * double(g.vy),
+                           double(g.oz) - 0.5 * double(g.vz) };
+    const double vox[3] = { double(g.vx), double(g.vy), double(g.vz) };
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const double r = (double(sv.detS[k]) + u * double(sv.detU[k]) + v * double(sv.detV[k])) - double(sv.src[k]);
+        len2 += r * r;
+        S[k] = (double(sv.src[k]) - lo[k]) / vox[k];
+        R[k] = r / vox[k];
+    }
+    const bool ymain = !(fabs(R[0]) >= fabs(R[1]));
+    const double r0 = ymain ? R[1] : R[0], s0 = ymain ? S[1] : S[0];
+    const double r1 = ymain ? R[0] : R[1], s1 = ymain ? S[0] : S[1];
+    const int n0 = ymain ? g.ny : g.nx, n1 = ymain ? g.nx : g.ny, n2 = g.nz;
+    const double rc = 1.0 / r0;
+    const double ta = -s0 * rc, tb = (double(n0) - s0) * rc;
+    const bool slabs = fabs(R[2]) <= fabs(r0) && fmin(ta, tb) >= 0.0 && fmax(ta, tb) <= 1.0 && *flag == 0;
+    const double mid = 0.5 * double(n0) - s0;
+    const SiddonMinor m1 = siddon_minor(s1 + mid * (r1 * rc), r1 * rc);
+    const SiddonMinor m2 = siddon_minor(S[2] + mid * (R[2] * rc), R[2] * rc);
+    const float len = float(sqrt(len2) * fabs(rc));
+    const float half0 = 0.5f * float(n0);
+    float flo = 0.f, fhi = float(n0 - 1);
+    siddon_slab_range(m1, half0, n1, flo, fhi);
+    siddon_slab_range(m2, half0, n2, flo, fhi);
+    const bool live = pix && slabs && flo <= fhi;
+    const int clo = live ? int(flo) : 0x7fffffff, chi = live ? int(fhi) : -1;
+    // past both crossings: the slopes agree in sign -> min(h1, h2), else
+    // h1 - min(h1, 1 - h2): with y = sa h2 + sb and m = min(h1, y), sa m + sb h1
+    const bool agree = (m1.slope < 0.f) == (m2.slope < 0.f);
+    const float sa = agree ? 1.f : -1.f, sb = agree ? 0.f : 1.f;
+    float acc = 0.f;
+    // waves near a diagonal hold rays of both main axes: one pass for each
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+        const bool mine = live && ymain == (pass == 1);
+        if (!__any(mine)) continue;
+        int wlo = mine ? clo : 0x7fffffff, whi = mine ? chi : -1;
+        for (int off = 32; off > 0; off >>= 1) {
+            wlo = min(wlo, __shfl_xor(wlo, off, 64));
+            whi = max(whi, __shfl_xor(whi, off, 64));
+        }
+        wlo = __builtin_amdgcn_readfirstlane(wlo);
+        whi = __builtin_amdgcn_readfirstlane(whi);
+        if (!mine) continue;
+        const int p1 = (pass ? g.nx : g.ny) + 2 * kJosephGuard;
+        const size_t slab_bytes = size_t(n2 + 2 * kJosephGuard - 1) * size_t(p1) * 8u;
+        const float top1 = float(pass ? g.nx : g.ny), top2 = float(n2);
+        const char* sl = reinterpret_cast<const char*>(pass ? gy : gx) + size_t(wlo) * slab_bytes;
+        float c = float(wlo) - half0;  // exact half-integers
+        auto taps = [&](float& h1, float& h2) {
+            const float f1 = fmaf(m1.slope, c, m1.base), f2 = fmaf(m2.slope, c, m2.base);
+            c += 1.f;
+            const float g1 = floorf(f1), g2 = floorf(f2);
+            h1 = __builtin_amdgcn_fmed3f(fmaf(f1 - g1, m1.inv, m1.off), 0.f, 1.f);
+            h2 = __builtin_amdgcn_fmed3f(fmaf(f2 - g2, m2.inv, m2.off), 0.f, 1.f);
+            // outside [-1, n] both taps of an axis are guards
+            const int j1 = int(__builtin_amdgcn_fmed3f(g1, -2.f, top1)) + kJosephGuard;
+            const int j2 = int(__builtin_amdgcn_fmed3f(g2, -2.f, top2)) + kJosephGuard;
+            const float4u q = *reinterpret_cast<const float4u*>(sl + unsigned(__mul24(j2, p1) + j1) * 8u);
+            sl += slab_bytes;
+            return q;
+        };
+        auto sum = [&](const float4u& q, float h1, float h2) {
+            const float m = fminf(h1, fmaf(sa, h2, sb));
+            const float w = fmaf(sa, m, sb * h1);
+            // q: (j2, j1), (j2 + 1, j1), (j2, j1 + 1), (j2 + 1, j1 + 1)
+            const float d2 = q.y - q.x, d1 = q.z - q.x;
+            const float both = (q.w - q.y) - d1;
+            acc += fmaf(w, both, fmaf(h2, d2, fmaf(h1, d1, q.x)));
+        };
+        int s = wlo;
+        constexpr int kUnroll = 4;
+        for (; s + kUnroll - 1 <= whi; s += kUnroll) {
+            float4u q[kUnroll];
+            float h1[kUnroll], h2[kUnroll];
+#pragma unroll
+            for (int k = 0; k < kUnroll; ++k) q[k] = taps(h1[k], h2[k]);
+#pragma unroll
+            for (int k = 0; k < kUnroll; ++k) sum(q[k], h1[k], h2[k]);
+        }
+        for (; s <= whi; ++s) {
+            float h1, h2;
+            const float4u q = taps(h1, h2);
+            sum(q, h1, h2);
+        }
+    }
+    if (!pix) return;
+    const float out = slabs ? acc * len : siddon_walk(vol, sv, g, u, v);
+    float* dst = proj + ((size_t)i * nv + v) * nu + u;
+    *dst = accumulate ? *dst + out : out;
 }
 
 // t-interval of the walk inside cell c of one axis: the forward walk's own
@@ -1361,6 +1539,18 @@ void launch_siddon_fp(const SiddonLaunch& p, hipStream_t s)
     dim3 block(256), grid((p.nu + 7) / 8, (p.nv + 3) / 4, (p.count + 7) / 8);
     hipLaunchKernelGGL(siddon_fp_kernel, grid, block, 0, s, p.volume, p.proj, p.views, p.vol, p.nu,
         p.nv, p.count, p.accumulate);
+    YK_HIP(hipGetLastError());
+}
+
+void launch_siddon_fp_slab(const SiddonSlabFpLaunch& p, hipStream_t s)
+{
+    const size_t n = size_t(p.vol.nx) * p.vol.ny * p.vol.nz;
+    hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(1), 0, s, p.flag);
+    hipLaunchKernelGGL(siddon_value_check_kernel, dim3(unsigned(std::min<size_t>(4096, (n + 255) / 256))), dim3(256), 0, s,
+        p.volume, n, p.flag);
+    dim3 block(64, 8), grid((p.nu + 63) / 64, p.nv, (p.count + 7) / 8);
+    hipLaunchKernelGGL(siddon_fp_slab_kernel, grid, block, 0, s, p.vol_x, p.vol_y, p.volume, p.flag, p.proj, p.views,
+        p.vol, p.nu, p.nv, p.count, p.accumulate);
     YK_HIP(hipGetLastError());
 }
 

@@ -19,6 +19,14 @@ void grow(DeviceArray<T>& a, size_t n)
     if (a.size() < n) a.resize(n);
 }
 
+// rays x main-axis slabs per voxel from which the Siddon projection makes its
+// volume copies: at 3 (one view of 512 x 384 at 256^3) the copies and the slab
+// kernel take 223 us against the walk's 316, at 6 304 against 429, at 24 411
+// against 999; one view at 128^3 48 against 90, at 64^3 28 against 39.  Below
+// 1 the copies are most of the work and the walk reads only what its few rays
+// cross.
+constexpr double kSiddonSlabRatio = 1.0;
+
 }  // namespace
 
 yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
@@ -112,6 +120,33 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
     YK_HIP(hipStreamSynchronize(s));
 }
 
+// both paired slab copies of the volume into w's scratch; false when the walk,
+// which needs none, has to serve the call: the copies do not fit in memory, a
+// stream capture allows no allocation, or the slab kernel's grid or 32-bit
+// slab offsets cannot hold the sizes
+bool yk_projector::siddon_copies(yk_projector& w, const float* d_volume)
+{
+    const size_t need_x = joseph_pair_size(grid.nx, grid.ny, grid.nz, true, true);
+    const size_t need_y = joseph_pair_size(grid.nx, grid.ny, grid.nz, false, true);
+    if (nv > 65535 || need_x / grid.nx > (size_t(1) << 29) || need_y / grid.ny > (size_t(1) << 29)) return false;
+    if (w.d_vol_zx.size() < need_x || w.d_vol_zy.size() < need_y || !w.d_flag.get()) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) return false;
+    }
+    try {
+        grow(w.d_vol_zx, need_x);
+        grow(w.d_vol_zy, need_y);
+        grow(w.d_flag, 1);
+    } catch (const Error&) {
+        (void)hipGetLastError();  // the failed allocation's, not the call's
+        return false;
+    }
+    launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, true, ctx->stream);
+    launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, true, ctx->stream);
+    return true;
+}
+
 void yk_projector::project(int kind, const float* d_volume, float* d_proj, int first, int count,
     int accumulate)
 {
@@ -184,10 +219,24 @@ void yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
         p.accumulate = accumulate;
         launch_joseph_fp(p, s);
     } else if (kind == YK_FP_SIDDON) {
-        // every view set walks the [z][y][x] volume with siddon_fp_kernel:
-        // its view-grouped tiles measured faster than the separable
-        // wave-per-column walk over a Z-fastest copy on untilted scans too
-        // (27.5 against 33.3 ms at 256^3 x 360), with bit-identical results
+        // The slab kernel reads paired copies of the volume along both axes,
+        // made on each call, so it takes the calls whose rays' slabs outnumber
+        // the voxels kSiddonSlabRatio times; the walk the others.
+        const double slabs = double(count) * nu * nv * std::max(grid.nx, grid.ny);
+        if (slabs >= kSiddonSlabRatio * double(grid.nx) * grid.ny * grid.nz && siddon_copies(w, d_volume)) {
+            SiddonSlabFpLaunch p{};
+            p.volume = d_volume;
+            p.vol_x = w.d_vol_zx.get();
+            p.vol_y = w.d_vol_zy.get();
+            p.flag = w.d_flag.get();
+            p.proj = d_proj;
+            p.views = d_sviews.get() + first;
+            p.vol = vol;
+            p.nu = nu; p.nv = nv; p.count = count;
+            p.accumulate = accumulate;
+            launch_siddon_fp_slab(p, s);
+            return;
+        }
         SiddonLaunch p{};
         p.volume = d_volume;
         p.proj = d_proj;

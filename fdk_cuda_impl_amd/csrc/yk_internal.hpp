@@ -354,6 +354,22 @@ struct SiddonLaunch {
 };
 void launch_siddon_fp(const SiddonLaunch& p, hipStream_t s);
 
+// Siddon projection over the paired slab copies of the volume (made by
+// launch_joseph_pair_copy with slab); both copies are needed: the main axis is
+// chosen per ray
+struct SiddonSlabFpLaunch {
+    const float* volume;        // [z][y][x]
+    const float* vol_x;         // paired slab copy, X-main
+    const float* vol_y;         // paired slab copy, Y-main
+    int* flag;                  // scratch word: the volume holds values only the walk can carry
+    float* proj;                // [count][nv][nu]
+    const SiddonViewDev* views; // device, `count`
+    VolumeGeom vol;
+    int nu, nv, count;
+    int accumulate;
+};
+void launch_siddon_fp_slab(const SiddonSlabFpLaunch& p, hipStream_t s);
+
 struct SiddonAdjointLaunch {
     const float* proj;
     float* volume;

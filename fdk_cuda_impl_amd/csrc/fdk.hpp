@@ -90,6 +90,8 @@ struct yk_projector {
     void backproject(int kind, const float* d_proj, float* d_volume, int first, int count, int accumulate);
     double dot(const float* a, const float* b, size_t n);
     bool siddon_copies(yk_projector& w, const float* d_volume);
+    bool gather_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
+        int accumulate);
 
     yk_ctx* ctx;
     int nu, nv, n_views;
@@ -104,12 +106,6 @@ struct yk_projector {
     yk::DeviceArray<float4> d_ray_ab;  // Joseph transpose ray table, one view chunk
     yk::DeviceArray<float> d_ray_len;
     std::vector<char> separable;       // per view: main axis X/Y and detV along Z only
-    yk::DeviceArray<float2> d_sep_ab1; // separable Joseph transpose ray table, one view chunk
-    yk::DeviceArray<float2> d_sep_ab2;
-    yk::DeviceArray<float> d_sep_pl;
-    std::vector<char> siddon_separable;  // per view: detV along Z only
-    yk::DeviceArray<float2> d_sid_col;   // separable Siddon transpose ray table, one view chunk
-    yk::DeviceArray<float2> d_sid_ray;
     // projector whose scratch arrays (volume copies, ray tables) this one uses;
     // null: its own.  Operators of one volume grid that run one after another
     // on one stream can share them.
@@ -117,6 +113,9 @@ struct yk_projector {
     yk::DeviceArray<float> d_vol_t;
     yk::DeviceArray<float> d_vol_zx;   // paired volume copies of the Joseph and Siddon projections
     yk::DeviceArray<float> d_vol_zy;
+    std::vector<char> joseph_gather, siddon_gather;  // per view: the gather transposes cover it
+    yk::DeviceArray<yk::GatherViewDev> d_gather;
+    yk::DeviceArray<float> d_gather_q; // ray values of the gather transposes, one view chunk
     yk::DeviceArray<int> d_flag;       // one word: see siddon_value_check_kernel
     yk::DeviceArray<double> d_partials;
     yk::DeviceArray<yk::OpBpViewDev> d_opviews;  // operator-form FDK backprojection records

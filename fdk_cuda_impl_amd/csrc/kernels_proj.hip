@@ -22,71 +22,11 @@
 
 #include <algorithm>
 
+#include "ray_geometry.hpp"
 #include "yk_internal.hpp"
 
 namespace yk {
 namespace {
-
-struct AxisInfo {
-    int p0, p1, p2;     // component index of c0, c1, c2
-    int n0, n1, n2;
-    float v0, v1, v2;
-};
-
-__device__ __forceinline__ AxisInfo axis_info(int axis, const VolumeGeom& g)
-{
-    AxisInfo a;
-    if (axis == 0) { a.p0 = 0; a.p1 = 1; a.p2 = 2; a.n0 = g.nx; a.n1 = g.ny; a.n2 = g.nz; a.v0 = g.vx; a.v1 = g.vy; a.v2 = g.vz; }
-    else if (axis == 1) { a.p0 = 1; a.p1 = 0; a.p2 = 2; a.n0 = g.ny; a.n1 = g.nx; a.n2 = g.nz; a.v0 = g.vy; a.v1 = g.vx; a.v2 = g.vz; }
-    else { a.p0 = 2; a.p1 = 0; a.p2 = 1; a.n0 = g.nz; a.n1 = g.nx; a.n2 = g.ny; a.v0 = g.vz; a.v1 = g.vx; a.v2 = g.vy; }
-    return a;
-}
-
-template <typename T>
-__device__ __forceinline__ T pick(int k, T a, T b, T c) { return k == 0 ? a : (k == 1 ? b : c); }
-
-struct JRay {
-    float a1, b1, a2, b2, L;
-};
-
-// Per-ray Joseph line in volume-centred voxel units.  Shared by the forward
-// kernel and the transpose's ray table, with contraction disabled so both
-// evaluate the same IEEE operations and obtain bit-identical parameters.
-__device__ __forceinline__ bool joseph_ray(const ProjViewDev& pv, const AxisInfo& ax,
-    int u, int v, JRay& r)
-{
-#pragma clang fp contract(off)
-    const float dx = (pv.detS[0] + float(u) * pv.detU[0]) + float(v) * pv.detV[0];
-    const float dy = (pv.detS[1] + float(u) * pv.detU[1]) + float(v) * pv.detV[1];
-    const float dz = (pv.detS[2] + float(u) * pv.detU[2]) + float(v) * pv.detV[2];
-    const float sx = pv.src[0], sy = pv.src[1], sz = pv.src[2];
-    const float s0 = pick(ax.p0, sx, sy, sz), s1 = pick(ax.p1, sx, sy, sz), s2 = pick(ax.p2, sx, sy, sz);
-    const float d0 = pick(ax.p0, dx, dy, dz), d1 = pick(ax.p1, dx, dy, dz), d2 = pick(ax.p2, dx, dy, dz);
-    const float den = s0 - d0;
-    if (den == 0.f) return false;
-    r.a1 = (s1 - d1) / den;
-    r.a2 = (s2 - d2) / den;
-    r.b1 = s1 - r.a1 * s0;
-    r.b2 = s2 - r.a2 * s0;
-    const float t1 = r.a1 * ax.v1, t2 = r.a2 * ax.v2;
-    r.L = sqrtf(ax.v0 * ax.v0 + t1 * t1 + t2 * t2);
-    return true;
-}
-
-// centred main-axis coordinate of slice s
-__device__ __forceinline__ float joseph_c0(int s, int n0)
-{
-#pragma clang fp contract(off)
-    return float(s) - 0.5f * float(n0 - 1);
-}
-
-// one minor-axis sample position (index space, texel k at k) of the line
-// c = a c0 + b
-__device__ __forceinline__ float joseph_minor(float a, float b, float c0, int n)
-{
-#pragma clang fp contract(off)
-    return (a * c0 + b) + 0.5f * float(n - 1);
-}
 
 // minor-axis sample position of slice s
 __device__ __forceinline__ void joseph_sample(const JRay& r, const AxisInfo& ax, int s, float& f1, float& f2)
@@ -640,186 +580,6 @@ joseph_adjoint_kernel(const float* __restrict__ proj, float* __restrict__ volume
 }
 
 // ---------------------------------------------------------------------------
-// Joseph transpose for separable views: main axis X or Y and detector columns
-// parallel to Z (detV has no component on the main or first minor axis, as
-// for an untilted circular scan).  Then d0 and d1 of a ray do not depend on v,
-// so a1, b1 - and the first-minor sample f1 of every slice - are those of the
-// whole detector column u, while f2 is affine in v.
-// ---------------------------------------------------------------------------
-
-// Column-major ray table of the separable transpose: ab1[view][u] = (a1, b1)
-// of column u; ab2[view][u][v] = (a2, b2) and pl[view][u][v] = p * L of ray
-// (u, v) (0 for a ray the forward projector skips), each column padded to
-// nvp = nv + kSepPad entries with zeros.  Same joseph_ray as the
-// forward kernel; the 32 x 32 tile is transposed through LDS so both the
-// projection reads and the table writes are contiguous.
-__global__ void __launch_bounds__(256)
-joseph_sep_table_kernel(const float* __restrict__ proj, const ProjViewDev* __restrict__ views,
-    VolumeGeom g, int nu, int nv, int nvp, float2* __restrict__ ab1, float2* __restrict__ ab2,
-    float* __restrict__ pl)
-{
-    __shared__ float2 s_ab[32][33];
-    __shared__ float s_pl[32][33];
-    const int i = blockIdx.z;
-    const int u0 = blockIdx.x * 32, v0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    const ProjViewDev pv = views[i];
-    const AxisInfo ax = axis_info(pv.axis, g);
-    const float* pi = proj + (size_t)i * nu * nv;
-    for (int k = ty; k < 32; k += 8) {
-        const int u = u0 + tx, v = v0 + k;
-        float2 ab = make_float2(0.f, 0.f);
-        float w = 0.f;
-        if (u < nu && v < nv) {
-            JRay r;
-            const bool ok = joseph_ray(pv, ax, u, v, r);
-            if (ok) {
-                ab = make_float2(r.a2, r.b2);
-                w = pi[(size_t)v * nu + u] * r.L;
-            }
-            if (v == 0) ab1[(size_t)i * nu + u] = ok ? make_float2(r.a1, r.b1) : make_float2(0.f, 0.f);
-        }
-        s_ab[k][tx] = ab;
-        s_pl[k][tx] = w;
-    }
-    __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-        const int u = u0 + k, v = v0 + tx;
-        if (u < nu && v < nvp) {
-            const size_t o = ((size_t)i * nu + u) * nvp + v;
-            ab2[o] = s_ab[tx][k];
-            pl[o] = s_pl[tx][k];
-        }
-    }
-}
-
-// world projective map (u or v numerator row r, denominator row d) of a point
-__device__ __forceinline__ float proj_coord(const float* c, int row, float x, float y, float z, float rd)
-{
-    return (c[row] * x + c[row + 1] * y + c[row + 2] * z + c[row + 3]) * rd;
-}
-
-// One lane per (x, y) column of kSepZ voxels, 16 x 16 columns per workgroup.
-// Per view the column sits on one main-axis slice s and one first-minor index
-// i1, so its candidate rays are whole detector columns u with
-// floor(f1(u)) in {i1 - 1, i1}, and in each such column the rays whose f2
-// lies in [z0 - 1, z0 + kSepZ).  Those are walked in v order; every ray adds
-// p L wa (1 - w2) and p L wa w2 to the two voxels its sample straddles.  The
-// sums live in LDS slots private to the lane (slot-major, lane-minor: no
-// bank conflicts, no sharing: plain read-modify-write, no atomics), so the
-// order of additions per voxel is fixed and the result deterministic.  Candidate ranges come from the FP32
-// projective map with 0.05 px of margin; membership is decided only by the
-// forward kernel's own f1, f2.
-constexpr int kSepZ = 32;
-constexpr int kSepU = kSepPad;  // rays of a column loaded before any is consumed
-
-__global__ void __launch_bounds__(256)
-joseph_adjoint_sep_kernel(const float2* __restrict__ ab1, const float2* __restrict__ ab2,
-    const float* __restrict__ pl, const ProjViewDev* __restrict__ views, const float* __restrict__ c32,
-    VolumeGeom g, int nu, int nv, int nvp, int count, int accumulate, float* __restrict__ volume)
-{
-    __shared__ float slot[(kSepZ + 2) * 256];
-    const int lane = threadIdx.x;
-    const int x = blockIdx.x * 16 + (lane & 15);
-    const int y = blockIdx.y * 16 + (lane >> 4);
-    const int z0 = blockIdx.z * kSepZ;
-#pragma unroll
-    for (int k = 0; k < kSepZ + 2; ++k) slot[k * 256 + lane] = 0.f;
-    if (x >= g.nx || y >= g.ny) return;
-    const float margin = 0.05f;
-    const float zlo = g.oz + float(z0 - 1) * g.vz;
-    const float zhi = g.oz + float(z0 + kSepZ) * g.vz;
-    const float zmid = g.oz + (float(z0) + 0.5f * float(kSepZ - 1)) * g.vz;
-    for (int i = 0; i < count; ++i) {
-        const ProjViewDev pv = views[i];
-        const AxisInfo ax = axis_info(pv.axis, g);
-        const bool xmain = pv.axis == 0;
-        const int s = xmain ? x : y, i1 = xmain ? y : x;
-        const float c0 = joseph_c0(s, ax.n0);
-        const float* c = c32 + (size_t)i * 12;
-        const float m0 = (xmain ? g.ox : g.oy) + float(s) * ax.v0;
-        const float o1 = xmain ? g.oy : g.ox;
-        // detector columns whose rays cross slice s within (i1 - 1, i1 + 1)
-        float ua, ub;
-        {
-            const float ma = o1 + float(i1 - 1) * ax.v1, mb = o1 + float(i1 + 1) * ax.v1;
-            const float xa = xmain ? m0 : ma, ya = xmain ? ma : m0;
-            const float xb = xmain ? m0 : mb, yb = xmain ? mb : m0;
-            const float da = c[8] * xa + c[9] * ya + c[10] * zmid + c[11];
-            const float db = c[8] * xb + c[9] * yb + c[10] * zmid + c[11];
-            if (!(da > 1e-6f) || !(db > 1e-6f)) continue;
-            ua = proj_coord(c, 0, xa, ya, zmid, 1.f / da);
-            ub = proj_coord(c, 0, xb, yb, zmid, 1.f / db);
-        }
-        const int ulo = max(0, int(ceilf(fminf(ua, ub) - margin)));
-        const int uhi = min(nu - 1, int(floorf(fmaxf(ua, ub) + margin)));
-        for (int u = ulo; u <= uhi; ++u) {
-            const float2 q1 = ab1[(size_t)i * nu + u];
-            const float f1 = joseph_minor(q1.x, q1.y, c0, ax.n1);
-            const float g1 = floorf(f1);
-            if (g1 < -1.f || g1 > float(ax.n1 - 1)) continue;
-            const int j1 = int(g1);
-            const float w1 = f1 - g1;
-            float wa;
-            if (j1 == i1) wa = 1.f - w1;
-            else if (j1 + 1 == i1) wa = w1;
-            else continue;
-            // rays of column u whose f2 falls in [z0 - 1, z0 + kSepZ)
-            const float m1 = o1 + f1 * ax.v1;
-            const float xc = xmain ? m0 : m1, yc = xmain ? m1 : m0;
-            const float dl = c[8] * xc + c[9] * yc + c[10] * zlo + c[11];
-            const float dh = c[8] * xc + c[9] * yc + c[10] * zhi + c[11];
-            if (!(dl > 1e-6f) || !(dh > 1e-6f)) continue;
-            const float va = proj_coord(c, 4, xc, yc, zlo, 1.f / dl);
-            const float vb = proj_coord(c, 4, xc, yc, zhi, 1.f / dh);
-            const int vlo = max(0, int(ceilf(fminf(va, vb) - margin)));
-            const int vhi = min(nv - 1, int(floorf(fmaxf(va, vb) + margin)));
-            // kSepU rays per step, loads first; the column carries kSepU
-            // zero-weight pad entries, so a step may run past vhi (rays
-            // beyond the candidate range fall outside the slots by f2)
-            const float2* q2 = ab2 + ((size_t)i * nu + u) * nvp + vlo;
-            const float* w = pl + ((size_t)i * nu + u) * nvp + vlo;
-            const int nr = vhi - vlo + 1;
-            for (int r0 = 0; r0 < nr; r0 += kSepU) {
-                float2 q[kSepU];
-                float pw[kSepU];
-#pragma unroll
-                for (int j = 0; j < kSepU; ++j) {
-                    q[j] = q2[r0 + j];
-                    pw[j] = w[r0 + j];
-                }
-#pragma unroll
-                for (int j = 0; j < kSepU; ++j) {
-                    const float f2 = joseph_minor(q[j].x, q[j].y, c0, ax.n2);
-                    const float g2 = floorf(f2);
-                    // slot of voxel floor(f2): 0 .. kSepZ covers f2 in
-                    // [z0 - 1, z0 + kSepZ); slots of voxels outside the
-                    // volume are never stored, which stands in for the
-                    // forward kernel's g2 range test
-                    const int k = int(g2) - (z0 - 1);
-                    const bool live = unsigned(k) <= unsigned(kSepZ);
-                    const float w2 = f2 - g2;
-                    const float cw = live ? pw[j] * wa : 0.f;
-                    float* sk = slot + ((live ? k : 0) * 256 + lane);
-                    sk[0] += cw * (1.f - w2);
-                    sk[256] += cw * w2;
-                }
-            }
-        }
-    }
-    const size_t plane = (size_t)g.nx * g.ny;
-    const size_t colx = (size_t)y * g.nx + x;
-#pragma unroll
-    for (int k = 1; k <= kSepZ; ++k) {
-        const int z = z0 + k - 1;
-        if (z >= g.nz) break;
-        const float val = slot[k * 256 + lane];
-        float* dst = volume + z * plane + colx;
-        *dst = accumulate ? *dst + val : val;
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Siddon
 // ---------------------------------------------------------------------------
 struct Box {
@@ -858,15 +618,6 @@ __device__ __forceinline__ bool clip_ray(const float* src, const float* ray, con
     for (int k = 0; k < 3; ++k)
         if (!slab_clip(src[k], ray[k], lo[k], hi[k], t0, t1)) return false;
     return t0 < t1;
-}
-
-__device__ __forceinline__ void siddon_ray_geom(const SiddonViewDev& sv, int u, int v, float* src, float* ray)
-{
-#pragma clang fp contract(off)
-    for (int k = 0; k < 3; ++k) {
-        src[k] = sv.src[k];
-        ray[k] = (sv.detS[k] + float(u) * sv.detU[k] + float(v) * sv.detV[k]) - sv.src[k];
-    }
 }
 
 // Exact Amanatides-Woo walk of one ray through the [z][y][x] volume, clipped
@@ -1121,6 +872,12 @@ __device__ __forceinline__ void cell_interval(float s, float r, float lo, float 
     }
 }
 
+// world projective map (u or v numerator row r, denominator row d) of a point
+__device__ __forceinline__ float proj_coord(const float* c, int row, float x, float y, float z, float rd)
+{
+    return (c[row] * x + c[row + 1] * y + c[row + 2] * z + c[row + 3]) * rd;
+}
+
 // Siddon transpose: one thread per voxel; for each view the candidate rays
 // are the pixels inside the projection of the voxel cube, and each candidate
 // contributes y * |segment inside the cube, clipped like the forward walk|.
@@ -1196,158 +953,6 @@ siddon_adjoint_kernel(const float* __restrict__ proj, float* __restrict__ volume
     }
     float* dst = volume + ((size_t)z * g.ny + y) * g.nx + x;
     *dst = accumulate ? *dst + acc : acc;
-}
-
-// ---------------------------------------------------------------------------
-// Siddon transpose for separable views (detV along Z only).  The rays of a
-// detector column u share ray_x and ray_y (independent of v), hence their XY
-// path: the t-interval of an (x, y) cell and the XY part of the volume clip
-// are column constants, and each ray only resolves the Z voxels it crosses
-// inside that interval.  Lane / slot layout of the separable Joseph transpose,
-// with kSidSepZ slices per lane column.
-// ---------------------------------------------------------------------------
-
-// col_xy[view][u] = (ray_x, ray_y) of column u; ray_wz[view][u][v] =
-// (p L, ray_z) of ray (u, v), L = |ray|, each column padded to nvp entries of
-// zeros (p L = 0 marks a ray that adds nothing)
-__global__ void __launch_bounds__(256)
-siddon_sep_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __restrict__ views,
-    int nu, int nv, int nvp, float2* __restrict__ col_xy, float2* __restrict__ ray_wz)
-{
-    __shared__ float2 s_t[32][33];
-    const int i = blockIdx.z;
-    const int u0 = blockIdx.x * 32, v0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    const SiddonViewDev sv = views[i];
-    const float* pi = proj + (size_t)i * nu * nv;
-    for (int k = ty; k < 32; k += 8) {
-        const int u = u0 + tx, v = v0 + k;
-        float2 e = make_float2(0.f, 0.f);
-        if (u < nu && v < nv) {
-            float src[3], ray[3];
-            siddon_ray_geom(sv, u, v, src, ray);
-            const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
-            e = make_float2(pi[(size_t)v * nu + u] * len, ray[2]);
-            if (v == 0) col_xy[(size_t)i * nu + u] = make_float2(ray[0], ray[1]);
-        }
-        s_t[k][tx] = e;
-    }
-    __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-        const int u = u0 + k, v = v0 + tx;
-        if (u < nu && v < nvp) ray_wz[((size_t)i * nu + u) * nvp + v] = s_t[tx][k];
-    }
-}
-
-// z-slices per lane column of the Siddon transpose: 16 (18 LDS slots a lane,
-// 8 workgroups per CU) measured 18 % faster than 32 at 256^3 x 360; the
-// Joseph transpose keeps kSepZ = 32, where 16 measured 12 % slower
-constexpr int kSidSepZ = 16;
-
-__global__ void __launch_bounds__(256)
-siddon_adjoint_sep_kernel(const float2* __restrict__ col_xy, const float2* __restrict__ ray_wz,
-    const SiddonViewDev* __restrict__ views, const float* __restrict__ c32, VolumeGeom g, int nu, int nv,
-    int nvp, int count, int accumulate, float* __restrict__ volume)
-{
-    __shared__ float slot[(kSidSepZ + 2) * 256];
-    const int lane = threadIdx.x;
-    const int x = blockIdx.x * 16 + (lane & 15);
-    const int y = blockIdx.y * 16 + (lane >> 4);
-    const int z0 = blockIdx.z * kSidSepZ;
-#pragma unroll
-    for (int k = 0; k < kSidSepZ + 2; ++k) slot[k * 256 + lane] = 0.f;
-    if (x >= g.nx || y >= g.ny) return;
-    const Box b = volume_box(g);
-    const float margin = 0.05f;
-    const int zend = min(z0 + kSidSepZ, g.nz);  // one past the block's last slice
-    const float xl = b.lo[0] + float(x) * g.vx, xh = b.lo[0] + float(x + 1) * g.vx;
-    const float yl = b.lo[1] + float(y) * g.vy, yh = b.lo[1] + float(y + 1) * g.vy;
-    const float zl = b.lo[2] + float(z0) * g.vz, zh = b.lo[2] + float(zend) * g.vz;
-    const float inv_vz = 1.f / g.vz;
-    // only a block holding the volume's first or last slice can see the Z
-    // faces of the volume clip bind inside its voxels
-    const bool zface = z0 == 0 || zend == g.nz;
-    for (int i = 0; i < count; ++i) {
-        const float* c = c32 + (size_t)i * 12;
-        // detector range of the cell x block (8 corners, FP32 map, margin)
-        float umin = 3.0e38f, umax = -3.0e38f, vmin = 3.0e38f, vmax = -3.0e38f;
-        bool ok = true;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float X = (k & 1) ? xh : xl, Y = (k & 2) ? yh : yl, Z = (k & 4) ? zh : zl;
-            const float den = c[8] * X + c[9] * Y + c[10] * Z + c[11];
-            ok = ok && den > 1e-6f;
-            const float rd = 1.f / den;
-            const float uu = proj_coord(c, 0, X, Y, Z, rd), vv = proj_coord(c, 4, X, Y, Z, rd);
-            umin = fminf(umin, uu); umax = fmaxf(umax, uu);
-            vmin = fminf(vmin, vv); vmax = fmaxf(vmax, vv);
-        }
-        if (!ok) continue;
-        const int ulo = max(0, int(ceilf(umin - margin)));
-        const int uhi = min(nu - 1, int(floorf(umax + margin)));
-        const int vlo = max(0, int(ceilf(vmin - margin)));
-        const int vhi = min(nv - 1, int(floorf(vmax + margin)));
-        const SiddonViewDev sv = views[i];
-        const float sx = sv.src[0], sy = sv.src[1], sz = sv.src[2];
-        for (int u = ulo; u <= uhi; ++u) {
-            const float2 r = col_xy[(size_t)i * nu + u];
-            // XY part of the volume clip and of the cell, shared by the column
-            float a0 = 0.f, e0 = 1.f;
-            if (!slab_clip(sx, r.x, b.lo[0], b.hi[0], a0, e0)) continue;
-            if (!slab_clip(sy, r.y, b.lo[1], b.hi[1], a0, e0)) continue;
-            float ca = -3.0e38f, cb = 3.0e38f;
-            cell_interval(sx, r.x, b.lo[0], g.vx, x, g.nx, ca, cb);
-            cell_interval(sy, r.y, b.lo[1], g.vy, y, g.ny, ca, cb);
-            a0 = fmaxf(a0, ca);
-            e0 = fminf(e0, cb);
-            if (!(e0 > a0)) continue;
-            const float2* q = ray_wz + ((size_t)i * nu + u) * nvp + vlo;
-            const int nr = vhi - vlo + 1;
-            for (int r0 = 0; r0 < nr; r0 += kSepU) {
-                float2 e[kSepU];
-#pragma unroll
-                for (int j = 0; j < kSepU; ++j) e[j] = q[r0 + j];
-#pragma unroll
-                for (int j = 0; j < kSepU; ++j) {
-                    const float pw = e[j].x, rz = e[j].y;
-                    float a = a0, t1 = e0;
-                    bool live = pw != 0.f;
-                    if (zface) live = live && slab_clip(sz, rz, b.lo[2], b.hi[2], a, t1);
-                    live = live && t1 > a;
-                    if (!live) continue;
-                    // Z voxels of the block the ray crosses inside [a, t1]
-                    const bool zvalid = fabsf(rz) > 1e-8f;
-                    const float rc = zvalid ? 1.f / rz : 0.f;
-                    const float za = sz + a * rz, zb = sz + t1 * rz;
-                    int ka = int(floorf((fminf(za, zb) - b.lo[2]) * inv_vz));
-                    int kb = int(floorf((fmaxf(za, zb) - b.lo[2]) * inv_vz));
-                    ka = max(ka, z0);
-                    kb = min(kb, zend - 1);
-                    for (int k = ka; k <= kb; ++k) {
-                        float lo = a, hi = t1;
-                        if (zvalid) {
-                            const float tl = (b.lo[2] + float(k) * g.vz - sz) * rc;
-                            const float th = (b.lo[2] + float(k + 1) * g.vz - sz) * rc;
-                            lo = fmaxf(lo, fminf(tl, th));
-                            hi = fminf(hi, fmaxf(tl, th));
-                        }
-                        const float seg = hi - lo;
-                        if (seg > 0.f) slot[(k - z0 + 1) * 256 + lane] += pw * seg;
-                    }
-                }
-            }
-        }
-    }
-    const size_t plane = (size_t)g.nx * g.ny;
-    const size_t colx = (size_t)y * g.nx + x;
-#pragma unroll
-    for (int k = 1; k <= kSidSepZ; ++k) {
-        const int z = z0 + k - 1;
-        if (z >= g.nz) break;
-        const float val = slot[k * 256 + lane];
-        float* dst = volume + z * plane + colx;
-        *dst = accumulate ? *dst + val : val;
-    }
 }
 
 // Operator-form FDK backprojections, the iterative B of the reference's
@@ -1522,18 +1127,6 @@ void launch_joseph_adjoint(const JosephAdjointLaunch& p, hipStream_t s)
     YK_HIP(hipGetLastError());
 }
 
-void launch_joseph_adjoint_sep(const JosephSepLaunch& p, hipStream_t s)
-{
-    const int nvp = p.nv + kSepPad;
-    dim3 tb(256), tg((p.nu + 31) / 32, (nvp + 31) / 32, p.count);
-    hipLaunchKernelGGL(joseph_sep_table_kernel, tg, tb, 0, s, p.proj, p.views, p.vol, p.nu, p.nv, nvp, p.ab1,
-        p.ab2, p.pl);
-    dim3 block(256), grid((p.vol.nx + 15) / 16, (p.vol.ny + 15) / 16, (p.vol.nz + kSepZ - 1) / kSepZ);
-    hipLaunchKernelGGL(joseph_adjoint_sep_kernel, grid, block, 0, s, p.ab1, p.ab2, p.pl, p.views, p.coeff32,
-        p.vol, p.nu, p.nv, nvp, p.count, p.accumulate, p.volume);
-    YK_HIP(hipGetLastError());
-}
-
 void launch_siddon_fp(const SiddonLaunch& p, hipStream_t s)
 {
     dim3 block(256), grid((p.nu + 7) / 8, (p.nv + 3) / 4, (p.count + 7) / 8);
@@ -1551,18 +1144,6 @@ void launch_siddon_fp_slab(const SiddonSlabFpLaunch& p, hipStream_t s)
     dim3 block(64, 8), grid((p.nu + 63) / 64, p.nv, (p.count + 7) / 8);
     hipLaunchKernelGGL(siddon_fp_slab_kernel, grid, block, 0, s, p.vol_x, p.vol_y, p.volume, p.flag, p.proj, p.views,
         p.vol, p.nu, p.nv, p.count, p.accumulate);
-    YK_HIP(hipGetLastError());
-}
-
-void launch_siddon_adjoint_sep(const SiddonSepLaunch& p, hipStream_t s)
-{
-    const int nvp = p.nv + kSepPad;
-    dim3 tb(256), tg((p.nu + 31) / 32, (nvp + 31) / 32, p.count);
-    hipLaunchKernelGGL(siddon_sep_table_kernel, tg, tb, 0, s, p.proj, p.views, p.nu, p.nv, nvp, p.col_xy,
-        p.ray_wz);
-    dim3 block(256), grid((p.vol.nx + 15) / 16, (p.vol.ny + 15) / 16, (p.vol.nz + kSidSepZ - 1) / kSidSepZ);
-    hipLaunchKernelGGL(siddon_adjoint_sep_kernel, grid, block, 0, s, p.col_xy, p.ray_wz, p.views, p.coeff32,
-        p.vol, p.nu, p.nv, nvp, p.count, p.accumulate, p.volume);
     YK_HIP(hipGetLastError());
 }
 

@@ -27,6 +27,60 @@ void grow(DeviceArray<T>& a, size_t n)
 // cross.
 constexpr double kSiddonSlabRatio = 1.0;
 
+// record of the gather transposes of a view whose main axis is X or Y, from
+// the forward kernel's voxel-normalized floats and the projective map of world
+// points
+void gather_view(const ProjViewDev& p, int nu, int nv, const double map[12], const VolumeGeom& g, GatherViewDev& o)
+{
+    std::memset(&o, 0, sizeof(o));
+    o.axis = p.axis;
+    const int order[3] = { p.axis, p.axis == 0 ? 1 : 0, 2 };
+    double most = 0.0;
+    for (int a = 0; a < 4; ++a)
+        most = std::max(most, std::fabs(double(p.detS[p.axis]) - p.src[p.axis] +
+            ((a & 1) ? nu - 1 : 0) * double(p.detU[p.axis]) + ((a & 2) ? nv - 1 : 0) * double(p.detV[p.axis])));
+    int e = 0;
+    std::frexp(most, &e);
+    const double scale = std::ldexp(1.0, -e);
+    o.scale = float(scale);
+    double* rows[3] = { o.d, o.e1, o.e2 };
+    for (int k = 0; k < 3; ++k) {
+        const int c = order[k];
+        o.src[k] = p.src[c];
+        rows[k][0] = (double(p.detS[c]) - p.src[c]) * scale;
+        rows[k][1] = p.detU[c] * scale;
+        rows[k][2] = p.detV[c] * scale;
+    }
+    // the map at voxel index (i, j, k): X = origin + index x voxel
+    const double vox[3] = { g.vx, g.vy, g.vz }, org[3] = { g.ox, g.oy, g.oz };
+    float* maps[3] = { o.mu, o.mv, o.md };
+    for (int m = 0; m < 3; ++m) {
+        const double* c = map + 4 * m;
+        for (int k = 0; k < 3; ++k) maps[m][k] = float(c[k] * vox[k]);
+        maps[m][3] = float(c[0] * org[0] + c[1] * org[1] + c[2] * org[2] + c[3]);
+    }
+}
+
+// least and largest distance of the volume's voxels, grown by `xy` and `z`
+// voxels on each side, from the source plane (row 2 of the map), over the
+// detector plane's
+void depth_range(const yk_view& w, const double map[12], const VolumeGeom& g, double xy, double z, double& least,
+    double& most)
+{
+    const ViewD d = widen(w);
+    const double plane = map[8] * d.detS[0] + map[9] * d.detS[1] + map[10] * d.detS[2] + map[11];
+    least = 1e300;
+    most = -1e300;
+    for (int a = 0; a < 8; ++a) {
+        const double X = g.ox + ((a & 1) ? g.nx - 1 + xy : -xy) * double(g.vx);
+        const double Y = g.oy + ((a & 2) ? g.ny - 1 + xy : -xy) * double(g.vy);
+        const double Z = g.oz + ((a & 4) ? g.nz - 1 + z : -z) * double(g.vz);
+        const double depth = (map[8] * X + map[9] * Y + map[10] * Z + map[11]) / plane;
+        least = std::min(least, depth);
+        most = std::max(most, depth);
+    }
+}
+
 }  // namespace
 
 yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
@@ -43,6 +97,7 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
     std::vector<ProjViewDev> jv(n);
     std::vector<SiddonViewDev> sv(n);
     std::vector<double> c64(size_t(n) * 12);
+    std::vector<GatherViewDev> gv(n);
     const double vox[3] = { grid.voxel_x_mm, grid.voxel_y_mm, grid.voxel_z_mm };
     const double cen[3] = { grid.center_mm[0], grid.center_mm[1], grid.center_mm[2] };
     for (int i = 0; i < n; ++i) {
@@ -65,7 +120,6 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
         // d0 and d1 of every ray independent of v (exact zeros, so bit-exact)
         separable.push_back(p.axis != 2 && p.detV[p.axis == 0 ? 0 : 1] == 0.f &&
                             p.detV[p.axis == 0 ? 1 : 0] == 0.f);
-        siddon_separable.push_back(w.detV[0] == 0.f && w.detV[1] == 0.f);
         SiddonViewDev& s = sv[i];
         std::memset(&s, 0, sizeof(s));
         std::memcpy(s.src, w.src, sizeof(s.src));
@@ -73,7 +127,23 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
         std::memcpy(s.detU, w.detU, sizeof(s.detU));
         std::memcpy(s.detV, w.detV, sizeof(s.detV));
         projection_map(w, &c64[size_t(i) * 12]);
+        // Gather transposes.  Their kernels take every support of a run of
+        // kGatherRun voxels to lie before the source, and the Siddon one that
+        // t in [0, 1] clips no ray inside the volume.
+        if (p.axis != 2) {
+            const double* map = &c64[size_t(i) * 12];
+            double least, most, inner, outer;
+            depth_range(w, map, vol, 2.0, kGatherRun + 2.0, least, most);
+            depth_range(w, map, vol, 0.5, 0.5, inner, outer);
+            gather_view(p, nu, nv, map, vol, gv[i]);
+            joseph_gather.push_back(least > 1e-3);
+            siddon_gather.push_back(least > 1e-3 && outer < 1.0);
+        } else {
+            joseph_gather.push_back(0);
+            siddon_gather.push_back(0);
+        }
     }
+    d_gather.upload(gv.data(), gv.size(), ctx->stream);
     // operator-form FDK backprojection records (FP64 geometry over the whole
     // view sequence, like FdkAffineCoeff in .../FDK/kernels/YkFDKBpPrecompute.cu:14-138)
     std::vector<DerivedD> der;
@@ -250,6 +320,49 @@ void yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
     }
 }
 
+// Transposes of views of any orientation by the gather kernels, a chunk of
+// views' table at a time (at most 1 GiB); false when they do not apply: a view
+// outside their forms, rows past 32-bit offsets, or no memory for the table
+// (none may be allocated under a stream capture)
+bool yk_projector::gather_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
+    int accumulate)
+{
+    const std::vector<char>& ok = siddon ? siddon_gather : joseph_gather;
+    if (!std::all_of(ok.begin() + first, ok.begin() + first + count, [](char c) { return c != 0; })) return false;
+    const int pitch = nu + kGatherPad;
+    const size_t per_view = size_t(nv + kGatherPadRows) * pitch * (siddon ? 4 : 1);  // floats
+    if (nv + kGatherPadRows > 65535 || per_view > (size_t(1) << 30)) return false;
+    const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
+    if (w.d_gather_q.size() < per_view * chunk || !w.d_flag.get()) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) return false;
+        try {
+            grow(w.d_gather_q, per_view * chunk);
+            grow(w.d_flag, 1);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    for (int c0 = 0; c0 < count; c0 += chunk) {
+        GatherLaunch p{};
+        p.proj = d_proj + size_t(nu) * nv * c0;
+        p.volume = d_volume;
+        p.views = d_jviews.get() + first + c0;
+        p.sviews = d_sviews.get() + first + c0;
+        p.gviews = d_gather.get() + first + c0;
+        p.q = w.d_gather_q.get();
+        p.flag = w.d_flag.get();
+        p.vol = vol;
+        p.nu = nu; p.nv = nv; p.pitch = pitch; p.count = std::min(chunk, count - c0);
+        p.siddon = siddon;
+        p.accumulate = c0 > 0 ? 1 : accumulate;
+        launch_gather_transpose(p, ctx->stream);
+    }
+    return true;
+}
+
 void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, int first, int count,
     int accumulate)
 {
@@ -257,31 +370,7 @@ void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, i
     if (!d_volume || !d_proj) fail(YK_ERR_INVALID_BUFFER, "null device buffer");
     hipStream_t s = ctx->stream;
     yk_projector& w = scratch_owner ? *scratch_owner : *this;  // scratch arrays
-    bool all_sep = true;
-    for (int i = first; i < first + count; ++i) all_sep = all_sep && separable[i];
-    if (kind == YK_BP_JOSEPH_ADJOINT && all_sep) {
-        // column-major ray table of a chunk of views at a time (at most 1 GiB)
-        const size_t per_view = size_t(nu) * nv;
-        const size_t table = size_t(nu) * (nv + kSepPad);
-        const int chunk = int(std::max<size_t>(1, std::min<size_t>(size_t(count),
-            (size_t(1) << 30) / (table * (sizeof(float2) + sizeof(float)) + size_t(nu) * sizeof(float2)))));
-        w.d_sep_ab1.resize(std::max(w.d_sep_ab1.size(), size_t(nu) * chunk));
-        w.d_sep_ab2.resize(std::max(w.d_sep_ab2.size(), table * chunk));
-        w.d_sep_pl.resize(std::max(w.d_sep_pl.size(), table * chunk));
-        for (int c0 = 0; c0 < count; c0 += chunk) {
-            JosephSepLaunch p{};
-            p.proj = d_proj + per_view * c0;
-            p.volume = d_volume;
-            p.views = d_jviews.get() + first + c0;
-            p.coeff32 = d_c32.get() + size_t(first + c0) * 12;
-            p.ab1 = w.d_sep_ab1.get();
-            p.ab2 = w.d_sep_ab2.get();
-            p.pl = w.d_sep_pl.get();
-            p.vol = vol;
-            p.nu = nu; p.nv = nv; p.count = std::min(chunk, count - c0);
-            p.accumulate = c0 > 0 ? 1 : accumulate;
-            launch_joseph_adjoint_sep(p, s);
-        }
+    if (kind == YK_BP_JOSEPH_ADJOINT && gather_transpose(w, false, d_proj, d_volume, first, count, accumulate)) {
     } else if (kind == YK_BP_JOSEPH_ADJOINT) {
         // the ray table holds a chunk of views at a time (at most 1 GiB)
         const size_t per_view = size_t(nu) * nv;
@@ -302,29 +391,7 @@ void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, i
             p.accumulate = c0 > 0 ? 1 : accumulate;
             launch_joseph_adjoint(p, s);
         }
-    } else if (kind == YK_BP_SIDDON_ADJOINT && std::all_of(siddon_separable.begin() + first,
-                                                            siddon_separable.begin() + first + count,
-                                                            [](char c) { return c != 0; })) {
-        // column-major ray table of a chunk of views at a time (at most 1 GiB)
-        const size_t per_view = size_t(nu) * nv;
-        const size_t table = size_t(nu) * (nv + kSepPad);
-        const int chunk = int(std::max<size_t>(1, std::min<size_t>(size_t(count),
-            (size_t(1) << 30) / ((table + nu) * sizeof(float2)))));
-        w.d_sid_col.resize(std::max(w.d_sid_col.size(), size_t(nu) * chunk));
-        w.d_sid_ray.resize(std::max(w.d_sid_ray.size(), table * chunk));
-        for (int c0 = 0; c0 < count; c0 += chunk) {
-            SiddonSepLaunch p{};
-            p.proj = d_proj + per_view * c0;
-            p.volume = d_volume;
-            p.views = d_sviews.get() + first + c0;
-            p.coeff32 = d_c32.get() + size_t(first + c0) * 12;
-            p.col_xy = w.d_sid_col.get();
-            p.ray_wz = w.d_sid_ray.get();
-            p.vol = vol;
-            p.nu = nu; p.nv = nv; p.count = std::min(chunk, count - c0);
-            p.accumulate = c0 > 0 ? 1 : accumulate;
-            launch_siddon_adjoint_sep(p, s);
-        }
+    } else if (kind == YK_BP_SIDDON_ADJOINT && gather_transpose(w, true, d_proj, d_volume, first, count, accumulate)) {
     } else if (kind == YK_BP_SIDDON_ADJOINT) {
         SiddonAdjointLaunch p{};
         p.proj = d_proj;

@@ -1,0 +1,82 @@
+// Device-side ray setup shared by the projection kernels and their transposes.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "yk_internal.hpp"
+
+namespace yk {
+namespace {
+
+struct AxisInfo {
+    int p0, p1, p2;     // component index of c0, c1, c2
+    int n0, n1, n2;
+    float v0, v1, v2;
+};
+
+__device__ __forceinline__ AxisInfo axis_info(int axis, const VolumeGeom& g)
+{
+    AxisInfo a;
+    if (axis == 0) { a.p0 = 0; a.p1 = 1; a.p2 = 2; a.n0 = g.nx; a.n1 = g.ny; a.n2 = g.nz; a.v0 = g.vx; a.v1 = g.vy; a.v2 = g.vz; }
+    else if (axis == 1) { a.p0 = 1; a.p1 = 0; a.p2 = 2; a.n0 = g.ny; a.n1 = g.nx; a.n2 = g.nz; a.v0 = g.vy; a.v1 = g.vx; a.v2 = g.vz; }
+    else { a.p0 = 2; a.p1 = 0; a.p2 = 1; a.n0 = g.nz; a.n1 = g.nx; a.n2 = g.ny; a.v0 = g.vz; a.v1 = g.vx; a.v2 = g.vy; }
+    return a;
+}
+
+template <typename T>
+__device__ __forceinline__ T pick(int k, T a, T b, T c) { return k == 0 ? a : (k == 1 ? b : c); }
+
+struct JRay {
+    float a1, b1, a2, b2, L;
+};
+
+// Per-ray Joseph line in volume-centred voxel units.  Shared by the forward
+// kernel and the transpose's ray table, with contraction disabled so both
+// evaluate the same IEEE operations and obtain bit-identical parameters.
+__device__ __forceinline__ bool joseph_ray(const ProjViewDev& pv, const AxisInfo& ax,
+    int u, int v, JRay& r)
+{
+#pragma clang fp contract(off)
+    const float dx = (pv.detS[0] + float(u) * pv.detU[0]) + float(v) * pv.detV[0];
+    const float dy = (pv.detS[1] + float(u) * pv.detU[1]) + float(v) * pv.detV[1];
+    const float dz = (pv.detS[2] + float(u) * pv.detU[2]) + float(v) * pv.detV[2];
+    const float sx = pv.src[0], sy = pv.src[1], sz = pv.src[2];
+    const float s0 = pick(ax.p0, sx, sy, sz), s1 = pick(ax.p1, sx, sy, sz), s2 = pick(ax.p2, sx, sy, sz);
+    const float d0 = pick(ax.p0, dx, dy, dz), d1 = pick(ax.p1, dx, dy, dz), d2 = pick(ax.p2, dx, dy, dz);
+    const float den = s0 - d0;
+    if (den == 0.f) return false;
+    r.a1 = (s1 - d1) / den;
+    r.a2 = (s2 - d2) / den;
+    r.b1 = s1 - r.a1 * s0;
+    r.b2 = s2 - r.a2 * s0;
+    const float t1 = r.a1 * ax.v1, t2 = r.a2 * ax.v2;
+    r.L = sqrtf(ax.v0 * ax.v0 + t1 * t1 + t2 * t2);
+    return true;
+}
+
+// centred main-axis coordinate of slice s
+__device__ __forceinline__ float joseph_c0(int s, int n0)
+{
+#pragma clang fp contract(off)
+    return float(s) - 0.5f * float(n0 - 1);
+}
+
+// one minor-axis sample position (index space, texel k at k) of the line
+// c = a c0 + b
+__device__ __forceinline__ float joseph_minor(float a, float b, float c0, int n)
+{
+#pragma clang fp contract(off)
+    return (a * c0 + b) + 0.5f * float(n - 1);
+}
+
+__device__ __forceinline__ void siddon_ray_geom(const SiddonViewDev& sv, int u, int v, float* src, float* ray)
+{
+#pragma clang fp contract(off)
+    for (int k = 0; k < 3; ++k) {
+        src[k] = sv.src[k];
+        ray[k] = (sv.detS[k] + float(u) * sv.detU[k] + float(v) * sv.detV[k]) - sv.src[k];
+    }
+}
+
+}  // namespace
+}  // namespace yk

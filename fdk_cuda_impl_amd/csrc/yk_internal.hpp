@@ -325,24 +325,39 @@ struct JosephAdjointLaunch {
 };
 void launch_joseph_adjoint(const JosephAdjointLaunch& p, hipStream_t s);
 
-// zero entries closing each detector column of the separable ray table
-constexpr int kSepPad = 8;
+// per-view record of the gather transposes (kernels_gather.hip): the map that
+// bounds the candidates of either model and, for Joseph, source and pixel
+// offsets in volume-centred voxel units, component 0 the main axis, 1 the
+// other of x and y, 2 z; pixel minus source is d / e1 / e2 = [0] + u [1] +
+// v [2] on components 0 / 1 / 2, times `scale`, a power of two that brings |d|
+// into [0, 1] over the detector
+struct GatherViewDev {
+    double src[3];
+    double d[3], e1[3], e2[3];
+    float mu[4], mv[4], md[4];  // projective map of voxel indices [x, y, z, 1]: u = mu / md, v = mv / md
+    float scale;
+    int axis;                   // 0 X, 1 Y
+};
 
-// Transpose of the Joseph projector for separable views (main axis X or Y,
-// detV with no X/Y component); the ray table arrays are scratch of `count` views.
-struct JosephSepLaunch {
+struct GatherLaunch {
     const float* proj;          // [count][nv][nu]
     float* volume;              // [z][y][x]
-    const ProjViewDev* views;   // device, `count`
-    const float* coeff32;       // device, per view cu[4] cv[4] cd[4] (world projective map)
-    float2* ab1;                // scratch [count][nu]
-    float2* ab2;                // scratch [count][nu][nv + kSepPad]
-    float* pl;                  // scratch [count][nu][nv + kSepPad]
+    const ProjViewDev* views;   // device, `count` (Joseph)
+    const SiddonViewDev* sviews; // device, `count` (Siddon)
+    const GatherViewDev* gviews; // device, `count`
+    float* q;                   // scratch [count][nv + kGatherPadRows][pitch] floats (Joseph) or float4s (Siddon)
+    int* flag;                  // scratch word
     VolumeGeom vol;
-    int nu, nv, count;
+    int nu, nv, pitch, count;
+    int siddon;                 // 0 Joseph
     int accumulate;
 };
-void launch_joseph_adjoint_sep(const JosephSepLaunch& p, hipStream_t s);
+void launch_gather_transpose(const GatherLaunch& p, hipStream_t s);
+// zero columns closing each row, and zero rows closing each view, of the
+// gather transposes' table (a chunk of candidates may run past the last pixel)
+constexpr int kGatherPad = 4;
+constexpr int kGatherPadRows = 3;
+constexpr int kGatherRun = 8;  // voxels along z of a lane
 
 struct SiddonLaunch {
     const float* volume;
@@ -380,21 +395,6 @@ struct SiddonAdjointLaunch {
     int accumulate;
 };
 void launch_siddon_adjoint(const SiddonAdjointLaunch& p, hipStream_t s);
-
-// Transpose of the Siddon projector for separable views (detV along Z only);
-// the ray table arrays are scratch of `count` views.
-struct SiddonSepLaunch {
-    const float* proj;          // [count][nv][nu]
-    float* volume;              // [z][y][x]
-    const SiddonViewDev* views; // device, `count`
-    const float* coeff32;       // device, per view cu[4] cv[4] cd[4] (world projective map)
-    float2* col_xy;             // scratch [count][nu]
-    float2* ray_wz;             // scratch [count][nu][nv + kSepPad]
-    VolumeGeom vol;
-    int nu, nv, count;
-    int accumulate;
-};
-void launch_siddon_adjoint_sep(const SiddonSepLaunch& p, hipStream_t s);
 
 // per-view record of the operator-form FDK backprojections (world units)
 struct OpBpViewDev {

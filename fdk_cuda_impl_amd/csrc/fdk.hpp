@@ -80,6 +80,9 @@ struct yk_fdk {
 
 private:
     void build_tiles();
+    int part_count(int count) const;
+    void split_views(yk::BpLaunch& p) const;
+    yk::DeviceArray<float> d_parts;    // the parts' volumes of a small volume's backprojection
 };
 
 struct yk_projector {

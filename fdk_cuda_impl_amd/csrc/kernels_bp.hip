@@ -700,15 +700,25 @@ fdk_bp_kernel(const void* __restrict__ proj, const unsigned* __restrict__ row_fa
     const int* __restrict__ gscale_bits, const BpCoeff* __restrict__ coeffs,
     const short4* __restrict__ tiles, const uint2* __restrict__ stage, int tile_stride, int tile_offset,
     float* __restrict__ volume, VolumeGeom vol, int nu, int nv, int count, int accumulate,
-    unsigned buf_bytes, int double_buffer)
+    unsigned buf_bytes, int double_buffer, int nbz, int part_views)
 {
+    // views [part * part_views, + part_views) of the call, into the part's own
+    // volume when there are several (launch_bz)
+    const int part = int(blockIdx.z) / nbz;
+    const int first = part * part_views;
+    count = min(part_views, count - first);
+    volume += size_t(part) * vol.nx * vol.ny * vol.nz;
+    coeffs += first;
+    tile_offset += first;
+    proj = static_cast<const char*>(proj) + size_t(first) * nu * nv * (STORAGE == YK_F32 ? 4 : 2);
+    if constexpr (has_factors(STORAGE)) row_factors += size_t(first) * nv;
     // one LDS tile buffer, or two alternating ones (then a single barrier per
     // view orders the writes of view i+1 after every read of view i-1)
     constexpr bool Q32 = bp_float_quads(STORAGE, GEO);
     extern __shared__ float4 lds_raw[];
     char* const lds0 = reinterpret_cast<char*>(lds_raw);
     unsigned cur = 0, nxt = double_buffer ? buf_bytes : 0u;
-    const int bxi = blockIdx.x, byi = blockIdx.y, bzi = blockIdx.z;
+    const int bxi = blockIdx.x, byi = blockIdx.y, bzi = int(blockIdx.z) - part * nbz;
     // lane -> column: each wave covers 16 x 4 columns, and every 8 consecutive
     // lanes a 4 x 2 patch, so the lanes one LDS cycle serves read nearby quads
     // of distinct banks whatever the view angle
@@ -821,10 +831,22 @@ fdk_bp_kernel(const void* __restrict__ proj, const unsigned* __restrict__ row_fa
     }
 }
 
+// sum of the parts' volumes (in FP64, so the split adds no rounding to speak
+// of), onto the volume when it accumulates
+__global__ void __launch_bounds__(256)
+sum_parts_kernel(const float* __restrict__ parts, int n_parts, size_t n, float* __restrict__ volume, int accumulate)
+{
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    double s = accumulate ? double(volume[i]) : 0.0;
+    for (int k = 0; k < n_parts; ++k) s += double(parts[size_t(k) * n + i]);
+    volume[i] = float(s);
+}
+
 template <int STORAGE, int BZ, int GEO, bool KAHAN>
 void launch_bz(const BpLaunch& p, const int* gbits, hipStream_t s)
 {
-    dim3 grid(p.nbx, p.nby, p.nbz), block(kThreads);
+    dim3 grid(p.nbx, p.nby, p.nbz * p.parts), block(kThreads);
     const size_t buf = size_t(p.lds_quads) * (bp_float_quads(STORAGE, GEO) ? 16 : 8);
     auto k = fdk_bp_kernel<STORAGE, BZ, GEO, KAHAN>;
     // double-buffer the tile when that costs no occupancy: workgroups per CU
@@ -840,8 +862,13 @@ void launch_bz(const BpLaunch& p, const int* gbits, hipStream_t s)
     YK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k),
         hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     hipLaunchKernelGGL(k, grid, block, lds, s, p.proj, p.row_factors, gbits, p.coeffs, p.tiles, p.stage,
-        p.tile_view_stride, p.tile_view_offset, p.volume, p.vol, p.nu, p.nv, p.count, p.accumulate,
-        unsigned(buf), db);
+        p.tile_view_stride, p.tile_view_offset, p.parts > 1 ? p.part_volumes : p.volume, p.vol, p.nu, p.nv, p.count,
+        p.parts > 1 ? 0 : p.accumulate, unsigned(buf), db, p.nbz, p.part_views);
+    if (p.parts > 1) {
+        const size_t n = size_t(p.vol.nx) * p.vol.ny * p.vol.nz;
+        hipLaunchKernelGGL(sum_parts_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, p.part_volumes, p.parts, n,
+            p.volume, p.accumulate);
+    }
 }
 
 template <int STORAGE, int GEO, bool KAHAN>

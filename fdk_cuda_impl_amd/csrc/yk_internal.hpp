@@ -233,6 +233,9 @@ struct BpLaunch {
     int nbx, nby, nbz;
     int bz;                     // z slices per workgroup (32, 16 or 8)
     int lds_quads;              // LDS capacity in quads
+    int parts;                  // parts of part_views views each, in workgroups of their own
+    int part_views;
+    float* part_volumes;        // `parts` volumes when parts > 1
 };
 void launch_fdk_bp(const BpLaunch& p, hipStream_t s);
 // BpLaunch::storage of half texels already normalized by launch_normalize_rows

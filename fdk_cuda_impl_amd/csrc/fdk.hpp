@@ -93,6 +93,7 @@ struct yk_projector {
     void backproject(int kind, const float* d_proj, float* d_volume, int first, int count, int accumulate);
     double dot(const float* a, const float* b, size_t n);
     bool siddon_copies(yk_projector& w, const float* d_volume);
+    int op_chunk(yk_projector& w, int count) const;
     bool gather_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
         int accumulate);
 
@@ -119,9 +120,11 @@ struct yk_projector {
     std::vector<char> joseph_gather, siddon_gather;  // per view: the gather transposes cover it
     yk::DeviceArray<yk::GatherViewDev> d_gather;
     yk::DeviceArray<float> d_gather_q; // ray values of the gather transposes, one view chunk
+    yk::DeviceArray<float> d_paired_views;  // paired views of the operator-form backprojections, one chunk
     yk::DeviceArray<int> d_flag;       // one word: see siddon_value_check_kernel
     yk::DeviceArray<double> d_partials;
     yk::DeviceArray<yk::OpBpViewDev> d_opviews;  // operator-form FDK backprojection records
+    std::vector<char> op_front;        // per view: no voxel needs the operator backprojections' sample tests
     std::vector<double> op_scale;      // per first view: vx vy vz / (du dv)
 };
 

@@ -968,6 +968,7 @@ siddon_adjoint_kernel(const float* __restrict__ proj, float* __restrict__ volume
 //   of X - src through one voxel along its main axis m = argmax |d_k / v_k|
 //   (ties X, then Y): v_m |d| / |d_m|.
 constexpr int kOpBpZ = 8;
+constexpr int kViewGuard = 1;  // zero pixels around a paired view
 enum OpBpMode { kOpFdk = 0, kOpMatched = 1, kOpJosephVoxel = 2 };
 
 __device__ __forceinline__ float bilinear_view(const float* __restrict__ p, int nu, int nv, float u, float v)
@@ -984,7 +985,73 @@ __device__ __forceinline__ float bilinear_view(const float* __restrict__ p, int 
     return (1.f - b) * ((1.f - a) * t00 + a * t01) + b * ((1.f - a) * t10 + a * t11);
 }
 
+// square root to half an ulp for a normal x > 0: one Newton step on the
+// hardware's reciprocal root (16 cycles, the library's scaled form takes ~40)
+__device__ __forceinline__ float op_sqrt(float x)
+{
+    const float r = __builtin_amdgcn_rsqf(x), s = x * r;
+    return fmaf(fmaf(-s, s, x), 0.5f * r, s);
+}
+
+// the part of a view's sample weight that a voxel column shares
 template <int MODE>
+struct OpColumn {
+    float xy2, inv, base;  // |X - src|^2 in the plane; 1 / main-axis steps (Joseph); FDK denominator at Z = 0
+    bool zmain;            // some lane of the wave may have main axis Z (Joseph)
+
+    __device__ __forceinline__ OpColumn(const OpBpViewDev& c, const VolumeGeom& g, float X, float Y, float Za, float Zb)
+    {
+        const float dx = X - c.src[0], dy = Y - c.src[1];
+        xy2 = dx * dx + dy * dy;
+        inv = base = 0.f;
+        zmain = false;
+        if constexpr (MODE == kOpJosephVoxel) {
+            base = fmaxf(fabsf(dx / g.vx), fabsf(dy / g.vy));
+            inv = __builtin_amdgcn_rcpf(base);
+            zmain = __any(!(fmaxf(fabsf(Za - c.src[2]), fabsf(Zb - c.src[2])) <= base * g.vz));
+        } else if constexpr (MODE == kOpFdk) {
+            base = c.cc[0] * X + c.cc[1] * Y + c.cc[3];
+        }
+    }
+
+    // weight of the sample at (u, v) of the column's voxel at height Z; `ok`
+    // is cleared when it adds nothing
+    __device__ __forceinline__ float weight(const OpBpViewDev& c, float ivz, float scale, float Z, float u, float v,
+        bool& ok) const
+    {
+        if constexpr (MODE == kOpJosephVoxel) {
+            // v_m |d| / |d_m|, m the axis of the largest |d_k / v_k|
+            const float dz = Z - c.src[2];
+            const float len = op_sqrt(fmaf(dz, dz, xy2));
+            return zmain ? len * __builtin_amdgcn_rcpf(fmaxf(base, fabsf(dz * ivz))) : len * inv;
+        } else if constexpr (MODE == kOpMatched) {
+            const float L2 = c.l2[0] + u * (c.l2[1] + u * c.l2[3]) + v * (c.l2[2] + u * c.l2[4] + v * c.l2[5]);
+            const float dz = Z - c.src[2], lsq = fmaf(dz, dz, xy2);
+            ok = ok && L2 >= 1e-8f && lsq >= 1e-8f;
+            return L2 * op_sqrt(L2) * __builtin_amdgcn_rcpf(lsq) * c.inv_sdd_plane * scale;
+        } else {
+            const float cn = fmaf(c.cc[2], Z, base);
+            const float rc = __builtin_amdgcn_rcpf(cn);
+            ok = ok && fabsf(cn) >= 1e-8f;
+            return c.wbase * rc * rc;
+        }
+    }
+};
+
+// One lane per (x, y) column of kOpBpZ voxels.
+// PAIRED: the samples come from a paired guarded copy of the views
+// (pair_views_kernel), one 16-byte load each at a position clamped into the
+// copy, with no bounds branches; the loads of kOpBatch slices are issued
+// together.  Otherwise four bounds-checked taps of the views themselves.
+// FRONT: every voxel (and the run's overhang past the last slice) lies before
+// the source of every view with a weight that is not singular, so no sample is
+// tested.
+// Bound of the paired form: about 100 VALU cycles (25 a CU) and one 16-cycle
+// gather a sample.  256^3 x 360 views of 512 x 384, four taps -> paired: FDK
+// 10.2 -> 4.4 ms, pseudo-matched 11.4 -> 6.1, voxel-driven Joseph 11.1 -> 5.9,
+// the copy included.
+constexpr int kOpBatch = 4;
+template <int MODE, bool PAIRED, bool FRONT>
 __global__ void __launch_bounds__(256)
 fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volume,
     const OpBpViewDev* __restrict__ views, VolumeGeom g, int nu, int nv, int count, float scale,
@@ -995,53 +1062,76 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
     const int z0 = blockIdx.z * kOpBpZ;
     if (x >= g.nx || y >= g.ny) return;
     const float X = g.ox + x * g.vx, Y = g.oy + y * g.vy;
+    const float Za = g.oz + z0 * g.vz, Zb = g.oz + (z0 + kOpBpZ - 1) * g.vz;
     float acc[kOpBpZ];
 #pragma unroll
     for (int k = 0; k < kOpBpZ; ++k) acc[k] = 0.f;
-    // reciprocal voxel sizes for the voxel-driven Joseph main-axis test
-    const float ivx = 1.f / g.vx, ivy = 1.f / g.vy, ivz = 1.f / g.vz;
+    const float ivz = 1.f / g.vz;
+    const int pitch = nu + 2 * kViewGuard + 1, rows = nv + 2 * kViewGuard;
+#pragma unroll 1
     for (int i = 0; i < count; ++i) {
-        const OpBpViewDev c = views[i];
-        const float* p = proj + (size_t)i * nu * nv;
+        const OpBpViewDev& c = views[i];
+        const OpColumn<MODE> col(c, g, X, Y, Za, Zb);
         // the view's map at this voxel column; each slice adds its Z term
         const float d0 = fmaf(c.cd[1], Y, fmaf(c.cd[0], X, c.cd[3]));
         const float u0 = fmaf(c.cu[1], Y, fmaf(c.cu[0], X, c.cu[3]));
         const float v0 = fmaf(c.cv[1], Y, fmaf(c.cv[0], X, c.cv[3]));
-#pragma unroll
-        for (int k = 0; k < kOpBpZ; ++k) {
-            if (z0 + k >= g.nz) break;
-            const float Z = g.oz + (z0 + k) * g.vz;
+        // numerators of u and v and the reciprocal depth at slice k: one
+        // Newton step on the hardware reciprocal brings u and v within an ulp
+        // or so of the quotients (the sample position is the sensitive
+        // input), for two FMAs instead of two divisions
+        auto project = [&](int k, float& Z, float& un, float& vn, float& rd) {
+            Z = g.oz + (z0 + k) * g.vz;
             const float den = fmaf(c.cd[2], Z, d0);
-            if (!(den >= 1e-8f)) continue;
-            // one Newton step on the hardware reciprocal: u and v within an
-            // ulp or so of the quotients (the sample position is the
-            // sensitive input), for two FMAs instead of two divisions
-            float rd = __builtin_amdgcn_rcpf(den);
+            rd = __builtin_amdgcn_rcpf(den);
             rd = fmaf(rd, fmaf(-den, rd, 1.f), rd);
-            const float u = fmaf(c.cu[2], Z, u0) * rd;
-            const float v = fmaf(c.cv[2], Z, v0) * rd;
-            float w;
-            if constexpr (MODE == kOpJosephVoxel) {
-                const float dx = X - c.src[0], dy = Y - c.src[1], dz = Z - c.src[2];
-                const float ax = fabsf(dx * ivx), ay = fabsf(dy * ivy), az = fabsf(dz * ivz);
-                const bool mx = ax >= ay && ax >= az, my = !mx && ay >= az;
-                const float vm = mx ? g.vx : my ? g.vy : g.vz;
-                const float dm = mx ? dx : my ? dy : dz;
-                w = vm * sqrtf(dx * dx + dy * dy + dz * dz) * __builtin_amdgcn_rcpf(fabsf(dm));
-            } else if constexpr (MODE == kOpMatched) {
-                const float L2 = c.l2[0] + u * (c.l2[1] + u * c.l2[3]) + v * (c.l2[2] + u * c.l2[4] + v * c.l2[5]);
-                if (!(L2 >= 1e-8f)) continue;
-                const float dx = X - c.src[0], dy = Y - c.src[1], dz = Z - c.src[2];
-                const float lsq = dx * dx + dy * dy + dz * dz;
-                if (!(lsq >= 1e-8f)) continue;
-                w = L2 * sqrtf(L2) * __builtin_amdgcn_rcpf(lsq) * c.inv_sdd_plane * scale;
-            } else {
-                const float cn = c.cc[0] * X + c.cc[1] * Y + c.cc[2] * Z + c.cc[3];
-                if (!(fabsf(cn) >= 1e-8f)) continue;
-                const float rc = __builtin_amdgcn_rcpf(cn);
-                w = c.wbase * rc * rc;
+            un = fmaf(c.cu[2], Z, u0);
+            vn = fmaf(c.cv[2], Z, v0);
+            return den >= 1e-8f;
+        };
+        if constexpr (PAIRED) {
+            const char* p = reinterpret_cast<const char*>(proj) + size_t(i) * rows * pitch * 8u;
+            const float umax = float(nu + 1), vmax = float(nv + 1);
+            const unsigned row_bytes = unsigned(pitch) * 8u;
+#pragma unroll
+            for (int k0 = 0; k0 < kOpBpZ; k0 += kOpBatch) {
+                float4u q[kOpBatch];
+                float a[kOpBatch], b[kOpBatch], w[kOpBatch];
+                bool on[kOpBatch];
+#pragma unroll
+                for (int k = 0; k < kOpBatch; ++k) {
+                    float Z, un, vn, rd;
+                    on[k] = project(k0 + k, Z, un, vn, rd);
+                    w[k] = col.weight(c, ivz, scale, Z, un * rd, vn * rd, on[k]);
+                    // positions in the copy (pixel + guard); past its guards
+                    // the clamped sample lies on zeros only
+                    const float u = __builtin_amdgcn_fmed3f(fmaf(un, rd, 1.f), 0.f, umax);
+                    const float v = __builtin_amdgcn_fmed3f(fmaf(vn, rd, 1.f), 0.f, vmax);
+                    a[k] = __builtin_amdgcn_fractf(u);
+                    b[k] = __builtin_amdgcn_fractf(v);
+                    q[k] = *reinterpret_cast<const float4u*>(p + (__umul24(unsigned(int(v)), row_bytes) + unsigned(int(u)) * 8u));
+                }
+#pragma unroll
+                for (int k = 0; k < kOpBatch; ++k) {
+                    // q: (row, col), (row + 1, col), (row, col + 1), (row + 1, col + 1)
+                    const float a0 = 1.f - a[k], b0 = 1.f - b[k];
+                    const float s = fmaf(b[k], fmaf(a[k], q[k].w, a0 * q[k].y), b0 * fmaf(a[k], q[k].z, a0 * q[k].x));
+                    const float t = fmaf(s, w[k], acc[k0 + k]);
+                    acc[k0 + k] = FRONT || on[k] ? t : acc[k0 + k];
+                }
             }
-            acc[k] += bilinear_view(p, nu, nv, u, v) * w;
+        } else {
+            const float* p = proj + (size_t)i * nu * nv;
+#pragma unroll
+            for (int k = 0; k < kOpBpZ; ++k) {
+                if (z0 + k >= g.nz) break;
+                float Z, un, vn, rd;
+                bool ok = project(k, Z, un, vn, rd);
+                const float u = un * rd, v = vn * rd;
+                const float w = col.weight(c, ivz, scale, Z, u, v, ok);
+                if (!ok) continue;
+                acc[k] += bilinear_view(p, nu, nv, u, v) * w;
+            }
         }
     }
 #pragma unroll
@@ -1050,6 +1140,24 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
         float* dst = volume + ((size_t)(z0 + k) * g.ny + y) * g.nx + x;
         *dst = accumulate ? *dst + acc[k] : acc[k];
     }
+}
+
+// Paired guarded copy of `count` views: entry (row r, column c) holds pixels
+// (r, c) and (r + 1, c), for rows and columns from -kViewGuard up to one guard
+// past the last (and a further column, read with the last guard), zero
+// outside the detector.
+__global__ void __launch_bounds__(256)
+pair_views_kernel(const float* __restrict__ proj, float2* __restrict__ out, int nu, int nv)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int pitch = nu + 2 * kViewGuard + 1;
+    if (e >= pitch) return;
+    const int c = e - kViewGuard, r = int(blockIdx.y) - kViewGuard;
+    const float* p = proj + size_t(blockIdx.z) * nu * nv;
+    const bool in = c >= 0 && c < nu;
+    const float a = in && r >= 0 && r < nv ? p[size_t(r) * nu + c] : 0.f;
+    const float b = in && r + 1 >= 0 && r + 1 < nv ? p[size_t(r + 1) * nu + c] : 0.f;
+    out[(size_t(blockIdx.z) * gridDim.y + blockIdx.y) * pitch + e] = make_float2(a, b);
 }
 
 }  // namespace
@@ -1155,18 +1263,32 @@ void launch_siddon_adjoint(const SiddonAdjointLaunch& p, hipStream_t s)
     YK_HIP(hipGetLastError());
 }
 
-void launch_fdk_operator_bp(const OpBpLaunch& p, hipStream_t s)
+size_t paired_view_floats(int nu, int nv) { return size_t(nv + 2 * kViewGuard) * (nu + 2 * kViewGuard + 1) * 2; }
+
+namespace {
+
+template <int MODE>
+void launch_op(const OpBpLaunch& p, hipStream_t s)
 {
     dim3 block(256), grid((p.vol.nx + 15) / 16, (p.vol.ny + 15) / 16, (p.vol.nz + kOpBpZ - 1) / kOpBpZ);
-    if (p.mode == kOpMatched)
-        hipLaunchKernelGGL(fdk_operator_bp_kernel<kOpMatched>, grid, block, 0, s, p.proj, p.volume, p.views,
-            p.vol, p.nu, p.nv, p.count, p.scale, p.accumulate);
-    else if (p.mode == kOpJosephVoxel)
-        hipLaunchKernelGGL(fdk_operator_bp_kernel<kOpJosephVoxel>, grid, block, 0, s, p.proj, p.volume, p.views,
-            p.vol, p.nu, p.nv, p.count, p.scale, p.accumulate);
-    else
-        hipLaunchKernelGGL(fdk_operator_bp_kernel<kOpFdk>, grid, block, 0, s, p.proj, p.volume, p.views, p.vol,
-            p.nu, p.nv, p.count, p.scale, p.accumulate);
+    auto k = !p.paired ? fdk_operator_bp_kernel<MODE, false, false>
+        : p.front      ? fdk_operator_bp_kernel<MODE, true, true>
+                       : fdk_operator_bp_kernel<MODE, true, false>;
+    hipLaunchKernelGGL(k, grid, block, 0, s, p.paired ? p.paired : p.proj, p.volume, p.views, p.vol, p.nu, p.nv, p.count,
+        p.scale, p.accumulate);
+}
+
+}  // namespace
+
+void launch_fdk_operator_bp(const OpBpLaunch& p, hipStream_t s)
+{
+    if (p.paired) {
+        dim3 grid((p.nu + 2 * kViewGuard + 1 + 255) / 256, p.nv + 2 * kViewGuard, p.count);
+        hipLaunchKernelGGL(pair_views_kernel, grid, dim3(256), 0, s, p.proj, reinterpret_cast<float2*>(p.paired), p.nu, p.nv);
+    }
+    if (p.mode == kOpMatched) launch_op<kOpMatched>(p, s);
+    else if (p.mode == kOpJosephVoxel) launch_op<kOpJosephVoxel>(p, s);
+    else launch_op<kOpFdk>(p, s);
     YK_HIP(hipGetLastError());
 }
 

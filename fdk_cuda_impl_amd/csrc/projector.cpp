@@ -19,6 +19,14 @@ void grow(DeviceArray<T>& a, size_t n)
     if (a.size() < n) a.resize(n);
 }
 
+// Samples (voxels x views) or views from which the operator-form
+// backprojections sample a paired copy of the views, and the voxels per pixel
+// below which the copy is most of the work: one view at 64^3 takes 8.7 us with
+// the copy and 6.4 without, two 8.5 and 9.1, four 10.0 and 15.4; one view at
+// 128^3 8.8 and 10.0, at 256^3 29 and 43; four views at 32^3 9.9 and 14.6.
+constexpr double kOpPairSamples = 1e6, kOpPairRatio = 0.5;
+constexpr int kOpPairViews = 3;
+
 // rays x main-axis slabs per voxel from which the Siddon projection makes its
 // volume copies: at 3 (one view of 512 x 384 at 256^3) the copies and the slab
 // kernel take 223 us against the walk's 316, at 6 304 against 429, at 24 411
@@ -178,6 +186,18 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
         o.l2[5] = float(dot(w.detV, w.detV));
         o.wbase = float(cf[i].wbase);
         o.inv_sdd_plane = std::fabs(der[i].sdd_plane) > 1e-12 ? float(1.0 / std::fabs(der[i].sdd_plane)) : 0.f;
+        // depth and FDK weight denominator (both affine) over the voxels and
+        // a run's overhang past the last slice
+        double least = 1e300;
+        for (int a = 0; a < 8; ++a) {
+            const double X = vol.ox + ((a & 1) ? (vol.nx - 1) * double(vol.vx) : 0.0);
+            const double Y = vol.oy + ((a & 2) ? (vol.ny - 1) * double(vol.vy) : 0.0);
+            const double Z = vol.oz + ((a & 4) ? (vol.nz + 7) * double(vol.vz) : 0.0);
+            const double* d = cf[i].cd;
+            least = std::min({ least, (d[0] * X + d[1] * Y + d[2] * Z + d[3]) / der[i].sdd_plane,
+                               1.0 - (w.src[0] * X + w.src[1] * Y + w.src[2] * Z) / (sod * sod) });
+        }
+        op_front.push_back(least > 1e-3);
         op_scale[i] = vox[0] * vox[1] * vox[2] / der[i].du / der[i].dv;
     }
     hipStream_t s = ctx->stream;
@@ -320,6 +340,30 @@ void yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
     }
 }
 
+// views per paired copy of the operator-form backprojections; 0: sample the
+// views themselves (few samples for the copy's launch and pass, sizes past its
+// grid or 24-bit row products, or no memory)
+int yk_projector::op_chunk(yk_projector& w, int count) const
+{
+    const size_t per_view = paired_view_floats(nu, nv);
+    const double samples = double(grid.nx) * grid.ny * grid.nz * count;
+    if ((samples < kOpPairSamples && count < kOpPairViews) || samples < kOpPairRatio * double(nu) * nv * count) return 0;
+    if (nv > 65000 || nu > 2000000 || per_view > (size_t(1) << 29)) return 0;
+    const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
+    if (w.d_paired_views.size() < per_view * chunk) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) return 0;
+        try {
+            grow(w.d_paired_views, per_view * chunk);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            return 0;
+        }
+    }
+    return chunk;
+}
+
 // Transposes of views of any orientation by the gather kernels, a chunk of
 // views' table at a time (at most 1 GiB); false when they do not apply: a view
 // outside their forms, rows past 32-bit offsets, or no memory for the table
@@ -403,16 +447,23 @@ void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, i
         p.accumulate = accumulate;
         launch_siddon_adjoint(p, s);
     } else if (kind == YK_BP_FDK || kind == YK_BP_FDK_PSEUDO_MATCHED || kind == YK_BP_JOSEPH_VOXEL) {
-        OpBpLaunch p{};
-        p.proj = d_proj;
-        p.volume = d_volume;
-        p.views = d_opviews.get() + first;
-        p.vol = vol;
-        p.nu = nu; p.nv = nv; p.count = count;
-        p.scale = float(op_scale[first]);
-        p.mode = kind == YK_BP_FDK_PSEUDO_MATCHED ? 1 : kind == YK_BP_JOSEPH_VOXEL ? 2 : 0;
-        p.accumulate = accumulate;
-        launch_fdk_operator_bp(p, s);
+        // a chunk of views (at most 1 GiB) at a time through the paired copy,
+        // or all of them without it
+        const int chunk = op_chunk(w, count);
+        for (int c0 = 0; c0 < count; c0 += chunk > 0 ? chunk : count) {
+            OpBpLaunch p{};
+            p.proj = d_proj + size_t(nu) * nv * c0;
+            p.volume = d_volume;
+            p.views = d_opviews.get() + first + c0;
+            p.vol = vol;
+            p.nu = nu; p.nv = nv; p.count = chunk > 0 ? std::min(chunk, count - c0) : count;
+            p.scale = float(op_scale[first]);
+            p.mode = kind == YK_BP_FDK_PSEUDO_MATCHED ? 1 : kind == YK_BP_JOSEPH_VOXEL ? 2 : 0;
+            p.accumulate = c0 > 0 ? 1 : accumulate;
+            p.front = std::all_of(op_front.begin() + first, op_front.begin() + first + count, [](char f) { return f != 0; });
+            p.paired = chunk > 0 ? w.d_paired_views.get() : nullptr;
+            launch_fdk_operator_bp(p, s);
+        }
     } else {
         fail(YK_ERR_UNSUPPORTED, "unknown back projector");
     }

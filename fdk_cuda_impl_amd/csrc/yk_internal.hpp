@@ -418,7 +418,10 @@ struct OpBpLaunch {
     float scale;                // vx vy vz / (du dv) of the first view (matched weight)
     int mode;                   // 0 FDK weight, 1 pseudo-matched, 2 voxel-driven Joseph
     int accumulate;
+    int front;                  // every voxel lies before every source, with regular weights (projector.cpp)
+    float* paired;              // scratch of count x paired_view_floats: sample a paired copy (null: the views)
 };
+size_t paired_view_floats(int nu, int nv);
 void launch_fdk_operator_bp(const OpBpLaunch& p, hipStream_t s);
 
 // vector helpers

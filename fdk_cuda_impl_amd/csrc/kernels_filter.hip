@@ -49,7 +49,8 @@ template <int C>
 __device__ __forceinline__ int slot(int i) { return i + C * (i >> 5); }
 
 // pad slots of the layout a pass of span ns writes, and of the one it reads
-constexpr int fft_out_pad(int ns) { return ns == 8 ? 4 : 1; }
+// (the last pass writes the layout that the crop and the first pass read)
+constexpr int fft_out_pad(int n, int ns) { return ns == 8 && n > 64 ? 4 : 1; }
 constexpr int fft_in_pad(int ns) { return ns == 64 ? 4 : 1; }
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
@@ -142,8 +143,8 @@ __device__ float2* fft_forward(float2* a, float2* b, const float2* tw, int n)
     return src;
 }
 
-// The same transform for a length known at compile time (n = NPT x the
-// workgroup size, every length of 512 and above): the pass sequence, spans
+// The same transform for a length known at compile time (64 to 4096), by the G
+// lanes of a group (`gl`: this lane's place in it): the pass sequence, spans
 // and lane loops are constants, so the index arithmetic folds to shifts and
 // masks, and the first pass (span 1, all twiddles 1) multiplies by nothing.
 // Every lane keeps the twiddles of its butterflies (and the filter weights
@@ -153,7 +154,7 @@ __device__ float2* fft_forward(float2* a, float2* b, const float2* tw, int n)
 constexpr int fft_radix(int n, int ns) { return ns * 8 <= n ? 8 : (ns * 4 <= n ? 4 : 2); }
 
 // butterflies per lane of a pass of radix r
-constexpr int fft_iters(int n, int r) { return (n / r + kFilterThreads - 1) / kFilterThreads; }
+constexpr int fft_iters(int n, int r, int g) { return (n / r + g - 1) / g; }
 
 // The span-8 pass has 8 distinct twiddle sets (k = lane mod 8): it reads
 // them from a 56-entry LDS copy (8 distinct addresses per read: no bank
@@ -163,17 +164,17 @@ constexpr int kTwLdsSpan = 8;
 constexpr bool fft_tw_in_regs(int ns) { return ns > kTwLdsSpan; }
 
 // registers of a pass's twiddles
-constexpr int fft_pass_tw_regs(int n, int ns)
+constexpr int fft_pass_tw_regs(int n, int ns, int g)
 {
-    return fft_tw_in_regs(ns) ? fft_iters(n, fft_radix(n, ns)) * (fft_radix(n, ns) - 1) : 0;
+    return fft_tw_in_regs(ns) ? fft_iters(n, fft_radix(n, ns), g) * (fft_radix(n, ns) - 1) : 0;
 }
 
 // twiddle registers of the passes from span ns on
-constexpr int fft_tw_regs(int n, int ns)
+constexpr int fft_tw_regs(int n, int ns, int g)
 {
     int total = 0;
     while (ns < n) {
-        total += fft_pass_tw_regs(n, ns);
+        total += fft_pass_tw_regs(n, ns, g);
         ns *= fft_radix(n, ns);
     }
     return total;
@@ -188,38 +189,38 @@ constexpr int fft_last_ns(int n)
 }
 
 // this lane's twiddles of the passes from span NS on (tw: that pass's block)
-template <int N, int NS>
-__device__ __forceinline__ void load_twiddles(float2* reg, const float2* __restrict__ tw)
+template <int N, int NS, int G>
+__device__ __forceinline__ void load_twiddles(float2* reg, const float2* __restrict__ tw, int gl)
 {
     if constexpr (NS < N) {
-        constexpr int R = fft_radix(N, NS), M = N / R, IT = fft_iters(N, R);
+        constexpr int R = fft_radix(N, NS), M = N / R, IT = fft_iters(N, R, G);
         if constexpr (fft_tw_in_regs(NS)) {
 #pragma unroll
             for (int it = 0; it < IT; ++it) {
-                const int j = it * kFilterThreads + int(threadIdx.x);
+                const int j = it * G + gl;
                 const int k = j & (NS - 1);
-                const bool live = M % kFilterThreads == 0 || j < M;
+                const bool live = M % G == 0 || j < M;
 #pragma unroll
                 for (int r = 1; r < R; ++r)
                     reg[it * (R - 1) + r - 1] = live ? tw[(r - 1) * NS + k] : make_float2(0.f, 0.f);
             }
         }
-        load_twiddles<N, NS * R>(reg + fft_pass_tw_regs(N, NS), tw + (R - 1) * NS);
+        load_twiddles<N, NS * R, G>(reg + fft_pass_tw_regs(N, NS, G), tw + (R - 1) * NS, gl);
     }
 }
 
 // this lane's filter weights of the last pass: bin idx + r NS of each of its
 // butterflies, w[b] for b <= N/2 and w[N - b] above (the response is even)
-template <int N>
-__device__ __forceinline__ void load_spectral_weights(float* reg, const float* __restrict__ weights)
+template <int N, int G>
+__device__ __forceinline__ void load_spectral_weights(float* reg, const float* __restrict__ weights, int gl)
 {
-    constexpr int NS = fft_last_ns(N), R = fft_radix(N, NS), M = N / R, IT = fft_iters(N, R);
+    constexpr int NS = fft_last_ns(N), R = fft_radix(N, NS), M = N / R, IT = fft_iters(N, R, G);
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int j = it * kFilterThreads + int(threadIdx.x);
+        const int j = it * G + gl;
         const int k = j & (NS - 1);
         const int idx = (j - k) * R + k;
-        const bool live = M % kFilterThreads == 0 || j < M;
+        const bool live = M % G == 0 || j < M;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int b = idx + r * NS;
@@ -228,15 +229,15 @@ __device__ __forceinline__ void load_spectral_weights(float* reg, const float* _
     }
 }
 
-template <int R, int N, int NS, bool SPECTRAL = false>
+template <int R, int N, int NS, int G, bool SPECTRAL = false>
 __device__ __forceinline__ void stockham_pass_ct(const float2* src, float2* dst, const float2* twr,
-    const float* wr, const float2* tw_lds)
+    const float* wr, const float2* tw_lds, int gl)
 {
     constexpr int m = N / R;
 #pragma unroll
-    for (int it = 0; it < fft_iters(N, R); ++it) {
-        const int j = it * kFilterThreads + int(threadIdx.x);
-        if (m % kFilterThreads != 0 && j >= m) break;
+    for (int it = 0; it < fft_iters(N, R, G); ++it) {
+        const int j = it * G + gl;
+        if (m % G != 0 && j >= m) break;
         const int k = j & (NS - 1);
         float2 v[R];
 #pragma unroll
@@ -257,25 +258,25 @@ __device__ __forceinline__ void stockham_pass_ct(const float2* src, float2* dst,
                 const float w = wr[it * R + r];
                 v[r] = make_float2(v[r].x * w, -v[r].y * w);
             }
-            dst[slot<fft_out_pad(NS)>(idx + r * NS)] = v[r];
+            dst[slot<fft_out_pad(N, NS)>(idx + r * NS)] = v[r];
         }
     }
 }
 
 // SPECTRAL: the last pass also applies the filter weights and conjugates.
 // twr: the twiddle registers of the passes of span NS and after.
-template <int N, int NS, bool SPECTRAL>
+template <int N, int NS, int G, bool SPECTRAL>
 __device__ __forceinline__ float2* fft_forward_ct(float2* src, float2* dst, const float2* twr, const float* wr,
-    const float2* tw_lds)
+    const float2* tw_lds, int gl)
 {
     if constexpr (NS >= N) {
-        (void)dst; (void)twr; (void)wr; (void)tw_lds;
+        (void)dst; (void)twr; (void)wr; (void)tw_lds; (void)gl;
         return src;
     } else {
         constexpr int R = fft_radix(N, NS);
-        stockham_pass_ct<R, N, NS, SPECTRAL && NS * R >= N>(src, dst, twr, wr, tw_lds);
+        stockham_pass_ct<R, N, NS, G, SPECTRAL && NS * R >= N>(src, dst, twr, wr, tw_lds, gl);
         __syncthreads();
-        return fft_forward_ct<N, NS * R, SPECTRAL>(dst, src, twr + fft_pass_tw_regs(N, NS), wr, tw_lds);
+        return fft_forward_ct<N, NS * R, G, SPECTRAL>(dst, src, twr + fft_pass_tw_regs(N, NS, G), wr, tw_lds, gl);
     }
 }
 
@@ -312,21 +313,31 @@ __device__ __forceinline__ float row_weight(const RowWeight& w, int u)
     return x;
 }
 
-// wave maxima of a and b (both rows of a pair at once), stored to red[wave]
-// for the reads after the next workgroup barrier (wave_max2_read)
-__device__ __forceinline__ void wave_max2_store(float a, float b, float2* red)
+// maxima of a and b over a group of G lanes: within a wave by shuffles; larger
+// groups (whole workgroups) combine their waves' through red, read after the
+// next workgroup barrier
+template <int G>
+__device__ __forceinline__ void group_max2(float& a, float& b, float2* red)
 {
-    for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+    for (int off = (G < 64 ? G : 64) / 2; off > 0; off >>= 1) {
         a = fmaxf(a, __shfl_xor(a, off, 64));
         b = fmaxf(b, __shfl_xor(b, off, 64));
     }
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(a, b);
+    if constexpr (G > 64) {
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(a, b);
+    }
 }
 
-__device__ __forceinline__ float2 wave_max2_read(const float2* red)
+template <int G>
+__device__ __forceinline__ float2 group_max2_read(float a, float b, const float2* red)
 {
-    float2 m = red[0];
-    for (int w = 1; w < kFilterThreads / 64; ++w) m = make_float2(fmaxf(m.x, red[w].x), fmaxf(m.y, red[w].y));
+    float2 m = make_float2(a, b);
+    if constexpr (G > 64) {
+        m = red[0];
+#pragma unroll
+        for (int w = 1; w < G / 64; ++w) m = make_float2(fmaxf(m.x, red[w].x), fmaxf(m.y, red[w].y));
+    }
     return m;
 }
 
@@ -344,11 +355,26 @@ __device__ __forceinline__ int row_scale_exp(float maxabs)
     return e - 14;
 }
 
+// Lanes and rows of the filter workgroups of padded length N (0: any length
+// below 64, at run time).  A compile-time length takes N / 8 lanes a row pair
+// (at most 256), one radix-8 butterfly each, so no lane idles in a pass:
+// lengths of 512 and below fit a wave, whose passes need no workgroup barrier,
+// and share it among 512 / N pairs.  With 256 lanes a pair whatever the length,
+// three quarters of them idled at N = 512: 180 x 256 rows of 256 pixels 85 -> 46
+// us (94 MB); N = 1024, 401 x 239 rows 221 -> 158 us (half storage 265 -> 205);
+// N = 256, 90 x 96 rows 23.5 -> 9.4 us.  N = 2048 and 4096 are unchanged.
+template <int N>
+struct FilterShape {
+    static constexpr int kLanes = N == 0 ? kFilterThreads : (N / 8 < 256 ? N / 8 : 256);
+    static constexpr int kThreads = kLanes < 64 ? 64 : kLanes;
+    static constexpr int kPairs = kThreads / kLanes;
+    static constexpr int kPerLane = N == 0 ? 1 : N / kLanes;
+};
+
 // LDS index of the rows entering and leaving the transforms: the layout the
-// first pass reads and the last pass writes (pad 1 per 32 for compile-time
-// lengths; every pass sequence of n >= 512 ends on a span other than 8)
-template <int NPT>
-__device__ __forceinline__ int io_slot(int i) { return NPT > 1 ? slot<1>(i) : pidx(i); }
+// first pass reads and the last pass writes
+template <int N>
+__device__ __forceinline__ int io_slot(int i) { return N > 0 ? slot<1>(i) : pidx(i); }
 
 template <int STORAGE>
 __device__ __forceinline__ void store_row(void* out, size_t base, int a, float val, float inv_scale)
@@ -375,56 +401,66 @@ __device__ __forceinline__ RowRef row_ref(int r, int nv)
     return x;
 }
 
-// Persistent workgroups: each filters row pairs p = blockIdx.x, + gridDim.x,
-// ... .  The raw texels of the next pair (NPT padded positions per lane and
-// row) are loaded into registers while the current pair is stored.  Lengths
-// of 512 and above run at most 128 registers per lane (4 workgroups per CU,
-// the LDS limit at n = 2048); 4096 at 2 workgroups per CU.
-template <int STORAGE, int NPT>
-__global__ void __launch_bounds__(kFilterThreads, NPT >= 16 ? 2 : 4)
+// Persistent workgroups: each filters kPairs row pairs at a time, from pair
+// blockIdx.x kPairs on.  The raw texels of the next pair (kPerLane padded
+// positions per lane and row) are loaded into registers while the current pair
+// is stored.  At most 128 registers per lane (four waves per SIMD, the LDS
+// limit at n = 2048), 4096 at two.
+template <int STORAGE, int N>
+__global__ void __launch_bounds__(FilterShape<N>::kThreads, N >= 4096 ? 2 : 4)
 fdk_filter_kernel(const float* __restrict__ proj, void* __restrict__ out,
     float* __restrict__ row_scales, const FilterView* __restrict__ views,
     const float* __restrict__ parker, const float* __restrict__ weights,
     const float2* __restrict__ tw, int nu, int nv, int rows, int n, float response_l1)
 {
+    using Shape = FilterShape<N>;
+    constexpr int G = Shape::kLanes, NPL = Shape::kPerLane;
     extern __shared__ float4 smem_raw[];
+    const int grp = Shape::kPairs > 1 ? int(threadIdx.x) / G : 0;
+    const int gl = Shape::kPairs > 1 ? int(threadIdx.x) % G : int(threadIdx.x);
     const int padded = pidx(n);
-    float2* bufa = reinterpret_cast<float2*>(smem_raw);
+    float2* bufa = reinterpret_cast<float2*>(smem_raw) + grp * 2 * padded;
     float2* bufb = bufa + padded;
     __shared__ float2 red[kFilterThreads / 64];
     // compile-time lengths: this lane's twiddles and last-pass filter
     // weights, loaded once (the pass-ordered table and the weights)
-    constexpr int NC = NPT > 1 ? NPT * kFilterThreads : 2;
-    float2 twr[NPT > 1 ? fft_tw_regs(NC, 1) : 1];
-    float wr[NPT > 1 ? fft_iters(NC, fft_radix(NC, fft_last_ns(NC))) * fft_radix(NC, fft_last_ns(NC)) : 1];
+    constexpr int NC = N > 0 ? N : 64;
+    constexpr int kTwRegs = fft_tw_regs(NC, 1, G), kLastR = fft_radix(NC, fft_last_ns(NC));
+    float2 twr[N > 0 && kTwRegs > 0 ? kTwRegs : 1];
+    float wr[N > 0 ? fft_iters(NC, kLastR, G) * kLastR : 1];
     __shared__ float2 tw_lds[7 * kTwLdsSpan];
-    if constexpr (NPT > 1) {
-        load_twiddles<NC, 1>(twr, tw);
-        load_spectral_weights<NC>(wr, weights);
+    if constexpr (N > 0) {
+        load_twiddles<NC, 1, G>(twr, tw, gl);
+        load_spectral_weights<NC, G>(wr, weights, gl);
         // the span-8 block of the pass-ordered table (after the 7 entries of span 1)
         if (threadIdx.x < 7 * kTwLdsSpan) tw_lds[threadIdx.x] = tw[7 + threadIdx.x];
         __syncthreads();
     }
 
     const int pairs = (rows + 1) / 2;
-    float xa[NPT], xb[NPT];
+    float xa[NPL], xb[NPL];
+    // a group past the last pair repeats it and stores nothing
     auto prefetch = [&](int p) {
+        p = Shape::kPairs > 1 ? min(p, pairs - 1) : p;
         const int ra = 2 * p, rb = ra + 1;
         const RowRef A = row_ref(ra, nv), B = row_ref(rb < rows ? rb : ra, nv);
         const int sa = views[A.view].start_u, sb = views[B.view].start_u;
         const float* pa = proj + ((size_t)A.view * nv + A.v) * nu;
         const float* pb = proj + ((size_t)B.view * nv + B.v) * nu;
 #pragma unroll
-        for (int e = 0; e < NPT; ++e) {
-            const int m = int(threadIdx.x) + e * kFilterThreads;
+        for (int e = 0; e < NPL; ++e) {
+            const int m = gl + e * G;
             const int ua = m - sa, ub = m - sb;
             xa[e] = (m < n && ua >= 0 && ua < nu) ? pa[ua] : 0.f;
             xb[e] = (m < n && rb < rows && ub >= 0 && ub < nu) ? pb[ub] : 0.f;
         }
     };
-    if (int(blockIdx.x) < pairs) prefetch(blockIdx.x);
+    const int stride = int(gridDim.x) * Shape::kPairs;
+    if (int(blockIdx.x) * Shape::kPairs < pairs) prefetch(int(blockIdx.x) * Shape::kPairs + grp);
 
-    for (int p = blockIdx.x; p < pairs; p += gridDim.x) {
+    for (int pb = int(blockIdx.x) * Shape::kPairs; pb < pairs; pb += stride) {
+        const bool live = Shape::kPairs == 1 || pb + grp < pairs;
+        const int p = Shape::kPairs > 1 ? min(pb + grp, pairs - 1) : pb;
         const int ra = 2 * p, rb = ra + 1;
         const bool has_b = rb < rows;
         const RowRef A = row_ref(ra, nv), B = row_ref(has_b ? rb : ra, nv);
@@ -432,31 +468,31 @@ fdk_filter_kernel(const float* __restrict__ proj, void* __restrict__ out,
         const FilterView fb = views[B.view];
         const RowWeight wta = row_weight_setup(fa, parker ? parker + (size_t)A.view * nu : nullptr, A.v);
         const RowWeight wtb = row_weight_setup(fb, parker ? parker + (size_t)B.view * nu : nullptr, B.v);
+        float ma = 0.f, mb = 0.f;
         // Y = conj(X W): the second forward transform then yields conj(IFFT(X W))
         float2* spec;
-        if constexpr (NPT >= 8) {
+        if constexpr (N > 0) {
             // The first radix-8 pass (span 1, no twiddles) reads elements
-            // j + r N/8, which for N/8 a multiple of the workgroup size are
+            // j + r N/8, which for N/8 a multiple of the group size are
             // this lane's own prefetched texels: weight them (cosine and
             // Parker) in registers and transform them straight into LDS.
-            constexpr int N = NPT * kFilterThreads, M = N / 8, S = M / kFilterThreads;
-            float2 wv[NPT];
+            constexpr int M = N / 8, S = M / G;
+            float2 wv[NPL];
 #pragma unroll
-            for (int e = 0; e < NPT; ++e) {
-                const int m = int(threadIdx.x) + e * kFilterThreads;
+            for (int e = 0; e < NPL; ++e) {
+                const int m = gl + e * G;
                 const int ua = m - fa.start_u, ub = m - fb.start_u;
                 const float wa = (ua >= 0 && ua < nu) ? row_weight(wta, ua) : 0.f;
                 const float wb = (has_b && ub >= 0 && ub < nu) ? row_weight(wtb, ub) : 0.f;
                 wv[e] = make_float2(xa[e] * wa, xb[e] * wb);
             }
             if constexpr (STORAGE != YK_F32) {
-                float ma = 0.f, mb = 0.f;
 #pragma unroll
-                for (int e = 0; e < NPT; ++e) {
+                for (int e = 0; e < NPL; ++e) {
                     ma = fmaxf(ma, fabsf(wv[e].x));
                     mb = fmaxf(mb, fabsf(wv[e].y));
                 }
-                wave_max2_store(ma, mb, red);
+                group_max2<G>(ma, mb, red);
             }
 #pragma unroll
             for (int t = 0; t < S; ++t) {
@@ -464,19 +500,18 @@ fdk_filter_kernel(const float* __restrict__ proj, void* __restrict__ out,
 #pragma unroll
                 for (int r = 0; r < 8; ++r) v[r] = wv[t + r * S];
                 dft<8>(v);
-                const int j = t * kFilterThreads + int(threadIdx.x);
+                const int j = t * G + gl;
 #pragma unroll
-                for (int r = 0; r < 8; ++r) bufb[slot<fft_out_pad(1)>(j * 8 + r)] = v[r];
+                for (int r = 0; r < 8; ++r) bufb[slot<fft_out_pad(N, 1)>(j * 8 + r)] = v[r];
             }
             __syncthreads();
             __builtin_amdgcn_s_setprio(0);
-            spec = fft_forward_ct<N, 8, true>(bufb, bufa, twr, wr, tw_lds);
+            spec = fft_forward_ct<N, 8, G, true>(bufb, bufa, twr, wr, tw_lds, gl);
         } else {
             // cosine (and Parker) weights on the way into LDS
-            float ma = 0.f, mb = 0.f;
 #pragma unroll
-            for (int e = 0; e < NPT; ++e) {
-                const int m = int(threadIdx.x) + e * kFilterThreads;
+            for (int e = 0; e < NPL; ++e) {
+                const int m = gl + e * G;
                 if (m < n) {
                     const int ua = m - fa.start_u, ub = m - fb.start_u;
                     const float wa = (ua >= 0 && ua < nu) ? row_weight(wta, ua) : 0.f;
@@ -484,40 +519,36 @@ fdk_filter_kernel(const float* __restrict__ proj, void* __restrict__ out,
                     const float2 x = make_float2(xa[e] * wa, xb[e] * wb);
                     ma = fmaxf(ma, fabsf(x.x));
                     mb = fmaxf(mb, fabsf(x.y));
-                    bufa[io_slot<NPT>(m)] = x;
+                    bufa[io_slot<N>(m)] = x;
                 }
             }
-            if constexpr (STORAGE != YK_F32) wave_max2_store(ma, mb, red);
+            if constexpr (STORAGE != YK_F32) group_max2<G>(ma, mb, red);
             __syncthreads();
             __builtin_amdgcn_s_setprio(0);
-            if constexpr (NPT > 1) {
-                spec = fft_forward_ct<NC, 1, true>(bufa, bufb, twr, wr, tw_lds);
-            } else {
-                spec = fft_forward(bufa, bufb, tw, n);
-                for (int k = threadIdx.x; k < n; k += kFilterThreads) {
-                    const float w = weights[k <= n / 2 ? k : n - k];
-                    const float2 x = spec[pidx(k)];
-                    spec[pidx(k)] = make_float2(x.x * w, -x.y * w);
-                }
-                __syncthreads();
+            spec = fft_forward(bufa, bufb, tw, n);
+            for (int k = threadIdx.x; k < n; k += kFilterThreads) {
+                const float w = weights[k <= n / 2 ? k : n - k];
+                const float2 x = spec[pidx(k)];
+                spec[pidx(k)] = make_float2(x.x * w, -x.y * w);
             }
+            __syncthreads();
         }
         float2* other = spec == bufa ? bufb : bufa;
         float2* res;
-        if constexpr (NPT > 1) res = fft_forward_ct<NC, 1, false>(spec, other, twr, nullptr, tw_lds);
+        if constexpr (N > 0) res = fft_forward_ct<N, 1, G, false>(spec, other, twr, nullptr, tw_lds, gl);
         else res = fft_forward(spec, other, tw, n);
 
         // crop: row a = Re(res), row b = -Im(res)
         float inv_a = 1.f, inv_b = 1.f;
         if constexpr (STORAGE != YK_F32) {
-            // red holds the wave maxima of the weighted inputs, stored before
-            // the first barrier of this pair's transforms
-            const float2 mx = wave_max2_read(red);
+            // the maxima of the weighted inputs, reduced before the first
+            // barrier of this pair's transforms
+            const float2 mx = group_max2_read<G>(ma, mb, red);
             const int ea = row_scale_exp(mx.x * response_l1), eb = row_scale_exp(mx.y * response_l1);
             const float sa = ldexpf(1.f, ea), sb = ldexpf(1.f, eb);
             inv_a = ldexpf(1.f, -ea);
             inv_b = ldexpf(1.f, -eb);
-            if (threadIdx.x == 0) {
+            if (gl == 0 && live) {
                 row_scales[ra] = sa;
                 if (has_b) row_scales[rb] = sb;
             }
@@ -532,14 +563,16 @@ fdk_filter_kernel(const float* __restrict__ proj, void* __restrict__ out,
         // transforms over those inside one: -6 % for the FP16 output at
         // n = 2048, -7 % for the FP32 output at n = 4096.
         __builtin_amdgcn_s_setprio(3);
-        if (p + int(gridDim.x) < pairs) prefetch(p + gridDim.x);
-        const size_t base_a = (size_t)ra * nu, base_b = (size_t)rb * nu;
-        for (int a = threadIdx.x; a < nu; a += kFilterThreads) {
-            const int ja = fa.start_u + a;
-            store_row<STORAGE>(out, base_a, a, (ja >= 0 && ja < n) ? res[io_slot<NPT>(ja)].x : 0.f, inv_a);
-            if (has_b) {
-                const int jb = fb.start_u + a;
-                store_row<STORAGE>(out, base_b, a, (jb >= 0 && jb < n) ? -res[io_slot<NPT>(jb)].y : 0.f, inv_b);
+        if (pb + stride < pairs) prefetch(pb + stride + grp);
+        if (live) {
+            const size_t base_a = (size_t)ra * nu, base_b = (size_t)rb * nu;
+            for (int a = gl; a < nu; a += G) {
+                const int ja = fa.start_u + a;
+                store_row<STORAGE>(out, base_a, a, (ja >= 0 && ja < n) ? res[io_slot<N>(ja)].x : 0.f, inv_a);
+                if (has_b) {
+                    const int jb = fb.start_u + a;
+                    store_row<STORAGE>(out, base_b, a, (jb >= 0 && jb < n) ? -res[io_slot<N>(jb)].y : 0.f, inv_b);
+                }
             }
         }
         // the next pair overwrites bufa, which the crop (res) may be
@@ -548,33 +581,42 @@ fdk_filter_kernel(const float* __restrict__ proj, void* __restrict__ out,
     __builtin_amdgcn_s_setprio(0);
 }
 
-template <int STORAGE, int NPT>
-void launch_npt(const FilterLaunch& p, int rows, size_t lds, hipStream_t s)
+template <int STORAGE, int N>
+void launch_length(const FilterLaunch& p, int rows, size_t lds, hipStream_t s)
 {
-    auto k = fdk_filter_kernel<STORAGE, NPT>;
+    using Shape = FilterShape<N>;
+    auto k = fdk_filter_kernel<STORAGE, N>;
+    lds *= Shape::kPairs;
     YK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
         int(lds)));
     int dev = 0, cus = 256;
     YK_HIP(hipGetDevice(&dev));
     YK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int per_cu = std::max(1, int((160 * 1024) / lds));
-    const int pairs = (rows + 1) / 2;
-    const int grid = std::max(1, std::min(pairs, cus * std::min(per_cu, 8)));
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kFilterThreads), lds, s, p.proj, p.out, p.row_scales, p.views,
+    // as many workgroups as fit a CU: by LDS, and by waves (sixteen of the
+    // compile-time lengths at 128 registers)
+    const int waves = N == 0 ? 8 : 16 * 64 / Shape::kThreads;
+    const int per_cu = std::max(1, std::min(int((160 * 1024) / lds), waves));
+    const int groups = ((rows + 1) / 2 + Shape::kPairs - 1) / Shape::kPairs;
+    const int grid = std::max(1, std::min(groups, cus * per_cu));
+    hipLaunchKernelGGL(k, dim3(grid), dim3(Shape::kThreads), lds, s, p.proj, p.out, p.row_scales, p.views,
         p.parker, p.weights, p.twiddles, p.nu, p.nv, rows, p.n, p.response_l1);
 }
 
 template <int STORAGE>
 void launch_storage(const FilterLaunch& p, int rows, size_t lds, hipStream_t s)
 {
-    const int npt = std::max(1, p.n / kFilterThreads);
-    switch (npt) {
-    case 1: launch_npt<STORAGE, 1>(p, rows, lds, s); break;
-    case 2: launch_npt<STORAGE, 2>(p, rows, lds, s); break;
-    case 4: launch_npt<STORAGE, 4>(p, rows, lds, s); break;
-    case 8: launch_npt<STORAGE, 8>(p, rows, lds, s); break;
-    case 16: launch_npt<STORAGE, 16>(p, rows, lds, s); break;
-    default: fail(YK_ERR_UNSUPPORTED, "padded row length outside the filter kernel's range");
+    switch (p.n) {
+    case 64: launch_length<STORAGE, 64>(p, rows, lds, s); break;
+    case 128: launch_length<STORAGE, 128>(p, rows, lds, s); break;
+    case 256: launch_length<STORAGE, 256>(p, rows, lds, s); break;
+    case 512: launch_length<STORAGE, 512>(p, rows, lds, s); break;
+    case 1024: launch_length<STORAGE, 1024>(p, rows, lds, s); break;
+    case 2048: launch_length<STORAGE, 2048>(p, rows, lds, s); break;
+    case 4096: launch_length<STORAGE, 4096>(p, rows, lds, s); break;
+    default:
+        if (p.n > 64) fail(YK_ERR_UNSUPPORTED, "padded row length outside the filter kernel's range");
+        launch_length<STORAGE, 0>(p, rows, lds, s);
+        break;
     }
 }
 

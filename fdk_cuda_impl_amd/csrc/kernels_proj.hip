@@ -141,7 +141,7 @@ __device__ __forceinline__ void finish_joseph(float* proj, int i, int nu, int nv
     *dst = accumulate ? *dst + out : out;
 }
 
-// Paired guarded volume copies of the Joseph projections.  A guarded copy
+// Paired guarded volume copies of the slab projections.  A guarded copy
 // has kJosephGuard zero planes on both sides of both minor axes; its paired
 // form stores, at entry (slice c, row r, column e), the two guarded values
 // of rows r and r + 1 in column e.  One 16-byte load at (c, r, e) then
@@ -154,119 +154,202 @@ constexpr int kJosephGuard = 2;
 typedef float float4u __attribute__((ext_vector_type(4), aligned(8)));
 
 // Joseph projection for separable views (main axis X or Y, detV along Z
-// only).  One wave per detector column (64 consecutive rays in v): a1, b1 and
-// hence f1 and its taps are the same for every lane, and the lanes' Z taps are
-// neighbouring entries of a paired Z-fastest copy (rows along y, columns
-// along z for X-main views; rows along x for Y-main views), so the gathers of
-// a sample touch a few cache lines per wave.  With the sample position
-// clamped to [-2, n] every tap lies in the copy, and a position outside
-// (-1, n) reads only zeros, so the kernel needs no per-sample range test (a
-// slice outside a lane's own range is outside (-1, n) on some minor axis).
-// A sample is one 16-byte load and three lerps; the first-minor weight and
-// tap row come from a per-wave LDS table built 64 slices at a time.  Sample
-// positions are those of joseph_fp_kernel (the same IEEE operations) and the
-// ray sum keeps its slice order.
-template <int CW>
-__global__ void __launch_bounds__(512)
-joseph_fp_sep_kernel(const float* __restrict__ vzx, const float* __restrict__ vzy,
+// only).  A wave takes one detector column u and 64 K of its rays in v.  a1,
+// b1 - hence f1, its weight and its two tap rows in a slice - are the same for
+// all of them, so per slice the wave interpolates the tap rows once, lanes
+// along z (two coalesced 16-byte loads of a Z-fastest copy a lane), leaves the
+// column in LDS, and each ray takes a linear sample of it, lanes along v.  A
+// sample is two LDS words and a few FP32 instructions where a bilinear gather
+// of 16 bytes took 16 cycles of the CU's vector memory pipe; the loads of the
+// next slice are in flight while a slice is sampled.
+// The copy has kJosephGuard zero planes on both sides of both minor axes, and
+// sample positions are clamped to [-2, n], so a position outside (-1, n) reads
+// only zeros and no sample is tested for range.
+// Bound: the vector memory pipe (two rows of the volume a column and slice;
+// without these loads 25 % less) with VALU issue close behind (without loads
+// and LDS reads 47 % less).  Six waves a SIMD hide the slice's chain: with
+// four 5 % slower, with eight the spills cost as much again.  Copies included,
+// with gathers -> here: 256^3 x 360 views of 512 x 384 9.2 -> 5.7 ms, 512^3 x
+// 90 of 1024 x 768 23.7 -> 15.0 ms, 128^3 x 12 of 256 x 192 69 -> 55 us.
+constexpr int kColumnChunk = 256;  // z a wave loads at a time, four a lane
+// values of a copy's row: whole 16-byte groups
+__host__ __device__ __forceinline__ int column_pitch(int nz) { return (nz + 2 * kJosephGuard + 3) & ~3; }
+
+constexpr int kColumnWaves = 8;
+// LDS floats of a wave: its column (and, split, its K rays a lane at the end)
+__host__ __device__ __forceinline__ int column_words(int nz, int k, bool split)
+{
+    return split && column_pitch(nz) < 64 * k ? 64 * k : column_pitch(nz);
+}
+
+template <int K, bool SPLIT>
+__global__ void __launch_bounds__(64 * kColumnWaves, 6)
+joseph_fp_column_kernel(const float* __restrict__ vzx, const float* __restrict__ vzy,
     float* __restrict__ proj, const ProjViewDev* __restrict__ views, VolumeGeom g,
     int nu, int nv, int count, int accumulate)
 {
-    // per wave, 64 slices at a time: the first-minor weight and the byte
-    // offset of its tap row (the same in every lane: a1, b1 are exact
-    // functions of the column u), built once per slice by one lane each and
-    // read back per sample by a broadcast LDS read
-    __shared__ uint2 tab[8][64];
-    const int wave = int(threadIdx.x >> 6), lane = int(threadIdx.x & 63);
-    // The eight waves take CW neighbouring detector columns of 8 / CW
-    // consecutive views: their rays nearly coincide, so the repeats of a tap
-    // row hit the CU's L1 (eight views measured 8 % faster than four at
-    // 512^3 x 720, sixteen 7 % slower than eight).  Column groups are remapped so that each XCD
-    // (workgroups go round-robin to the 8 XCDs; gridDim.x is a multiple of
-    // 8) sweeps a contiguous range of columns, whose neighbouring rays share
-    // tap rows in its L2.
-    const int group = int(blockIdx.x & 7u) * int(gridDim.x >> 3) + int(blockIdx.x >> 3);
-    const int u = group * CW + wave % CW;
-    const int v = blockIdx.y * 64 + lane;
-    const int i = int(blockIdx.z) * (8 / CW) + wave / CW;
-    if (u >= nu || i >= count) return;  // whole wave
-    const bool pix = v < nv;
+    // per wave, 64 slices at a time: x = weight of the second tap row, y =
+    // byte offset of the first row at the column's first z, z, w = tau and
+    // base of f = base + tau e, a ray's position from there (e: its z offset
+    // from the detector's middle row, the same in every slice); and the
+    // largest f, two less than the column's values
+    __shared__ float4 tab[kColumnWaves][64];
+    __shared__ float tab_top[kColumnWaves][64];
+    extern __shared__ float4 column_raw[];
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = int(threadIdx.x & 63);
+    // The waves of a workgroup take one column of consecutive views (their
+    // rays nearly coincide, so the repeats of a tap row hit the CU's L1) or,
+    // SPLIT, equal parts of the slices of one column of one view, added at the
+    // end: for calls of too few columns to fill the GPU.
+    // Columns are remapped so that each XCD (workgroups go round-robin to the
+    // 8 XCDs; gridDim.x is a multiple of 8) sweeps a contiguous range of them,
+    // whose neighbouring rays share tap rows in its L2.
+    const int u = int(blockIdx.x & 7u) * int(gridDim.x >> 3) + int(blockIdx.x >> 3);
+    const int v0 = int(blockIdx.y) * 64 * K;
+    const int waves = int(blockDim.x >> 6);
+    const int i = SPLIT ? int(blockIdx.z) : int(blockIdx.z) * waves + wave;
+    if (u >= nu || i >= count) return;  // whole wave, SPLIT: whole workgroup
+    const int words = column_words(g.nz, K, SPLIT);
+    float* const column = reinterpret_cast<float*>(column_raw) + wave * words;
     const ProjViewDev pv = views[i];
     const AxisInfo ax = axis_info(pv.axis, g);
-    const float* base = pv.axis == 0 ? vzx : vzy;
-    JRay r{};
-    int lo = 1, hi = 0;
-    if (pix && joseph_ray(pv, ax, u, v, r)) joseph_slice_range(r, ax, lo, hi);
-    int wlo = lo <= hi ? lo : 0x7fffffff, whi = lo <= hi ? hi : -1;
-    for (int off = 32; off > 0; off >>= 1) {
-        wlo = min(wlo, __shfl_xor(wlo, off, 64));
-        whi = max(whi, __shfl_xor(whi, off, 64));
+    const float s0 = pick(ax.p0, pv.src[0], pv.src[1], 0.f), s1 = pick(ax.p1, pv.src[0], pv.src[1], 0.f), s2 = pv.src[2];
+    const float dv2 = pv.detV[2], vmid = 0.5f * float(nv - 1);
+    const float h1 = 0.5f * float(ax.n1 - 1), h2 = 0.5f * float(ax.n2 - 1) + float(kJosephGuard);
+    // the column's offsets from the source (at the middle row)
+    const float d0 = (pick(ax.p0, pv.detS[0], pv.detS[1], 0.f) + float(u) * pick(ax.p0, pv.detU[0], pv.detU[1], 0.f)) - s0;
+    const float d1 = (pick(ax.p1, pv.detS[0], pv.detS[1], 0.f) + float(u) * pick(ax.p1, pv.detU[0], pv.detU[1], 0.f)) - s1;
+    const float d2 = (pv.detS[2] + float(u) * pv.detU[2] + vmid * dv2) - s2;
+    const float rd0 = d0 != 0.f ? 1.f / d0 : 0.f;
+    float e[K], acc[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        // rays past the last one repeat it and store nothing
+        e[k] = (float(min(v0 + 64 * k + lane, nv - 1)) - vmid) * dv2;
+        acc[k] = 0.f;
+    }
+    const float eF = (float(v0) - vmid) * dv2, eE = (float(min(v0 + 64 * K, nv) - 1) - vmid) * dv2;
+    // slices in which the column can lie inside (-1, n) on the first minor
+    // axis, with a slice of margin (z needs no range: outside reads zeros)
+    int wlo = 1, whi = 0;
+    if (d0 != 0.f) {
+        JRay r{};
+        r.a1 = d1 * rd0;
+        r.b1 = s1 - r.a1 * s0;
+        joseph_slice_range(r, ax, wlo, whi);
     }
     wlo = __builtin_amdgcn_readfirstlane(wlo);
     whi = __builtin_amdgcn_readfirstlane(whi);
-    // lane 0 (v = 64 blockIdx.y < nv) holds the column's a1, b1
-    const float a1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r.a1)));
-    const float b1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r.b1)));
-    const int p2 = ax.n2 + 2 * kJosephGuard;
-    const unsigned row_bytes = unsigned(p2) * 8u;
-    const size_t slice_bytes = size_t(ax.n1 + 2 * kJosephGuard - 1) * row_bytes;
-    const float f1max = float(ax.n1), f2max = float(ax.n2);
-    float acc = 0.f;
-    uint2* t = tab[wave];
+    if constexpr (SPLIT) {
+        const int part = (whi - wlo + waves) / waves;
+        wlo += wave * part;
+        whi = min(whi, wlo + part - 1);
+    }
+    const int p2 = column_pitch(ax.n2);
+    const size_t slice_bytes = size_t(ax.n1 + 2 * kJosephGuard) * p2 * 4u;
+    const float f1max = float(ax.n1), f2max = float(ax.n2 + kJosephGuard);
+    float4* const t = tab[wave];
+    float* const tt = tab_top[wave];
+    const char* sl = reinterpret_cast<const char*>(pv.axis == 0 ? vzx : vzy) + size_t(wlo) * slice_bytes;
+    float4 ra, rb;
+    // Issues the loads of a column of the slice at p (rows at byte offset o,
+    // which is a multiple of 16, top + 2 values): four values of either tap
+    // row a lane.
+    const float first = float(4 * lane - 2);
+    auto load = [&](const char* p, unsigned o, float top) {
+        if (first < top) {
+            const char* a = p + (o + unsigned(lane) * 16u);
+            ra = *reinterpret_cast<const float4*>(a);
+            rb = *reinterpret_cast<const float4*>(a + size_t(p2) * 4u);
+        }
+    };
+    auto lerp4 = [](float w, const float4& a, const float4& b) {
+        return make_float4(fmaf(w, b.x - a.x, a.x), fmaf(w, b.y - a.y, a.y), fmaf(w, b.z - a.z, a.z), fmaf(w, b.w - a.w, a.w));
+    };
     for (int c = wlo; c <= whi; c += 64) {
+        const int end = min(c + 63, whi);
+        int chunks;
         {
-            const int st = min(c + lane, whi);
-            float f1 = joseph_minor(a1, b1, joseph_c0(st, ax.n0), ax.n1);
-            f1 = __builtin_amdgcn_fmed3f(f1, -2.f, f1max);
-            const int j1 = int(floorf(f1)) + kJosephGuard;
-            t[lane] = make_uint2(__float_as_uint(__builtin_amdgcn_fractf(f1)), unsigned(j1) * row_bytes);
+            // the column's line in this slice: f = s + d (c0 - s0) / d0
+            const float c0 = joseph_c0(min(c + lane, end), ax.n0);
+            const float tau = (c0 - s0) * rd0;
+            const float f1 = __builtin_amdgcn_fmed3f(fmaf(d1, tau, s1) + h1, -2.f, f1max);
+            const float q = fmaf(d2, tau, s2);
+            const float fF = __builtin_amdgcn_fmed3f(fmaf(eF, tau, q + h2), 0.f, f2max);
+            const float fE = __builtin_amdgcn_fmed3f(fmaf(eE, tau, q + h2), 0.f, f2max);
+            // the rays' positions are monotonic in v up to rounding: one z to
+            // spare below the lower end, and above the upper end's second tap
+            // (from a whole 16-byte group on)
+            const int zlo = max(int(fminf(fF, fE)) - 1, 0) & ~3, zhi = min(int(fmaxf(fF, fE)) + 2, ax.n2 + 2 * kJosephGuard - 1);
+            const int row = int(floorf(f1)) + kJosephGuard;
+            t[lane] = make_float4(__builtin_amdgcn_fractf(f1), __uint_as_float(unsigned(row * p2 + zlo) * 4u), tau,
+                q + (h2 - float(zlo)));
+            tt[lane] = float(zhi - zlo - 1);
+            chunks = (zhi - zlo + kColumnChunk) / kColumnChunk;
+            for (int off = 32; off > 0; off >>= 1) chunks = max(chunks, __shfl_xor(chunks, off, 64));
+            chunks = __builtin_amdgcn_readfirstlane(chunks);
         }
         __builtin_amdgcn_wave_barrier();
-        const int cnt = min(64, whi - c + 1);
-        // the slice coordinate steps by exactly 1 (half-integers below 2^22);
-        // the slice base is wave-uniform
-        float c0 = joseph_c0(c, ax.n0);
-        const char* sl = reinterpret_cast<const char*>(base) + size_t(c) * slice_bytes;
-        int k = 0;
-        constexpr int kUnroll = 4;
-        for (; k + kUnroll <= cnt; k += kUnroll) {
-            float4u q[kUnroll];
-            float w1[kUnroll], w2[kUnroll];
-#pragma unroll
-            for (int j = 0; j < kUnroll; ++j) {
-                const uint2 e = t[k + j];
-                float f2 = joseph_minor(r.a2, r.b2, c0, ax.n2);
-                c0 += 1.f;
-                f2 = __builtin_amdgcn_fmed3f(f2, -2.f, f2max);
-                w1[j] = __uint_as_float(e.x);
-                w2[j] = __builtin_amdgcn_fractf(f2);
-                const unsigned o = e.y + unsigned(int(floorf(f2)) + kJosephGuard) * 8u;
-                q[j] = *reinterpret_cast<const float4u*>(sl + o);
+        // cur is sampled while nxt loads, and the entry after it is read
+        float4 cur = t[0], nxt = t[min(1, end - c)];
+        float ctop = tt[0], ntop = tt[min(1, end - c)];
+        load(sl, __float_as_uint(cur.y), ctop);
+        for (int s = c; s <= end; ++s) {
+            const float4 after = t[min(s + 2, end) - c];
+            const float atop = tt[min(s + 2, end) - c];
+            float4* const col4 = reinterpret_cast<float4*>(column);
+            if (first < ctop) col4[lane] = lerp4(cur.x, ra, rb);
+            if (chunks > 1) {  // a longer column: the rest, not loaded ahead
+                const char* p = sl + __float_as_uint(cur.y);
+                for (int z = kColumnChunk + 4 * lane; z < int(ctop) + 2; z += kColumnChunk)
+                    col4[z / 4] = lerp4(cur.x, *reinterpret_cast<const float4*>(p + size_t(z) * 4u),
+                                        *reinterpret_cast<const float4*>(p + (size_t(z) + p2) * 4u));
+            }
+            if (s < whi) {
+                // (past the table's last slice: reloads it, unused)
+                load(sl + (s < end ? slice_bytes : 0), __float_as_uint(nxt.y), ntop);
                 sl += slice_bytes;
             }
+            __builtin_amdgcn_wave_barrier();
+            float lo[K], hi[K], w[K];
 #pragma unroll
-            for (int j = 0; j < kUnroll; ++j) {
-                const float a = fmaf(w2[j], q[j].z - q[j].x, q[j].x);
-                const float b = fmaf(w2[j], q[j].w - q[j].y, q[j].y);
-                acc += fmaf(w1[j], b - a, a);
+            for (int k = 0; k < K; ++k) {
+                const float f = __builtin_amdgcn_fmed3f(fmaf(e[k], cur.z, cur.w), 0.f, ctop);
+                const float* p = column + int(f);
+                lo[k] = p[0];
+                hi[k] = p[1];
+                w[k] = __builtin_amdgcn_fractf(f);
             }
+#pragma unroll
+            for (int k = 0; k < K; ++k) acc[k] += fmaf(w[k], hi[k] - lo[k], lo[k]);
+            __builtin_amdgcn_wave_barrier();
+            cur = nxt;
+            ctop = ntop;
+            nxt = after;
+            ntop = atop;
         }
-        for (; k < cnt; ++k) {
-            const uint2 e = t[k];
-            float f2 = joseph_minor(r.a2, r.b2, c0, ax.n2);
-            c0 += 1.f;
-            f2 = __builtin_amdgcn_fmed3f(f2, -2.f, f2max);
-            const float w2 = __builtin_amdgcn_fractf(f2);
-            const unsigned o = e.y + unsigned(int(floorf(f2)) + kJosephGuard) * 8u;
-            const float4u q = *reinterpret_cast<const float4u*>(sl + o);
-            sl += slice_bytes;
-            const float a = fmaf(w2, q.z - q.x, q.x);
-            const float b = fmaf(w2, q.w - q.y, q.y);
-            acc += fmaf(__uint_as_float(e.x), b - a, a);
-        }
-        __builtin_amdgcn_wave_barrier();
     }
-    finish_joseph(proj, i, nu, nv, u, v, pix, lo <= hi, acc, r.L, accumulate);
+    auto store = [&](int v, float sum) {
+        if (v >= nv) return;
+        JRay r{};
+        const float out = joseph_ray(pv, ax, u, v, r) ? sum * r.L : 0.f;
+        float* dst = proj + ((size_t)i * nv + v) * nu + u;
+        *dst = accumulate ? *dst + out : out;
+    };
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) column[64 * k + lane] = acc[k];
+        __syncthreads();
+        const float* const sums = reinterpret_cast<const float*>(column_raw);
+        for (int k = wave; k < K; k += waves) {
+            float sum = 0.f;
+            for (int w = 0; w < waves; ++w) sum += sums[w * words + 64 * k + lane];
+            store(v0 + 64 * k + lane, sum);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) store(v0 + 64 * k + lane, acc[k]);
+    }
 }
 
 // Joseph projection for any X- or Y-main view set (tilted detectors, lifted
@@ -274,7 +357,7 @@ joseph_fp_sep_kernel(const float* __restrict__ vzx, const float* __restrict__ vz
 // rows along z and columns along the first minor axis (y for X-main, x for
 // Y-main views).  A slice of the main axis is one contiguous slab (scalar
 // base, 32-bit lane offsets); the lanes of a wave (consecutive u) read
-// neighbouring columns.  As in joseph_fp_sep_kernel the sample position is
+// neighbouring columns.  As in joseph_fp_column_kernel the sample position is
 // clamped to [-2, n], positions outside (-1, n) read only zeros, and a
 // sample is one 16-byte load and three lerps.
 __global__ void __launch_bounds__(512)
@@ -360,56 +443,30 @@ joseph_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy
 // OS-SART sweep of 10 subsets at 128 x 128 x 100 x 120 views went from 5.66 to
 // 5.32 ms, a SART sweep at 64 x 60 x 48 x 40 views from 2.09 to 1.92 ms).
 //
-// paired separable copy, X-main: [x][row y + guard][column z + guard];
-// blockIdx.z is the row, 32 x 32 (x, column) tiles of the two source rows
-// through LDS
-__global__ void pair_zfast_x_kernel(const float* __restrict__ in, float2* __restrict__ out,
-    int nx, int ny, int nz)
+// Z-fastest copy for joseph_fp_column_kernel: [slice][row + guard][z + guard],
+// slices along x and rows along y (X-main), or the reverse; 32 x 32 tiles
+// through LDS, blockIdx.z is y + guard (X-main) or y (Y-main), blockIdx.x tiles x
+// (with its guards for Y-main rows).
+template <bool XMAIN>
+__global__ void zfast_copy_kernel(const float* __restrict__ in, float* __restrict__ out, int nx, int ny, int nz)
 {
-    __shared__ float tile[2][32][33];
-    const int r = blockIdx.z;
-    const int x0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
-    const size_t rows = size_t(ny) + 2 * kJosephGuard - 1, cols = size_t(nz) + 2 * kJosephGuard;
+    __shared__ float tile[32][33];
+    const int x0 = int(blockIdx.x) * 32 - (XMAIN ? 0 : kJosephGuard), e0 = blockIdx.y * 32;
+    const int y = int(blockIdx.z) - (XMAIN ? kJosephGuard : 0);
+    const int cols = column_pitch(nz);
     for (int k = threadIdx.y; k < 32; k += 8) {
-        const int z = e0 + k - kJosephGuard, x = x0 + threadIdx.x;
-        const bool in_xz = x < nx && z >= 0 && z < nz;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int y = r + h - kJosephGuard;
-            tile[h][k][threadIdx.x] = in_xz && y >= 0 && y < ny ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
-        }
+        const int z = e0 + k - kJosephGuard, x = x0 + int(threadIdx.x);
+        const bool in_range = x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz;
+        tile[k][threadIdx.x] = in_range ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
     }
     __syncthreads();
     for (int k = threadIdx.y; k < 32; k += 8) {
         const int x = x0 + k, e = e0 + threadIdx.x;
-        if (x < nx && e < int(cols))
-            out[(size_t(x) * rows + r) * cols + e] = make_float2(tile[0][threadIdx.x][k], tile[1][threadIdx.x][k]);
-    }
-}
-
-// paired separable copy, Y-main: [y][row x + guard][column z + guard];
-// blockIdx.z is y, 32 x 32 (row, column) tiles (33 source columns of x)
-// through LDS
-__global__ void pair_zfast_y_kernel(const float* __restrict__ in, float2* __restrict__ out,
-    int nx, int ny, int nz)
-{
-    __shared__ float tile[32][34];
-    const int y = blockIdx.z;
-    const int r0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
-    const int rows = nx + 2 * kJosephGuard - 1;
-    const size_t cols = size_t(nz) + 2 * kJosephGuard;
-    for (int k = threadIdx.y; k < 32; k += 8) {
-        const int z = e0 + k - kJosephGuard;
-        for (int t = threadIdx.x; t < 33; t += 32) {
-            const int x = r0 + t - kJosephGuard;
-            tile[k][t] = z >= 0 && z < nz && x >= 0 && x < nx ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
-        }
-    }
-    __syncthreads();
-    for (int k = threadIdx.y; k < 32; k += 8) {
-        const int r = r0 + k, e = e0 + threadIdx.x;
-        if (r < rows && e < int(cols))
-            out[(size_t(y) * rows + r) * cols + e] = make_float2(tile[threadIdx.x][k], tile[threadIdx.x][k + 1]);
+        const bool in_range = XMAIN ? x < nx : x < nx + kJosephGuard;
+        if (!in_range || e >= cols) continue;
+        const size_t slice = XMAIN ? x : y, row = XMAIN ? y + kJosephGuard : x + kJosephGuard;
+        const size_t rows = size_t(XMAIN ? ny : nx) + 2 * kJosephGuard;
+        out[(slice * rows + row) * cols + e] = tile[threadIdx.x][k];
     }
 }
 
@@ -1170,37 +1227,92 @@ void launch_joseph_fp(const JosephLaunch& p, hipStream_t s)
     YK_HIP(hipGetLastError());
 }
 
-void launch_joseph_fp_sep(const JosephSepFpLaunch& p, hipStream_t s)
+size_t joseph_column_size(int nx, int ny, int nz, bool x_main)
 {
-    constexpr int kCols = 1;  // columns per workgroup (the other waves: further views)
-    const int groups = (p.nu + kCols - 1) / kCols;
-    dim3 block(512), grid((groups + 7) / 8 * 8, (p.nv + 63) / 64, (p.count + 8 / kCols - 1) / (8 / kCols));
-    hipLaunchKernelGGL(joseph_fp_sep_kernel<kCols>, grid, block, 0, s, p.vol_zx, p.vol_zy, p.proj, p.views,
-        p.vol, p.nu, p.nv, p.count, p.accumulate);
+    const size_t g = 2 * kJosephGuard;
+    return size_t(x_main ? nx : ny) * ((x_main ? ny : nx) + g) * column_pitch(nz);
+}
+
+void launch_joseph_column_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s)
+{
+    const int g = 2 * kJosephGuard;
+    dim3 block(32, 8);
+    if (x_main)
+        hipLaunchKernelGGL(zfast_copy_kernel<true>, dim3((nx + 31) / 32, (column_pitch(nz) + 31) / 32, ny + g), block, 0, s, in, out,
+            nx, ny, nz);
+    else
+        hipLaunchKernelGGL(zfast_copy_kernel<false>, dim3((nx + g + 31) / 32, (column_pitch(nz) + 31) / 32, ny), block, 0, s, in, out,
+            nx, ny, nz);
     YK_HIP(hipGetLastError());
 }
 
-size_t joseph_pair_size(int nx, int ny, int nz, bool x_main, bool slab)
+namespace {
+
+template <int K, bool SPLIT>
+void launch_column_kernel(const JosephSepFpLaunch& p, hipStream_t s)
+{
+    const size_t column = size_t(column_words(p.vol.nz, K, SPLIT)) * sizeof(float);
+    // the waves' columns in 32 KiB; a longer column has a workgroup to itself
+    const int waves = column <= 4096 ? kColumnWaves : column <= 8192 ? 4 : column <= 16384 ? 2 : 1;
+    if (waves == 1)
+        YK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(joseph_fp_column_kernel<K, SPLIT>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, int(column)));
+    dim3 grid((p.nu + 7) / 8 * 8, (p.nv + 64 * K - 1) / (64 * K), SPLIT ? p.count : (p.count + waves - 1) / waves);
+    hipLaunchKernelGGL((joseph_fp_column_kernel<K, SPLIT>), grid, dim3(64 * waves), column * waves, s, p.vol_zx, p.vol_zy,
+        p.proj, p.views, p.vol, p.nu, p.nv, p.count, p.accumulate);
+}
+
+// A call with fewer columns than this (2 waves for each of 1024 SIMDs) takes
+// SPLIT.  256^3 / 512 x 384, whole calls, not split and split: 1 view 163 and
+// 65 us, 4 views 172 and 125 us, 8192 columns and more: the same to 10 % slower.
+constexpr size_t kSplitColumns = 4096;
+
+template <int K>
+void launch_column(const JosephSepFpLaunch& p, hipStream_t s)
+{
+    const size_t columns = size_t(p.nu) * p.count * ((p.nv + 64 * K - 1) / (64 * K));
+    if (columns < kSplitColumns && p.count <= 65535) launch_column_kernel<K, true>(p, s);
+    else launch_column_kernel<K, false>(p, s);
+}
+
+}  // namespace
+
+bool joseph_column_fits(const VolumeGeom& g)
+{
+    const size_t g2 = 2 * kJosephGuard;
+    const size_t slice = (size_t(std::max(g.nx, g.ny)) + g2) * size_t(column_pitch(g.nz)) * sizeof(float);
+    // 144 KB of LDS for the longest column, 32-bit byte offsets in a slice
+    return g.nz <= 36000 && slice < (size_t(1) << 32);
+}
+
+void launch_joseph_fp_column(const JosephSepFpLaunch& p, hipStream_t s)
+{
+    // rays a lane: the detector's rows in equal blocks of at most 384
+    const int lanes = (p.nv + 63) / 64, blocks = (lanes + 5) / 6;
+    switch ((lanes + blocks - 1) / blocks) {
+    case 1: launch_column<1>(p, s); break;
+    case 2: launch_column<2>(p, s); break;
+    case 3: launch_column<3>(p, s); break;
+    case 4: launch_column<4>(p, s); break;
+    case 5: launch_column<5>(p, s); break;
+    default: launch_column<6>(p, s); break;
+    }
+    YK_HIP(hipGetLastError());
+}
+
+size_t joseph_pair_size(int nx, int ny, int nz, bool x_main)
 {
     const size_t n0 = size_t(x_main ? nx : ny), n1 = size_t(x_main ? ny : nx);
     const size_t g = 2 * kJosephGuard;
-    // rows x columns of float2 per slice: (n_r + 2g - 1) x (n_e + 2g)
-    const size_t rows = (slab ? size_t(nz) : n1) + g - 1, cols = (slab ? n1 : size_t(nz)) + g;
-    return n0 * rows * cols * 2;
+    // rows x columns of float2 per slice: (nz + 2g - 1) x (n1 + 2g)
+    return n0 * (size_t(nz) + g - 1) * (n1 + g) * 2;
 }
 
-void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, bool slab,
-    hipStream_t s)
+void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s)
 {
     float2* o = reinterpret_cast<float2*>(out);
     const int g = 2 * kJosephGuard;
-    if (!slab && x_main) {
-        dim3 block(32, 8), grid((nx + 31) / 32, (nz + g + 31) / 32, ny + g - 1);
-        hipLaunchKernelGGL(pair_zfast_x_kernel, grid, block, 0, s, in, o, nx, ny, nz);
-    } else if (!slab) {
-        dim3 block(32, 8), grid((nx + g - 1 + 31) / 32, (nz + g + 31) / 32, ny);
-        hipLaunchKernelGGL(pair_zfast_y_kernel, grid, block, 0, s, in, o, nx, ny, nz);
-    } else if (x_main) {
+    if (x_main) {
         dim3 block(32, 8), grid((nx + 31) / 32, (ny + g + 31) / 32, nz + g - 1);
         hipLaunchKernelGGL(pair_slab_x_kernel, grid, block, 0, s, in, o, nx, ny, nz);
     } else {

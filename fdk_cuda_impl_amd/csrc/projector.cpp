@@ -216,8 +216,8 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
 // slab offsets cannot hold the sizes
 bool yk_projector::siddon_copies(yk_projector& w, const float* d_volume)
 {
-    const size_t need_x = joseph_pair_size(grid.nx, grid.ny, grid.nz, true, true);
-    const size_t need_y = joseph_pair_size(grid.nx, grid.ny, grid.nz, false, true);
+    const size_t need_x = joseph_pair_size(grid.nx, grid.ny, grid.nz, true);
+    const size_t need_y = joseph_pair_size(grid.nx, grid.ny, grid.nz, false);
     if (nv > 65535 || need_x / grid.nx > (size_t(1) << 29) || need_y / grid.ny > (size_t(1) << 29)) return false;
     if (w.d_vol_zx.size() < need_x || w.d_vol_zy.size() < need_y || !w.d_flag.get()) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -232,8 +232,8 @@ bool yk_projector::siddon_copies(yk_projector& w, const float* d_volume)
         (void)hipGetLastError();  // the failed allocation's, not the call's
         return false;
     }
-    launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, true, ctx->stream);
-    launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, true, ctx->stream);
+    launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, ctx->stream);
+    launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, ctx->stream);
     return true;
 }
 
@@ -252,15 +252,15 @@ void yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
         any_y = any_y || ax == 1;
         any_z = any_z || ax == 2;
     }
-    if (kind == YK_FP_JOSEPH && all_sep) {
-        // paired guarded copies (every call rewrites the copy it reads)
+    if (kind == YK_FP_JOSEPH && all_sep && joseph_column_fits(vol)) {
+        // guarded copies (every call rewrites the copy it reads)
         if (any_x) {
-            grow(w.d_vol_zx, joseph_pair_size(grid.nx, grid.ny, grid.nz, true, false));
-            launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, false, s);
+            grow(w.d_vol_zx, joseph_column_size(grid.nx, grid.ny, grid.nz, true));
+            launch_joseph_column_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, s);
         }
         if (any_y) {
-            grow(w.d_vol_zy, joseph_pair_size(grid.nx, grid.ny, grid.nz, false, false));
-            launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, false, s);
+            grow(w.d_vol_zy, joseph_column_size(grid.nx, grid.ny, grid.nz, false));
+            launch_joseph_column_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, s);
         }
         JosephSepFpLaunch p{};
         p.vol_zx = any_x ? w.d_vol_zx.get() : nullptr;
@@ -270,16 +270,16 @@ void yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
         p.vol = vol;
         p.nu = nu; p.nv = nv; p.count = count;
         p.accumulate = accumulate;
-        launch_joseph_fp_sep(p, s);
+        launch_joseph_fp_column(p, s);
     } else if (kind == YK_FP_JOSEPH && !any_z) {
         // X/Y-main views of any orientation: paired slab copies
         if (any_x) {
-            grow(w.d_vol_zx, joseph_pair_size(grid.nx, grid.ny, grid.nz, true, true));
-            launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, true, s);
+            grow(w.d_vol_zx, joseph_pair_size(grid.nx, grid.ny, grid.nz, true));
+            launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, s);
         }
         if (any_y) {
-            grow(w.d_vol_zy, joseph_pair_size(grid.nx, grid.ny, grid.nz, false, true));
-            launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, true, s);
+            grow(w.d_vol_zy, joseph_pair_size(grid.nx, grid.ny, grid.nz, false));
+            launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, s);
         }
         JosephSepFpLaunch p{};
         p.vol_zx = any_x ? w.d_vol_zx.get() : nullptr;

@@ -291,29 +291,31 @@ struct JosephLaunch {
 void launch_joseph_fp(const JosephLaunch& p, hipStream_t s);
 void launch_transpose_xy(const float* in, float* out, int nx, int ny, int nz, hipStream_t s);
 
-// Joseph projection for separable views from paired Z-fastest volume copies
+// Joseph projection from volume copies
 struct JosephSepFpLaunch {
-    const float* vol_zx;        // paired copy for X-main views (may be null if none)
-    const float* vol_zy;        // paired copy for Y-main views (may be null if none)
+    const float* vol_zx;        // copy for X-main views (may be null if none)
+    const float* vol_zy;        // copy for Y-main views (may be null if none)
     float* proj;                // [count][nv][nu]
     const ProjViewDev* views;   // device, `count`
     VolumeGeom vol;
     int nu, nv, count;
     int accumulate;
 };
-void launch_joseph_fp_sep(const JosephSepFpLaunch& p, hipStream_t s);
-// Joseph projection of X- or Y-main views of any orientation from paired
-// slab copies (vol_zx / vol_zy made by launch_joseph_pair_copy with slab)
+// separable views, from Z-fastest copies (launch_joseph_column_copy) of
+// joseph_column_size floats: [slice][row][z] of a [z][y][x] volume, slices along
+// the main axis (x for x_main, else y), rows along the other of x and y, two
+// zero planes before and after each minor axis
+void launch_joseph_fp_column(const JosephSepFpLaunch& p, hipStream_t s);
+void launch_joseph_column_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s);
+size_t joseph_column_size(int nx, int ny, int nz, bool x_main);
+bool joseph_column_fits(const VolumeGeom& g);
+// X- or Y-main views of any orientation, from paired slab copies
+// (launch_joseph_pair_copy) of joseph_pair_size floats: float2 entries (value
+// at z row r, value at row r + 1), columns along the other of x and y, two
+// zero planes around both minor axes
 void launch_joseph_fp_slab(const JosephSepFpLaunch& p, hipStream_t s);
-// Paired guarded copy of a [z][y][x] volume for the Joseph projections:
-// float2 entries (value at row r, value at row r + 1) of a copy with two zero
-// planes before and after each minor axis.  Separable layout (slab false):
-// slices along the main axis (x for x_main, else y), rows along the other
-// of x and y, columns along z.  Slab layout: rows along z, columns along the
-// other of x and y.  joseph_pair_size floats.
-void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, bool slab,
-    hipStream_t s);
-size_t joseph_pair_size(int nx, int ny, int nz, bool x_main, bool slab);
+void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s);
+size_t joseph_pair_size(int nx, int ny, int nz, bool x_main);
 
 struct JosephAdjointLaunch {
     const float* proj;          // [count][nv][nu]

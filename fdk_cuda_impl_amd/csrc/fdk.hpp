@@ -1,6 +1,8 @@
 // FDK plan and projection-operator plan (library-owned handles of the C ABI).
 #pragma once
 
+#include <atomic>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -85,9 +87,43 @@ private:
     yk::DeviceArray<float> d_parts;    // the parts' volumes of a small volume's backprojection
 };
 
+struct yk_projector;
+
+// What the algebraic solvers keep with their projector between calls: work
+// arrays, and operators made from its views (their contents hold nothing from
+// one call for the next).  Arrays beyond kKeep bytes in all are given back
+// when the call ends; the rest with the projector.
+struct SolverScratch {
+    static constexpr size_t kKeep = size_t(1) << 30;
+    yk::DeviceArray<float> arrays[9];
+    std::unique_ptr<yk_projector> subset_op;  // the views in the order of subset_op_units interleaved subsets
+    int subset_op_units = 0;
+    std::unique_ptr<yk_projector> coarse;     // the TIGRE row weights' support volume
+    // array k with room for n floats; another call's array of any size is kept
+    // if it has
+    float* array(int k, size_t n);
+    ~SolverScratch();
+    std::atomic<bool> busy{ false };
+};
+
+// One solver call: takes the projector's scratch, or scratch of its own where
+// another call (a progress callback's, another thread's) holds that; its queued
+// work is done and the large arrays are freed when it ends, by return or by error
+struct SolverCall {
+    SolverScratch own;
+    SolverScratch& ws;
+    hipStream_t stream;
+    SolverCall(SolverScratch& kept, hipStream_t s) : ws(kept.busy.exchange(true) ? own : kept), stream(s) {}
+    SolverCall(const SolverCall&) = delete;
+    SolverCall& operator=(const SolverCall&) = delete;
+    ~SolverCall();
+};
+
 struct yk_projector {
+    // `segments`: counts of consecutive views that are view sequences of their
+    // own for the operator-form backprojections (null: all views are one)
     yk_projector(yk_ctx* ctx, const yk_view* views, int n_views, int nu, int nv,
-        const yk_volume_grid& grid, float scan_range);
+        const yk_volume_grid& grid, float scan_range, const std::vector<int>* segments = nullptr);
 
     void project(int kind, const float* d_volume, float* d_proj, int first, int count, int accumulate);
     void backproject(int kind, const float* d_proj, float* d_volume, int first, int count, int accumulate);
@@ -126,6 +162,7 @@ struct yk_projector {
     yk::DeviceArray<yk::OpBpViewDev> d_opviews;  // operator-form FDK backprojection records
     std::vector<char> op_front;        // per view: no voxel needs the operator backprojections' sample tests
     std::vector<double> op_scale;      // per first view: vx vy vz / (du dv)
+    SolverScratch solver;
 };
 
 // unified SIRT / SART / OS-SART (algebraic.cpp); throws through fail()

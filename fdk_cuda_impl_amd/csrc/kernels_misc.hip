@@ -65,14 +65,17 @@ __global__ void fill_kernel(float* __restrict__ y, float v, size_t n)
 // (src/Reconstruction/Iterative/Common/kernels/YkIterKernels.cu:202-256, 299-318):
 //   mode 0: res = row > eps ? (b - res) / row : 0     (residual, divide_launch)
 //   mode 1: res = (b - res) * row                     (residual, multiply_launch)
+// for `count` views of res and row, view_n values each; b's lie b_stride views apart
 __global__ void algebraic_residual_kernel(float* __restrict__ res, const float* __restrict__ b,
-    const float* __restrict__ row, float eps, int mode, size_t n)
+    const float* __restrict__ row, float eps, int mode, size_t view_n, int count, int b_stride)
 {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float r = b[i] - res[i];
-        const float w = row[i];
-        res[i] = mode == 0 ? (w > eps ? r / w : 0.f) : r * w;
-    }
+    for (int j = blockIdx.y; j < count; j += gridDim.y)
+        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < view_n; i += (size_t)gridDim.x * blockDim.x) {
+            const size_t k = size_t(j) * view_n + i;
+            const float r = b[size_t(j) * b_stride * view_n + i] - res[k];
+            const float w = row[k];
+            res[k] = mode == 0 ? (w > eps ? r / w : 0.f) : r * w;
+        }
 }
 
 // x += lambda bp / (col + eps), then the optional bounds (update_launch,
@@ -222,10 +225,11 @@ void launch_fill(float* y, float v, size_t n, hipStream_t s)
     YK_HIP(hipGetLastError());
 }
 
-void algebraic_residual(float* res, const float* b, const float* row, float eps, int mode, size_t n,
-    hipStream_t s)
+void algebraic_residual(float* res, const float* b, const float* row, float eps, int mode, size_t view_n, int count,
+    int b_stride, hipStream_t s)
 {
-    hipLaunchKernelGGL(algebraic_residual_kernel, dim3(grid_for(n)), dim3(256), 0, s, res, b, row, eps, mode, n);
+    hipLaunchKernelGGL(algebraic_residual_kernel, dim3(grid_for(view_n), count < 65535 ? count : 65535), dim3(256), 0, s, res, b,
+        row, eps, mode, view_n, count, b_stride);
     YK_HIP(hipGetLastError());
 }
 

@@ -92,7 +92,7 @@ void depth_range(const yk_view& w, const double map[12], const VolumeGeom& g, do
 }  // namespace
 
 yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
-    const yk_volume_grid& g, float range)
+    const yk_volume_grid& g, float range, const std::vector<int>* segments)
     : ctx(c), nu(nu_), nv(nv_), n_views(n), grid(g),
       scan_range(range > 0.f ? double(range) : 6.28318530717958647692)
 {
@@ -156,8 +156,22 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
     // view sequence, like FdkAffineCoeff in .../FDK/kernels/YkFDKBpPrecompute.cu:14-138)
     std::vector<DerivedD> der;
     std::vector<CoeffD> cf;
-    derive_geometry(views, nu, nv, scan_range, der);
-    fdk_coefficients(views, der, cf);
+    if (segments) {
+        std::vector<DerivedD> sder;
+        std::vector<CoeffD> scf;
+        auto at = views.begin();
+        for (int k : *segments) {
+            const std::vector<yk_view> part(at, at + k);
+            derive_geometry(part, nu, nv, scan_range, sder);
+            fdk_coefficients(part, sder, scf);
+            der.insert(der.end(), sder.begin(), sder.end());
+            cf.insert(cf.end(), scf.begin(), scf.end());
+            at += k;
+        }
+    } else {
+        derive_geometry(views, nu, nv, scan_range, der);
+        fdk_coefficients(views, der, cf);
+    }
     std::vector<OpBpViewDev> ov(n);
     op_scale.resize(n);
     for (int i = 0; i < n; ++i) {
@@ -208,6 +222,24 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
     d_c32.upload(c32.data(), c32.size(), s);
     d_partials.resize(1024);
     YK_HIP(hipStreamSynchronize(s));
+}
+
+float* SolverScratch::array(int k, size_t n)
+{
+    grow(arrays[k], n);
+    return arrays[k].get();
+}
+
+SolverScratch::~SolverScratch() = default;
+
+SolverCall::~SolverCall()
+{
+    (void)hipStreamSynchronize(stream);
+    size_t bytes = 0;
+    for (const auto& a : ws.arrays) bytes += a.size() * sizeof(float);
+    if (bytes > SolverScratch::kKeep)
+        for (auto& a : ws.arrays) a.reset();
+    ws.busy = false;
 }
 
 // both paired slab copies of the volume into w's scratch; false when the walk,

@@ -433,9 +433,10 @@ void launch_axpy(float* y, const float* x, float a, size_t n, hipStream_t s);   
 void launch_xpby(float* y, const float* x, float b, size_t n, hipStream_t s);        // y = x + b y
 void launch_scale_copy(float* y, const float* x, float a, size_t n, hipStream_t s);  // y = a x
 void launch_fill(float* y, float v, size_t n, hipStream_t s);
-// algebraic steps: mode 0 res = row > eps ? (b - res) / row : 0, mode 1 res = (b - res) row
-void algebraic_residual(float* res, const float* b, const float* row, float eps, int mode, size_t n,
-    hipStream_t s);
+// algebraic steps: mode 0 res = row > eps ? (b - res) / row : 0, mode 1 res = (b - res) row,
+// over `count` views of view_n values; consecutive views of b lie b_stride views apart
+void algebraic_residual(float* res, const float* b, const float* row, float eps, int mode, size_t view_n, int count,
+    int b_stride, hipStream_t s);
 // x += lambda bp / (col + eps), then optional bounds
 void algebraic_update(float* x, const float* bp, const float* col, float lambda, float eps, int use_min,
     float lo, int use_max, float hi, size_t n, hipStream_t s);

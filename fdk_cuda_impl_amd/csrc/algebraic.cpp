@@ -179,8 +179,17 @@ void run_algebraic(yk_projector* p, const yk_algebraic_desc& d, const float* d_b
         (tigre ? ws.coarse.get() : op)->project(d.forward_kind, ones_vol, rows + size_t(at) * view_n, at,
             std::min(kRowViews, na - at), 0);
     if (tigre) weight_prepare(rows, 0.5f * min_voxel, 1, size_t(na) * view_n, s);
-    if (cache_cols)
-        for (int k = 0; k < nu_units; ++k) column_weights(units[k], cols + size_t(k) * nx);
+    if (cache_cols) {
+        // one launch for all units where their operators are one sequence
+        std::vector<int> counts;
+        bool one_op = true;
+        for (const Unit& u : units) {
+            counts.push_back(u.count);
+            one_op = one_op && u.op == op;
+        }
+        if (!one_op || !op->column_weights(d.back_kind, ones_proj, counts, mask_cols, cols))
+            for (int k = 0; k < nu_units; ++k) column_weights(units[k], cols + size_t(k) * nx);
+    }
 
     // convergence monitor state (AlgebraicReconstructorEx::prepareConvergence_, :236-256)
     const bool watch_residual = d.relative_residual_tolerance > 0.f || d.relative_improvement_tolerance > 0.f;
@@ -209,8 +218,17 @@ void run_algebraic(yk_projector* p, const yk_algebraic_desc& d, const float* d_b
             u.op->project(d.forward_kind, d_x, fwd, u.op_first, u.count, 0);
             algebraic_residual(fwd, d_b + size_t(u.b_first) * view_n, rows + size_t(u.first) * view_n, d.epsilon, tigre ? 1 : 0,
                 view_n, u.count, u.b_stride, s);
-            u.op->backproject(d.back_kind, fwd, bp, u.op_first, u.count, 0);
-            algebraic_update(d_x, bp, c, lambda, d.epsilon, d.use_min, d.min_value, d.use_max, d.max_value, nx, s);
+            OpBpStore update{};
+            update.x = d_x;
+            update.col = c;
+            update.lambda = lambda;
+            update.eps = d.epsilon;
+            update.use_min = d.use_min; update.use_max = d.use_max;
+            update.lo = d.min_value; update.hi = d.max_value;
+            if (!u.op->backproject_update(d.back_kind, fwd, u.op_first, u.count, update)) {
+                u.op->backproject(d.back_kind, fwd, bp, u.op_first, u.count, 0);
+                algebraic_update(d_x, bp, c, lambda, d.epsilon, d.use_min, d.min_value, d.use_max, d.max_value, nx, s);
+            }
             lambda *= per_update;
         }
         if (tigre) lambda *= d.relaxation_reduction;

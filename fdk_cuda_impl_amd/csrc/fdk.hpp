@@ -127,9 +127,12 @@ struct yk_projector {
 
     void project(int kind, const float* d_volume, float* d_proj, int first, int count, int accumulate);
     void backproject(int kind, const float* d_proj, float* d_volume, int first, int count, int accumulate);
+    bool backproject_update(int kind, const float* d_proj, int first, int count, const yk::OpBpStore& update);
+    bool column_weights(int kind, const float* d_ones, const std::vector<int>& counts, bool mask, float* out);
+    yk::OpBpLaunch op_launch(int kind, const float* d_proj, int first, int count) const;
     double dot(const float* a, const float* b, size_t n);
     bool siddon_copies(yk_projector& w, const float* d_volume);
-    int op_chunk(yk_projector& w, int count) const;
+    int op_chunk(yk_projector& w, int count, bool one_view = false) const;
     bool gather_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
         int accumulate);
 
@@ -160,6 +163,7 @@ struct yk_projector {
     yk::DeviceArray<int> d_flag;       // one word: see siddon_value_check_kernel
     yk::DeviceArray<double> d_partials;
     yk::DeviceArray<yk::OpBpViewDev> d_opviews;  // operator-form FDK backprojection records
+    yk::DeviceArray<yk::OpBpUnit> d_op_units;  // units of a column_weights launch
     std::vector<char> op_front;        // per view: no voxel needs the operator backprojections' sample tests
     std::vector<double> op_scale;      // per first view: vx vy vz / (du dv)
     SolverScratch solver;

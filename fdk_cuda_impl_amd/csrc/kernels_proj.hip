@@ -1025,6 +1025,7 @@ siddon_adjoint_kernel(const float* __restrict__ proj, float* __restrict__ volume
 //   of X - src through one voxel along its main axis m = argmax |d_k / v_k|
 //   (ties X, then Y): v_m |d| / |d_m|.
 constexpr int kOpBpZ = 8;
+constexpr int kOpBpShortZ = 2;
 constexpr int kViewGuard = 1;  // zero pixels around a paired view
 enum OpBpMode { kOpFdk = 0, kOpMatched = 1, kOpJosephVoxel = 2 };
 
@@ -1107,22 +1108,38 @@ struct OpColumn {
 // gather a sample.  256^3 x 360 views of 512 x 384, four taps -> paired: FDK
 // 10.2 -> 4.4 ms, pseudo-matched 11.4 -> 6.1, voxel-driven Joseph 11.1 -> 5.9,
 // the copy included.
+// A launch serves one unit of views or, with `units`, a volume for each of
+// several; view_step 0 gives every view the first one's pixels: the column
+// weights of all subsets of a solver are one launch, and its update is made by
+// the store (SART at 64 x 60 x 48 x 40 single views 1.26 -> 0.80 ms, OS-SART of
+// 10 subsets at 128 x 128 x 100 x 120 views 1.86 -> 1.65 ms).
 constexpr int kOpBatch = 4;
-template <int MODE, bool PAIRED, bool FRONT>
+template <int MODE, bool PAIRED, bool FRONT, int ZR>
 __global__ void __launch_bounds__(256)
 fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volume,
     const OpBpViewDev* __restrict__ views, VolumeGeom g, int nu, int nv, int count, float scale,
-    int accumulate)
+    int view_step, const OpBpUnit* __restrict__ units, int z_blocks, OpBpStore st)
 {
     const int x = blockIdx.x * 16 + int(threadIdx.x % 16);
     const int y = blockIdx.y * 16 + int(threadIdx.x / 16);
-    const int z0 = blockIdx.z * kOpBpZ;
+    int z_block = int(blockIdx.z);
+    if (units) {
+        const int k = z_block / z_blocks;
+        z_block -= k * z_blocks;
+        const OpBpUnit unit = units[k];
+        views += unit.first;
+        count = unit.count;
+        scale = unit.scale;
+        volume += (size_t)k * g.nz * g.ny * g.nx;
+    }
+    const int z0 = z_block * ZR;
     if (x >= g.nx || y >= g.ny) return;
     const float X = g.ox + x * g.vx, Y = g.oy + y * g.vy;
-    const float Za = g.oz + z0 * g.vz, Zb = g.oz + (z0 + kOpBpZ - 1) * g.vz;
-    float acc[kOpBpZ];
+    const float Za = g.oz + z0 * g.vz, Zb = g.oz + (z0 + ZR - 1) * g.vz;
+    constexpr int kBatch = ZR < kOpBatch ? ZR : kOpBatch;
+    float acc[ZR];
 #pragma unroll
-    for (int k = 0; k < kOpBpZ; ++k) acc[k] = 0.f;
+    for (int k = 0; k < ZR; ++k) acc[k] = 0.f;
     const float ivz = 1.f / g.vz;
     const int pitch = nu + 2 * kViewGuard + 1, rows = nv + 2 * kViewGuard;
 #pragma unroll 1
@@ -1147,16 +1164,16 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
             return den >= 1e-8f;
         };
         if constexpr (PAIRED) {
-            const char* p = reinterpret_cast<const char*>(proj) + size_t(i) * rows * pitch * 8u;
+            const char* p = reinterpret_cast<const char*>(proj) + size_t(i * view_step) * rows * pitch * 8u;
             const float umax = float(nu + 1), vmax = float(nv + 1);
             const unsigned row_bytes = unsigned(pitch) * 8u;
 #pragma unroll
-            for (int k0 = 0; k0 < kOpBpZ; k0 += kOpBatch) {
-                float4u q[kOpBatch];
-                float a[kOpBatch], b[kOpBatch], w[kOpBatch];
-                bool on[kOpBatch];
+            for (int k0 = 0; k0 < ZR; k0 += kBatch) {
+                float4u q[kBatch];
+                float a[kBatch], b[kBatch], w[kBatch];
+                bool on[kBatch];
 #pragma unroll
-                for (int k = 0; k < kOpBatch; ++k) {
+                for (int k = 0; k < kBatch; ++k) {
                     float Z, un, vn, rd;
                     on[k] = project(k0 + k, Z, un, vn, rd);
                     w[k] = col.weight(c, ivz, scale, Z, un * rd, vn * rd, on[k]);
@@ -1169,7 +1186,7 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
                     q[k] = *reinterpret_cast<const float4u*>(p + (__umul24(unsigned(int(v)), row_bytes) + unsigned(int(u)) * 8u));
                 }
 #pragma unroll
-                for (int k = 0; k < kOpBatch; ++k) {
+                for (int k = 0; k < kBatch; ++k) {
                     // q: (row, col), (row + 1, col), (row, col + 1), (row + 1, col + 1)
                     const float a0 = 1.f - a[k], b0 = 1.f - b[k];
                     const float s = fmaf(b[k], fmaf(a[k], q[k].w, a0 * q[k].y), b0 * fmaf(a[k], q[k].z, a0 * q[k].x));
@@ -1178,9 +1195,9 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
                 }
             }
         } else {
-            const float* p = proj + (size_t)i * nu * nv;
+            const float* p = proj + (size_t)(i * view_step) * nu * nv;
 #pragma unroll
-            for (int k = 0; k < kOpBpZ; ++k) {
+            for (int k = 0; k < ZR; ++k) {
                 if (z0 + k >= g.nz) break;
                 float Z, un, vn, rd;
                 bool ok = project(k, Z, un, vn, rd);
@@ -1192,10 +1209,19 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
         }
     }
 #pragma unroll
-    for (int k = 0; k < kOpBpZ; ++k) {
+    for (int k = 0; k < ZR; ++k) {
         if (z0 + k >= g.nz) break;
-        float* dst = volume + ((size_t)(z0 + k) * g.ny + y) * g.nx + x;
-        *dst = accumulate ? *dst + acc[k] : acc[k];
+        const size_t at = ((size_t)(z0 + k) * g.ny + y) * g.nx + x;
+        if (st.mode == OpBpStore::kUpdate) {
+            float v = st.x[at] + st.lambda * acc[k] / (st.col[at] + st.eps);
+            if (st.use_min && v < st.lo) v = st.lo;
+            if (st.use_max && v > st.hi) v = st.hi;
+            st.x[at] = v;
+        } else if (st.mode == OpBpStore::kWeight) {
+            volume[at] = acc[k] <= 0.f ? 1e30f : acc[k];
+        } else {
+            volume[at] = st.mode == OpBpStore::kAdd ? volume[at] + acc[k] : acc[k];
+        }
     }
 }
 
@@ -1379,15 +1405,32 @@ size_t paired_view_floats(int nu, int nv) { return size_t(nv + 2 * kViewGuard) *
 
 namespace {
 
+// Workgroups of kOpBpZ slices from which a launch takes them; below, a lane runs
+// 2 slices in four times the workgroups, else the GPU is not filled.  Whole
+// calls of voxel-driven Joseph, 8 and 2 slices: 60 views at 32^3 116 and 52 us,
+// 64^3 120 and 58, 96^3 137 and 107, 128^3 (1024 workgroups) 199 and 202, 160^3
+// 311 and 347; one view at 64^3 19.0 and 16.4, at 256^3 43 and 48.
+constexpr long kOpWideBlocks = 1024;
+
+template <int MODE, int ZR>
+void launch_op_run(const OpBpLaunch& p, hipStream_t s)
+{
+    const int z_blocks = (p.vol.nz + ZR - 1) / ZR;
+    dim3 block(256), grid((p.vol.nx + 15) / 16, (p.vol.ny + 15) / 16, z_blocks * (p.units ? p.n_units : 1));
+    auto k = !p.paired ? fdk_operator_bp_kernel<MODE, false, false, ZR>
+        : p.front      ? fdk_operator_bp_kernel<MODE, true, true, ZR>
+                       : fdk_operator_bp_kernel<MODE, true, false, ZR>;
+    hipLaunchKernelGGL(k, grid, block, 0, s, p.paired ? p.paired : p.proj, p.volume, p.views, p.vol, p.nu, p.nv, p.count,
+        p.scale, p.one_view ? 0 : 1, p.units, z_blocks, p.store);
+}
+
 template <int MODE>
 void launch_op(const OpBpLaunch& p, hipStream_t s)
 {
-    dim3 block(256), grid((p.vol.nx + 15) / 16, (p.vol.ny + 15) / 16, (p.vol.nz + kOpBpZ - 1) / kOpBpZ);
-    auto k = !p.paired ? fdk_operator_bp_kernel<MODE, false, false>
-        : p.front      ? fdk_operator_bp_kernel<MODE, true, true>
-                       : fdk_operator_bp_kernel<MODE, true, false>;
-    hipLaunchKernelGGL(k, grid, block, 0, s, p.paired ? p.paired : p.proj, p.volume, p.views, p.vol, p.nu, p.nv, p.count,
-        p.scale, p.accumulate);
+    const long wide = long((p.vol.nx + 15) / 16) * ((p.vol.ny + 15) / 16) * ((p.vol.nz + kOpBpZ - 1) / kOpBpZ) *
+        (p.units ? p.n_units : 1);
+    if (wide >= kOpWideBlocks) launch_op_run<MODE, kOpBpZ>(p, s);
+    else launch_op_run<MODE, kOpBpShortZ>(p, s);
 }
 
 }  // namespace
@@ -1395,7 +1438,7 @@ void launch_op(const OpBpLaunch& p, hipStream_t s)
 void launch_fdk_operator_bp(const OpBpLaunch& p, hipStream_t s)
 {
     if (p.paired) {
-        dim3 grid((p.nu + 2 * kViewGuard + 1 + 255) / 256, p.nv + 2 * kViewGuard, p.count);
+        dim3 grid((p.nu + 2 * kViewGuard + 1 + 255) / 256, p.nv + 2 * kViewGuard, p.one_view ? 1 : p.count);
         hipLaunchKernelGGL(pair_views_kernel, grid, dim3(256), 0, s, p.proj, reinterpret_cast<float2*>(p.paired), p.nu, p.nv);
     }
     if (p.mode == kOpMatched) launch_op<kOpMatched>(p, s);

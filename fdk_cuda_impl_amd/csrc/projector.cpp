@@ -35,6 +35,13 @@ constexpr int kOpPairViews = 3;
 // cross.
 constexpr double kSiddonSlabRatio = 1.0;
 
+bool operator_form(int kind)
+{
+    return kind == YK_BP_FDK || kind == YK_BP_FDK_PSEUDO_MATCHED || kind == YK_BP_JOSEPH_VOXEL;
+}
+
+int op_mode(int kind) { return kind == YK_BP_FDK_PSEUDO_MATCHED ? 1 : kind == YK_BP_JOSEPH_VOXEL ? 2 : 0; }
+
 // record of the gather transposes of a view whose main axis is X or Y, from
 // the forward kernel's voxel-normalized floats and the projective map of world
 // points
@@ -372,16 +379,19 @@ void yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
     }
 }
 
-// views per paired copy of the operator-form backprojections; 0: sample the
+// views per paired copy of the operator-form backprojections (one_view: the
+// copy holds one view, which serves all `count`); 0: sample the
 // views themselves (few samples for the copy's launch and pass, sizes past its
 // grid or 24-bit row products, or no memory)
-int yk_projector::op_chunk(yk_projector& w, int count) const
+int yk_projector::op_chunk(yk_projector& w, int count, bool one_view) const
 {
     const size_t per_view = paired_view_floats(nu, nv);
     const double samples = double(grid.nx) * grid.ny * grid.nz * count;
-    if ((samples < kOpPairSamples && count < kOpPairViews) || samples < kOpPairRatio * double(nu) * nv * count) return 0;
+    const double copied = double(nu) * nv * (one_view ? 1 : count);
+    if ((samples < kOpPairSamples && count < kOpPairViews) || samples < kOpPairRatio * copied) return 0;
     if (nv > 65000 || nu > 2000000 || per_view > (size_t(1) << 29)) return 0;
-    const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
+    const int chunk = one_view ? 1
+        : int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
     if (w.d_paired_views.size() < per_view * chunk) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
@@ -478,27 +488,83 @@ void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, i
         p.nu = nu; p.nv = nv; p.count = count;
         p.accumulate = accumulate;
         launch_siddon_adjoint(p, s);
-    } else if (kind == YK_BP_FDK || kind == YK_BP_FDK_PSEUDO_MATCHED || kind == YK_BP_JOSEPH_VOXEL) {
+    } else if (operator_form(kind)) {
         // a chunk of views (at most 1 GiB) at a time through the paired copy,
         // or all of them without it
         const int chunk = op_chunk(w, count);
         for (int c0 = 0; c0 < count; c0 += chunk > 0 ? chunk : count) {
-            OpBpLaunch p{};
-            p.proj = d_proj + size_t(nu) * nv * c0;
-            p.volume = d_volume;
-            p.views = d_opviews.get() + first + c0;
-            p.vol = vol;
-            p.nu = nu; p.nv = nv; p.count = chunk > 0 ? std::min(chunk, count - c0) : count;
+            OpBpLaunch p = op_launch(kind, d_proj + size_t(nu) * nv * c0, first + c0, chunk > 0 ? std::min(chunk, count - c0) : count);
             p.scale = float(op_scale[first]);
-            p.mode = kind == YK_BP_FDK_PSEUDO_MATCHED ? 1 : kind == YK_BP_JOSEPH_VOXEL ? 2 : 0;
-            p.accumulate = c0 > 0 ? 1 : accumulate;
-            p.front = std::all_of(op_front.begin() + first, op_front.begin() + first + count, [](char f) { return f != 0; });
+            p.volume = d_volume;
+            p.store.mode = c0 > 0 || accumulate ? OpBpStore::kAdd : OpBpStore::kSet;
             p.paired = chunk > 0 ? w.d_paired_views.get() : nullptr;
             launch_fdk_operator_bp(p, s);
         }
     } else {
         fail(YK_ERR_UNSUPPORTED, "unknown back projector");
     }
+}
+
+// x += lambda B y / (col + eps), bounded, in the backprojection's own store;
+// false when the back model has no such store or takes several launches
+bool yk_projector::backproject_update(int kind, const float* d_proj, int first, int count, const OpBpStore& update)
+{
+    if (!operator_form(kind)) return false;
+    yk_projector& w = scratch_owner ? *scratch_owner : *this;
+    const int chunk = op_chunk(w, count);
+    if (chunk > 0 && chunk < count) return false;
+    OpBpLaunch p = op_launch(kind, d_proj, first, count);
+    p.store = update;
+    p.store.mode = OpBpStore::kUpdate;
+    p.paired = chunk > 0 ? w.d_paired_views.get() : nullptr;
+    launch_fdk_operator_bp(p, ctx->stream);
+    return true;
+}
+
+// the backprojections of a view of ones by consecutive units of `counts` views
+// from the first on, a volume each in `out`; false when the back model has no
+// launch for several units
+bool yk_projector::column_weights(int kind, const float* d_ones, const std::vector<int>& counts, bool mask, float* out)
+{
+    if (!operator_form(kind)) return false;
+    yk_projector& w = scratch_owner ? *scratch_owner : *this;
+    std::vector<OpBpUnit> units;
+    int at = 0;
+    for (int k : counts) {
+        units.push_back(OpBpUnit{ at, k, float(op_scale[at]), 0 });
+        at += k;
+    }
+    hipStream_t s = ctx->stream;
+    if (w.d_op_units.size() < units.size()) w.d_op_units.resize(units.size());
+    YK_HIP(hipMemcpyAsync(w.d_op_units.get(), units.data(), units.size() * sizeof(OpBpUnit), hipMemcpyHostToDevice, s));
+    OpBpLaunch p = op_launch(kind, d_ones, 0, n_views);
+    p.store.mode = mask ? OpBpStore::kWeight : OpBpStore::kSet;
+    p.one_view = 1;
+    p.paired = op_chunk(w, n_views, true) > 0 ? w.d_paired_views.get() : nullptr;
+    // (at most 65535 workgroups along z of a launch)
+    const size_t per = std::max<size_t>(1, size_t(60000) / size_t(grid.nz));
+    for (size_t k = 0; k < units.size(); k += per) {
+        p.units = w.d_op_units.get() + k;
+        p.n_units = int(std::min(per, units.size() - k));
+        p.volume = out + k * size_t(grid.nx) * grid.ny * grid.nz;
+        launch_fdk_operator_bp(p, s);
+    }
+    YK_HIP(hipStreamSynchronize(s));  // (`units` is host memory)
+    return true;
+}
+
+// launch of the operator-form backprojection of views [first, first + count)
+OpBpLaunch yk_projector::op_launch(int kind, const float* d_proj, int first, int count) const
+{
+    OpBpLaunch p{};
+    p.proj = d_proj;
+    p.views = d_opviews.get() + first;
+    p.vol = vol;
+    p.nu = nu; p.nv = nv; p.count = count;
+    p.scale = float(op_scale[first]);
+    p.mode = op_mode(kind);
+    p.front = std::all_of(op_front.begin() + first, op_front.begin() + first + count, [](char f) { return f != 0; });
+    return p;
 }
 
 double yk_projector::dot(const float* a, const float* b, size_t n)

@@ -411,6 +411,24 @@ struct OpBpViewDev {
     float inv_sdd_plane;
 };
 
+// views [first, first + count) of a launch's, backprojected into a volume of their own
+struct OpBpUnit {
+    int first, count;
+    float scale;
+    int pad;
+};
+
+// what becomes of a backprojected value
+struct OpBpStore {
+    enum Mode { kSet, kAdd, kWeight, kUpdate };
+    int mode;                   // volume =, volume +=, volume = (value > 0 ? value : 1e30), x += lambda value / (col + eps)
+    float* x;                   // (kUpdate) then bounded
+    const float* col;
+    float lambda, eps;
+    int use_min, use_max;
+    float lo, hi;
+};
+
 struct OpBpLaunch {
     const float* proj;          // [count][nv][nu], unfiltered
     float* volume;              // [z][y][x]
@@ -419,7 +437,10 @@ struct OpBpLaunch {
     int nu, nv, count;
     float scale;                // vx vy vz / (du dv) of the first view (matched weight)
     int mode;                   // 0 FDK weight, 1 pseudo-matched, 2 voxel-driven Joseph
-    int accumulate;
+    OpBpStore store;
+    const OpBpUnit* units;      // device, n_units, volume [unit][z][y][x]; null: one unit of `count` views
+    int n_units;
+    int one_view;               // every view has the pixels of proj's first
     int front;                  // every voxel lies before every source, with regular weights (projector.cpp)
     float* paired;              // scratch of count x paired_view_floats: sample a paired copy (null: the views)
 };

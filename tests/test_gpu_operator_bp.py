@@ -48,3 +48,17 @@ def test_matches_oracle(ctx, oracle, name, kind, views):
     base = np.full_like(got, np.abs(ref).max())
     acc = P.adjoint(part, kind=kind, first=first, out=torch.from_numpy(base).cuda(), accumulate=True).cpu().numpy()
     assert rel_rmse(acc, ref + base) < tolerance(name, g)
+
+
+@pytest.mark.parametrize("views", [1, 4])
+@pytest.mark.parametrize("kind", ["fdk", "fdk_pseudo_matched", "joseph_voxel"])
+def test_long_runs(ctx, oracle, kind, views):
+    """A volume of enough workgroups for the runs of eight slices, the last one of a single slice."""
+    g = small_geometry(volume=(250, 243, 33), voxel_mm=(0.11, 0.1, 0.5), total_views=4, views_per_turn=4, **OFF)
+    P = yk.Projector(ctx, g.views(), g.nu, g.nv, g.grid())
+    y = np.random.default_rng(15).standard_normal((4, g.nv, g.nu)).astype(np.float32)
+    y[views:] = 0.0
+    ref = oracle.bp_fdk_operator(oracle.views_from_float(P.views), y.astype(np.float64), oracle_volume(oracle, g),
+                                 matched={"fdk": 0, "fdk_pseudo_matched": 1, "joseph_voxel": 2}[kind])
+    got = P.adjoint(torch.from_numpy(y[:views]).cuda(), kind=kind).cpu().numpy()
+    assert rel_rmse(got, ref) < tolerance("long_runs", g), rel_rmse(got, ref)

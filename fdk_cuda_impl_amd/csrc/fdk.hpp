@@ -130,6 +130,7 @@ struct yk_projector {
     bool backproject_update(int kind, const float* d_proj, int first, int count, const yk::OpBpStore& update);
     bool column_weights(int kind, const float* d_ones, const std::vector<int>& counts, bool mask, float* out);
     yk::OpBpLaunch op_launch(int kind, const float* d_proj, int first, int count) const;
+    bool column_transpose(yk_projector& w, const float* d_proj, float* d_volume, int first, int count, int accumulate);
     double dot(const float* a, const float* b, size_t n);
     bool siddon_copies(yk_projector& w, const float* d_volume);
     int op_chunk(yk_projector& w, int count, bool one_view = false) const;
@@ -156,6 +157,8 @@ struct yk_projector {
     yk::DeviceArray<float> d_vol_t;
     yk::DeviceArray<float> d_vol_zx;   // paired volume copies of the Joseph and Siddon projections
     yk::DeviceArray<float> d_vol_zy;
+    std::vector<char> joseph_column;   // per view: the column transpose covers it
+    yk::DeviceArray<float> d_column_x, d_column_y;  // its volumes of the X- and Y-main views
     std::vector<char> joseph_gather, siddon_gather;  // per view: the gather transposes cover it
     yk::DeviceArray<yk::GatherViewDev> d_gather;
     yk::DeviceArray<float> d_gather_q; // ray values of the gather transposes, one view chunk

@@ -15,8 +15,7 @@
 // table value, where evaluating its line took 24 bytes of table and a floor /
 // compare chain for each.  N_k at a reference pixel near the voxel is formed in
 // FP64 (its terms are a thousand times the result) and carried to the
-// candidates in FP32 steps.  The source and pixel positions are the forward
-// kernel's (float records), so the transpose matches it up to rounding.
+// candidates in FP32 steps.
 //
 // Siddon: the segment of a ray in a voxel lies between its crossings of the
 // voxel's six planes, (plane - src) * (1 / ray); the reciprocals come from a

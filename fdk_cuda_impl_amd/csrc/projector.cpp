@@ -35,6 +35,12 @@ constexpr int kOpPairViews = 3;
 // cross.
 constexpr double kSiddonSlabRatio = 1.0;
 
+// Voxels from which the Joseph transpose of separable views goes by columns:
+// 96^3 x 60 views take 169 us against the gather's 237, 128^3 x 4 49 against
+// 50, 64^3 x 60 110 against 113, 64^3 x 4 33 against 27 (three launches
+// and two volumes more, and too few waves).
+constexpr size_t kColumnVoxels = 500000;
+
 bool operator_form(int kind)
 {
     return kind == YK_BP_FDK || kind == YK_BP_FDK_PSEUDO_MATCHED || kind == YK_BP_JOSEPH_VOXEL;
@@ -43,17 +49,18 @@ bool operator_form(int kind)
 int op_mode(int kind) { return kind == YK_BP_FDK_PSEUDO_MATCHED ? 1 : kind == YK_BP_JOSEPH_VOXEL ? 2 : 0; }
 
 // record of the gather transposes of a view whose main axis is X or Y, from
-// the forward kernel's voxel-normalized floats and the projective map of world
-// points
-void gather_view(const ProjViewDev& p, int nu, int nv, const double map[12], const VolumeGeom& g, GatherViewDev& o)
+// its vectors in volume-centred voxel units and the projective map of world
+// points.  In FP64: the forward kernel's float records of a source 1500 voxels
+// away put a ray 4e-5 voxels aside.
+void gather_view(const ViewD& w, int axis, int nu, int nv, const double map[12], const VolumeGeom& g, GatherViewDev& o)
 {
     std::memset(&o, 0, sizeof(o));
-    o.axis = p.axis;
-    const int order[3] = { p.axis, p.axis == 0 ? 1 : 0, 2 };
+    o.axis = axis;
+    const int order[3] = { axis, axis == 0 ? 1 : 0, 2 };
     double most = 0.0;
     for (int a = 0; a < 4; ++a)
-        most = std::max(most, std::fabs(double(p.detS[p.axis]) - p.src[p.axis] +
-            ((a & 1) ? nu - 1 : 0) * double(p.detU[p.axis]) + ((a & 2) ? nv - 1 : 0) * double(p.detV[p.axis])));
+        most = std::max(most, std::fabs(w.detS[axis] - w.src[axis] + ((a & 1) ? nu - 1 : 0) * w.detU[axis] +
+            ((a & 2) ? nv - 1 : 0) * w.detV[axis]));
     int e = 0;
     std::frexp(most, &e);
     const double scale = std::ldexp(1.0, -e);
@@ -61,10 +68,10 @@ void gather_view(const ProjViewDev& p, int nu, int nv, const double map[12], con
     double* rows[3] = { o.d, o.e1, o.e2 };
     for (int k = 0; k < 3; ++k) {
         const int c = order[k];
-        o.src[k] = p.src[c];
-        rows[k][0] = (double(p.detS[c]) - p.src[c]) * scale;
-        rows[k][1] = p.detU[c] * scale;
-        rows[k][2] = p.detV[c] * scale;
+        o.src[k] = w.src[c];
+        rows[k][0] = (w.detS[c] - w.src[c]) * scale;
+        rows[k][1] = w.detU[c] * scale;
+        rows[k][2] = w.detV[c] * scale;
     }
     // the map at voxel index (i, j, k): X = origin + index x voxel
     const double vox[3] = { g.vx, g.vy, g.vz }, org[3] = { g.ox, g.oy, g.oz };
@@ -74,6 +81,19 @@ void gather_view(const ProjViewDev& p, int nu, int nv, const double map[12], con
         for (int k = 0; k < 3; ++k) maps[m][k] = float(c[k] * vox[k]);
         maps[m][3] = float(c[0] * org[0] + c[1] * org[1] + c[2] * org[2] + c[3]);
     }
+}
+
+// The column transpose takes separable views in which at most eight rays of a
+// detector column pass within a voxel along z, of a detector whose row
+// numbers times FP32 rounding stay far below its 0.01 pixels of margin
+bool column_view(const ProjViewDev& p, int nu, int nv, const VolumeGeom& g)
+{
+    const int a = p.axis;
+    const double h = 0.5 * ((a == 0 ? g.nx : g.ny) - 1);
+    const double near = std::fabs(double(p.src[a])) - h;  // least distance of a slice from the source
+    double far = 0.0;
+    for (int u : { 0, nu - 1 }) far = std::max(far, std::fabs(double(p.detS[a]) + u * double(p.detU[a]) - p.src[a]));
+    return near > 0.0 && nv <= 8192 && far <= 3.9 * near * std::fabs(double(p.detV[2]));
 }
 
 // least and largest distance of the volume's voxels, grown by `xy` and `z`
@@ -150,12 +170,21 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
             double least, most, inner, outer;
             depth_range(w, map, vol, 2.0, kGatherRun + 2.0, least, most);
             depth_range(w, map, vol, 0.5, 0.5, inner, outer);
-            gather_view(p, nu, nv, map, vol, gv[i]);
+            ViewD n{};
+            for (int k = 0; k < 3; ++k) {
+                n.src[k] = (double(w.src[k]) - cen[k]) / vox[k];
+                n.detS[k] = (double(w.detS[k]) - cen[k]) / vox[k];
+                n.detU[k] = double(w.detU[k]) / vox[k];
+                n.detV[k] = double(w.detV[k]) / vox[k];
+            }
+            gather_view(n, p.axis, nu, nv, map, vol, gv[i]);
             joseph_gather.push_back(least > 1e-3);
             siddon_gather.push_back(least > 1e-3 && outer < 1.0);
+            joseph_column.push_back(separable.back() && joseph_gather.back() && column_view(p, nu, nv, vol));
         } else {
             joseph_gather.push_back(0);
             siddon_gather.push_back(0);
+            joseph_column.push_back(0);
         }
     }
     d_gather.upload(gv.data(), gv.size(), ctx->stream);
@@ -449,6 +478,54 @@ bool yk_projector::gather_transpose(yk_projector& w, bool siddon, const float* d
     return true;
 }
 
+// Joseph transpose of separable views by detector columns, a chunk of views'
+// table at a time (at most 1 GiB); false when the gather has to serve the call:
+// a view outside its form, sizes past its grids, few voxels, or no memory
+bool yk_projector::column_transpose(yk_projector& w, const float* d_proj, float* d_volume, int first, int count, int accumulate)
+{
+    if (!std::all_of(joseph_column.begin() + first, joseph_column.begin() + first + count, [](char c) { return c != 0; }))
+        return false;
+    const size_t voxels = size_t(grid.nx) * grid.ny * grid.nz;
+    if (voxels < kColumnVoxels || grid.ny > 65535 || grid.nx > 500000 || grid.nz > 2000000) return false;
+    const int pitch = nv + 2 * kColumnPad;
+    const size_t per_view = size_t(nu) * pitch;
+    if (per_view > (size_t(1) << 30)) return false;
+    const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
+    bool any_x = false, any_y = false;
+    for (int i = first; i < first + count; ++i) (main_axis(views[i], nu, nv) == 0 ? any_x : any_y) = true;
+    if (w.d_gather_q.size() < per_view * chunk || !w.d_flag.get() || (any_x && w.d_column_x.size() < voxels) ||
+        (any_y && w.d_column_y.size() < voxels)) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) return false;
+        try {
+            grow(w.d_gather_q, per_view * chunk);
+            grow(w.d_flag, 1);
+            if (any_x) grow(w.d_column_x, voxels);
+            if (any_y) grow(w.d_column_y, voxels);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    for (int c0 = 0; c0 < count; c0 += chunk) {
+        ColumnTransposeLaunch p{};
+        p.proj = d_proj + size_t(nu) * nv * c0;
+        p.volume = d_volume;
+        p.views = d_jviews.get() + first + c0;
+        p.gviews = d_gather.get() + first + c0;
+        p.q = w.d_gather_q.get();
+        p.part_x = any_x ? w.d_column_x.get() : nullptr;
+        p.part_y = any_y ? w.d_column_y.get() : nullptr;
+        p.flag = w.d_flag.get();
+        p.vol = vol;
+        p.nu = nu; p.nv = nv; p.pitch = pitch; p.count = std::min(chunk, count - c0);
+        p.accumulate = c0 > 0 ? 1 : accumulate;
+        launch_joseph_column_transpose(p, ctx->stream);
+    }
+    return true;
+}
+
 void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, int first, int count,
     int accumulate)
 {
@@ -456,7 +533,8 @@ void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, i
     if (!d_volume || !d_proj) fail(YK_ERR_INVALID_BUFFER, "null device buffer");
     hipStream_t s = ctx->stream;
     yk_projector& w = scratch_owner ? *scratch_owner : *this;  // scratch arrays
-    if (kind == YK_BP_JOSEPH_ADJOINT && gather_transpose(w, false, d_proj, d_volume, first, count, accumulate)) {
+    if (kind == YK_BP_JOSEPH_ADJOINT && column_transpose(w, d_proj, d_volume, first, count, accumulate)) {
+    } else if (kind == YK_BP_JOSEPH_ADJOINT && gather_transpose(w, false, d_proj, d_volume, first, count, accumulate)) {
     } else if (kind == YK_BP_JOSEPH_ADJOINT) {
         // the ray table holds a chunk of views at a time (at most 1 GiB)
         const size_t per_view = size_t(nu) * nv;

@@ -364,6 +364,25 @@ constexpr int kGatherPad = 4;
 constexpr int kGatherPadRows = 3;
 constexpr int kGatherRun = 8;  // voxels along z of a lane
 
+// Joseph transpose of separable views by detector columns (kernels_column.hip)
+struct ColumnTransposeLaunch {
+    const float* proj;          // [count][nv][nu]
+    float* volume;              // [z][y][x]
+    const ProjViewDev* views;   // device, `count`
+    const GatherViewDev* gviews; // device, `count`
+    float* q;                   // scratch [count][nu][pitch], pitch = nv + 2 kColumnPad
+    float* part_x;              // scratch [x][y][z] (null: no X-main view)
+    float* part_y;              // scratch [y][x][z] (null: no Y-main view)
+    int* flag;                  // scratch word
+    VolumeGeom vol;
+    int nu, nv, pitch, count;
+    int accumulate;
+};
+void launch_joseph_column_transpose(const ColumnTransposeLaunch& p, hipStream_t s);
+constexpr int kColumnPad = 8;      // zeros on either side of a table's column
+constexpr int kColumnSlices = 4;   // consecutive slices of a workgroup, a wave each
+constexpr int kColumnGroups = 4;   // 64-voxel groups along z of a wave, at most
+
 struct SiddonLaunch {
     const float* volume;
     float* proj;

@@ -42,6 +42,8 @@ namespace yk {
 namespace {
 
 typedef float float4a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float float3a4 __attribute__((ext_vector_type(3), aligned(4)));
+typedef float float2a4 __attribute__((ext_vector_type(2), aligned(4)));
 
 // clamp to [0, 1]: the output modifier of the instruction that forms x
 __device__ __forceinline__ float sat(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, 1.f); }
@@ -97,6 +99,31 @@ siddon_gather_table_kernel(const float* __restrict__ proj, const SiddonViewDev* 
     q[((size_t)i * gridDim.y + v) * pitch + u] = w;
 }
 
+// The same of views whose detector rows and columns lie along the main axes'
+// plane and z (separable, no z in a row's step): a ray's x and y do not depend
+// on v, nor its z on u, so the reciprocals are one entry a column, ru [view]
+// [pitch] (1 / x, 1 / y), and one a row, rv [view][nv + kGatherPadRows]; q is
+// p |ray| alone.
+__global__ void __launch_bounds__(256)
+siddon_flat_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __restrict__ views, int nu, int nv, int pitch,
+    float* __restrict__ q, float2* __restrict__ ru, float* __restrict__ rv, int* __restrict__ flag)
+{
+    const int u = blockIdx.x * 256 + threadIdx.x;
+    const int v = blockIdx.y, i = blockIdx.z;
+    if (u >= pitch) return;
+    float w = 0.f, rc[3] = { 0.f, 0.f, 0.f };
+    float src[3], ray[3];
+    siddon_ray_geom(views[i], u, v, src, ray);
+    for (int k = 0; k < 3; ++k) rc[k] = fabsf(ray[k]) > 1e-8f ? 1.f / ray[k] : 1e30f;
+    if (u < nu && v < nv) {
+        w = proj[((size_t)i * nv + v) * nu + u] * sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
+        if (!(fabsf(w) <= 3.4e38f)) atomicOr(flag, 1);
+    }
+    q[((size_t)i * gridDim.y + v) * pitch + u] = w;
+    if (v == 0) ru[(size_t)i * pitch + u] = make_float2(rc[0], rc[1]);
+    if (u == 0) rv[(size_t)i * gridDim.y + v] = rc[2];
+}
+
 // Where the candidates of a lane's run of ZR voxels along z lie on one view.
 // A lane walks its run two voxels at a time: a pair shares the rows both see
 // (for Joseph 5.1 instead of 2 x 3.4 at a magnified voxel of 1.7 pixels).  The
@@ -109,6 +136,7 @@ struct CandidateBox {
     float u0, v0, d0;  // numerators of u and v, and depth, at (x, y, 0)
     float u_z, v_z, a_z;
     float um, vm;      // the middle of the run
+    float v_zd;        // v a voxel along z, of views whose depth does not vary along z
     float hu, hv;      // half widths of a pair's box anywhere in the run
 
     __device__ __forceinline__ CandidateBox(const GatherViewDev& r, int x, int y, int z0, float h_main, float h_1,
@@ -135,6 +163,7 @@ struct CandidateBox {
         const float rb = __builtin_amdgcn_rcpf(dm - fmaf(0.5f * float(ZR), fabsf(a_z), dhalf));
         um = fmaf(u_z, zm, u0) * rm;
         vm = fmaf(v_z, zm, v0) * rm;
+        v_zd = v_z * rm;
         const float ku = fabsf(fmaf(-um, a_z, u_z)) * rb, kv = fabsf(fmaf(-vm, a_z, v_z)) * rb;
         const float su = 0.5f * float(ZR) * ku, sv = 0.5f * float(ZR) * kv;
         hu = fmaf(h_z, ku, fmaf(h_1, fabsf(fmaf(-um, a_1, u_1)) * rb, fmaf(su * dhalf, rb, 0.05f)));
@@ -295,11 +324,79 @@ __device__ __forceinline__ void siddon_gather(const float4* __restrict__ q, cons
     }
 }
 
-template <bool SIDDON, int ZR>
+// Views of siddon_flat_table_kernel.  Depth, the candidate columns and the part
+// of each column's rays over the voxel column's x and y planes hold for the
+// whole run, and a row's z planes for all its candidates, so a candidate takes 7
+// instructions and 4 bytes where siddon_gather takes 16 and 16: 256^3 x 360
+// views of 512 x 384 17.2 -> 10.4 ms, 128^3 x 120 891 -> 570 us, 64^3 x 60 116
+// -> 102.  (Pixels x rows a chunk at 256^3: 3 x 1 12.9 ms, 3 x 3 11.2, 2 x 2
+// 22.3, 4 x 2 10.9.)
+template <int ZR, bool SAFE>
+__device__ __forceinline__ void siddon_flat_gather(const float* __restrict__ q, const float2* __restrict__ ru,
+    const float* __restrict__ rv, const GatherViewDev* __restrict__ views, const SiddonViewDev* __restrict__ sviews,
+    const VolumeGeom& g, int nu, int nv, int pitch, int count, int x, int y, int z0, float (&acc)[ZR])
+{
+    constexpr int kWidth = 3, kRows = 2;
+    const float lox = g.ox - 0.5f * g.vx, loy = g.oy - 0.5f * g.vy, loz = g.oz - 0.5f * g.vz;
+#pragma unroll 1
+    for (int i = 0; i < count; ++i) {
+        const size_t rows = size_t(i) * (nv + kGatherPadRows);
+        const float* qi = q + rows * pitch;
+        const float* rvi = rv + rows;
+        const CandidateBox<ZR> box(views[i], x, y, z0, 0.5f, 0.5f, 1.f);
+        const SiddonViewDev& sv = sviews[i];
+        const float x0 = plane_offset(lox, g.vx, x, sv.src[0]), x1 = plane_offset(lox, g.vx, x + 1, sv.src[0]);
+        const float y0 = plane_offset(loy, g.vy, y, sv.src[1]), y1 = plane_offset(loy, g.vy, y + 1, sv.src[1]);
+        const int ulo = int(fmaxf(0.f, ceilf(box.um - box.hu))), uhi = int(fminf(float(nu - 1), floorf(box.um + box.hu)));
+#pragma unroll 1
+        for (int u = ulo; u <= uhi; u += kWidth) {
+            float ya[kWidth], yb[kWidth];
+#pragma unroll
+            for (int k = 0; k < kWidth; ++k) {
+                const float2 c = ru[(size_t)i * pitch + (u + k)];
+                const float tx0 = x0 * c.x, tx1 = x1 * c.x;
+                ya[k] = __builtin_amdgcn_fmed3f(y0 * c.y, tx0, tx1);
+                yb[k] = __builtin_amdgcn_fmed3f(y1 * c.y, tx0, tx1);
+            }
+#pragma unroll
+            for (int p = 0; p < ZR; p += 2) {
+                const float vc = fmaf(box.v_zd, float(p) + 0.5f - 0.5f * float(ZR - 1), box.vm);
+                const int vlo = int(fmaxf(0.f, ceilf(vc - box.hv))), vhi = int(fminf(float(nv - 1), floorf(vc + box.hv)));
+                const float za = plane_offset(loz, g.vz, z0 + p, sv.src[2]);
+                const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.src[2]);
+                const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.src[2]);
+                unsigned row = unsigned(vlo) * unsigned(pitch) + unsigned(u);
+#pragma unroll 1
+                for (int v = vlo; v <= vhi; v += kRows) {
+                    float3a4 w[kRows];
+#pragma unroll
+                    for (int j = 0; j < kRows; ++j) w[j] = *reinterpret_cast<const float3a4*>(qi + (row + unsigned(j * pitch)));
+                    const float2a4 r = *reinterpret_cast<const float2a4*>(rvi + unsigned(v));
+#pragma unroll
+                    for (int j = 0; j < kRows; ++j) {
+                        const float za_t = za * r[j], zb_t = zb * r[j], zc_t = zc * r[j];
+#pragma unroll
+                        for (int k = 0; k < kWidth; ++k) {
+                            const float ta = __builtin_amdgcn_fmed3f(za_t, ya[k], yb[k]);
+                            const float tb = __builtin_amdgcn_fmed3f(zb_t, ya[k], yb[k]);
+                            const float tc = __builtin_amdgcn_fmed3f(zc_t, ya[k], yb[k]);
+                            const float sa = fabsf(tb - ta), sb = fabsf(tc - tb);
+                            if (!SAFE || sa > 0.f) acc[p] = fmaf(sa, w[j][k], acc[p]);
+                            if (!SAFE || sb > 0.f) acc[p + 1] = fmaf(sb, w[j][k], acc[p + 1]);
+                        }
+                    }
+                    row += unsigned(kRows * pitch);
+                }
+            }
+        }
+    }
+}
+
+template <int MODEL, int ZR>
 __global__ void __launch_bounds__(256)
-gather_transpose_kernel(const void* __restrict__ q, float* __restrict__ volume,
-    const GatherViewDev* __restrict__ views, const SiddonViewDev* __restrict__ sviews, const int* __restrict__ flag, VolumeGeom g, int nu, int nv, int pitch,
-    int count, int accumulate)
+gather_transpose_kernel(const void* __restrict__ q, const float2* __restrict__ ru, const float* __restrict__ rv,
+    float* __restrict__ volume, const GatherViewDev* __restrict__ views, const SiddonViewDev* __restrict__ sviews,
+    const int* __restrict__ flag, VolumeGeom g, int nu, int nv, int pitch, int count, int accumulate)
 {
     const int x = blockIdx.x * 16 + (threadIdx.x & 15);
     const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
@@ -309,7 +406,11 @@ gather_transpose_kernel(const void* __restrict__ q, float* __restrict__ volume,
 #pragma unroll
     for (int k = 0; k < ZR; ++k) acc[k] = 0.f;
     const bool plain = __builtin_amdgcn_readfirstlane(*flag) == 0;
-    if constexpr (SIDDON) {
+    if constexpr (MODEL == kGatherSiddonFlat) {
+        const float* t = static_cast<const float*>(q);
+        if (plain) siddon_flat_gather<ZR, false>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
+        else siddon_flat_gather<ZR, true>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
+    } else if constexpr (MODEL == kGatherSiddon) {
         const float4* t = static_cast<const float4*>(q);
         if (plain) siddon_gather<ZR, false>(t, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
         else siddon_gather<ZR, true>(t, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
@@ -327,17 +428,17 @@ gather_transpose_kernel(const void* __restrict__ q, float* __restrict__ volume,
     }
 }
 
-template <bool SIDDON, int ZR>
+template <int MODEL, int ZR>
 void launch_run(const GatherLaunch& p, hipStream_t s)
 {
     const VolumeGeom& g = p.vol;
     dim3 grid((g.nx + 15) / 16, (g.ny + 15) / 16, (g.nz + ZR - 1) / ZR);
-    hipLaunchKernelGGL((gather_transpose_kernel<SIDDON, ZR>), grid, dim3(256), 0, s, p.q, p.volume, p.gviews, p.sviews, p.flag, g,
-        p.nu, p.nv, p.pitch, p.count, p.accumulate);
+    hipLaunchKernelGGL((gather_transpose_kernel<MODEL, ZR>), grid, dim3(256), 0, s, p.q, p.ru, p.rv, p.volume, p.gviews, p.sviews,
+        p.flag, g, p.nu, p.nv, p.pitch, p.count, p.accumulate);
     YK_HIP(hipGetLastError());
 }
 
-template <bool SIDDON>
+template <int MODEL>
 void launch_gather(const GatherLaunch& p, hipStream_t s)
 {
     const VolumeGeom& g = p.vol;
@@ -346,8 +447,8 @@ void launch_gather(const GatherLaunch& p, hipStream_t s)
     // one has four times the workgroups: at 60 views and 128^3 = 1024
     // workgroups both take 432 us, at 160^3 724 against 811, at 112^3 346
     // against 304, at 64^3 236 against 96)
-    if (wide >= 1024) launch_run<SIDDON, kGatherRun>(p, s);
-    else launch_run<SIDDON, 2>(p, s);
+    if (wide >= 1024) launch_run<MODEL, kGatherRun>(p, s);
+    else launch_run<MODEL, 2>(p, s);
 }
 
 }  // namespace
@@ -356,14 +457,18 @@ void launch_gather_transpose(const GatherLaunch& p, hipStream_t s)
 {
     hipLaunchKernelGGL(gather_clear_kernel, dim3(1), dim3(1), 0, s, p.flag);
     dim3 tg((p.pitch + 255) / 256, p.nv + kGatherPadRows, p.count);
-    if (p.siddon) {
+    if (p.model == kGatherSiddonFlat) {
+        hipLaunchKernelGGL(siddon_flat_table_kernel, tg, dim3(256), 0, s, p.proj, p.sviews, p.nu, p.nv, p.pitch, p.q, p.ru, p.rv,
+            p.flag);
+        launch_gather<kGatherSiddonFlat>(p, s);
+    } else if (p.model == kGatherSiddon) {
         hipLaunchKernelGGL(siddon_gather_table_kernel, tg, dim3(256), 0, s, p.proj, p.sviews, p.nu, p.nv, p.pitch,
             reinterpret_cast<float4*>(p.q), p.flag);
-        launch_gather<true>(p, s);
+        launch_gather<kGatherSiddon>(p, s);
     } else {
         hipLaunchKernelGGL(joseph_gather_table_kernel, tg, dim3(256), 0, s, p.proj, p.views, p.gviews, p.vol, p.nu, p.nv,
             p.pitch, p.q, p.flag);
-        launch_gather<false>(p, s);
+        launch_gather<kGatherJoseph>(p, s);
     }
 }
 

@@ -180,11 +180,13 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
             gather_view(n, p.axis, nu, nv, map, vol, gv[i]);
             joseph_gather.push_back(least > 1e-3);
             siddon_gather.push_back(least > 1e-3 && outer < 1.0);
+            siddon_flat.push_back(separable.back() && w.detU[2] == 0.f);
             joseph_column.push_back(separable.back() && joseph_gather.back() && column_view(p, nu, nv, vol));
         } else {
             joseph_gather.push_back(0);
             siddon_gather.push_back(0);
             joseph_column.push_back(0);
+            siddon_flat.push_back(0);
         }
     }
     d_gather.upload(gv.data(), gv.size(), ctx->stream);
@@ -444,8 +446,12 @@ bool yk_projector::gather_transpose(yk_projector& w, bool siddon, const float* d
 {
     const std::vector<char>& ok = siddon ? siddon_gather : joseph_gather;
     if (!std::all_of(ok.begin() + first, ok.begin() + first + count, [](char c) { return c != 0; })) return false;
+    const bool flat = siddon && std::all_of(siddon_flat.begin() + first, siddon_flat.begin() + first + count,
+        [](char c) { return c != 0; });
     const int pitch = nu + kGatherPad;
-    const size_t per_view = size_t(nv + kGatherPadRows) * pitch * (siddon ? 4 : 1);  // floats
+    // floats (flat: an entry a column and a row more, columns' aligned to 8 bytes)
+    const size_t rows = size_t(nv) + kGatherPadRows;
+    const size_t per_view = flat ? rows * pitch + 2 * size_t(pitch) + rows + 1 : rows * pitch * (siddon ? 4 : 1);
     if (nv + kGatherPadRows > 65535 || per_view > (size_t(1) << 30)) return false;
     const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
     if (w.d_gather_q.size() < per_view * chunk || !w.d_flag.get()) {
@@ -471,7 +477,12 @@ bool yk_projector::gather_transpose(yk_projector& w, bool siddon, const float* d
         p.flag = w.d_flag.get();
         p.vol = vol;
         p.nu = nu; p.nv = nv; p.pitch = pitch; p.count = std::min(chunk, count - c0);
-        p.siddon = siddon;
+        p.model = flat ? kGatherSiddonFlat : siddon ? kGatherSiddon : kGatherJoseph;
+        if (flat) {
+            const size_t q_size = (rows * pitch * p.count + 1) & ~size_t(1);
+            p.ru = reinterpret_cast<float2*>(p.q + q_size);
+            p.rv = p.q + q_size + 2 * size_t(pitch) * p.count;
+        }
         p.accumulate = c0 > 0 ? 1 : accumulate;
         launch_gather_transpose(p, ctx->stream);
     }

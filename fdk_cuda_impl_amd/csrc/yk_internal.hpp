@@ -344,17 +344,21 @@ struct GatherViewDev {
     int axis;                   // 0 X, 1 Y
 };
 
+// (flat: separable views whose row steps have no z component)
+enum GatherModel { kGatherJoseph, kGatherSiddon, kGatherSiddonFlat };
 struct GatherLaunch {
     const float* proj;          // [count][nv][nu]
     float* volume;              // [z][y][x]
     const ProjViewDev* views;   // device, `count` (Joseph)
     const SiddonViewDev* sviews; // device, `count` (Siddon)
     const GatherViewDev* gviews; // device, `count`
-    float* q;                   // scratch [count][nv + kGatherPadRows][pitch] floats (Joseph) or float4s (Siddon)
+    float* q;                   // scratch [count][nv + kGatherPadRows][pitch] floats or float4s (kGatherSiddon)
+    float2* ru;                 // scratch [count][pitch] (kGatherSiddonFlat)
+    float* rv;                  // scratch [count][nv + kGatherPadRows] (kGatherSiddonFlat)
     int* flag;                  // scratch word
     VolumeGeom vol;
     int nu, nv, pitch, count;
-    int siddon;                 // 0 Joseph
+    int model;
     int accumulate;
 };
 void launch_gather_transpose(const GatherLaunch& p, hipStream_t s);

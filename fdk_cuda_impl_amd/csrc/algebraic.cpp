@@ -163,10 +163,8 @@ void run_algebraic(yk_projector* p, const yk_algebraic_desc& d, const float* d_b
     float* const cols = ws.array(1, cache_cols ? nx * nu_units : nx);
     float* const fwd = ws.array(2, size_t(max_k) * view_n);
     float* const bp = ws.array(3, nx);
-    float* const ones_vol = ws.array(4, tigre ? 8 : nx);
-    float* const ones_proj = ws.array(5, size_t(max_k) * view_n);
-    float* const grad = d.tv_iterations > 0 && d.tv_strength > 0.f ? ws.array(6, nx) : nullptr;
-    launch_fill(ones_vol, 1.f, tigre ? 8 : nx, s);
+    float* const ones_proj = ws.array(4, size_t(max_k) * view_n);
+    float* const grad = d.tv_iterations > 0 && d.tv_strength > 0.f ? ws.array(5, nx) : nullptr;
     launch_fill(ones_proj, 1.f, size_t(max_k) * view_n, s);
     // the SIRT batch backend and the TIGRE backend mask voxels no ray reaches
     const bool mask_cols = tigre || nu_units == 1;
@@ -174,10 +172,7 @@ void run_algebraic(yk_projector* p, const yk_algebraic_desc& d, const float* d_b
         u.op->backproject(d.back_kind, ones_proj, out, u.op_first, u.count, 0);
         if (mask_cols) weight_prepare(out, 0.f, 0, nx, s);
     };
-    constexpr int kRowViews = 32768;  // (grids of single views hold 65535)
-    for (int at = 0; at < na; at += kRowViews)
-        (tigre ? ws.coarse.get() : op)->project(d.forward_kind, ones_vol, rows + size_t(at) * view_n, at,
-            std::min(kRowViews, na - at), 0);
+    (tigre ? ws.coarse.get() : op)->project_ones(d.forward_kind, rows, 0, na);
     if (tigre) weight_prepare(rows, 0.5f * min_voxel, 1, size_t(na) * view_n, s);
     if (cache_cols) {
         // one launch for all units where their operators are one sequence
@@ -194,8 +189,8 @@ void run_algebraic(yk_projector* p, const yk_algebraic_desc& d, const float* d_b
     // convergence monitor state (AlgebraicReconstructorEx::prepareConvergence_, :236-256)
     const bool watch_residual = d.relative_residual_tolerance > 0.f || d.relative_improvement_tolerance > 0.f;
     const bool watch_update = d.relative_update_tolerance > 0.f;
-    float* const resid = watch_residual ? ws.array(7, size_t(na) * view_n) : nullptr;
-    float* const prev = watch_update ? ws.array(8, nx) : nullptr;
+    float* const resid = watch_residual ? ws.array(6, size_t(na) * view_n) : nullptr;
+    float* const prev = watch_update ? ws.array(7, nx) : nullptr;
     if (watch_update) YK_HIP(hipMemcpyAsync(prev, d_x, nx * sizeof(float), hipMemcpyDeviceToDevice, s));
     const double measured = watch_residual ? std::sqrt(std::max(0.0, p->dot(d_b, d_b, size_t(na) * view_n))) : 0.0;
     const double eps = d.epsilon;

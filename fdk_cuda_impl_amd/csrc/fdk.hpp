@@ -95,7 +95,7 @@ struct yk_projector;
 // when the call ends; the rest with the projector.
 struct SolverScratch {
     static constexpr size_t kKeep = size_t(1) << 30;
-    yk::DeviceArray<float> arrays[9];
+    yk::DeviceArray<float> arrays[8];
     std::unique_ptr<yk_projector> subset_op;  // the views in the order of subset_op_units interleaved subsets
     int subset_op_units = 0;
     std::unique_ptr<yk_projector> coarse;     // the TIGRE row weights' support volume
@@ -126,6 +126,7 @@ struct yk_projector {
         const yk_volume_grid& grid, float scan_range, const std::vector<int>* segments = nullptr);
 
     void project(int kind, const float* d_volume, float* d_proj, int first, int count, int accumulate);
+    void project_ones(int kind, float* d_proj, int first, int count);  // of a volume of ones
     void backproject(int kind, const float* d_proj, float* d_volume, int first, int count, int accumulate);
     bool backproject_update(int kind, const float* d_proj, int first, int count, const yk::OpBpStore& update);
     bool column_weights(int kind, const float* d_ones, const std::vector<int>& counts, bool mask, float* out);

@@ -722,6 +722,70 @@ __device__ __forceinline__ float siddon_walk(const float* __restrict__ vol, cons
     return acc * len;
 }
 
+// The projections of a volume of ones, the algebraic solvers' row weights, in
+// closed form: no volume, copies or gathers.
+//
+// Joseph: a slice adds the weights of its taps inside the volume, the product
+// over both minor axes of min(f + 1, n - f) clamped to [0, 1].  It is 1 in every
+// slice where the ray lies inside [0, n - 1] on both axes, so only the slices at
+// the ends (and one more on either side) are evaluated.
+// (OS-SART of 10 subsets at 128 x 128 x 100 x 120 views of 256 x 192: 1.65 ms
+// with the projection of a volume of ones, 350 us with its copies, 1.36 here.)
+__global__ void __launch_bounds__(256)
+joseph_ones_kernel(float* __restrict__ proj, const ProjViewDev* __restrict__ views, VolumeGeom g, int nu, int nv)
+{
+    const int u = blockIdx.x * 64 + threadIdx.x;
+    const int v = blockIdx.y * 4 + threadIdx.y;
+    const int i = blockIdx.z;
+    if (u >= nu || v >= nv) return;
+    const ProjViewDev pv = views[i];
+    const AxisInfo ax = axis_info(pv.axis, g);
+    JRay r{};
+    int lo = 1, hi = 0;
+    if (joseph_ray(pv, ax, u, v, r)) joseph_slice_range(r, ax, lo, hi);
+    // slices inside on both axes
+    float slo = float(lo), shi = float(hi);
+    const float h0 = 0.5f * float(ax.n0 - 1);
+    const float a[2] = { r.a1, r.a2 }, n[2] = { float(ax.n1), float(ax.n2) };
+    const float b[2] = { r.b1 + 0.5f * float(ax.n1 - 1), r.b2 + 0.5f * float(ax.n2 - 1) };
+    for (int k = 0; k < 2; ++k) {
+        if (fabsf(a[k]) > 1e-12f) {
+            const float t0 = -b[k] / a[k] + h0, t1 = (n[k] - 1.f - b[k]) / a[k] + h0;
+            slo = fmaxf(slo, fminf(t0, t1));
+            shi = fminf(shi, fmaxf(t0, t1));
+        } else if (!(b[k] >= 0.f && b[k] <= n[k] - 1.f)) {
+            shi = -1.f;
+        }
+    }
+    const int ilo = int(ceilf(fminf(slo, float(hi)))) + 1, ihi = int(floorf(fmaxf(shi, -1.f))) - 1;
+    float sum = ilo <= ihi ? float(ihi - ilo + 1) : 0.f;
+    for (int s = lo; s <= hi; ++s) {
+        if (s == ilo && ilo <= ihi) s = ihi + 1;  // (<= hi: shi and a slice less)
+        float f1, f2;
+        joseph_sample(r, ax, s, f1, f2);
+        sum += __builtin_amdgcn_fmed3f(fminf(f1 + 1.f, n[0] - f1), 0.f, 1.f) *
+            __builtin_amdgcn_fmed3f(fminf(f2 + 1.f, n[1] - f2), 0.f, 1.f);
+    }
+    proj[((size_t)i * nv + v) * nu + u] = sum * r.L;
+}
+
+// Siddon: the length of the ray inside the volume, between the ends the walk
+// clips it to
+__global__ void __launch_bounds__(256)
+siddon_ones_kernel(float* __restrict__ proj, const SiddonViewDev* __restrict__ views, VolumeGeom g, int nu, int nv)
+{
+    const int u = blockIdx.x * 64 + threadIdx.x;
+    const int v = blockIdx.y * 4 + threadIdx.y;
+    const int i = blockIdx.z;
+    if (u >= nu || v >= nv) return;
+    float src[3], ray[3], t0, t1;
+    siddon_ray_geom(views[i], u, v, src, ray);
+    const Box b = volume_box(g);
+    const bool hit = clip_ray(src, ray, b.lo, b.hi, t0, t1);
+    const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
+    proj[((size_t)i * nv + v) * nu + u] = hit ? (t1 - t0) * len : 0.f;
+}
+
 // Siddon projection by the walk, one lane per ray.  It serves the calls whose
 // rays are too few to pay for the volume copies of siddon_fp_slab_kernel.
 __global__ void __launch_bounds__(256)
@@ -1370,6 +1434,20 @@ void launch_joseph_adjoint(const JosephAdjointLaunch& p, hipStream_t s)
     dim3 block(256), grid((p.vol.nx + 15) / 16, (p.vol.ny + 15) / 16, p.vol.nz);
     hipLaunchKernelGGL(joseph_adjoint_kernel, grid, block, 0, s, p.proj, p.volume, p.views, p.coeff32,
         p.ray_ab, p.ray_len, p.vol, p.nu, p.nv, p.count, p.accumulate);
+    YK_HIP(hipGetLastError());
+}
+
+void launch_joseph_ones(const JosephLaunch& p, hipStream_t s)
+{
+    dim3 block(64, 4), grid((p.nu + 63) / 64, (p.nv + 3) / 4, p.count);
+    hipLaunchKernelGGL(joseph_ones_kernel, grid, block, 0, s, p.proj, p.views, p.vol, p.nu, p.nv);
+    YK_HIP(hipGetLastError());
+}
+
+void launch_siddon_ones(const SiddonLaunch& p, hipStream_t s)
+{
+    dim3 block(64, 4), grid((p.nu + 63) / 64, (p.nv + 3) / 4, p.count);
+    hipLaunchKernelGGL(siddon_ones_kernel, grid, block, 0, s, p.proj, p.views, p.vol, p.nu, p.nv);
     YK_HIP(hipGetLastError());
 }
 

@@ -410,6 +410,29 @@ void yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
     }
 }
 
+void yk_projector::project_ones(int kind, float* d_proj, int first, int count)
+{
+    constexpr int kViews = 32768;  // (a grid holds 65535)
+    for (int at = 0; at < count; at += kViews) {
+        float* proj = d_proj + size_t(nu) * nv * at;
+        if (kind == YK_FP_JOSEPH) {
+            JosephLaunch p{};
+            p.proj = proj;
+            p.views = d_jviews.get() + first + at;
+            p.vol = vol;
+            p.nu = nu; p.nv = nv; p.count = std::min(kViews, count - at);
+            launch_joseph_ones(p, ctx->stream);
+        } else {
+            SiddonLaunch p{};
+            p.proj = proj;
+            p.views = d_sviews.get() + first + at;
+            p.vol = vol;
+            p.nu = nu; p.nv = nv; p.count = std::min(kViews, count - at);
+            launch_siddon_ones(p, ctx->stream);
+        }
+    }
+}
+
 // views per paired copy of the operator-form backprojections (one_view: the
 // copy holds one view, which serves all `count`); 0: sample the
 // views themselves (few samples for the copy's launch and pass, sizes past its

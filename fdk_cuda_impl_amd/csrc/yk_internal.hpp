@@ -289,6 +289,7 @@ struct JosephLaunch {
     int accumulate;
 };
 void launch_joseph_fp(const JosephLaunch& p, hipStream_t s);
+void launch_joseph_ones(const JosephLaunch& p, hipStream_t s);  // of a volume of ones (volume unused)
 void launch_transpose_xy(const float* in, float* out, int nx, int ny, int nz, hipStream_t s);
 
 // Joseph projection from volume copies
@@ -396,6 +397,7 @@ struct SiddonLaunch {
     int accumulate;
 };
 void launch_siddon_fp(const SiddonLaunch& p, hipStream_t s);
+void launch_siddon_ones(const SiddonLaunch& p, hipStream_t s);  // of a volume of ones (volume unused)
 
 // Siddon projection over the paired slab copies of the volume (made by
 // launch_joseph_pair_copy with slab); both copies are needed: the main axis is

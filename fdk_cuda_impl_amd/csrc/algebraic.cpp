@@ -210,9 +210,16 @@ void run_algebraic(yk_projector* p, const yk_algebraic_desc& d, const float* d_b
             const Unit& u = units[order[k]];
             float* c = cols + (cache_cols ? size_t(order[k]) * nx : 0);
             if (!cache_cols) column_weights(u, c);
-            u.op->project(d.forward_kind, d_x, fwd, u.op_first, u.count, 0);
-            algebraic_residual(fwd, d_b + size_t(u.b_first) * view_n, rows + size_t(u.first) * view_n, d.epsilon, tigre ? 1 : 0,
-                view_n, u.count, u.b_stride, s);
+            const float* b = d_b + size_t(u.b_first) * view_n;
+            const float* row = rows + size_t(u.first) * view_n;
+            FpStore residual{};
+            residual.mode = tigre ? FpStore::kResidualMultiply : FpStore::kResidualDivide;
+            residual.eps = d.epsilon;
+            residual.b = b;
+            residual.row = row;
+            residual.b_view = size_t(u.b_stride) * view_n;
+            if (!u.op->project(d.forward_kind, d_x, fwd, u.op_first, u.count, 0, &residual))
+                algebraic_residual(fwd, b, row, d.epsilon, tigre ? 1 : 0, view_n, u.count, u.b_stride, s);
             OpBpStore update{};
             update.x = d_x;
             update.col = c;

@@ -125,7 +125,10 @@ struct yk_projector {
     yk_projector(yk_ctx* ctx, const yk_view* views, int n_views, int nu, int nv,
         const yk_volume_grid& grid, float scan_range, const std::vector<int>* segments = nullptr);
 
-    void project(int kind, const float* d_volume, float* d_proj, int first, int count, int accumulate);
+    // `residual`: the store to make of the values where the kernel has it; false
+    // when they are stored as they are
+    bool project(int kind, const float* d_volume, float* d_proj, int first, int count, int accumulate,
+        const yk::FpStore* residual = nullptr);
     void project_ones(int kind, float* d_proj, int first, int count);  // of a volume of ones
     void backproject(int kind, const float* d_proj, float* d_volume, int first, int count, int accumulate);
     bool backproject_update(int kind, const float* d_proj, int first, int count, const yk::OpBpStore& update);

@@ -292,6 +292,17 @@ void launch_joseph_fp(const JosephLaunch& p, hipStream_t s);
 void launch_joseph_ones(const JosephLaunch& p, hipStream_t s);  // of a volume of ones (volume unused)
 void launch_transpose_xy(const float* in, float* out, int nx, int ny, int nz, hipStream_t s);
 
+// what becomes of a projected value a: proj =, proj +=, or the algebraic
+// solvers' residual, proj = row > eps ? (b - a) / row : 0 or proj = (b - a) row
+struct FpStore {
+    enum Mode { kSet, kAdd, kResidualDivide, kResidualMultiply };
+    int mode;
+    float eps;
+    const float* b;             // views b_view floats apart
+    const float* row;           // as proj
+    size_t b_view;
+};
+
 // Joseph projection from volume copies
 struct JosephSepFpLaunch {
     const float* vol_zx;        // copy for X-main views (may be null if none)
@@ -300,7 +311,7 @@ struct JosephSepFpLaunch {
     const ProjViewDev* views;   // device, `count`
     VolumeGeom vol;
     int nu, nv, count;
-    int accumulate;
+    FpStore store;
 };
 // separable views, from Z-fastest copies (launch_joseph_column_copy) of
 // joseph_column_size floats: [slice][row][z] of a [z][y][x] volume, slices along

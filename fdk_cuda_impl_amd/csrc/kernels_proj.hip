@@ -1350,12 +1350,20 @@ void launch_joseph_column_copy(const float* in, float* out, int nx, int ny, int 
 
 namespace {
 
+// Columns from which a column's slices are split over four waves instead of
+// eight (each wave forms tables for its part and leaves a sum): 12 views of 256 x
+// 192 at 128^3 (3072 columns) 78.6 -> 71.8 us, 30 of 128 x 96 at 64^3 (3840) 56.5
+// -> 49.5; one view (256 and 128 columns) 31.9 -> 35.9 and 23.6 -> 25.4.  Between,
+// eight keep a view's rounding the same however few views a call has.
+constexpr size_t kFewColumns = 2048;
+
 template <int K, bool SPLIT>
 void launch_column_kernel(const JosephSepFpLaunch& p, hipStream_t s)
 {
     const size_t column = size_t(column_words(p.vol.nz, K, SPLIT)) * sizeof(float);
     // the waves' columns in 32 KiB; a longer column has a workgroup to itself
-    const int waves = column <= 4096 ? kColumnWaves : column <= 8192 ? 4 : column <= 16384 ? 2 : 1;
+    int waves = column <= 4096 ? kColumnWaves : column <= 8192 ? 4 : column <= 16384 ? 2 : 1;
+    if (SPLIT && size_t(p.nu) * p.count >= kFewColumns) waves = std::min(waves, 4);
     if (waves == 1)
         YK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(joseph_fp_column_kernel<K, SPLIT>),
             hipFuncAttributeMaxDynamicSharedMemorySize, int(column)));

@@ -46,3 +46,17 @@ def test_forward_matches_oracle(ctx, oracle, name):
     acc = P.forward(torch.from_numpy(x).cuda(), out=torch.ones(g.total_views, g.nv, g.nu, device="cuda"),
                     accumulate=True).cpu().numpy()
     assert rel_rmse(acc - 1.0, ref) < 2e-5 * index
+
+
+@pytest.mark.parametrize("views", [19, 18])
+@pytest.mark.parametrize("volume", [(23, 21, 18), (5, 70, 9)])
+def test_split_over_four_and_eight_waves(ctx, oracle, views, volume):
+    """2052 and 1944 columns: either side of the split of a column's slices over fewer waves."""
+    g = small_geometry(total_views=views, views_per_turn=views, channels=108, channel_mm=0.4, volume=volume, start_angle_rad=0.1,
+                       offset_unv_mm=(0.3, 0.0, 0.2))
+    P = yk.Projector(ctx, g.views(), g.nu, g.nv, g.grid())
+    x = np.random.default_rng(8).random((volume[2], volume[1], volume[0])).astype(np.float32)
+    got = P.forward(torch.from_numpy(x).cuda()).cpu().numpy()
+    ref = oracle.fp_joseph(oracle.views_from_float(P.views), g.nu, g.nv, oracle_volume(oracle, g), x)
+    assert rel_rmse(got, ref) < 1e-5, rel_rmse(got, ref)
+    assert max_abs(got, ref) < 1e-4 * np.abs(ref).max()

@@ -641,7 +641,7 @@ yk_status yk_tv_gradient(yk_ctx* ctx, const yk_volume_grid* volume, const float*
         validate_volume(*volume);
         require(std::isfinite(eps) && eps > 0.f, YK_ERR_INVALID_CONFIG, "epsilon must be positive");
         ctx->activate();
-        const int parts = 1024;
+        const int parts = kTvPartials;
         ctx->reduce_scratch.resize(parts);
         launch_tv_gradient(d_x, d_gradient, ctx->reduce_scratch.get(), parts, volume_geom(*volume), eps,
             ctx->stream);
@@ -662,7 +662,7 @@ yk_status yk_dot(yk_ctx* ctx, const float* a, const float* b, size_t n, double* 
         require(ctx && a && b && out, YK_ERR_INVALID_BUFFER, "null argument");
         ctx->activate();
         const int parts = int(std::min<size_t>(1024, std::max<size_t>(1, (n + 255) / 256)));
-        ctx->reduce_scratch.resize(1024);
+        ctx->reduce_scratch.resize(kTvPartials);
         launch_dot(a, b, n, ctx->reduce_scratch.get(), parts, ctx->stream);
         std::vector<double> h(parts);
         YK_HIP(hipMemcpyAsync(h.data(), ctx->reduce_scratch.get(), parts * sizeof(double),

@@ -132,28 +132,46 @@ __device__ __forceinline__ void tv_field(const float* __restrict__ x, int i, int
 // gradient = -div(grad x / sqrt(|grad x|^2 + eps^2)), value = sum sqrt(...)
 // (YkTvRegularizationKernels.cu:41-73; doc/algorithms.md:257-261)
 // (iz = 0: the slice-wise 2-D form, no z differences; TvDimensionality::Slice2D)
+// A workgroup takes 256 voxels of a plane at a time, so a voxel costs one 32-bit
+// division for its place (Index; 64 bits for planes past 2^31 voxels) where three
+// 64-bit ones were over half its instructions.  Bound: VALU issue (four square
+// roots and six divisions a voxel).
+template <typename Index>
 __global__ void __launch_bounds__(kThreads)
 tv_kernel(const float* __restrict__ x, float* __restrict__ grad, double* __restrict__ partials,
     VolumeGeom g, float eps, float iz)
 {
     __shared__ double red[kThreads / 64];
     const float ix = 1.f / g.vx, iy = 1.f / g.vy;
-    const size_t n = (size_t)g.nx * g.ny * g.nz;
+    const Index nx = Index(g.nx), plane = nx * Index(g.ny);
+    const Index chunks = (plane + (kThreads - 1)) / kThreads;  // of a plane
+    // (plane k, chunk) of the items from blockIdx.x on in steps of the grid
+    const Index dk = gridDim.x / chunks, dchunk = gridDim.x - dk * chunks;
+    Index k = blockIdx.x / chunks, chunk = blockIdx.x - k * chunks;
     double val = 0.0;
-    for (size_t c = (size_t)blockIdx.x * kThreads + threadIdx.x; c < n; c += (size_t)gridDim.x * kThreads) {
-        const int i = int(c % g.nx);
-        const int j = int((c / g.nx) % g.ny);
-        const int k = int(c / ((size_t)g.nx * g.ny));
-        float px, py, pz, den, qx, qy, qz, d2;
-        tv_field(x, i, j, k, g, ix, iy, iz, eps, px, py, pz, den);
-        val += den;
-        float div = 0.f;
-        float pxm = 0.f, pym = 0.f, pzm = 0.f;
-        if (i > 0) { tv_field(x, i - 1, j, k, g, ix, iy, iz, eps, qx, qy, qz, d2); pxm = qx; }
-        if (j > 0) { tv_field(x, i, j - 1, k, g, ix, iy, iz, eps, qx, qy, qz, d2); pym = qy; }
-        if (k > 0) { tv_field(x, i, j, k - 1, g, ix, iy, iz, eps, qx, qy, qz, d2); pzm = qz; }
-        div = (px - pxm) * ix + (py - pym) * iy + (pz - pzm) * iz;
-        if (grad) grad[c] = -div;
+    while (k < Index(g.nz)) {
+        const Index p = chunk * kThreads + threadIdx.x;
+        if (p < plane) {
+            const int j = int(p / nx), i = int(p - Index(j) * nx);
+            const size_t c = size_t(k) * plane + p;
+            const int z = int(k);
+            float px, py, pz, den, qx, qy, qz, d2;
+            tv_field(x, i, j, z, g, ix, iy, iz, eps, px, py, pz, den);
+            val += den;
+            float div = 0.f;
+            float pxm = 0.f, pym = 0.f, pzm = 0.f;
+            if (i > 0) { tv_field(x, i - 1, j, z, g, ix, iy, iz, eps, qx, qy, qz, d2); pxm = qx; }
+            if (j > 0) { tv_field(x, i, j - 1, z, g, ix, iy, iz, eps, qx, qy, qz, d2); pym = qy; }
+            if (z > 0) { tv_field(x, i, j, z - 1, g, ix, iy, iz, eps, qx, qy, qz, d2); pzm = qz; }
+            div = (px - pxm) * ix + (py - pym) * iy + (pz - pzm) * iz;
+            if (grad) grad[c] = -div;
+        }
+        k += dk;
+        chunk += dchunk;
+        if (chunk >= chunks) {
+            chunk -= chunks;
+            ++k;
+        }
     }
     const double s = block_sum(val, red);
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
@@ -256,8 +274,9 @@ void weight_prepare(float* x, float threshold, int reciprocal, size_t n, hipStre
 void launch_tv_gradient(const float* x, float* grad, double* partials, int n_partials,
     const VolumeGeom& g, float eps, hipStream_t s, int dims)
 {
-    hipLaunchKernelGGL(tv_kernel, dim3(n_partials), dim3(kThreads), 0, s, x, grad, partials, g, eps,
-        dims == 2 ? 0.f : 1.f / g.vz);
+    const bool wide = size_t(g.nx) * g.ny >= (size_t(1) << 31) - kThreads;
+    hipLaunchKernelGGL(wide ? tv_kernel<size_t> : tv_kernel<unsigned>, dim3(n_partials), dim3(kThreads), 0, s, x, grad, partials,
+        g, eps, dims == 2 ? 0.f : 1.f / g.vz);
     YK_HIP(hipGetLastError());
 }
 

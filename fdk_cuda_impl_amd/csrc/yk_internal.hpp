@@ -501,6 +501,10 @@ void launch_bounds_clamp(float* x, int use_min, float lo, int use_max, float hi,
 // x <= threshold -> 1e30, then optionally x = 1 / x
 void weight_prepare(float* x, float threshold, int reciprocal, size_t n, hipStream_t s);
 // smoothed TV value partials and gradient; dims 3 (volume) or 2 (each z slice alone)
+// (16 workgroups a CU: with four, and three 64-bit divisions a voxel for its
+// place, an OS-SART sweep with three steps on 1.6 million voxels took 1.304 ms
+// instead of 1.285)
+constexpr int kTvPartials = 4096;
 void launch_tv_gradient(const float* x, float* grad, double* partials, int n_partials,
     const VolumeGeom& g, float eps, hipStream_t s, int dims = 3);
 void launch_phantom(const float* ellipsoids, int n, const VolumeGeom& g, int clamp,

@@ -161,6 +161,7 @@ struct yk_projector {
     yk::DeviceArray<float> d_vol_t;
     yk::DeviceArray<float> d_vol_zx;   // paired volume copies of the Joseph and Siddon projections
     yk::DeviceArray<float> d_vol_zy;
+    std::vector<char> siddon_main;     // per view: no ray runs across the main axis
     std::vector<char> siddon_flat;     // per view: a ray's x and y depend on the column alone, its z on the row
     std::vector<char> joseph_column;   // per view: the column transpose covers it
     yk::DeviceArray<float> d_column_x, d_column_y;  // its volumes of the X- and Y-main views

@@ -18,19 +18,20 @@
 // candidates in FP32 steps.
 //
 // Siddon: the segment of a ray in a voxel lies between its crossings of the
-// voxel's six planes, (plane - src) * (1 / ray); the reciprocals come from a
-// table of the view's rays (16 bytes with p |ray|) instead of three divisions
-// per candidate.
+// voxel's six planes, at (plane - src) * (main / minor component) along the main
+// axis; the quotients come from a table of the view's rays (12 bytes with
+// p |ray / main|) instead of three divisions per candidate.
 //
 // 256^3 x 360 views of 512 x 384, detector tilted: Joseph 118.7 -> 15.9 ms,
 // Siddon 139.7 -> 20.9 ms against one thread per voxel with every candidate's
-// line evaluated; untilted 25.5 -> 15.8 and 39.5 -> 20.6 ms against lane
-// columns over column-major ray tables (64^3 x 60 views of 128 x 96: 1.15 ->
-// 0.09 and 1.75 -> 0.12 ms).  Medians in place of sorted Siddon intervals took
-// a forward and a transpose of 240 x 231 x 190 x 240 views of 480 x 360, tilted,
-// from 18.0 to 15.8 ms.  Bound: VALU issue (Joseph: 324 instructions a
-// voxel pair and view, of which 218 weigh its 5.4 rows of 4 candidates; the
-// texture addressers are 63 % busy).
+// line evaluated; then, for Siddon, medians in place of sorted intervals -> 16.5
+// and quotients along the main axis (12 bytes and 14 instructions a candidate
+// for 16 and 16) -> 16.1.  64^3 x 60 views of 128 x 96: 1.15 -> 0.09 and 1.75 ->
+// 0.11 ms.  Untilted views have forms of their own where they are faster
+// (kernels_column.hip, siddon_flat_gather).
+// Bound: VALU issue (Joseph: 324 instructions a voxel pair and view, of which 218
+// weigh its 5.4 rows of 4 candidates; the texture addressers are 63 % busy;
+// Siddon: its six 12-byte loads for 84 instructions keep those busier).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -77,26 +78,31 @@ joseph_gather_table_kernel(const float* __restrict__ proj, const ProjViewDev* __
     q[((size_t)i * gridDim.y + v) * pitch + u] = w;
 }
 
-// (1 / ray, p |ray|) of every ray, same layout; a component the ray does not
-// move along (below 1e-8 mm) has a reciprocal so large that its cell either
-// bounds nothing or leaves no segment
+// (main / first minor, main / z component, p |ray / main|) of every ray, same
+// layout; a minor component the ray does not move along (below 1e-8 mm) has a
+// quotient so large that its cell either bounds nothing or leaves no segment
 __global__ void __launch_bounds__(256)
-siddon_gather_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __restrict__ views, int nu, int nv,
-    int pitch, float4* __restrict__ q, int* __restrict__ flag)
+siddon_gather_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __restrict__ views,
+    const GatherViewDev* __restrict__ gviews, int nu, int nv, int pitch, float* __restrict__ q, int* __restrict__ flag)
 {
     const int u = blockIdx.x * 256 + threadIdx.x;
     const int v = blockIdx.y, i = blockIdx.z;
     if (u >= pitch) return;
-    float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+    float r1 = 0.f, r2 = 0.f, w = 0.f;
     if (u < nu && v < nv) {
-        float src[3], ray[3], rc[3];
+        float src[3], ray[3];
         siddon_ray_geom(views[i], u, v, src, ray);
-        for (int k = 0; k < 3; ++k) rc[k] = fabsf(ray[k]) > 1e-8f ? 1.f / ray[k] : 1e30f;
-        const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
-        w = make_float4(rc[0], rc[1], rc[2], proj[((size_t)i * nv + v) * nu + u] * len);
-        if (!(fabsf(w.w) <= 3.4e38f)) atomicOr(flag, 1);
+        const bool xmain = gviews[i].axis == 0;
+        const float m0 = xmain ? ray[0] : ray[1], m1 = xmain ? ray[1] : ray[0];
+        r1 = fabsf(m1) > 1e-8f ? m0 / m1 : 1e30f;
+        r2 = fabsf(ray[2]) > 1e-8f ? m0 / ray[2] : 1e30f;
+        w = proj[((size_t)i * nv + v) * nu + u] * (sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]) / fabsf(m0));
+        if (!(fabsf(w) <= 3.4e38f)) atomicOr(flag, 1);
     }
-    q[((size_t)i * gridDim.y + v) * pitch + u] = w;
+    float* dst = q + 3 * (((size_t)i * gridDim.y + v) * pitch + u);
+    dst[0] = r1;
+    dst[1] = r2;
+    dst[2] = w;
 }
 
 // The same of views whose detector rows and columns lie along the main axes'
@@ -265,7 +271,7 @@ __device__ __forceinline__ void joseph_gather(const float* __restrict__ q, const
 __device__ __forceinline__ float plane_offset(float lo, float vox, int c, float s) { return lo + float(c) * vox - s; }
 
 template <int ZR, bool SAFE>
-__device__ __forceinline__ void siddon_gather(const float4* __restrict__ q, const GatherViewDev* __restrict__ views,
+__device__ __forceinline__ void siddon_gather(const float* __restrict__ q, const GatherViewDev* __restrict__ views,
     const SiddonViewDev* __restrict__ sviews, const VolumeGeom& g, int nu, int nv, int pitch, int count, int x, int y,
     int z0, float (&acc)[ZR])
 {
@@ -275,11 +281,13 @@ __device__ __forceinline__ void siddon_gather(const float4* __restrict__ q, cons
     const float lox = g.ox - 0.5f * g.vx, loy = g.oy - 0.5f * g.vy, loz = g.oz - 0.5f * g.vz;
 #pragma unroll 1
     for (int i = 0; i < count; ++i) {
-        const float4* qi = q + (size_t)i * (nv + kGatherPadRows) * pitch;
+        const float* qi = q + 3 * ((size_t)i * (nv + kGatherPadRows) * pitch);
         const CandidateBox<ZR> box(views[i], x, y, z0, 0.5f, 0.5f, 1.f);
         const SiddonViewDev& sv = sviews[i];
         const float x0 = plane_offset(lox, g.vx, x, sv.src[0]), x1 = plane_offset(lox, g.vx, x + 1, sv.src[0]);
         const float y0 = plane_offset(loy, g.vy, y, sv.src[1]), y1 = plane_offset(loy, g.vy, y + 1, sv.src[1]);
+        const bool xmain = views[i].axis == 0;
+        const float m0 = xmain ? x0 : y0, m1 = xmain ? x1 : y1, n0 = xmain ? y0 : x0, n1 = xmain ? y1 : x1;
 #pragma unroll
         for (int p = 0; p < ZR; p += 2) {
             int ulo, uhi, vlo, vhi;
@@ -292,30 +300,30 @@ __device__ __forceinline__ void siddon_gather(const float4* __restrict__ q, cons
             for (int v = vlo; v <= vhi; v += kRows) {
 #pragma unroll 1
                 for (int u = ulo; u <= uhi; u += kWidth) {
-                    float4 w[kRows][kWidth];
+                    float3a4 w[kRows][kWidth];
 #pragma unroll
                     for (int j = 0; j < kRows; ++j)
 #pragma unroll
-                        for (int k = 0; k < kWidth; ++k) w[j][k] = qi[row + unsigned(j * pitch + u + k)];
+                        for (int k = 0; k < kWidth; ++k)
+                            w[j][k] = *reinterpret_cast<const float3a4*>(qi + 3u * (row + unsigned(j * pitch + u + k)));
 #pragma unroll
                     for (int j = 0; j < kRows; ++j)
 #pragma unroll
                         for (int k = 0; k < kWidth; ++k) {
-                            const float4 c = w[j][k];
-                            const float tx0 = x0 * c.x, tx1 = x1 * c.x, ty0 = y0 * c.y, ty1 = y1 * c.y;
-                            // The ray is between the voxel's planes along x while t
-                            // lies between tx0 and tx1, whichever is less; a median
-                            // moves the y planes into that interval and the z planes
-                            // into what is left (empty: onto one point), with no
-                            // interval sorted.  25 -> 16 instructions a candidate
-                            // against sorted ends, with the same differences.
-                            const float y0t = __builtin_amdgcn_fmed3f(ty0, tx0, tx1), y1t = __builtin_amdgcn_fmed3f(ty1, tx0, tx1);
-                            const float ta = __builtin_amdgcn_fmed3f(za * c.z, y0t, y1t);
-                            const float tb = __builtin_amdgcn_fmed3f(zb * c.z, y0t, y1t);
-                            const float tc = __builtin_amdgcn_fmed3f(zc * c.z, y0t, y1t);
+                            const float3a4 c = w[j][k];
+                            // Along the main axis the ray is between the voxel's
+                            // planes from m0 to m1; a median moves the crossings of
+                            // the minor planes into that interval and those of the z
+                            // planes into what is left (empty: onto one point), with
+                            // no interval sorted.  25 -> 14 instructions a candidate
+                            // against sorted ends of three axes.
+                            const float na = __builtin_amdgcn_fmed3f(n0 * c.x, m0, m1), nb = __builtin_amdgcn_fmed3f(n1 * c.x, m0, m1);
+                            const float ta = __builtin_amdgcn_fmed3f(za * c.y, na, nb);
+                            const float tb = __builtin_amdgcn_fmed3f(zb * c.y, na, nb);
+                            const float tc = __builtin_amdgcn_fmed3f(zc * c.y, na, nb);
                             const float sa = fabsf(tb - ta), sb = fabsf(tc - tb);
-                            if (!SAFE || sa > 0.f) acc[p] = fmaf(sa, c.w, acc[p]);
-                            if (!SAFE || sb > 0.f) acc[p + 1] = fmaf(sb, c.w, acc[p + 1]);
+                            if (!SAFE || sa > 0.f) acc[p] = fmaf(sa, c.z, acc[p]);
+                            if (!SAFE || sb > 0.f) acc[p + 1] = fmaf(sb, c.z, acc[p + 1]);
                         }
                 }
                 row += unsigned(kRows * pitch);
@@ -327,7 +335,8 @@ __device__ __forceinline__ void siddon_gather(const float4* __restrict__ q, cons
 // Views of siddon_flat_table_kernel.  Depth, the candidate columns and the part
 // of each column's rays over the voxel column's x and y planes hold for the
 // whole run, and a row's z planes for all its candidates, so a candidate takes 7
-// instructions and 4 bytes where siddon_gather takes 16 and 16: 256^3 x 360
+// instructions and 4 bytes where siddon_gather takes 14 and 12.  Against 16
+// and 16: 256^3 x 360
 // views of 512 x 384 17.2 -> 10.4 ms, 128^3 x 120 891 -> 570 us, 64^3 x 60 116
 // -> 102.  (Pixels x rows a chunk at 256^3: 3 x 1 12.9 ms, 3 x 3 11.2, 2 x 2
 // 22.3, 4 x 2 10.9.)
@@ -411,7 +420,7 @@ gather_transpose_kernel(const void* __restrict__ q, const float2* __restrict__ r
         if (plain) siddon_flat_gather<ZR, false>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
         else siddon_flat_gather<ZR, true>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
     } else if constexpr (MODEL == kGatherSiddon) {
-        const float4* t = static_cast<const float4*>(q);
+        const float* t = static_cast<const float*>(q);
         if (plain) siddon_gather<ZR, false>(t, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
         else siddon_gather<ZR, true>(t, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
     } else {
@@ -462,8 +471,8 @@ void launch_gather_transpose(const GatherLaunch& p, hipStream_t s)
             p.flag);
         launch_gather<kGatherSiddonFlat>(p, s);
     } else if (p.model == kGatherSiddon) {
-        hipLaunchKernelGGL(siddon_gather_table_kernel, tg, dim3(256), 0, s, p.proj, p.sviews, p.nu, p.nv, p.pitch,
-            reinterpret_cast<float4*>(p.q), p.flag);
+        hipLaunchKernelGGL(siddon_gather_table_kernel, tg, dim3(256), 0, s, p.proj, p.sviews, p.gviews, p.nu, p.nv,
+            p.pitch, p.q, p.flag);
         launch_gather<kGatherSiddon>(p, s);
     } else {
         hipLaunchKernelGGL(joseph_gather_table_kernel, tg, dim3(256), 0, s, p.proj, p.views, p.gviews, p.vol, p.nu, p.nv,

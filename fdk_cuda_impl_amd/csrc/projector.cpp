@@ -89,6 +89,24 @@ void gather_view(const ViewD& w, int axis, int nu, int nv, const double map[12],
     }
 }
 
+// No ray of the view runs across its main axis: the general Siddon gather
+// measures segments along that axis
+bool along_main(const ViewD& w, int axis, int nu, int nv)
+{
+    double sign = 0.0;
+    for (int a = 0; a < 4; ++a) {
+        double r[3], len2 = 0.0;
+        for (int k = 0; k < 3; ++k) {
+            r[k] = w.detS[k] + ((a & 1) ? nu - 1 : 0) * w.detU[k] + ((a & 2) ? nv - 1 : 0) * w.detV[k] - w.src[k];
+            len2 += r[k] * r[k];
+        }
+        // (linear over the detector: its corners bound it)
+        if (sign == 0.0) sign = r[axis] < 0.0 ? -1.0 : 1.0;
+        if (!(sign * r[axis] > 1e-3 * std::sqrt(len2))) return false;
+    }
+    return true;
+}
+
 // The column transpose takes separable views in which at most eight rays of a
 // detector column pass within a voxel along z, of a detector whose row
 // numbers times FP32 rounding stay far below its 0.01 pixels of margin
@@ -187,12 +205,14 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
             joseph_gather.push_back(least > 1e-3);
             siddon_gather.push_back(least > 1e-3 && outer < 1.0);
             siddon_flat.push_back(separable.back() && w.detU[2] == 0.f);
+            siddon_main.push_back(along_main(widen(w), p.axis, nu, nv));
             joseph_column.push_back(separable.back() && joseph_gather.back() && column_view(p, nu, nv, vol));
         } else {
             joseph_gather.push_back(0);
             siddon_gather.push_back(0);
             joseph_column.push_back(0);
             siddon_flat.push_back(0);
+            siddon_main.push_back(0);
         }
     }
     d_gather.upload(gv.data(), gv.size(), ctx->stream);
@@ -484,10 +504,13 @@ bool yk_projector::gather_transpose(yk_projector& w, bool siddon, const float* d
     if (!std::all_of(ok.begin() + first, ok.begin() + first + count, [](char c) { return c != 0; })) return false;
     const bool flat = siddon && std::all_of(siddon_flat.begin() + first, siddon_flat.begin() + first + count,
         [](char c) { return c != 0; });
+    if (siddon && !flat && !std::all_of(siddon_main.begin() + first, siddon_main.begin() + first + count,
+        [](char c) { return c != 0; }))
+        return false;
     const int pitch = nu + kGatherPad;
     // floats (flat: an entry a column and a row more, columns' aligned to 8 bytes)
     const size_t rows = size_t(nv) + kGatherPadRows;
-    const size_t per_view = flat ? rows * pitch + 2 * size_t(pitch) + rows + 1 : rows * pitch * (siddon ? 4 : 1);
+    const size_t per_view = flat ? rows * pitch + 2 * size_t(pitch) + rows + 1 : rows * pitch * (siddon ? 3 : 1);
     if (nv + kGatherPadRows > 65535 || per_view > (size_t(1) << 30)) return false;
     const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
     if (w.d_gather_q.size() < per_view * chunk || !w.d_flag.get()) {

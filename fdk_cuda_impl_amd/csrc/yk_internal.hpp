@@ -364,7 +364,7 @@ struct GatherLaunch {
     const ProjViewDev* views;   // device, `count` (Joseph)
     const SiddonViewDev* sviews; // device, `count` (Siddon)
     const GatherViewDev* gviews; // device, `count`
-    float* q;                   // scratch [count][nv + kGatherPadRows][pitch] floats or float4s (kGatherSiddon)
+    float* q;                   // scratch [count][nv + kGatherPadRows][pitch] floats or float triples (kGatherSiddon)
     float2* ru;                 // scratch [count][pitch] (kGatherSiddonFlat)
     float* rv;                  // scratch [count][nv + kGatherPadRows] (kGatherSiddonFlat)
     int* flag;                  // scratch word

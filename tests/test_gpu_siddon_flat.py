@@ -60,3 +60,14 @@ def test_extreme_pixel_reaches_only_its_voxels(ctx, oracle, value):
     # (a ray within rounding of a voxel's edge may or may not meet it)
     assert np.isfinite(got[clear]).mean() > 0.999
     assert (np.abs(got[clear] - plain[clear]) <= 1e-5 * np.abs(plain).max()).mean() > 0.999
+
+
+def test_rays_across_the_main_axis(ctx, oracle):
+    """Tilted views with rays perpendicular to their main axis, which the general gather leaves to the search."""
+    g = small_geometry(sid_mm=40.0, sdd_mm=60.0, channels=170, channel_mm=1.0, tilt_rad=(0.02, 0.01, -0.03), volume=(24, 22, 18),
+                       start_angle_rad=0.78, offset_unv_mm=(0.3, 0.0, 0.2), total_views=3, views_per_turn=7)
+    P = yk.Projector(ctx, g.views(), g.nu, g.nv, g.grid())
+    y = np.random.default_rng(23).standard_normal((g.total_views, g.nv, g.nu)).astype(np.float32)
+    got = P.adjoint(torch.from_numpy(y).cuda(), kind="siddon").cpu().numpy()
+    tol = max(2e-5, 3.0 * 2.0**-24 * g.sdd_mm / min(g.voxel_mm))
+    assert rel_rmse(got, reference(oracle, g, P, y)) < tol

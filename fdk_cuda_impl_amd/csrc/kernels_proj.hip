@@ -13,11 +13,11 @@
 // src/FlatFpBp/FP/kernels/YkFPSiddonKernel.cu:19-124); voxel boundaries are
 // recomputed from integer indices instead of accumulated.
 //
-// Transposes are deterministic gathers (no atomics): for each voxel and view
-// the candidate rays are the detector pixels inside the projection of the
-// voxel's support, and each candidate ray is re-evaluated with exactly the
-// arithmetic of the forward kernel (shared functions below, FP contraction
-// off), so <A x, y> = <x, A^T y> up to summation order.
+// Transposes are deterministic gathers (no atomics).  The ones here serve the
+// views that kernels_gather.hip and kernels_column.hip leave: for each voxel and
+// view the candidate rays are the detector pixels inside the projection of the
+// voxel's support, and each is re-evaluated with exactly the arithmetic of the
+// forward kernel (shared functions below, FP contraction off).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

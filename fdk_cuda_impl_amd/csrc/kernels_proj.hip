@@ -1102,7 +1102,13 @@ siddon_adjoint_kernel(const float* __restrict__ proj, float* __restrict__ volume
 //   (ties X, then Y): v_m |d| / |d_m|.
 constexpr int kOpBpZ = 8;
 constexpr int kOpBpShortZ = 2;
-constexpr int kViewGuard = 1;  // zero pixels around a paired view
+// zero pixels before and after a paired view's rows and columns: two, as both
+// taps of a sample clamped off the detector must be zeros (one zero and one pixel
+// of weight zero would spread a pixel that is not finite)
+constexpr int kViewGuard = 2;
+// entries of a paired view's row, and its rows (the last one pairs with zeros)
+__host__ __device__ __forceinline__ int paired_pitch(int nu) { return nu + 2 * kViewGuard; }
+__host__ __device__ __forceinline__ int paired_rows(int nv) { return nv + 2 * kViewGuard - 1; }
 enum OpBpMode { kOpFdk = 0, kOpMatched = 1, kOpJosephVoxel = 2 };
 
 __device__ __forceinline__ float bilinear_view(const float* __restrict__ p, int nu, int nv, float u, float v)
@@ -1217,7 +1223,7 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
 #pragma unroll
     for (int k = 0; k < ZR; ++k) acc[k] = 0.f;
     const float ivz = 1.f / g.vz;
-    const int pitch = nu + 2 * kViewGuard + 1, rows = nv + 2 * kViewGuard;
+    const int pitch = paired_pitch(nu), rows = paired_rows(nv);
 #pragma unroll 1
     for (int i = 0; i < count; ++i) {
         const OpBpViewDev& c = views[i];
@@ -1241,7 +1247,8 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
         };
         if constexpr (PAIRED) {
             const char* p = reinterpret_cast<const char*>(proj) + size_t(i * view_step) * rows * pitch * 8u;
-            const float umax = float(nu + 1), vmax = float(nv + 1);
+            constexpr float kGuard = float(kViewGuard);
+            const float umax = float(nu) + kGuard, vmax = float(nv) + kGuard;
             const unsigned row_bytes = unsigned(pitch) * 8u;
 #pragma unroll
             for (int k0 = 0; k0 < ZR; k0 += kBatch) {
@@ -1253,10 +1260,10 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
                     float Z, un, vn, rd;
                     on[k] = project(k0 + k, Z, un, vn, rd);
                     w[k] = col.weight(c, ivz, scale, Z, un * rd, vn * rd, on[k]);
-                    // positions in the copy (pixel + guard); past its guards
-                    // the clamped sample lies on zeros only
-                    const float u = __builtin_amdgcn_fmed3f(fmaf(un, rd, 1.f), 0.f, umax);
-                    const float v = __builtin_amdgcn_fmed3f(fmaf(vn, rd, 1.f), 0.f, vmax);
+                    // positions in the copy (pixel + guard); a clamped sample
+                    // lies on guards only
+                    const float u = __builtin_amdgcn_fmed3f(fmaf(un, rd, kGuard), 0.f, umax);
+                    const float v = __builtin_amdgcn_fmed3f(fmaf(vn, rd, kGuard), 0.f, vmax);
                     a[k] = __builtin_amdgcn_fractf(u);
                     b[k] = __builtin_amdgcn_fractf(v);
                     q[k] = *reinterpret_cast<const float4u*>(p + (__umul24(unsigned(int(v)), row_bytes) + unsigned(int(u)) * 8u));
@@ -1302,14 +1309,13 @@ fdk_operator_bp_kernel(const float* __restrict__ proj, float* __restrict__ volum
 }
 
 // Paired guarded copy of `count` views: entry (row r, column c) holds pixels
-// (r, c) and (r + 1, c), for rows and columns from -kViewGuard up to one guard
-// past the last (and a further column, read with the last guard), zero
-// outside the detector.
+// (r, c) and (r + 1, c), for rows and columns from -kViewGuard up to the last
+// guard column and the last guard row but one, zero outside the detector.
 __global__ void __launch_bounds__(256)
 pair_views_kernel(const float* __restrict__ proj, float2* __restrict__ out, int nu, int nv)
 {
     const int e = blockIdx.x * 256 + threadIdx.x;
-    const int pitch = nu + 2 * kViewGuard + 1;
+    const int pitch = paired_pitch(nu);
     if (e >= pitch) return;
     const int c = e - kViewGuard, r = int(blockIdx.y) - kViewGuard;
     const float* p = proj + size_t(blockIdx.z) * nu * nv;
@@ -1499,7 +1505,7 @@ void launch_siddon_adjoint(const SiddonAdjointLaunch& p, hipStream_t s)
     YK_HIP(hipGetLastError());
 }
 
-size_t paired_view_floats(int nu, int nv) { return size_t(nv + 2 * kViewGuard) * (nu + 2 * kViewGuard + 1) * 2; }
+size_t paired_view_floats(int nu, int nv) { return size_t(paired_rows(nv)) * paired_pitch(nu) * 2; }
 
 namespace {
 
@@ -1536,7 +1542,7 @@ void launch_op(const OpBpLaunch& p, hipStream_t s)
 void launch_fdk_operator_bp(const OpBpLaunch& p, hipStream_t s)
 {
     if (p.paired) {
-        dim3 grid((p.nu + 2 * kViewGuard + 1 + 255) / 256, p.nv + 2 * kViewGuard, p.one_view ? 1 : p.count);
+        dim3 grid((paired_pitch(p.nu) + 255) / 256, paired_rows(p.nv), p.one_view ? 1 : p.count);
         hipLaunchKernelGGL(pair_views_kernel, grid, dim3(256), 0, s, p.proj, reinterpret_cast<float2*>(p.paired), p.nu, p.nv);
     }
     if (p.mode == kOpMatched) launch_op<kOpMatched>(p, s);

@@ -80,11 +80,14 @@ joseph_gather_table_kernel(const float* __restrict__ proj, const ProjViewDev* __
 }
 
 // (main / first minor, main / z component, p |ray / main|) of every ray, same
-// layout; a minor component the ray does not move along (below 1e-8 mm) has a
-// quotient so large that its cell either bounds nothing or leaves no segment
+// layout; a minor component the ray does not move along (siddon_stays) has a
+// quotient so large that its cell either bounds nothing or leaves no segment,
+// with the main component's sign: the cell's upper plane is then always the
+// farther one along the ray
 __global__ void __launch_bounds__(256)
 siddon_gather_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __restrict__ views,
-    const GatherViewDev* __restrict__ gviews, int nu, int nv, int pitch, float* __restrict__ q, int* __restrict__ flag)
+    const GatherViewDev* __restrict__ gviews, VolumeGeom g, int nu, int nv, int pitch, float* __restrict__ q,
+    int* __restrict__ flag)
 {
     const int u = blockIdx.x * 64 + threadIdx.x;
     const int v = blockIdx.y * 4 + threadIdx.y, i = blockIdx.z;
@@ -92,12 +95,16 @@ siddon_gather_table_kernel(const float* __restrict__ proj, const SiddonViewDev* 
     if (u >= pitch || v >= rows) return;
     float r1 = 0.f, r2 = 0.f, w = 0.f;
     if (u < nu && v < nv) {
-        float src[3], ray[3];
-        siddon_ray_geom(views[i], u, v, src, ray);
+        double r[3];
+        siddon_ray_geom(views[i], u, v, r);
         const bool xmain = gviews[i].axis == 0;
+        const int n0 = xmain ? g.nx : g.ny, n1 = xmain ? g.ny : g.nx;
+        const double along = (xmain ? r[0] : r[1]) * (xmain ? g.vy * g.vz : g.vx * g.vz);  // (cells, times vx vy vz)
+        const float ray[3] = { float(r[0]), float(r[1]), float(r[2]) };
         const float m0 = xmain ? ray[0] : ray[1], m1 = xmain ? ray[1] : ray[0];
-        r1 = fabsf(m1) > 1e-8f ? m0 / m1 : 1e30f;
-        r2 = fabsf(ray[2]) > 1e-8f ? m0 / ray[2] : 1e30f;
+        const float far = copysignf(1e30f, m0);
+        r1 = siddon_stays((xmain ? r[1] : r[0]) * (xmain ? g.vx * g.vz : g.vy * g.vz), n1, along, n0) ? far : m0 / m1;
+        r2 = siddon_stays(r[2] * (g.vx * g.vy), g.nz, along, n0) ? far : m0 / ray[2];
         w = proj[((size_t)i * nv + v) * nu + u] * (sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]) / fabsf(m0));
         if (!(fabsf(w) <= 3.4e38f)) atomicOr(flag, 1);
     }
@@ -113,8 +120,8 @@ siddon_gather_table_kernel(const float* __restrict__ proj, const SiddonViewDev* 
 // [pitch] (1 / x, 1 / y), and one a row, rv [view][nv + kGatherPadRows]; q is
 // p |ray| alone.
 __global__ void __launch_bounds__(256)
-siddon_flat_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __restrict__ views, int nu, int nv, int pitch,
-    float* __restrict__ q, float2* __restrict__ ru, float* __restrict__ rv, int* __restrict__ flag)
+siddon_flat_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __restrict__ views, VolumeGeom g, int nu, int nv,
+    int pitch, float* __restrict__ q, float2* __restrict__ ru, float* __restrict__ rv, int* __restrict__ flag)
 {
     const int u = blockIdx.x * 64 + threadIdx.x;
     const int v = blockIdx.y * 4 + threadIdx.y, i = blockIdx.z;
@@ -128,9 +135,17 @@ siddon_flat_table_kernel(const float* __restrict__ proj, const SiddonViewDev* __
         if (!(fabsf(w) <= 3.4e38f)) atomicOr(flag, 1);
     }
     q[((size_t)i * rows + v) * pitch + u] = w;
-    auto quotient = [](float r) { return fabsf(r) > 1e-8f ? 1.f / r : 1e30f; };
-    if (v == 0) ru[(size_t)i * pitch + u] = make_float2(quotient(ray[0]), quotient(ray[1]));
-    if (u == 0) rv[(size_t)i * rows + v] = quotient(ray[2]);
+    if (u > 0 && v > 0) return;
+    double r[3];
+    siddon_ray_geom(views[i], u, v, r);
+    // (cells, times vx vy vz)
+    const double cx = r[0] * (g.vy * g.vz), cy = r[1] * (g.vx * g.vz), cz = r[2] * (g.vx * g.vy);
+    const bool xmain = fabs(cx) >= fabs(cy);
+    auto quotient = [](bool stays, double r) { return stays || r == 0.0 ? 1e30f : 1.f / float(r); };
+    if (v == 0)
+        ru[(size_t)i * pitch + u] = make_float2(quotient(!xmain && siddon_stays(cx, g.nx, cy, g.ny), r[0]),
+            quotient(xmain && siddon_stays(cy, g.ny, cx, g.nx), r[1]));
+    if (u == 0) rv[(size_t)i * rows + v] = quotient(siddon_stays(cz, g.nz, xmain ? cx : cy, xmain ? g.nx : g.ny), r[2]);
 }
 
 // Where the candidates of a lane's run of ZR voxels along z lie on one view.
@@ -270,8 +285,11 @@ __device__ __forceinline__ void joseph_gather(const float* __restrict__ q, const
     }
 }
 
-// offset of a cell plane from the source, as the forward walk forms it
-__device__ __forceinline__ float plane_offset(float lo, float vox, int c, float s) { return lo + float(c) * vox - s; }
+// offset of plane c between cells from the source; exactly zero on the source's own plane
+__device__ __forceinline__ float plane_offset(float lo, float vox, int c, float s, int plane)
+{
+    return c == plane ? 0.f : lo + float(c) * vox - s;
+}
 
 template <int ZR, bool SAFE>
 __device__ __forceinline__ void siddon_gather(const float* __restrict__ q, const GatherViewDev* __restrict__ views,
@@ -287,17 +305,19 @@ __device__ __forceinline__ void siddon_gather(const float* __restrict__ q, const
         const float* qi = q + 3 * ((size_t)i * (nv + kGatherPadRows) * pitch);
         const CandidateBox<ZR> box(views[i], x, y, z0, 0.5f, 0.5f, 1.f);
         const SiddonViewDev& sv = sviews[i];
-        const float x0 = plane_offset(lox, g.vx, x, sv.src[0]), x1 = plane_offset(lox, g.vx, x + 1, sv.src[0]);
-        const float y0 = plane_offset(loy, g.vy, y, sv.src[1]), y1 = plane_offset(loy, g.vy, y + 1, sv.src[1]);
+        const float x0 = plane_offset(lox, g.vx, x, sv.src[0], sv.plane[0]);
+        const float x1 = plane_offset(lox, g.vx, x + 1, sv.src[0], sv.plane[0]);
+        const float y0 = plane_offset(loy, g.vy, y, sv.src[1], sv.plane[1]);
+        const float y1 = plane_offset(loy, g.vy, y + 1, sv.src[1], sv.plane[1]);
         const bool xmain = views[i].axis == 0;
         const float m0 = xmain ? x0 : y0, m1 = xmain ? x1 : y1, n0 = xmain ? y0 : x0, n1 = xmain ? y1 : x1;
 #pragma unroll
         for (int p = 0; p < ZR; p += 2) {
             int ulo, uhi, vlo, vhi;
             if (!box.pair(z0 + p, nu, nv, ulo, uhi, vlo, vhi)) continue;
-            const float za = plane_offset(loz, g.vz, z0 + p, sv.src[2]);
-            const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.src[2]);
-            const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.src[2]);
+            const float za = plane_offset(loz, g.vz, z0 + p, sv.src[2], sv.plane[2]);
+            const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.src[2], sv.plane[2]);
+            const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.src[2], sv.plane[2]);
             unsigned row = unsigned(vlo) * unsigned(pitch);
 #pragma unroll 1
             for (int v = vlo; v <= vhi; v += kRows) {
@@ -357,8 +377,10 @@ __device__ __forceinline__ void siddon_flat_gather(const float* __restrict__ q, 
         const float* rvi = rv + rows;
         const CandidateBox<ZR> box(views[i], x, y, z0, 0.5f, 0.5f, 1.f);
         const SiddonViewDev& sv = sviews[i];
-        const float x0 = plane_offset(lox, g.vx, x, sv.src[0]), x1 = plane_offset(lox, g.vx, x + 1, sv.src[0]);
-        const float y0 = plane_offset(loy, g.vy, y, sv.src[1]), y1 = plane_offset(loy, g.vy, y + 1, sv.src[1]);
+        const float x0 = plane_offset(lox, g.vx, x, sv.src[0], sv.plane[0]);
+        const float x1 = plane_offset(lox, g.vx, x + 1, sv.src[0], sv.plane[0]);
+        const float y0 = plane_offset(loy, g.vy, y, sv.src[1], sv.plane[1]);
+        const float y1 = plane_offset(loy, g.vy, y + 1, sv.src[1], sv.plane[1]);
         const int ulo = int(fmaxf(0.f, ceilf(box.um - box.hu))), uhi = int(fminf(float(nu - 1), floorf(box.um + box.hu)));
 #pragma unroll 1
         for (int u = ulo; u <= uhi; u += kWidth) {
@@ -374,9 +396,9 @@ __device__ __forceinline__ void siddon_flat_gather(const float* __restrict__ q, 
             for (int p = 0; p < ZR; p += 2) {
                 const float vc = fmaf(box.v_zd, float(p) + 0.5f - 0.5f * float(ZR - 1), box.vm);
                 const int vlo = int(fmaxf(0.f, ceilf(vc - box.hv))), vhi = int(fminf(float(nv - 1), floorf(vc + box.hv)));
-                const float za = plane_offset(loz, g.vz, z0 + p, sv.src[2]);
-                const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.src[2]);
-                const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.src[2]);
+                const float za = plane_offset(loz, g.vz, z0 + p, sv.src[2], sv.plane[2]);
+                const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.src[2], sv.plane[2]);
+                const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.src[2], sv.plane[2]);
                 unsigned row = unsigned(vlo) * unsigned(pitch) + unsigned(u);
 #pragma unroll 1
                 for (int v = vlo; v <= vhi; v += kRows) {
@@ -472,12 +494,12 @@ void launch_gather_transpose(const GatherLaunch& p, hipStream_t s)
     // pitch of 260; CGLS at 128^3 x 120 views of 256 x 192 5.84 -> 5.76 ms)
     dim3 tb(64, 4), tg((p.pitch + 63) / 64, (p.nv + kGatherPadRows + 3) / 4, p.count);
     if (p.model == kGatherSiddonFlat) {
-        hipLaunchKernelGGL(siddon_flat_table_kernel, tg, tb, 0, s, p.proj, p.sviews, p.nu, p.nv, p.pitch, p.q, p.ru, p.rv,
-            p.flag);
+        hipLaunchKernelGGL(siddon_flat_table_kernel, tg, tb, 0, s, p.proj, p.sviews, p.vol, p.nu, p.nv, p.pitch, p.q, p.ru,
+            p.rv, p.flag);
         launch_gather<kGatherSiddonFlat>(p, s);
     } else if (p.model == kGatherSiddon) {
-        hipLaunchKernelGGL(siddon_gather_table_kernel, tg, tb, 0, s, p.proj, p.sviews, p.gviews, p.nu, p.nv,
-            p.pitch, p.q, p.flag);
+        hipLaunchKernelGGL(siddon_gather_table_kernel, tg, tb, 0, s, p.proj, p.sviews, p.gviews, p.vol, p.nu,
+            p.nv, p.pitch, p.q, p.flag);
         launch_gather<kGatherSiddon>(p, s);
     } else {
         hipLaunchKernelGGL(joseph_gather_table_kernel, tg, tb, 0, s, p.proj, p.views, p.gviews, p.vol, p.nu, p.nv,

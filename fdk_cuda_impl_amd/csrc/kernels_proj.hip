@@ -841,9 +841,13 @@ struct SiddonMinor {
     float inv, off;     // 1 / |slope|, (|slope| - 1) / |slope|
 };
 
-__device__ __forceinline__ SiddonMinor siddon_minor(double at_mid, double slope)
+__device__ __forceinline__ SiddonMinor siddon_minor(double at_mid, double slope, int n, int n0, int plane)
 {
     SiddonMinor m;
+    if (siddon_stays(slope, n, 1.0, n0)) {
+        slope = 0.0;
+        if (plane >= 0) at_mid = double(plane);
+    }
     m.slope = float(slope);
     m.base = float(at_mid + fmin(slope, 0.0));
     const float a = fabsf(m.slope);
@@ -895,16 +899,16 @@ siddon_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy
     if (i >= count) return;  // whole wave
     const bool pix = u < nu;
     const SiddonViewDev sv = views[i];
-    double S[3], R[3], len2 = 0.0;
+    double S[3], R[3], r[3], len2 = 0.0;
+    siddon_ray_geom(sv, u, v, r);
     const double lo[3] = { double(g.ox) - 0.5 * double(g.vx), double(g.oy) - 0.5 * double(g.vy),
                            double(g.oz) - 0.5 * double(g.vz) };
     const double vox[3] = { double(g.vx), double(g.vy), double(g.vz) };
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const double r = (double(sv.detS[k]) + u * double(sv.detU[k]) + v * double(sv.detV[k])) - double(sv.src[k]);
-        len2 += r * r;
+        len2 += r[k] * r[k];
         S[k] = (double(sv.src[k]) - lo[k]) / vox[k];
-        R[k] = r / vox[k];
+        R[k] = r[k] / vox[k];
     }
     const bool ymain = !(fabs(R[0]) >= fabs(R[1]));
     const double r0 = ymain ? R[1] : R[0], s0 = ymain ? S[1] : S[0];
@@ -914,8 +918,8 @@ siddon_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy
     const double ta = -s0 * rc, tb = (double(n0) - s0) * rc;
     const bool slabs = fabs(R[2]) <= fabs(r0) && fmin(ta, tb) >= 0.0 && fmax(ta, tb) <= 1.0 && *flag == 0;
     const double mid = 0.5 * double(n0) - s0;
-    const SiddonMinor m1 = siddon_minor(s1 + mid * (r1 * rc), r1 * rc);
-    const SiddonMinor m2 = siddon_minor(S[2] + mid * (R[2] * rc), R[2] * rc);
+    const SiddonMinor m1 = siddon_minor(s1 + mid * (r1 * rc), r1 * rc, n1, n0, ymain ? sv.plane[0] : sv.plane[1]);
+    const SiddonMinor m2 = siddon_minor(S[2] + mid * (R[2] * rc), R[2] * rc, n2, n0, sv.plane[2]);
     const float len = float(sqrt(len2) * fabs(rc));
     const float half0 = 0.5f * float(n0);
     float flo = 0.f, fhi = float(n0 - 1);

@@ -89,6 +89,16 @@ void gather_view(const ViewD& w, int axis, int nu, int nv, const double map[12],
     }
 }
 
+// The plane between cells (0 .. n) on which the source lies along an axis, or
+// -1.  The tolerance is twice the rounding that the voxels' FP32 origin and size
+// bring to a plane: a centred scan has its source in the middle plane of an even
+// volume, whatever the voxel.
+int source_plane(double src, double centre, double voxel, int n)
+{
+    const double cell = (src - centre) / voxel + 0.5 * n, plane = std::rint(cell);
+    return plane >= 0.0 && plane <= n && std::fabs(cell - plane) <= n * 0x1p-23 ? int(plane) : -1;
+}
+
 // No ray of the view runs across its main axis: the general Siddon gather
 // measures segments along that axis
 bool along_main(const ViewD& w, int axis, int nu, int nv)
@@ -185,6 +195,8 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
         std::memcpy(s.detS, w.detS, sizeof(s.detS));
         std::memcpy(s.detU, w.detU, sizeof(s.detU));
         std::memcpy(s.detV, w.detV, sizeof(s.detV));
+        const int cells[3] = { grid.nx, grid.ny, grid.nz };
+        for (int k = 0; k < 3; ++k) s.plane[k] = source_plane(w.src[k], cen[k], vox[k], cells[k]);
         projection_map(w, &c64[size_t(i) * 12]);
         // Gather transposes.  Their kernels take every support of a run of
         // kGatherRun voxels to lie before the source, and the Siddon one that

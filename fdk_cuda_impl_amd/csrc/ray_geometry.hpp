@@ -78,5 +78,23 @@ __device__ __forceinline__ void siddon_ray_geom(const SiddonViewDev& sv, int u, 
     }
 }
 
+// the same in FP64: pixel minus source
+__device__ __forceinline__ void siddon_ray_geom(const SiddonViewDev& sv, int u, int v, double* ray)
+{
+    for (int k = 0; k < 3; ++k)
+        ray[k] = (double(sv.detS[k]) + u * double(sv.detU[k]) + v * double(sv.detV[k])) - double(sv.src[k]);
+}
+
+// A ray that moves `along` cells of its main axis, of n0, and `across` cells of
+// another, of n, in the same time stays in one cell layer of that axis if it moves
+// no further across the volume than FP32 resolves there.  If the source lies on a
+// plane between cells (SiddonViewDev::plane) the layer is the upper one.  The
+// projection and the transposes have to agree on that: the ray's whole
+// contribution is at stake, not a rounding of it.
+__device__ __forceinline__ bool siddon_stays(double across, int n, double along, int n0)
+{
+    return fabs(across) * n0 <= fabs(along) * (n * 0x1p-22);
+}
+
 }  // namespace
 }  // namespace yk

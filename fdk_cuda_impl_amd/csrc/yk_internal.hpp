@@ -277,6 +277,7 @@ struct SiddonViewDev {
     float detS[4];
     float detU[4];
     float detV[4];
+    int plane[4];               // per axis, the plane between cells that the source lies on, or -1 (projector.cpp)
 };
 
 struct JosephLaunch {

@@ -702,7 +702,7 @@ __device__ __forceinline__ float siddon_walk(const float* __restrict__ vol, cons
     const int dims[3] = { g.nx, g.ny, g.nz };
     const float vox[3] = { g.vx, g.vy, g.vz };
     float t0, t1, acc = 0.f;
-    if (!clip_ray(src, ray, b.lo, b.hi, t0, t1)) return 0.f;
+    if (!clip_ray(src, ray, b.lo, b.hi, t0, t1) || siddon_in_upper_face(sv, g, u, v)) return 0.f;
     const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
     int idx[3], step[3];
     float tn[3], rcp[3];
@@ -793,7 +793,7 @@ siddon_ones_kernel(float* __restrict__ proj, const SiddonViewDev* __restrict__ v
     float src[3], ray[3], t0, t1;
     siddon_ray_geom(views[i], u, v, src, ray);
     const Box b = volume_box(g);
-    const bool hit = clip_ray(src, ray, b.lo, b.hi, t0, t1);
+    const bool hit = clip_ray(src, ray, b.lo, b.hi, t0, t1) && !siddon_in_upper_face(views[i], g, u, v);
     const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
     proj[((size_t)i * nv + v) * nu + u] = hit ? (t1 - t0) * len : 0.f;
 }
@@ -1076,7 +1076,7 @@ siddon_adjoint_kernel(const float* __restrict__ proj, float* __restrict__ volume
                 if (!(e > a)) continue;
                 if (surface) {
                     float t0, t1;
-                    if (!clip_ray(src, ray, b.lo, b.hi, t0, t1)) continue;
+                    if (!clip_ray(src, ray, b.lo, b.hi, t0, t1) || siddon_in_upper_face(sv, g, uu, vv)) continue;
                     a = fmaxf(a, t0);
                     e = fminf(e, t1);
                 } else {

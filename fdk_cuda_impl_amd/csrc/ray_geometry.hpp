@@ -96,5 +96,24 @@ __device__ __forceinline__ bool siddon_stays(double across, int n, double along,
     return fabs(across) * n0 <= fabs(along) * (n * 0x1p-22);
 }
 
+// whether a ray lies in an upper face of the volume, and so in no cell
+__device__ __forceinline__ bool siddon_in_upper_face(const SiddonViewDev& sv, const VolumeGeom& g, int u, int v)
+{
+    const int n[3] = { g.nx, g.ny, g.nz };
+    if (sv.plane[0] != n[0] && sv.plane[1] != n[1] && sv.plane[2] != n[2]) return false;
+    double r[3];
+    siddon_ray_geom(sv, u, v, r);
+    r[0] /= g.vx;
+    r[1] /= g.vy;
+    r[2] /= g.vz;
+    int m = fabs(r[0]) >= fabs(r[1]) ? 0 : 1;
+    if (fabs(r[2]) > fabs(m == 0 ? r[0] : r[1])) m = 2;
+    const double along = m == 0 ? r[0] : m == 1 ? r[1] : r[2];
+    const int n0 = m == 0 ? n[0] : m == 1 ? n[1] : n[2];
+    bool in = false;
+    for (int k = 0; k < 3; ++k) in = in || (k != m && sv.plane[k] == n[k] && siddon_stays(r[k], n[k], along, n0));
+    return in;
+}
+
 }  // namespace
 }  // namespace yk

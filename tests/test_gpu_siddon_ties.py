@@ -1,9 +1,9 @@
 """Siddon projection and transpose of rays that lie in a plane between two cells:
 a centred source, an even number of cells and an odd number of pixels, as
 centred scans have them.  Such a ray belongs to the upper cell, for the
-projection and for its transpose, whatever the direction it runs in.  The views
-hold multiples of 1/1024 mm, so that the rays' zeros are exact in FP32 and FP64
-alike."""
+projection and for its transpose, whatever the direction it runs in; one in the
+upper face of the volume to none.  The views hold multiples of 1/1024 mm, so that
+the rays' zeros are exact in FP32 and FP64 alike."""
 import numpy as np
 import pytest
 import torch
@@ -58,3 +58,24 @@ def test_upper_cell(ctx, oracle, tilt, voxel):
         at = P.adjoint(torch.from_numpy(row).cuda(), kind="siddon", first=i).cpu().numpy().astype(np.float64)
         a = P.forward(torch.from_numpy(x).cuda(), kind="siddon", first=i, count=1).cpu().numpy().astype(np.float64)
         assert abs((at * x).sum() / (a * row).sum() - 1.0) < 1e-5, i
+
+
+@pytest.mark.parametrize("tilt", list(TILTS))
+def test_upper_face(ctx, oracle, tilt):
+    """The middle row lies in the volume's upper face: projection, transpose and the solvers' row weights leave it out."""
+    g, views = centred((1.0, 1.0, 1.0), TILTS[tilt], center_mm=(0.0, 0.0, -9.0))
+    P = yk.Projector(ctx, views, g.nu, g.nv, g.grid())
+    ov = oracle.views_from_float(P.views)
+    vol = oracle.volume(*g.volume, *g.voxel_mm, center=g.center_mm)
+    x = np.random.default_rng(42).random(P.volume_shape, dtype=np.float32)
+    ax = P.forward(torch.from_numpy(x).cuda(), kind="siddon").cpu().numpy()
+    assert rel_rmse(ax, oracle.fp_siddon(ov, g.nu, g.nv, vol, x)) < 1e-5
+    assert (ax[:, NV // 2] == 0.0).all()
+    row = np.zeros((8, NV, NU), dtype=np.float32)
+    row[:, NV // 2] = 1.0
+    assert float(P.adjoint(torch.from_numpy(row).cuda(), kind="siddon").abs().max()) == 0.0
+    b = ax.copy()
+    b[:, NV // 2] = 5.0
+    kw = dict(method="sirt", iterations=2, forward="siddon", back="joseph_voxel", relaxation=0.7)
+    got = P.algebraic(torch.from_numpy(b).cuda(), **kw).cpu().numpy()
+    assert rel_rmse(got, oracle.algebraic(ov, g.nu, g.nv, vol, b, **kw)) < 1e-4

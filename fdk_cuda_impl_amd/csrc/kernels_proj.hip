@@ -190,11 +190,10 @@ constexpr int kColumnChunk = 256;  // z a wave loads at a time, four a lane
 __host__ __device__ __forceinline__ int column_pitch(int nz) { return (nz + 2 * kJosephGuard + 3) & ~3; }
 
 constexpr int kColumnWaves = 8;
-// LDS floats of a wave: its column (and, split, its K rays a lane at the end)
-__host__ __device__ __forceinline__ int column_words(int nz, int k, bool split)
-{
-    return split && column_pitch(nz) < 64 * k ? 64 * k : column_pitch(nz);
-}
+// A column's slices are summed in this many equal parts, then the parts in
+// order, however many waves take them: a ray has the same bits in every call
+// (256^3 x 360 views 5.70 -> 5.78 ms for the parts' sums).
+constexpr int kColumnParts = 8;
 
 template <int K, bool SPLIT>
 __global__ void __launch_bounds__(64 * kColumnWaves, 6)
@@ -213,7 +212,7 @@ joseph_fp_column_kernel(const float* __restrict__ vzx, const float* __restrict__
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = int(threadIdx.x & 63);
     // The waves of a workgroup take one column of consecutive views (their
     // rays nearly coincide, so the repeats of a tap row hit the CU's L1) or,
-    // SPLIT, equal parts of the slices of one column of one view, added at the
+    // SPLIT, equal numbers of the parts of one column of one view, added at the
     // end: for calls of too few columns to fill the GPU.
     // Columns are remapped so that each XCD (workgroups go round-robin to the
     // 8 XCDs; gridDim.x is a multiple of 8) sweeps a contiguous range of them,
@@ -223,8 +222,10 @@ joseph_fp_column_kernel(const float* __restrict__ vzx, const float* __restrict__
     const int waves = int(blockDim.x >> 6);
     const int i = SPLIT ? int(blockIdx.z) : int(blockIdx.z) * waves + wave;
     if (u >= nu || i >= count) return;  // whole wave, SPLIT: whole workgroup
-    const int words = column_words(g.nz, K, SPLIT);
+    const int words = column_pitch(g.nz);
     float* const column = reinterpret_cast<float*>(column_raw) + wave * words;
+    // SPLIT: the parts' sums, 64 K floats each, behind the columns
+    float* const sums = reinterpret_cast<float*>(column_raw) + waves * words;
     const ProjViewDev pv = views[i];
     const AxisInfo ax = axis_info(pv.axis, g);
     const float s0 = pick(ax.p0, pv.src[0], pv.src[1], 0.f), s1 = pick(ax.p1, pv.src[0], pv.src[1], 0.f), s2 = pv.src[2];
@@ -235,12 +236,12 @@ joseph_fp_column_kernel(const float* __restrict__ vzx, const float* __restrict__
     const float d1 = (pick(ax.p1, pv.detS[0], pv.detS[1], 0.f) + float(u) * pick(ax.p1, pv.detU[0], pv.detU[1], 0.f)) - s1;
     const float d2 = (pv.detS[2] + float(u) * pv.detU[2] + vmid * dv2) - s2;
     const float rd0 = d0 != 0.f ? 1.f / d0 : 0.f;
-    float e[K], acc[K];
+    float e[K], acc[K], total[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         // rays past the last one repeat it and store nothing
         e[k] = (float(min(v0 + 64 * k + lane, nv - 1)) - vmid) * dv2;
-        acc[k] = 0.f;
+        acc[k] = total[k] = 0.f;
     }
     const float eF = (float(v0) - vmid) * dv2, eE = (float(min(v0 + 64 * K, nv) - 1) - vmid) * dv2;
     // slices in which the column can lie inside (-1, n) on the first minor
@@ -254,11 +255,26 @@ joseph_fp_column_kernel(const float* __restrict__ vzx, const float* __restrict__
     }
     wlo = __builtin_amdgcn_readfirstlane(wlo);
     whi = __builtin_amdgcn_readfirstlane(whi);
+    const int part = (whi - wlo + kColumnParts) / kColumnParts;  // slices
+    int part_at = 0, part_top = kColumnParts;
     if constexpr (SPLIT) {
-        const int part = (whi - wlo + waves) / waves;
-        wlo += wave * part;
-        whi = min(whi, wlo + part - 1);
+        const int parts = kColumnParts / waves;
+        part_at = wave * parts;
+        part_top = part_at + parts;
+        wlo += part_at * part;
+        whi = min(whi, wlo + parts * part - 1);
     }
+    int part_end = wlo + part - 1;
+    auto end_part = [&]() {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if constexpr (SPLIT) sums[(part_at * K + k) * 64 + lane] = acc[k];
+            else total[k] += acc[k];
+            acc[k] = 0.f;
+        }
+        ++part_at;
+        part_end += part;
+    };
     const int p2 = column_pitch(ax.n2);
     const size_t slice_bytes = size_t(ax.n1 + 2 * kJosephGuard) * p2 * 4u;
     const float f1max = float(ax.n1), f2max = float(ax.n2 + kJosephGuard);
@@ -308,39 +324,42 @@ joseph_fp_column_kernel(const float* __restrict__ vzx, const float* __restrict__
         float4 cur = t[0], nxt = t[min(1, end - c)];
         float ctop = tt[0], ntop = tt[min(1, end - c)];
         load(sl, __float_as_uint(cur.y), ctop);
-        for (int s = c; s <= end; ++s) {
-            const float4 after = t[min(s + 2, end) - c];
-            const float atop = tt[min(s + 2, end) - c];
-            float4* const col4 = reinterpret_cast<float4*>(column);
-            if (first < ctop) col4[lane] = lerp4(cur.x, ra, rb);
-            if (chunks > 1) {  // a longer column: the rest, not loaded ahead
-                const char* p = sl + __float_as_uint(cur.y);
-                for (int z = kColumnChunk + 4 * lane; z < int(ctop) + 2; z += kColumnChunk)
-                    col4[z / 4] = lerp4(cur.x, *reinterpret_cast<const float4*>(p + size_t(z) * 4u),
-                                        *reinterpret_cast<const float4*>(p + (size_t(z) + p2) * 4u));
-            }
-            if (s < whi) {
-                // (past the table's last slice: reloads it, unused)
-                load(sl + (s < end ? slice_bytes : 0), __float_as_uint(nxt.y), ntop);
-                sl += slice_bytes;
-            }
-            __builtin_amdgcn_wave_barrier();
-            float lo[K], hi[K], w[K];
+        for (int s = c; s <= end;) {
+            for (const int stop = min(end, part_end); s <= stop; ++s) {
+                const float4 after = t[min(s + 2, end) - c];
+                const float atop = tt[min(s + 2, end) - c];
+                float4* const col4 = reinterpret_cast<float4*>(column);
+                if (first < ctop) col4[lane] = lerp4(cur.x, ra, rb);
+                if (chunks > 1) {  // a longer column: the rest, not loaded ahead
+                    const char* p = sl + __float_as_uint(cur.y);
+                    for (int z = kColumnChunk + 4 * lane; z < int(ctop) + 2; z += kColumnChunk)
+                        col4[z / 4] = lerp4(cur.x, *reinterpret_cast<const float4*>(p + size_t(z) * 4u),
+                                            *reinterpret_cast<const float4*>(p + (size_t(z) + p2) * 4u));
+                }
+                if (s < whi) {
+                    // (past the table's last slice: reloads it, unused)
+                    load(sl + (s < end ? slice_bytes : 0), __float_as_uint(nxt.y), ntop);
+                    sl += slice_bytes;
+                }
+                __builtin_amdgcn_wave_barrier();
+                float lo[K], hi[K], w[K];
 #pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const float f = __builtin_amdgcn_fmed3f(fmaf(e[k], cur.z, cur.w), 0.f, ctop);
-                const float* p = column + int(f);
-                lo[k] = p[0];
-                hi[k] = p[1];
-                w[k] = __builtin_amdgcn_fractf(f);
-            }
+                for (int k = 0; k < K; ++k) {
+                    const float f = __builtin_amdgcn_fmed3f(fmaf(e[k], cur.z, cur.w), 0.f, ctop);
+                    const float* p = column + int(f);
+                    lo[k] = p[0];
+                    hi[k] = p[1];
+                    w[k] = __builtin_amdgcn_fractf(f);
+                }
 #pragma unroll
-            for (int k = 0; k < K; ++k) acc[k] += fmaf(w[k], hi[k] - lo[k], lo[k]);
-            __builtin_amdgcn_wave_barrier();
-            cur = nxt;
-            ctop = ntop;
-            nxt = after;
-            ntop = atop;
+                for (int k = 0; k < K; ++k) acc[k] += fmaf(w[k], hi[k] - lo[k], lo[k]);
+                __builtin_amdgcn_wave_barrier();
+                cur = nxt;
+                ctop = ntop;
+                nxt = after;
+                ntop = atop;
+            }
+            if (s > part_end) end_part();
         }
     }
     auto store = [&](int v, float sum) {
@@ -349,18 +368,16 @@ joseph_fp_column_kernel(const float* __restrict__ vzx, const float* __restrict__
         store_ray(proj, i, nu, nv, u, v, joseph_ray(pv, ax, u, v, r) ? sum * r.L : 0.f, st);
     };
     if constexpr (SPLIT) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) column[64 * k + lane] = acc[k];
+        while (part_at < part_top) end_part();  // the last one, and any that no slice is left for
         __syncthreads();
-        const float* const sums = reinterpret_cast<const float*>(column_raw);
         for (int k = wave; k < K; k += waves) {
             float sum = 0.f;
-            for (int w = 0; w < waves; ++w) sum += sums[w * words + 64 * k + lane];
+            for (int p = 0; p < kColumnParts; ++p) sum += sums[(p * K + k) * 64 + lane];
             store(v0 + 64 * k + lane, sum);
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < K; ++k) store(v0 + 64 * k + lane, acc[k]);
+        for (int k = 0; k < K; ++k) store(v0 + 64 * k + lane, total[k] + acc[k]);
     }
 }
 
@@ -1361,24 +1378,24 @@ void launch_joseph_column_copy(const float* in, float* out, int nx, int ny, int 
 namespace {
 
 // Columns from which a column's slices are split over four waves instead of
-// eight (each wave forms tables for its part and leaves a sum): 12 views of 256 x
-// 192 at 128^3 (3072 columns) 78.6 -> 71.8 us, 30 of 128 x 96 at 64^3 (3840) 56.5
-// -> 49.5; one view (256 and 128 columns) 31.9 -> 35.9 and 23.6 -> 25.4.  Between,
-// eight keep a view's rounding the same however few views a call has.
+// eight (each wave forms tables for its parts): 12 views of 256 x 192 at 128^3
+// (3072 columns) 78.6 -> 71.8 us, 30 of 128 x 96 at 64^3 (3840) 56.5 -> 49.5; one
+// view (256 and 128 columns) 31.9 -> 35.9 and 23.6 -> 25.4.
 constexpr size_t kFewColumns = 2048;
 
 template <int K, bool SPLIT>
 void launch_column_kernel(const JosephSepFpLaunch& p, hipStream_t s)
 {
-    const size_t column = size_t(column_words(p.vol.nz, K, SPLIT)) * sizeof(float);
+    const size_t column = size_t(column_pitch(p.vol.nz)) * sizeof(float);
     // the waves' columns in 32 KiB; a longer column has a workgroup to itself
     int waves = column <= 4096 ? kColumnWaves : column <= 8192 ? 4 : column <= 16384 ? 2 : 1;
     if (SPLIT && size_t(p.nu) * p.count >= kFewColumns) waves = std::min(waves, 4);
+    const size_t lds = column * waves + (SPLIT ? size_t(kColumnParts) * 64 * K * sizeof(float) : 0);
     if (waves == 1)
         YK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(joseph_fp_column_kernel<K, SPLIT>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, int(column)));
+            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     dim3 grid((p.nu + 7) / 8 * 8, (p.nv + 64 * K - 1) / (64 * K), SPLIT ? p.count : (p.count + waves - 1) / waves);
-    hipLaunchKernelGGL((joseph_fp_column_kernel<K, SPLIT>), grid, dim3(64 * waves), column * waves, s, p.vol_zx, p.vol_zy,
+    hipLaunchKernelGGL((joseph_fp_column_kernel<K, SPLIT>), grid, dim3(64 * waves), lds, s, p.vol_zx, p.vol_zy,
         p.proj, p.views, p.vol, p.nu, p.nv, p.count, p.store);
 }
 
@@ -1401,8 +1418,9 @@ bool joseph_column_fits(const VolumeGeom& g)
 {
     const size_t g2 = 2 * kJosephGuard;
     const size_t slice = (size_t(std::max(g.nx, g.ny)) + g2) * size_t(column_pitch(g.nz)) * sizeof(float);
-    // 144 KB of LDS for the longest column, 32-bit byte offsets in a slice
-    return g.nz <= 36000 && slice < (size_t(1) << 32);
+    // 128 KB of LDS for the longest column beside the tables and parts, 32-bit byte
+    // offsets in a slice
+    return g.nz <= 32767 && slice < (size_t(1) << 32);
 }
 
 void launch_joseph_fp_column(const JosephSepFpLaunch& p, hipStream_t s)

@@ -1399,16 +1399,21 @@ void launch_column_kernel(const JosephSepFpLaunch& p, hipStream_t s)
         p.proj, p.views, p.vol, p.nu, p.nv, p.count, p.store);
 }
 
-// A call with fewer columns than this (2 waves for each of 1024 SIMDs) takes
-// SPLIT.  256^3 / 512 x 384, whole calls, not split and split: 1 view 163 and
-// 65 us, 4 views 172 and 125 us, 8192 columns and more: the same to 10 % slower.
-constexpr size_t kSplitColumns = 4096;
+// A call of fewer columns than kSplitColumns (4 waves for each of 1024 SIMDs)
+// takes SPLIT, and one of kRoundColumns (the waves resident at six a SIMD) to
+// twice as many: a wave a column would leave the second round partly empty, and
+// four a column leave shorter ones.  Whole calls, not split and split: 256^3 of
+// 512 x 384, 1 view 163 and 65 us, 4 views 172 and 125; 128^3 of 128 x 96, 40
+// views (5120 columns) 74 and 77, 60 views (7680) 117 and 97, 120 views (15360)
+// 171 and 169; 192^3 of 192 x 144, 60 views (11520) 250 and 219.
+constexpr size_t kSplitColumns = 4096, kRoundColumns = 6144;
 
 template <int K>
 void launch_column(const JosephSepFpLaunch& p, hipStream_t s)
 {
     const size_t columns = size_t(p.nu) * p.count * ((p.nv + 64 * K - 1) / (64 * K));
-    if (columns < kSplitColumns && p.count <= 65535) launch_column_kernel<K, true>(p, s);
+    const bool split = columns < kSplitColumns || (columns > kRoundColumns && columns <= 2 * kRoundColumns);
+    if (split && p.count <= 65535) launch_column_kernel<K, true>(p, s);
     else launch_column_kernel<K, false>(p, s);
 }
 

@@ -709,7 +709,9 @@ __device__ __forceinline__ bool clip_ray(const float* src, const float* ray, con
 // Exact Amanatides-Woo walk of one ray through the [z][y][x] volume, clipped
 // to t in [0, 1] and to the volume box.  Plane crossings are recomputed from
 // integer indices as (plane - src) * (1 / ray), and the ray sum adds the
-// segments in walk order.
+// segments in walk order.  (For a ray outside the upper faces: the caller asks
+// siddon_in_upper_face, whose FP64 registers the slab kernel's loop has no room
+// for.)
 __device__ __forceinline__ float siddon_walk(const float* __restrict__ vol, const SiddonViewDev& sv, const VolumeGeom& g,
     int u, int v)
 {
@@ -719,7 +721,7 @@ __device__ __forceinline__ float siddon_walk(const float* __restrict__ vol, cons
     const int dims[3] = { g.nx, g.ny, g.nz };
     const float vox[3] = { g.vx, g.vy, g.vz };
     float t0, t1, acc = 0.f;
-    if (!clip_ray(src, ray, b.lo, b.hi, t0, t1) || siddon_in_upper_face(sv, g, u, v)) return 0.f;
+    if (!clip_ray(src, ray, b.lo, b.hi, t0, t1)) return 0.f;
     const float len = sqrtf(ray[0] * ray[0] + ray[1] * ray[1] + ray[2] * ray[2]);
     int idx[3], step[3];
     float tn[3], rcp[3];
@@ -828,7 +830,8 @@ siddon_fp_kernel(const float* __restrict__ vol, float* __restrict__ proj,
     const int v = blockIdx.y * 4 + ((threadIdx.x >> 3) & 3);
     const int i = int(blockIdx.z) * 8 + int(threadIdx.x >> 5);
     if (u >= nu || v >= nv || i >= count) return;
-    const float acc = siddon_walk(vol, views[i], g, u, v);
+    const SiddonViewDev& sv = views[i];
+    const float acc = siddon_in_upper_face(sv, g, u, v) ? 0.f : siddon_walk(vol, sv, g, u, v);
     float* dst = proj + ((size_t)i * nv + v) * nu + u;
     *dst = accumulate ? *dst + acc : acc;
 }
@@ -916,6 +919,7 @@ siddon_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy
     if (i >= count) return;  // whole wave
     const bool pix = u < nu;
     const SiddonViewDev sv = views[i];
+    const bool face = siddon_in_upper_face(sv, g, u, v);
     double S[3], R[3], r[3], len2 = 0.0;
     siddon_ray_geom(sv, u, v, r);
     const double lo[3] = { double(g.ox) - 0.5 * double(g.vx), double(g.oy) - 0.5 * double(g.vy),
@@ -1005,7 +1009,7 @@ siddon_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy
         }
     }
     if (!pix) return;
-    const float out = slabs ? acc * len : siddon_walk(vol, sv, g, u, v);
+    const float out = slabs ? acc * len : face ? 0.f : siddon_walk(vol, sv, g, u, v);
     float* dst = proj + ((size_t)i * nv + v) * nu + u;
     *dst = accumulate ? *dst + out : out;
 }

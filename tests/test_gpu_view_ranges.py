@@ -1,6 +1,7 @@
 """Every ray of a projection of a range of views has the bits that it has in a
 projection of all of them, whatever share of the views the range is: calls of
-few and many detector columns, which split a column's slices differently."""
+few and many detector columns (which split a column's slices differently) and of
+few and many rays for the volume (which sample it in place or from copies)."""
 import numpy as np
 import pytest
 import torch
@@ -26,7 +27,7 @@ GEOMS = {
 
 
 @pytest.mark.parametrize("name", list(GEOMS))
-@pytest.mark.parametrize("kind", ["joseph"])
+@pytest.mark.parametrize("kind", ["joseph", "siddon"])
 def test_range_has_the_bits_of_the_whole(ctx, kind, name):
     g = small_geometry(**GEOMS[name])
     P = yk.Projector(ctx, g.views(), g.nu, g.nv, g.grid())

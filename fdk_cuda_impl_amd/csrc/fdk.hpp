@@ -136,7 +136,7 @@ struct yk_projector {
     yk::OpBpLaunch op_launch(int kind, const float* d_proj, int first, int count) const;
     bool column_transpose(yk_projector& w, const float* d_proj, float* d_volume, int first, int count, int accumulate);
     double dot(const float* a, const float* b, size_t n);
-    bool siddon_copies(yk_projector& w, const float* d_volume);
+    bool siddon_copies(yk_projector& w, const float* d_volume, bool any_x, bool any_y);
     int op_chunk(yk_projector& w, int count, bool one_view = false) const;
     bool gather_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
         int accumulate);
@@ -169,7 +169,8 @@ struct yk_projector {
     yk::DeviceArray<yk::GatherViewDev> d_gather;
     yk::DeviceArray<float> d_gather_q; // ray values of the gather transposes, one view chunk
     yk::DeviceArray<float> d_paired_views;  // paired views of the operator-form backprojections, one chunk
-    yk::DeviceArray<int> d_flag;       // one word: see siddon_value_check_kernel
+    yk::DeviceArray<int> d_flag;       // one word: a copy or table holds values of an extreme size
+    std::vector<char> siddon_axes;     // per view: bit 0, 1: some ray may have the main axis X, Y
     yk::DeviceArray<double> d_partials;
     yk::DeviceArray<yk::OpBpViewDev> d_opviews;  // operator-form FDK backprojection records
     yk::DeviceArray<yk::OpBpUnit> d_op_units;  // units of a column_weights launch

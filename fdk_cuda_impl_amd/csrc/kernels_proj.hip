@@ -499,11 +499,19 @@ __global__ void zfast_copy_kernel(const float* __restrict__ in, float* __restric
     }
 }
 
+// A volume whose values the Siddon slab projection's differences of taps cannot
+// carry (infinities, NaN, values near the type's ends): its copy raises *flag and
+// the projection walks instead, which reads only the voxels a ray crosses.
+__device__ __forceinline__ void check_value(float v, int* flag)
+{
+    if (flag && !(fabsf(v) <= 1e37f)) atomicOr(flag, 1);
+}
+
 // paired slab copy, X-main: [x][row z + guard][column y + guard];
 // blockIdx.z is the row, 32 x 32 (x, column) tiles of the two source planes
 // through LDS
 __global__ void pair_slab_x_kernel(const float* __restrict__ in, float2* __restrict__ out,
-    int nx, int ny, int nz)
+    int nx, int ny, int nz, int* __restrict__ flag)
 {
     __shared__ float tile[2][32][33];
     const int r = blockIdx.z;
@@ -517,6 +525,7 @@ __global__ void pair_slab_x_kernel(const float* __restrict__ in, float2* __restr
             const int z = r + h - kJosephGuard;
             tile[h][k][threadIdx.x] = in_xy && z >= 0 && z < nz ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
         }
+        check_value(tile[0][k][threadIdx.x], flag);
     }
     __syncthreads();
     for (int k = threadIdx.y; k < 32; k += 8) {
@@ -529,7 +538,7 @@ __global__ void pair_slab_x_kernel(const float* __restrict__ in, float2* __restr
 // paired slab copy, Y-main: [y][row z + guard][column x + guard] (x stays
 // fastest: row copies)
 __global__ void pair_slab_y_kernel(const float* __restrict__ in, float2* __restrict__ out,
-    int nx, int ny, int nz)
+    int nx, int ny, int nz, int* __restrict__ flag)
 {
     const int e = blockIdx.x * 256 + threadIdx.x;
     const int y = blockIdx.y, r = blockIdx.z;
@@ -540,6 +549,7 @@ __global__ void pair_slab_y_kernel(const float* __restrict__ in, float2* __restr
     const float a = in_x && z >= 0 && z < nz ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
     const float b = in_x && z + 1 >= 0 && z + 1 < nz ? in[(size_t(z + 1) * ny + y) * nx + x] : 0.f;
     out[(size_t(y) * rows + r) * cols + e] = make_float2(a, b);
+    check_value(a, flag);
 }
 
 // [z][y][x] -> [z][x][y]
@@ -817,7 +827,7 @@ siddon_ones_kernel(float* __restrict__ proj, const SiddonViewDev* __restrict__ v
     proj[((size_t)i * nv + v) * nu + u] = hit ? (t1 - t0) * len : 0.f;
 }
 
-// Siddon projection by the walk, one lane per ray.  It serves the calls whose
+// Siddon projection by the walk, one lane per ray.  It serves the plans whose
 // rays are too few to pay for the volume copies of siddon_fp_slab_kernel.
 __global__ void __launch_bounds__(256)
 siddon_fp_kernel(const float* __restrict__ vol, float* __restrict__ proj,
@@ -834,19 +844,6 @@ siddon_fp_kernel(const float* __restrict__ vol, float* __restrict__ proj,
     const float acc = siddon_in_upper_face(sv, g, u, v) ? 0.f : siddon_walk(vol, sv, g, u, v);
     float* dst = proj + ((size_t)i * nv + v) * nu + u;
     *dst = accumulate ? *dst + acc : acc;
-}
-
-// A volume whose values the slab projection's differences of taps cannot
-// carry (infinities, NaN, values near the type's ends): *flag is raised and
-// the projection walks instead, which reads only the voxels a ray crosses.
-constexpr float kSiddonLargest = 1e37f;
-__global__ void __launch_bounds__(256)
-siddon_value_check_kernel(const float* __restrict__ vol, size_t n, int* __restrict__ flag)
-{
-    bool bad = false;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-        bad = bad || !(fabsf(vol[i]) <= kSiddonLargest);
-    if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
 }
 
 __global__ void clear_flag_kernel(int* __restrict__ flag) { *flag = 0; }
@@ -905,7 +902,8 @@ __device__ __forceinline__ void siddon_slab_range(const SiddonMinor& m, float ha
 // The ray is set up in FP64 about the middle of the volume, so positions carry
 // ~1e-5 voxel of rounding.  Rays that the slab form does not cover (steepest
 // along Z, or the source or the pixel inside the main-axis extent, where t in
-// [0, 1] can clip) walk, as do all rays of a flagged volume.
+// [0, 1] can clip) walk, as do all rays of a flagged volume.  A call whose rays all
+// have one main axis comes with that axis's copy alone.
 __global__ void __launch_bounds__(512)
 siddon_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy, const float* __restrict__ vol,
     const int* __restrict__ flag, float* __restrict__ proj, const SiddonViewDev* __restrict__ views, VolumeGeom g,
@@ -937,7 +935,7 @@ siddon_fp_slab_kernel(const float* __restrict__ gx, const float* __restrict__ gy
     const int n0 = ymain ? g.ny : g.nx, n1 = ymain ? g.nx : g.ny, n2 = g.nz;
     const double rc = 1.0 / r0;
     const double ta = -s0 * rc, tb = (double(n0) - s0) * rc;
-    const bool slabs = fabs(R[2]) <= fabs(r0) && fmin(ta, tb) >= 0.0 && fmax(ta, tb) <= 1.0 && *flag == 0;
+    const bool slabs = fabs(R[2]) <= fabs(r0) && fmin(ta, tb) >= 0.0 && fmax(ta, tb) <= 1.0 && (ymain ? gy : gx) && *flag == 0;
     const double mid = 0.5 * double(n0) - s0;
     const SiddonMinor m1 = siddon_minor(s1 + mid * (r1 * rc), r1 * rc, n1, n0, ymain ? sv.plane[0] : sv.plane[1]);
     const SiddonMinor m2 = siddon_minor(S[2] + mid * (R[2] * rc), R[2] * rc, n2, n0, sv.plane[2]);
@@ -1455,16 +1453,16 @@ size_t joseph_pair_size(int nx, int ny, int nz, bool x_main)
     return n0 * (size_t(nz) + g - 1) * (n1 + g) * 2;
 }
 
-void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s)
+void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s, int* flag)
 {
     float2* o = reinterpret_cast<float2*>(out);
     const int g = 2 * kJosephGuard;
     if (x_main) {
         dim3 block(32, 8), grid((nx + 31) / 32, (ny + g + 31) / 32, nz + g - 1);
-        hipLaunchKernelGGL(pair_slab_x_kernel, grid, block, 0, s, in, o, nx, ny, nz);
+        hipLaunchKernelGGL(pair_slab_x_kernel, grid, block, 0, s, in, o, nx, ny, nz, flag);
     } else {
         dim3 block(256), grid((nx + g + 255) / 256, ny, nz + g - 1);
-        hipLaunchKernelGGL(pair_slab_y_kernel, grid, block, 0, s, in, o, nx, ny, nz);
+        hipLaunchKernelGGL(pair_slab_y_kernel, grid, block, 0, s, in, o, nx, ny, nz, flag);
     }
     YK_HIP(hipGetLastError());
 }
@@ -1516,12 +1514,14 @@ void launch_siddon_fp(const SiddonLaunch& p, hipStream_t s)
     YK_HIP(hipGetLastError());
 }
 
+void launch_clear_flag(int* flag, hipStream_t s)
+{
+    hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(1), 0, s, flag);
+    YK_HIP(hipGetLastError());
+}
+
 void launch_siddon_fp_slab(const SiddonSlabFpLaunch& p, hipStream_t s)
 {
-    const size_t n = size_t(p.vol.nx) * p.vol.ny * p.vol.nz;
-    hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(1), 0, s, p.flag);
-    hipLaunchKernelGGL(siddon_value_check_kernel, dim3(unsigned(std::min<size_t>(4096, (n + 255) / 256))), dim3(256), 0, s,
-        p.volume, n, p.flag);
     dim3 block(64, 8), grid((p.nu + 63) / 64, p.nv, (p.count + 7) / 8);
     hipLaunchKernelGGL(siddon_fp_slab_kernel, grid, block, 0, s, p.vol_x, p.vol_y, p.volume, p.flag, p.proj, p.views,
         p.vol, p.nu, p.nv, p.count, p.accumulate);

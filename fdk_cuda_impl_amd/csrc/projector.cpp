@@ -27,12 +27,14 @@ void grow(DeviceArray<T>& a, size_t n)
 constexpr double kOpPairSamples = 1e6, kOpPairRatio = 0.5;
 constexpr int kOpPairViews = 3;
 
-// rays x main-axis slabs per voxel from which the Siddon projection makes its
-// volume copies: at 3 (one view of 512 x 384 at 256^3) the copies and the slab
-// kernel take 223 us against the walk's 316, at 6 304 against 429, at 24 411
-// against 999; one view at 128^3 48 against 90, at 64^3 28 against 39.  Below
-// 1 the copies are most of the work and the walk reads only what its few rays
-// cross.
+// rays x main-axis slabs of all the plan's views per voxel from which the Siddon
+// projection makes its volume copies.  Calls of a plan of 60 views, walk and
+// copies with the slab kernel: at 128^3 one view of 128 x 96 59 and 34 us, all 301
+// and 114; at 256^3 one view of 256 x 192 145 and 120 us, all 3370 and 836, of
+// 64 x 48 136 and 116, 361 and 367; at 512^3 one view of 512 x 384 0.79 and 0.87
+// ms, all 32.7 and 8.3.  Few views of a coarse detector before a large volume lose
+// by it (512^3, one view of 256 x 192: 0.39 and 0.72 ms): the walk reads only what
+// their rays cross, but a ray must not depend on the call it is in.
 constexpr double kSiddonSlabRatio = 1.0;
 
 // Voxels from which the Joseph transpose of separable views goes by columns:
@@ -87,6 +89,26 @@ void gather_view(const ViewD& w, int axis, int nu, int nv, const double map[12],
         for (int k = 0; k < 3; ++k) maps[m][k] = float(c[k] * vox[k]);
         maps[m][3] = float(c[0] * org[0] + c[1] * org[1] + c[2] * org[2] + c[3]);
     }
+}
+
+// Which of X (1) and Y (2) may be the main axis, the larger |ray / voxel|, of some
+// ray of the view.  The ray is linear over the detector, so where one component
+// keeps its sign and exceeds the other's size at the corners it does everywhere.
+int ray_axes(const ViewD& w, const double vox[3], int nu, int nv)
+{
+    bool x_only = true, y_only = true;
+    double sign[2] = { 0.0, 0.0 };
+    for (int a = 0; a < 4; ++a) {
+        double r[2];
+        for (int k = 0; k < 2; ++k) {
+            r[k] = (w.detS[k] + ((a & 1) ? nu - 1 : 0) * w.detU[k] + ((a & 2) ? nv - 1 : 0) * w.detV[k] - w.src[k]) / vox[k];
+            if (sign[k] == 0.0) sign[k] = r[k] < 0.0 ? -1.0 : 1.0;
+        }
+        // (a margin for the kernel's own rounding)
+        x_only = x_only && sign[0] * r[0] > 1.000001 * std::fabs(r[1]);
+        y_only = y_only && sign[1] * r[1] > 1.000001 * std::fabs(r[0]);
+    }
+    return x_only ? 1 : y_only ? 2 : 3;
 }
 
 // The plane between cells (0 .. n) on which the source lies along an axis, or
@@ -195,6 +217,7 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
         std::memcpy(s.detS, w.detS, sizeof(s.detS));
         std::memcpy(s.detU, w.detU, sizeof(s.detU));
         std::memcpy(s.detV, w.detV, sizeof(s.detV));
+        siddon_axes.push_back(char(ray_axes(widen(w), vox, nu, nv)));
         const int cells[3] = { grid.nx, grid.ny, grid.nz };
         for (int k = 0; k < 3; ++k) s.plane[k] = source_plane(w.src[k], cen[k], vox[k], cells[k]);
         projection_map(w, &c64[size_t(i) * 12]);
@@ -318,15 +341,16 @@ SolverCall::~SolverCall()
     ws.busy = false;
 }
 
-// both paired slab copies of the volume into w's scratch; false when the walk,
-// which needs none, has to serve the call: the copies do not fit in memory, a
-// stream capture allows no allocation, or the slab kernel's grid or 32-bit
-// slab offsets cannot hold the sizes
-bool yk_projector::siddon_copies(yk_projector& w, const float* d_volume)
+// the paired slab copies of the volume for rays of either main axis into w's
+// scratch; false when the walk, which needs none, has to serve the call: the
+// copies do not fit in memory, a stream capture allows no allocation, or the slab
+// kernel's grid or 32-bit slab offsets cannot hold the sizes
+bool yk_projector::siddon_copies(yk_projector& w, const float* d_volume, bool any_x, bool any_y)
 {
-    const size_t need_x = joseph_pair_size(grid.nx, grid.ny, grid.nz, true);
-    const size_t need_y = joseph_pair_size(grid.nx, grid.ny, grid.nz, false);
-    if (nv > 65535 || need_x / grid.nx > (size_t(1) << 29) || need_y / grid.ny > (size_t(1) << 29)) return false;
+    const size_t size_x = joseph_pair_size(grid.nx, grid.ny, grid.nz, true);
+    const size_t size_y = joseph_pair_size(grid.nx, grid.ny, grid.nz, false);
+    if (nv > 65535 || size_x / grid.nx > (size_t(1) << 29) || size_y / grid.ny > (size_t(1) << 29)) return false;
+    const size_t need_x = any_x ? size_x : 0, need_y = any_y ? size_y : 0;
     if (w.d_vol_zx.size() < need_x || w.d_vol_zy.size() < need_y || !w.d_flag.get()) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
@@ -340,8 +364,10 @@ bool yk_projector::siddon_copies(yk_projector& w, const float* d_volume)
         (void)hipGetLastError();  // the failed allocation's, not the call's
         return false;
     }
-    launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, ctx->stream);
-    launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, ctx->stream);
+    int* const flag = w.d_flag.get();
+    launch_clear_flag(flag, ctx->stream);
+    if (any_x) launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, ctx->stream, flag);
+    if (any_y) launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, ctx->stream, flag);
     return true;
 }
 
@@ -423,15 +449,18 @@ bool yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
         p.accumulate = accumulate;
         launch_joseph_fp(p, s);
     } else if (kind == YK_FP_SIDDON) {
-        // The slab kernel reads paired copies of the volume along both axes,
-        // made on each call, so it takes the calls whose rays' slabs outnumber
-        // the voxels kSiddonSlabRatio times; the walk the others.
-        const double slabs = double(count) * nu * nv * std::max(grid.nx, grid.ny);
-        if (slabs >= kSiddonSlabRatio * double(grid.nx) * grid.ny * grid.nz && siddon_copies(w, d_volume)) {
+        // The slab kernel reads paired copies of the volume, made on each call.
+        // Which form takes a ray is the plan's matter, not the call's: the two
+        // differ in rounding, and a range of views has the bits of the whole.
+        const double slabs = double(n_views) * nu * nv * std::max(grid.nx, grid.ny);
+        int axes = 0;
+        for (int i = first; i < first + count; ++i) axes |= siddon_axes[i];
+        if (slabs >= kSiddonSlabRatio * double(grid.nx) * grid.ny * grid.nz &&
+            siddon_copies(w, d_volume, (axes & 1) != 0, (axes & 2) != 0)) {
             SiddonSlabFpLaunch p{};
             p.volume = d_volume;
-            p.vol_x = w.d_vol_zx.get();
-            p.vol_y = w.d_vol_zy.get();
+            p.vol_x = (axes & 1) ? w.d_vol_zx.get() : nullptr;
+            p.vol_y = (axes & 2) ? w.d_vol_zy.get() : nullptr;
             p.flag = w.d_flag.get();
             p.proj = d_proj;
             p.views = d_sviews.get() + first;

@@ -325,9 +325,12 @@ bool joseph_column_fits(const VolumeGeom& g);
 // X- or Y-main views of any orientation, from paired slab copies
 // (launch_joseph_pair_copy) of joseph_pair_size floats: float2 entries (value
 // at z row r, value at row r + 1), columns along the other of x and y, two
-// zero planes around both minor axes
+// zero planes around both minor axes.  A copy raises *flag (null: unused) for
+// values that launch_siddon_fp_slab cannot take.
 void launch_joseph_fp_slab(const JosephSepFpLaunch& p, hipStream_t s);
-void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s);
+void launch_joseph_pair_copy(const float* in, float* out, int nx, int ny, int nz, bool x_main, hipStream_t s,
+    int* flag = nullptr);
+void launch_clear_flag(int* flag, hipStream_t s);
 size_t joseph_pair_size(int nx, int ny, int nz, bool x_main);
 
 struct JosephAdjointLaunch {
@@ -411,14 +414,14 @@ struct SiddonLaunch {
 void launch_siddon_fp(const SiddonLaunch& p, hipStream_t s);
 void launch_siddon_ones(const SiddonLaunch& p, hipStream_t s);  // of a volume of ones (volume unused)
 
-// Siddon projection over the paired slab copies of the volume (made by
-// launch_joseph_pair_copy with slab); both copies are needed: the main axis is
-// chosen per ray
+// Siddon projection over the paired slab copies of the volume
+// (launch_joseph_pair_copy).  The main axis is chosen per ray: a copy may be null
+// if no ray of the call has its axis.
 struct SiddonSlabFpLaunch {
     const float* volume;        // [z][y][x]
     const float* vol_x;         // paired slab copy, X-main
     const float* vol_y;         // paired slab copy, Y-main
-    int* flag;                  // scratch word: the volume holds values only the walk can carry
+    const int* flag;            // raised by the copies: the volume holds values only the walk can carry
     float* proj;                // [count][nv][nu]
     const SiddonViewDev* views; // device, `count`
     VolumeGeom vol;

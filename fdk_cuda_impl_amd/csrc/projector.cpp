@@ -37,11 +37,14 @@ constexpr int kOpPairViews = 3;
 // their rays cross, but a ray must not depend on the call it is in.
 constexpr double kSiddonSlabRatio = 1.0;
 
-// Voxels from which the Joseph transpose of separable views goes by columns:
-// 96^3 x 60 views take 169 us against the gather's 237, 128^3 x 4 49 against
-// 50, 64^3 x 60 110 against 113, 64^3 x 4 33 against 27 (three launches
-// and two volumes more, and too few waves).
-constexpr size_t kColumnVoxels = 500000;
+// Samples (voxels x views) from which the Joseph transpose of separable views goes
+// by columns; it takes three launches and passes over two volumes more than the
+// gather, so a single view never does.  Gather and columns, detector as wide as
+// the volume: 96^3 x 4 views 16 and 21 us, x 8 26 and 26, x 60 136 and 95; 128^3
+// x 1 12 and 19, x 4 28 and 26, x 60 251 and 126; 256^3 x 1 39 and 51, x 2 66 and
+// 58, x 60 1535 and 500; 64^3 x 30 37 and 39, x 60 63 and 61.
+constexpr double kColumnSamples = 8e6;
+constexpr int kColumnViews = 2;
 
 // Rays up to which a Joseph projection's store makes the solvers' residual: its
 // lanes run along detector columns, so the reads of b and the row weights it
@@ -591,13 +594,13 @@ bool yk_projector::gather_transpose(yk_projector& w, bool siddon, const float* d
 
 // Joseph transpose of separable views by detector columns, a chunk of views'
 // table at a time (at most 1 GiB); false when the gather has to serve the call:
-// a view outside its form, sizes past its grids, few voxels, or no memory
+// a view outside its form, few voxels or views, or no memory
 bool yk_projector::column_transpose(yk_projector& w, const float* d_proj, float* d_volume, int first, int count, int accumulate)
 {
     if (!std::all_of(joseph_column.begin() + first, joseph_column.begin() + first + count, [](char c) { return c != 0; }))
         return false;
     const size_t voxels = size_t(grid.nx) * grid.ny * grid.nz;
-    if (voxels < kColumnVoxels || grid.ny > 65535 || grid.nx > 500000 || grid.nz > 2000000) return false;
+    if (double(voxels) * count < kColumnSamples || count < kColumnViews) return false;
     const int pitch = nv + 2 * kColumnPad;
     const size_t per_view = size_t(nu) * pitch;
     if (per_view > (size_t(1) << 30)) return false;

@@ -138,7 +138,14 @@ struct yk_projector {
     double dot(const float* a, const float* b, size_t n);
     bool siddon_copies(yk_projector& w, const float* d_volume, bool any_x, bool any_y);
     int op_chunk(yk_projector& w, int count, bool one_view = false) const;
-    bool gather_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
+    bool gather_transpose(yk_projector& w, int model, const float* d_proj, float* d_volume, int first, int count, int accumulate);
+    enum TransposeForm { kUntilted, kGeneral, kSearch };
+    struct TransposeRun {
+        TransposeForm form;
+        int first, count;
+    };
+    std::vector<TransposeRun> transpose_runs(bool siddon, int first, int count) const;
+    void transpose(yk_projector& w, bool siddon, TransposeForm form, const float* d_proj, float* d_volume, int first, int count,
         int accumulate);
 
     yk_ctx* ctx;
@@ -161,11 +168,11 @@ struct yk_projector {
     yk::DeviceArray<float> d_vol_t;
     yk::DeviceArray<float> d_vol_zx;   // paired volume copies of the Joseph and Siddon projections
     yk::DeviceArray<float> d_vol_zy;
-    std::vector<char> siddon_main;     // per view: no ray runs across the main axis
-    std::vector<char> siddon_flat;     // per view: a ray's x and y depend on the column alone, its z on the row
+    std::vector<char> siddon_flat;     // per view: siddon_flat_gather covers it
     std::vector<char> joseph_column;   // per view: the column transpose covers it
     yk::DeviceArray<float> d_column_x, d_column_y;  // its volumes of the X- and Y-main views
     std::vector<char> joseph_gather, siddon_gather;  // per view: the gather transposes cover it
+    std::vector<char> near_source;     // per view: a voxel lies within their margin of the source plane, or behind it
     yk::DeviceArray<yk::GatherViewDev> d_gather;
     yk::DeviceArray<float> d_gather_q; // ray values of the gather transposes, one view chunk
     yk::DeviceArray<float> d_paired_views;  // paired views of the operator-form backprojections, one chunk

@@ -389,8 +389,9 @@ __device__ __forceinline__ void siddon_flat_gather(const float* __restrict__ q, 
             for (int k = 0; k < kWidth; ++k) {
                 const float2 c = ru[(size_t)i * pitch + (u + k)];
                 const float tx0 = x0 * c.x, tx1 = x1 * c.x;
-                ya[k] = __builtin_amdgcn_fmed3f(y0 * c.y, tx0, tx1);
-                yb[k] = __builtin_amdgcn_fmed3f(y1 * c.y, tx0, tx1);
+                // (the ray ends at its pixel, t = 1)
+                ya[k] = fminf(__builtin_amdgcn_fmed3f(y0 * c.y, tx0, tx1), 1.f);
+                yb[k] = fminf(__builtin_amdgcn_fmed3f(y1 * c.y, tx0, tx1), 1.f);
             }
 #pragma unroll
             for (int p = 0; p < ZR; p += 2) {

@@ -225,8 +225,8 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
         for (int k = 0; k < 3; ++k) s.plane[k] = source_plane(w.src[k], cen[k], vox[k], cells[k]);
         projection_map(w, &c64[size_t(i) * 12]);
         // Gather transposes.  Their kernels take every support of a run of
-        // kGatherRun voxels to lie before the source, and the Siddon one that
-        // t in [0, 1] clips no ray inside the volume.
+        // kGatherRun voxels to lie before the source, and the general Siddon one
+        // that the detector ends no ray inside the volume.
         if (p.axis != 2) {
             const double* map = &c64[size_t(i) * 12];
             double least, most, inner, outer;
@@ -244,7 +244,7 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
             near_source.push_back(!front);
             joseph_gather.push_back(front);
             siddon_gather.push_back(front && outer < 1.0 && along_main(widen(w), p.axis, nu, nv));
-            siddon_flat.push_back(front && outer < 1.0 && separable.back() && w.detU[2] == 0.f);
+            siddon_flat.push_back(front && separable.back() && w.detU[2] == 0.f);
             joseph_column.push_back(front && separable.back() && column_view(p, nu, nv, vol));
         } else {
             near_source.push_back(0);

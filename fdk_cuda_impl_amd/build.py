@@ -24,7 +24,7 @@ VMEM_COSTS = os.path.join(HERE, "yk_vmem_costs")
 ARCH = os.environ.get("YK_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["capi.cpp", "geometry.cpp", "fdk.cpp", "projector.cpp", "algebraic.cpp", "cgls.cpp", "diagnostics.cpp", "session.cpp",
-           "kernels_filter.hip", "kernels_bp.hip", "kernels_proj.hip", "kernels_gather.hip", "kernels_column.hip",
+           "kernels_filter.hip", "kernels_bp.hip", "kernels_proj.hip", "kernels_gather.hip", "kernels_column.hip", "kernels_scatter.hip",
            "kernels_misc.hip"]
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

@@ -139,12 +139,14 @@ struct yk_projector {
     bool siddon_copies(yk_projector& w, const float* d_volume, bool any_x, bool any_y);
     int op_chunk(yk_projector& w, int count, bool one_view = false) const;
     bool gather_transpose(yk_projector& w, int model, const float* d_proj, float* d_volume, int first, int count, int accumulate);
-    enum TransposeForm { kUntilted, kGeneral, kSearch };
+    enum TransposeForm { kUntilted, kGeneral, kScatter, kSearch };
     struct TransposeRun {
         TransposeForm form;
         int first, count;
     };
     std::vector<TransposeRun> transpose_runs(bool siddon, int first, int count) const;
+    bool scatter_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
+        int accumulate);
     void transpose(yk_projector& w, bool siddon, TransposeForm form, const float* d_proj, float* d_volume, int first, int count,
         int accumulate);
 
@@ -174,6 +176,7 @@ struct yk_projector {
     std::vector<char> joseph_gather, siddon_gather;  // per view: the gather transposes cover it
     std::vector<char> near_source;     // per view: a voxel lies within their margin of the source plane, or behind it
     yk::DeviceArray<yk::GatherViewDev> d_gather;
+    yk::DeviceArray<float> d_scatter;  // ray table of the scatter transposes, one view chunk
     yk::DeviceArray<float> d_gather_q; // ray values of the gather transposes, one view chunk
     yk::DeviceArray<float> d_paired_views;  // paired views of the operator-form backprojections, one chunk
     yk::DeviceArray<int> d_flag;       // one word: a copy or table holds values of an extreme size

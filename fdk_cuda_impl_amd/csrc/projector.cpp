@@ -546,7 +546,8 @@ int yk_projector::op_chunk(yk_projector& w, int count, bool one_view) const
 // over the volume.  Two kinds of views do decide for the call:
 // - a voxel within the gathers' margin of the source has thousands of candidates
 //   in few lanes, which launches of few views would wait for one after another
-//   (92 mm orbit around that volume, tilted: the search 31 ms, split 68);
+//   (92 mm orbit around that volume, tilted: the search 31 ms, split 68); untilted
+//   views are scattered then (7.4 ms);
 // - rays so dense that the columns take them in some views and not in others cost
 //   columns and gather alike, in twice the launches (125 mm: 1.66 ms, split 3.22).
 std::vector<yk_projector::TransposeRun> yk_projector::transpose_runs(bool siddon, int first, int count) const
@@ -554,11 +555,13 @@ std::vector<yk_projector::TransposeRun> yk_projector::transpose_runs(bool siddon
     constexpr int kShortRun = 8;
     const std::vector<char>& untilted = siddon ? siddon_flat : joseph_column;
     const std::vector<char>& general = siddon ? siddon_gather : joseph_gather;
-    bool columns = true;
+    bool columns = true, near = false, all_sep = true;
     for (int i = first; i < first + count; ++i) {
-        if (near_source[i]) return { TransposeRun{ kSearch, first, count } };
+        near = near || near_source[i];
+        all_sep = all_sep && separable[i];
         columns = columns && (siddon || untilted[i] || !general[i] || !separable[i]);
     }
+    if (near) return { TransposeRun{ all_sep ? kScatter : kSearch, first, count } };
     std::vector<TransposeRun> runs;
     for (int i = first; i < first + count; ++i) {
         const TransposeForm form = untilted[i] && columns ? kUntilted : general[i] ? kGeneral : kSearch;
@@ -672,14 +675,54 @@ bool yk_projector::column_transpose(yk_projector& w, const float* d_proj, float*
     return true;
 }
 
+// Untilted views by scattering, a chunk of views' table at a time (at most 1 GiB);
+// false when there is no memory for it (none may be allocated under a capture)
+bool yk_projector::scatter_transpose(yk_projector& w, bool siddon, const float* d_proj, float* d_volume, int first, int count,
+    int accumulate)
+{
+    // floats a view: Joseph (a2, b2) and p L of every ray, (a1, b1) of every column;
+    // Siddon two a ray and two a column
+    const size_t rays = size_t(nu) * (nv + kScatterPad);
+    const size_t per_view = (siddon ? 2 : 3) * rays + 2 * size_t(nu);
+    const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
+    if (w.d_scatter.size() < per_view * chunk) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) return false;
+        try {
+            grow(w.d_scatter, per_view * chunk);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    for (int c0 = 0; c0 < count; c0 += chunk) {
+        const int n = std::min(chunk, count - c0);
+        float2* const columns = reinterpret_cast<float2*>(w.d_scatter.get());
+        float2* const table = columns + size_t(nu) * n;
+        const float* proj = d_proj + size_t(nu) * nv * c0;
+        const float* map = d_c32.get() + size_t(first + c0) * 12;
+        const int add = c0 > 0 ? 1 : accumulate;
+        if (siddon) {
+            launch_siddon_scatter(SiddonScatterLaunch{ proj, d_volume, d_sviews.get() + first + c0, map, columns, table, vol, nu, nv,
+                n, add }, ctx->stream);
+        } else {
+            launch_joseph_scatter(JosephScatterLaunch{ proj, d_volume, d_jviews.get() + first + c0, map, columns, table,
+                reinterpret_cast<float*>(table + rays * n), vol, nu, nv, n, add }, ctx->stream);
+        }
+    }
+    return true;
+}
+
 // one run of transpose_runs
 void yk_projector::transpose(yk_projector& w, bool siddon, TransposeForm form, const float* d_proj, float* d_volume, int first,
     int count, int accumulate)
 {
     hipStream_t s = ctx->stream;
     const int model = !siddon ? kGatherJoseph : form == kUntilted ? kGatherSiddonFlat : kGatherSiddon;
+    if (form == kScatter && scatter_transpose(w, siddon, d_proj, d_volume, first, count, accumulate)) return;
     if (!siddon && form == kUntilted && column_transpose(w, d_proj, d_volume, first, count, accumulate)) {
-    } else if (form != kSearch && gather_transpose(w, model, d_proj, d_volume, first, count, accumulate)) {
+    } else if (form <= kGeneral && gather_transpose(w, model, d_proj, d_volume, first, count, accumulate)) {
     } else if (!siddon) {
         // the ray table holds a chunk of views at a time (at most 1 GiB)
         const size_t per_view = size_t(nu) * nv;

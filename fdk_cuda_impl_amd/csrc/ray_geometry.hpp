@@ -115,5 +115,65 @@ __device__ __forceinline__ bool siddon_in_upper_face(const SiddonViewDev& sv, co
     return in;
 }
 
+struct Box {
+    float lo[3], hi[3];
+};
+
+__device__ __forceinline__ Box volume_box(const VolumeGeom& g)
+{
+    Box b;
+    b.lo[0] = g.ox - 0.5f * g.vx; b.hi[0] = g.ox + (float(g.nx) - 0.5f) * g.vx;
+    b.lo[1] = g.oy - 0.5f * g.vy; b.hi[1] = g.oy + (float(g.ny) - 0.5f) * g.vy;
+    b.lo[2] = g.oz - 0.5f * g.vz; b.hi[2] = g.oz + (float(g.nz) - 0.5f) * g.vz;
+    return b;
+}
+
+// one slab of the box clip: narrows [t0, t1] to lo <= s + t r <= hi; a ray
+// parallel to the slab and outside it misses
+__device__ __forceinline__ bool slab_clip(float s, float r, float lo, float hi, float& t0, float& t1)
+{
+    if (fabsf(r) > 1e-8f) {
+        float ta = (lo - s) / r, tb = (hi - s) / r;
+        if (ta > tb) { const float t = ta; ta = tb; tb = t; }
+        t0 = fmaxf(t0, ta);
+        t1 = fminf(t1, tb);
+        return true;
+    }
+    return !(s < lo || s > hi);
+}
+
+// parametric segment [t0, t1] of src + t ray inside the box, clipped to [0, 1]
+__device__ __forceinline__ bool clip_ray(const float* src, const float* ray, const float* lo,
+    const float* hi, float& t0, float& t1)
+{
+    t0 = 0.f;
+    t1 = 1.f;
+    for (int k = 0; k < 3; ++k)
+        if (!slab_clip(src[k], ray[k], lo[k], hi[k], t0, t1)) return false;
+    return t0 < t1;
+}
+
+// t-interval of the walk inside cell c of one axis: the forward walk's own
+// plane crossings (plane - src) * (1 / ray); a ray parallel to the axis stays
+// in the cell its source coordinate lies in
+__device__ __forceinline__ void cell_interval(float s, float r, float lo, float vox, int c, int n,
+    float& ta, float& tb)
+{
+    if (fabsf(r) > 1e-8f) {
+        const float rc = 1.f / r;
+        const float t0 = (lo + float(c) * vox - s) * rc, t1 = (lo + float(c + 1) * vox - s) * rc;
+        ta = fmaxf(ta, fminf(t0, t1));
+        tb = fminf(tb, fmaxf(t0, t1));
+    } else if (min(n - 1, max(0, int(floorf((s - lo) / vox)))) != c) {
+        tb = -3.0e38f;
+    }
+}
+
+// world projective map (u or v numerator row r, denominator row d) of a point
+__device__ __forceinline__ float proj_coord(const float* c, int row, float x, float y, float z, float rd)
+{
+    return (c[row] * x + c[row + 1] * y + c[row + 2] * z + c[row + 3]) * rd;
+}
+
 }  // namespace
 }  // namespace yk

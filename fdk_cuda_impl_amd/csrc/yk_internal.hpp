@@ -441,6 +441,35 @@ struct SiddonAdjointLaunch {
 };
 void launch_siddon_adjoint(const SiddonAdjointLaunch& p, hipStream_t s);
 
+// Transposes of untilted views by scattering (kernels_scatter.hip); the ray table
+// arrays are scratch of `count` views, columns closed by kScatterPad zero entries
+constexpr int kScatterPad = 8;
+struct JosephScatterLaunch {
+    const float* proj;          // [count][nv][nu]
+    float* volume;              // [z][y][x]
+    const ProjViewDev* views;   // device, `count`
+    const float* coeff32;       // device, per view cu[4] cv[4] cd[4] (world projective map)
+    float2* ab1;                // scratch [count][nu]
+    float2* ab2;                // scratch [count][nu][nv + kScatterPad]
+    float* pl;                  // scratch [count][nu][nv + kScatterPad]
+    VolumeGeom vol;
+    int nu, nv, count;
+    int accumulate;
+};
+void launch_joseph_scatter(const JosephScatterLaunch& p, hipStream_t s);
+struct SiddonScatterLaunch {
+    const float* proj;          // [count][nv][nu]
+    float* volume;              // [z][y][x]
+    const SiddonViewDev* views; // device, `count`
+    const float* coeff32;       // device, per view cu[4] cv[4] cd[4] (world projective map)
+    float2* col_xy;             // scratch [count][nu]
+    float2* ray_wz;             // scratch [count][nu][nv + kScatterPad]
+    VolumeGeom vol;
+    int nu, nv, count;
+    int accumulate;
+};
+void launch_siddon_scatter(const SiddonScatterLaunch& p, hipStream_t s);
+
 // per-view record of the operator-form FDK backprojections (world units)
 struct OpBpViewDev {
     float cu[4], cv[4], cd[4];  // projective map u = Cu.[X,1] / Cd.[X,1], v likewise

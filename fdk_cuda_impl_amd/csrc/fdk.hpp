@@ -167,6 +167,20 @@ struct yk_projector {
     // null: its own.  Operators of one volume grid that run one after another
     // on one stream can share them.
     yk_projector* scratch_owner = nullptr;
+    // Scratch only grows: paths of different layouts share an array, and a
+    // reallocation would synchronize.  Once a call has been captured into a graph an
+    // array that has to grow is kept beside its successor until the projector goes:
+    // the graph's replays go on using it.
+    template <typename T>
+    void grow(yk::DeviceArray<T>& a, size_t n)
+    {
+        if (a.size() >= n) return;
+        if (captured && a.size()) retired.push_back(std::make_shared<yk::DeviceArray<T>>(std::move(a)));
+        a.resize(n);
+    }
+    void note_capture();               // sets the two flags for a call about to be made
+    bool capturing = false, captured = false;
+    std::vector<std::shared_ptr<void>> retired;
     yk::DeviceArray<float> d_vol_t;
     yk::DeviceArray<float> d_vol_zx;   // paired volume copies of the Joseph and Siddon projections
     yk::DeviceArray<float> d_vol_zy;

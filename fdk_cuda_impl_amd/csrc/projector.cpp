@@ -11,14 +11,6 @@ using namespace yk;
 
 namespace {
 
-// scratch that only grows: the separable paths alternate between layouts of
-// different sizes in one array, and a reallocation would synchronize
-template <typename T>
-void grow(DeviceArray<T>& a, size_t n)
-{
-    if (a.size() < n) a.resize(n);
-}
-
 // Samples (voxels x views) or views from which the operator-form
 // backprojections sample a paired copy of the views, and the voxels per pixel
 // below which the copy is most of the work: one view at 64^3 takes 8.7 us with
@@ -327,9 +319,17 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
     YK_HIP(hipStreamSynchronize(s));
 }
 
+void yk_projector::note_capture()
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    YK_HIP(hipStreamIsCapturing(ctx->stream, &status));
+    capturing = status != hipStreamCaptureStatusNone;
+    captured = captured || capturing;
+}
+
 float* SolverScratch::array(int k, size_t n)
 {
-    grow(arrays[k], n);
+    if (arrays[k].size() < n) arrays[k].resize(n);
     return arrays[k].get();
 }
 
@@ -356,14 +356,12 @@ bool yk_projector::siddon_copies(yk_projector& w, const float* d_volume, bool an
     if (nv > 65535 || size_x / grid.nx > (size_t(1) << 29) || size_y / grid.ny > (size_t(1) << 29)) return false;
     const size_t need_x = any_x ? size_x : 0, need_y = any_y ? size_y : 0;
     if (w.d_vol_zx.size() < need_x || w.d_vol_zy.size() < need_y || !w.d_flag.get()) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
-        if (capture != hipStreamCaptureStatusNone) return false;
+        if (w.capturing) return false;
     }
     try {
-        grow(w.d_vol_zx, need_x);
-        grow(w.d_vol_zy, need_y);
-        grow(w.d_flag, 1);
+        w.grow(w.d_vol_zx, need_x);
+        w.grow(w.d_vol_zy, need_y);
+        w.grow(w.d_flag, 1);
     } catch (const Error&) {
         (void)hipGetLastError();  // the failed allocation's, not the call's
         return false;
@@ -382,6 +380,7 @@ bool yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
     if (!d_volume || !d_proj) fail(YK_ERR_INVALID_BUFFER, "null device buffer");
     hipStream_t s = ctx->stream;
     yk_projector& w = scratch_owner ? *scratch_owner : *this;  // scratch arrays
+    w.note_capture();
     if (size_t(count) * nu * nv > kResidualRays) residual = nullptr;
     FpStore store{};
     store.mode = accumulate ? FpStore::kAdd : FpStore::kSet;
@@ -397,11 +396,11 @@ bool yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
     if (kind == YK_FP_JOSEPH && all_sep && joseph_column_fits(vol)) {
         // guarded copies (every call rewrites the copy it reads)
         if (any_x) {
-            grow(w.d_vol_zx, joseph_column_size(grid.nx, grid.ny, grid.nz, true));
+            w.grow(w.d_vol_zx, joseph_column_size(grid.nx, grid.ny, grid.nz, true));
             launch_joseph_column_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, s);
         }
         if (any_y) {
-            grow(w.d_vol_zy, joseph_column_size(grid.nx, grid.ny, grid.nz, false));
+            w.grow(w.d_vol_zy, joseph_column_size(grid.nx, grid.ny, grid.nz, false));
             launch_joseph_column_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, s);
         }
         JosephSepFpLaunch p{};
@@ -417,11 +416,11 @@ bool yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
     } else if (kind == YK_FP_JOSEPH && !any_z) {
         // X/Y-main views of any orientation: paired slab copies
         if (any_x) {
-            grow(w.d_vol_zx, joseph_pair_size(grid.nx, grid.ny, grid.nz, true));
+            w.grow(w.d_vol_zx, joseph_pair_size(grid.nx, grid.ny, grid.nz, true));
             launch_joseph_pair_copy(d_volume, w.d_vol_zx.get(), grid.nx, grid.ny, grid.nz, true, s);
         }
         if (any_y) {
-            grow(w.d_vol_zy, joseph_pair_size(grid.nx, grid.ny, grid.nz, false));
+            w.grow(w.d_vol_zy, joseph_pair_size(grid.nx, grid.ny, grid.nz, false));
             launch_joseph_pair_copy(d_volume, w.d_vol_zy.get(), grid.nx, grid.ny, grid.nz, false, s);
         }
         JosephSepFpLaunch p{};
@@ -440,7 +439,7 @@ bool yk_projector::project(int kind, const float* d_volume, float* d_proj, int f
         for (int i = first; i < first + count; ++i)
             if (main_axis(views[i], nu, nv) == 0) need_t = true;
         if (need_t) {
-            w.d_vol_t.resize(size_t(grid.nx) * grid.ny * grid.nz);
+            w.grow(w.d_vol_t, size_t(grid.nx) * grid.ny * grid.nz);
             launch_transpose_xy(d_volume, w.d_vol_t.get(), grid.nx, grid.ny, grid.nz, s);
         }
         JosephLaunch p{};
@@ -525,11 +524,9 @@ int yk_projector::op_chunk(yk_projector& w, int count, bool one_view) const
     const int chunk = one_view ? 1
         : int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
     if (w.d_paired_views.size() < per_view * chunk) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
-        if (capture != hipStreamCaptureStatusNone) return 0;
+        if (w.capturing) return 0;
         try {
-            grow(w.d_paired_views, per_view * chunk);
+            w.grow(w.d_paired_views, per_view * chunk);
         } catch (const Error&) {
             (void)hipGetLastError();
             return 0;
@@ -595,12 +592,10 @@ bool yk_projector::gather_transpose(yk_projector& w, int model, const float* d_p
     if (nv + kGatherPadRows > 65535 || per_view > (size_t(1) << 30)) return false;
     const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
     if (w.d_gather_q.size() < per_view * chunk || !w.d_flag.get()) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
-        if (capture != hipStreamCaptureStatusNone) return false;
+        if (w.capturing) return false;
         try {
-            grow(w.d_gather_q, per_view * chunk);
-            grow(w.d_flag, 1);
+            w.grow(w.d_gather_q, per_view * chunk);
+            w.grow(w.d_flag, 1);
         } catch (const Error&) {
             (void)hipGetLastError();
             return false;
@@ -644,14 +639,12 @@ bool yk_projector::column_transpose(yk_projector& w, const float* d_proj, float*
     for (int i = first; i < first + count; ++i) (main_axis(views[i], nu, nv) == 0 ? any_x : any_y) = true;
     if (w.d_gather_q.size() < per_view * chunk || !w.d_flag.get() || (any_x && w.d_column_x.size() < voxels) ||
         (any_y && w.d_column_y.size() < voxels)) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
-        if (capture != hipStreamCaptureStatusNone) return false;
+        if (w.capturing) return false;
         try {
-            grow(w.d_gather_q, per_view * chunk);
-            grow(w.d_flag, 1);
-            if (any_x) grow(w.d_column_x, voxels);
-            if (any_y) grow(w.d_column_y, voxels);
+            w.grow(w.d_gather_q, per_view * chunk);
+            w.grow(w.d_flag, 1);
+            if (any_x) w.grow(w.d_column_x, voxels);
+            if (any_y) w.grow(w.d_column_y, voxels);
         } catch (const Error&) {
             (void)hipGetLastError();
             return false;
@@ -686,11 +679,9 @@ bool yk_projector::scatter_transpose(yk_projector& w, bool siddon, const float* 
     const size_t per_view = (siddon ? 2 : 3) * rays + 2 * size_t(nu);
     const int chunk = int(std::max<size_t>(1, std::min({ size_t(count), size_t(65535), (size_t(1) << 28) / per_view })));
     if (w.d_scatter.size() < per_view * chunk) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        YK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
-        if (capture != hipStreamCaptureStatusNone) return false;
+        if (w.capturing) return false;
         try {
-            grow(w.d_scatter, per_view * chunk);
+            w.grow(w.d_scatter, per_view * chunk);
         } catch (const Error&) {
             (void)hipGetLastError();
             return false;
@@ -728,8 +719,8 @@ void yk_projector::transpose(yk_projector& w, bool siddon, TransposeForm form, c
         const size_t per_view = size_t(nu) * nv;
         const int chunk = int(std::max<size_t>(1, std::min<size_t>(size_t(count),
             (size_t(1) << 30) / (per_view * (sizeof(float4) + sizeof(float))))));
-        w.d_ray_ab.resize(std::max(w.d_ray_ab.size(), per_view * chunk));
-        w.d_ray_len.resize(std::max(w.d_ray_len.size(), per_view * chunk));
+        w.grow(w.d_ray_ab, per_view * chunk);
+        w.grow(w.d_ray_len, per_view * chunk);
         for (int c0 = 0; c0 < count; c0 += chunk) {
             JosephAdjointLaunch p{};
             p.proj = d_proj + per_view * c0;
@@ -763,6 +754,7 @@ void yk_projector::backproject(int kind, const float* d_proj, float* d_volume, i
     if (!d_volume || !d_proj) fail(YK_ERR_INVALID_BUFFER, "null device buffer");
     hipStream_t s = ctx->stream;
     yk_projector& w = scratch_owner ? *scratch_owner : *this;  // scratch arrays
+    w.note_capture();
     if (kind == YK_BP_JOSEPH_ADJOINT || kind == YK_BP_SIDDON_ADJOINT) {
         const bool siddon = kind == YK_BP_SIDDON_ADJOINT;
         for (const TransposeRun& r : transpose_runs(siddon, first, count)) {

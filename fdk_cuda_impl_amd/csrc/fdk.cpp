@@ -27,14 +27,20 @@ size_t storage_bytes(int storage)
 
 // View split of the backprojection (split_views): workgroups wanted (16 per
 // CU: four resident rounds, so the last one's idle tail is small), the fewest
-// views worth a part (the first view's staging is exposed), the most parts,
-// and the most bytes of part volumes, which then stay in the last-level cache
+// views worth a part (the first view's staging is exposed), the voxels that ask for
+// one more (a part is a pass over its volume and the sum's) and the most that is
+// asked, the most parts, and the most bytes of part volumes, which then stay in the last-level cache
 // (256 x 256 x 200 from 60 views in two or three parts measured 2 % slower).
 // Backprojection, one part -> split: 32 x 32 x 24 x 48 views 86 -> 16 us,
 // 64^3 x 90 158 -> 26, 128^3 x 180 385 -> 214 (1024 workgroups 258, 2048
-// 225), 201 x 187 x 150 x 401 tilted 1551 -> 1267 (1024 unchanged).
+// 225), 201 x 187 x 150 x 401 tilted 1551 -> 1267 (1024 unchanged).  Few views, one
+// part and parts of four or five: 128^3 x 10 22 and 26 us, 160^3 x 10 25 and 38, x
+// 20 57 and 69, x 40 133 and 105 (of eight); 200^3 x 40 half storage 210 and 177 (of
+// 13); 224^3 x 10 51 and 81, x 40 223 and 239 (of 20); 112^3 x 20 49 and 34.
 constexpr long kBpBlocks = 4096;
 constexpr int kBpPartViews = 4;
+constexpr int kBpMostPartViews = 13;
+constexpr size_t kBpPartVoxels = 400000;
 constexpr int kBpMaxParts = 16;
 constexpr size_t kBpPartBytes = size_t(96) << 20;
 
@@ -298,8 +304,10 @@ int yk_fdk::part_count(int count) const
 {
     const long blocks = long(nbx) * nby * nbz;
     const long want = (kBpBlocks + blocks - 1) / blocks;
-    const long room = long(kBpPartBytes / (size_t(grid.nx) * grid.ny * grid.nz * sizeof(float)));
-    return int(std::max(1L, std::min({ want, long(count / kBpPartViews), long(kBpMaxParts), room })));
+    const size_t voxels = size_t(grid.nx) * grid.ny * grid.nz;
+    const long room = long(kBpPartBytes / (voxels * sizeof(float)));
+    const long views = std::clamp(long((voxels + kBpPartVoxels - 1) / kBpPartVoxels), long(kBpPartViews), long(kBpMostPartViews));
+    return int(std::max(1L, std::min({ want, count / views, long(kBpMaxParts), room })));
 }
 
 void yk_fdk::backproject(const void* d_filtered, int storage, const float* d_scales, int first,

@@ -185,6 +185,7 @@ struct yk_projector {
     yk::DeviceArray<float> d_vol_zx;   // paired volume copies of the Joseph and Siddon projections
     yk::DeviceArray<float> d_vol_zy;
     std::vector<char> siddon_flat;     // per view: siddon_flat_gather covers it
+    std::vector<char> siddon_ends;     // per view: the detector may end rays inside the volume
     std::vector<char> joseph_column;   // per view: the column transpose covers it
     yk::DeviceArray<float> d_column_x, d_column_y;  // its volumes of the X- and Y-main views
     std::vector<char> joseph_gather, siddon_gather;  // per view: the gather transposes cover it

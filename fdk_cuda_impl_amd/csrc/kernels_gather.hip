@@ -285,11 +285,9 @@ __device__ __forceinline__ void joseph_gather(const float* __restrict__ q, const
     }
 }
 
-// offset of plane c between cells from the source; exactly zero on the source's own plane
-__device__ __forceinline__ float plane_offset(float lo, float vox, int c, float s, int plane)
-{
-    return c == plane ? 0.f : lo + float(c) * vox - s;
-}
+// offset of plane c between cells from the source (SiddonViewDev::on_plane):
+// exactly zero on the source's own plane
+__device__ __forceinline__ float plane_offset(float lo, float vox, int c, float s) { return fmaf(float(c), vox, lo) - s; }
 
 template <int ZR, bool SAFE>
 __device__ __forceinline__ void siddon_gather(const float* __restrict__ q, const GatherViewDev* __restrict__ views,
@@ -305,19 +303,19 @@ __device__ __forceinline__ void siddon_gather(const float* __restrict__ q, const
         const float* qi = q + 3 * ((size_t)i * (nv + kGatherPadRows) * pitch);
         const CandidateBox<ZR> box(views[i], x, y, z0, 0.5f, 0.5f, 1.f);
         const SiddonViewDev& sv = sviews[i];
-        const float x0 = plane_offset(lox, g.vx, x, sv.src[0], sv.plane[0]);
-        const float x1 = plane_offset(lox, g.vx, x + 1, sv.src[0], sv.plane[0]);
-        const float y0 = plane_offset(loy, g.vy, y, sv.src[1], sv.plane[1]);
-        const float y1 = plane_offset(loy, g.vy, y + 1, sv.src[1], sv.plane[1]);
+        const float x0 = plane_offset(lox, g.vx, x, sv.on_plane[0]);
+        const float x1 = plane_offset(lox, g.vx, x + 1, sv.on_plane[0]);
+        const float y0 = plane_offset(loy, g.vy, y, sv.on_plane[1]);
+        const float y1 = plane_offset(loy, g.vy, y + 1, sv.on_plane[1]);
         const bool xmain = views[i].axis == 0;
         const float m0 = xmain ? x0 : y0, m1 = xmain ? x1 : y1, n0 = xmain ? y0 : x0, n1 = xmain ? y1 : x1;
 #pragma unroll
         for (int p = 0; p < ZR; p += 2) {
             int ulo, uhi, vlo, vhi;
             if (!box.pair(z0 + p, nu, nv, ulo, uhi, vlo, vhi)) continue;
-            const float za = plane_offset(loz, g.vz, z0 + p, sv.src[2], sv.plane[2]);
-            const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.src[2], sv.plane[2]);
-            const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.src[2], sv.plane[2]);
+            const float za = plane_offset(loz, g.vz, z0 + p, sv.on_plane[2]);
+            const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.on_plane[2]);
+            const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.on_plane[2]);
             unsigned row = unsigned(vlo) * unsigned(pitch);
 #pragma unroll 1
             for (int v = vlo; v <= vhi; v += kRows) {
@@ -363,7 +361,9 @@ __device__ __forceinline__ void siddon_gather(const float* __restrict__ q, const
 // views of 512 x 384 17.2 -> 10.4 ms, 128^3 x 120 891 -> 570 us, 64^3 x 60 116
 // -> 102.  (Pixels x rows a chunk at 256^3: 3 x 1 12.9 ms, 3 x 3 11.2, 2 x 2
 // 22.3, 4 x 2 10.9.)
-template <int ZR, bool SAFE>
+// ENDS: a ray ends at its pixel, t = 1, inside the volume of some view (5 % on
+// the others).
+template <int ZR, bool SAFE, bool ENDS>
 __device__ __forceinline__ void siddon_flat_gather(const float* __restrict__ q, const float2* __restrict__ ru,
     const float* __restrict__ rv, const GatherViewDev* __restrict__ views, const SiddonViewDev* __restrict__ sviews,
     const VolumeGeom& g, int nu, int nv, int pitch, int count, int x, int y, int z0, float (&acc)[ZR])
@@ -377,10 +377,10 @@ __device__ __forceinline__ void siddon_flat_gather(const float* __restrict__ q, 
         const float* rvi = rv + rows;
         const CandidateBox<ZR> box(views[i], x, y, z0, 0.5f, 0.5f, 1.f);
         const SiddonViewDev& sv = sviews[i];
-        const float x0 = plane_offset(lox, g.vx, x, sv.src[0], sv.plane[0]);
-        const float x1 = plane_offset(lox, g.vx, x + 1, sv.src[0], sv.plane[0]);
-        const float y0 = plane_offset(loy, g.vy, y, sv.src[1], sv.plane[1]);
-        const float y1 = plane_offset(loy, g.vy, y + 1, sv.src[1], sv.plane[1]);
+        const float x0 = plane_offset(lox, g.vx, x, sv.on_plane[0]);
+        const float x1 = plane_offset(lox, g.vx, x + 1, sv.on_plane[0]);
+        const float y0 = plane_offset(loy, g.vy, y, sv.on_plane[1]);
+        const float y1 = plane_offset(loy, g.vy, y + 1, sv.on_plane[1]);
         const int ulo = int(fmaxf(0.f, ceilf(box.um - box.hu))), uhi = int(fminf(float(nu - 1), floorf(box.um + box.hu)));
 #pragma unroll 1
         for (int u = ulo; u <= uhi; u += kWidth) {
@@ -389,17 +389,20 @@ __device__ __forceinline__ void siddon_flat_gather(const float* __restrict__ q, 
             for (int k = 0; k < kWidth; ++k) {
                 const float2 c = ru[(size_t)i * pitch + (u + k)];
                 const float tx0 = x0 * c.x, tx1 = x1 * c.x;
-                // (the ray ends at its pixel, t = 1)
-                ya[k] = fminf(__builtin_amdgcn_fmed3f(y0 * c.y, tx0, tx1), 1.f);
-                yb[k] = fminf(__builtin_amdgcn_fmed3f(y1 * c.y, tx0, tx1), 1.f);
+                ya[k] = __builtin_amdgcn_fmed3f(y0 * c.y, tx0, tx1);
+                yb[k] = __builtin_amdgcn_fmed3f(y1 * c.y, tx0, tx1);
+                if constexpr (ENDS) {
+                    ya[k] = fminf(ya[k], 1.f);
+                    yb[k] = fminf(yb[k], 1.f);
+                }
             }
 #pragma unroll
             for (int p = 0; p < ZR; p += 2) {
                 const float vc = fmaf(box.v_zd, float(p) + 0.5f - 0.5f * float(ZR - 1), box.vm);
                 const int vlo = int(fmaxf(0.f, ceilf(vc - box.hv))), vhi = int(fminf(float(nv - 1), floorf(vc + box.hv)));
-                const float za = plane_offset(loz, g.vz, z0 + p, sv.src[2], sv.plane[2]);
-                const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.src[2], sv.plane[2]);
-                const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.src[2], sv.plane[2]);
+                const float za = plane_offset(loz, g.vz, z0 + p, sv.on_plane[2]);
+                const float zb = plane_offset(loz, g.vz, z0 + p + 1, sv.on_plane[2]);
+                const float zc = plane_offset(loz, g.vz, z0 + p + 2, sv.on_plane[2]);
                 unsigned row = unsigned(vlo) * unsigned(pitch) + unsigned(u);
 #pragma unroll 1
                 for (int v = vlo; v <= vhi; v += kRows) {
@@ -441,10 +444,11 @@ gather_transpose_kernel(const void* __restrict__ q, const float2* __restrict__ r
 #pragma unroll
     for (int k = 0; k < ZR; ++k) acc[k] = 0.f;
     const bool plain = __builtin_amdgcn_readfirstlane(*flag) == 0;
-    if constexpr (MODEL == kGatherSiddonFlat) {
+    if constexpr (MODEL == kGatherSiddonFlat || MODEL == kGatherSiddonFlatEnds) {
+        constexpr bool kEnds = MODEL == kGatherSiddonFlatEnds;
         const float* t = static_cast<const float*>(q);
-        if (plain) siddon_flat_gather<ZR, false>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
-        else siddon_flat_gather<ZR, true>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
+        if (plain) siddon_flat_gather<ZR, false, kEnds>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
+        else siddon_flat_gather<ZR, true, kEnds>(t, ru, rv, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
     } else if constexpr (MODEL == kGatherSiddon) {
         const float* t = static_cast<const float*>(q);
         if (plain) siddon_gather<ZR, false>(t, views, sviews, g, nu, nv, pitch, count, x, y, z0, acc);
@@ -494,10 +498,11 @@ void launch_gather_transpose(const GatherLaunch& p, hipStream_t s)
     // (64 x 4 rays a workgroup: 256 rays of one row left half of them idle at a
     // pitch of 260; CGLS at 128^3 x 120 views of 256 x 192 5.84 -> 5.76 ms)
     dim3 tb(64, 4), tg((p.pitch + 63) / 64, (p.nv + kGatherPadRows + 3) / 4, p.count);
-    if (p.model == kGatherSiddonFlat) {
+    if (p.model == kGatherSiddonFlat || p.model == kGatherSiddonFlatEnds) {
         hipLaunchKernelGGL(siddon_flat_table_kernel, tg, tb, 0, s, p.proj, p.sviews, p.vol, p.nu, p.nv, p.pitch, p.q, p.ru,
             p.rv, p.flag);
-        launch_gather<kGatherSiddonFlat>(p, s);
+        if (p.model == kGatherSiddonFlatEnds) launch_gather<kGatherSiddonFlatEnds>(p, s);
+        else launch_gather<kGatherSiddonFlat>(p, s);
     } else if (p.model == kGatherSiddon) {
         hipLaunchKernelGGL(siddon_gather_table_kernel, tg, tb, 0, s, p.proj, p.sviews, p.gviews, p.vol, p.nu,
             p.nv, p.pitch, p.q, p.flag);

@@ -214,7 +214,11 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
         std::memcpy(s.detV, w.detV, sizeof(s.detV));
         siddon_axes.push_back(char(ray_axes(widen(w), vox, nu, nv)));
         const int cells[3] = { grid.nx, grid.ny, grid.nz };
-        for (int k = 0; k < 3; ++k) s.plane[k] = source_plane(w.src[k], cen[k], vox[k], cells[k]);
+        const float lo[3] = { vol.ox - 0.5f * vol.vx, vol.oy - 0.5f * vol.vy, vol.oz - 0.5f * vol.vz };
+        for (int k = 0; k < 3; ++k) {
+            s.plane[k] = source_plane(w.src[k], cen[k], vox[k], cells[k]);
+            s.on_plane[k] = s.plane[k] < 0 ? w.src[k] : std::fma(float(s.plane[k]), float(vox[k]), lo[k]);
+        }
         projection_map(w, &c64[size_t(i) * 12]);
         // Gather transposes.  Their kernels take every support of a run of
         // kGatherRun voxels to lie before the source, and the general Siddon one
@@ -237,6 +241,7 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
             joseph_gather.push_back(front);
             siddon_gather.push_back(front && outer < 1.0 && along_main(widen(w), p.axis, nu, nv));
             siddon_flat.push_back(front && separable.back() && w.detU[2] == 0.f);
+            siddon_ends.push_back(!(outer < 1.0));
             joseph_column.push_back(front && separable.back() && column_view(p, nu, nv, vol));
         } else {
             near_source.push_back(0);
@@ -244,6 +249,7 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
             siddon_gather.push_back(0);
             joseph_column.push_back(0);
             siddon_flat.push_back(0);
+            siddon_ends.push_back(0);
         }
     }
     d_gather.upload(gv.data(), gv.size(), ctx->stream);
@@ -584,7 +590,7 @@ std::vector<yk_projector::TransposeRun> yk_projector::transpose_runs(bool siddon
 bool yk_projector::gather_transpose(yk_projector& w, int model, const float* d_proj, float* d_volume, int first, int count,
     int accumulate)
 {
-    const bool flat = model == kGatherSiddonFlat;
+    const bool flat = model == kGatherSiddonFlat || model == kGatherSiddonFlatEnds;
     const int pitch = nu + kGatherPad;
     // floats (flat: an entry a column and a row more, columns' aligned to 8 bytes)
     const size_t rows = size_t(nv) + kGatherPadRows;
@@ -710,7 +716,8 @@ void yk_projector::transpose(yk_projector& w, bool siddon, TransposeForm form, c
     int count, int accumulate)
 {
     hipStream_t s = ctx->stream;
-    const int model = !siddon ? kGatherJoseph : form == kUntilted ? kGatherSiddonFlat : kGatherSiddon;
+    const bool ends = std::any_of(siddon_ends.begin() + first, siddon_ends.begin() + first + count, [](char c) { return c != 0; });
+    const int model = !siddon ? kGatherJoseph : form != kUntilted ? kGatherSiddon : ends ? kGatherSiddonFlatEnds : kGatherSiddonFlat;
     if (form == kScatter && scatter_transpose(w, siddon, d_proj, d_volume, first, count, accumulate)) return;
     if (!siddon && form == kUntilted && column_transpose(w, d_proj, d_volume, first, count, accumulate)) {
     } else if (form <= kGeneral && gather_transpose(w, model, d_proj, d_volume, first, count, accumulate)) {

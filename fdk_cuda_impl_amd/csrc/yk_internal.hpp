@@ -278,6 +278,7 @@ struct SiddonViewDev {
     float detU[4];
     float detV[4];
     int plane[4];               // per axis, the plane between cells that the source lies on, or -1 (projector.cpp)
+    float on_plane[4];          // src, moved onto that plane as the gathers form it
 };
 
 struct JosephLaunch {
@@ -360,8 +361,9 @@ struct GatherViewDev {
     int axis;                   // 0 X, 1 Y
 };
 
-// (flat: separable views whose row steps have no z component)
-enum GatherModel { kGatherJoseph, kGatherSiddon, kGatherSiddonFlat };
+// (flat: separable views whose row steps have no z component; ends: rays may end
+// inside the volume)
+enum GatherModel { kGatherJoseph, kGatherSiddon, kGatherSiddonFlat, kGatherSiddonFlatEnds };
 struct GatherLaunch {
     const float* proj;          // [count][nv][nu]
     float* volume;              // [z][y][x]

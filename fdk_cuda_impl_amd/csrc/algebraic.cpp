@@ -237,7 +237,7 @@ void run_algebraic(yk_projector* p, const yk_algebraic_desc& d, const float* d_b
         if (d.tv_iterations > 0 && tv_strength > 0.f) {
             p->ctx->reduce_scratch.resize(kTvPartials);
             for (int j = 0; j < d.tv_iterations; ++j) {
-                launch_tv_gradient(d_x, grad, p->ctx->reduce_scratch.get(), kTvPartials, g, d.tv_epsilon, s,
+                launch_tv_gradient(d_x, grad, p->ctx->reduce_scratch.get(), tv_partials(g), g, d.tv_epsilon, s,
                     d.tv_dimensions == 2 ? 2 : 3);
                 launch_axpy(d_x, grad, -tv_strength, nx, s);
             }

@@ -641,10 +641,10 @@ yk_status yk_tv_gradient(yk_ctx* ctx, const yk_volume_grid* volume, const float*
         validate_volume(*volume);
         require(std::isfinite(eps) && eps > 0.f, YK_ERR_INVALID_CONFIG, "epsilon must be positive");
         ctx->activate();
-        const int parts = kTvPartials;
-        ctx->reduce_scratch.resize(parts);
-        launch_tv_gradient(d_x, d_gradient, ctx->reduce_scratch.get(), parts, volume_geom(*volume), eps,
-            ctx->stream);
+        const VolumeGeom g = volume_geom(*volume);
+        const int parts = tv_partials(g);
+        ctx->reduce_scratch.resize(kTvPartials);
+        launch_tv_gradient(d_x, d_gradient, ctx->reduce_scratch.get(), parts, g, eps, ctx->stream);
         std::vector<double> h(parts);
         YK_HIP(hipMemcpyAsync(h.data(), ctx->reduce_scratch.get(), parts * sizeof(double),
             hipMemcpyDeviceToHost, ctx->stream));

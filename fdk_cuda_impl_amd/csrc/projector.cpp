@@ -328,7 +328,10 @@ yk_projector::yk_projector(yk_ctx* c, const yk_view* v, int n, int nu_, int nv_,
 void yk_projector::note_capture()
 {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    YK_HIP(hipStreamIsCapturing(ctx->stream, &status));
+    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) {
+        (void)hipGetLastError();  // (the null stream beside another's capture: the launches say what is wrong)
+        status = hipStreamCaptureStatusNone;
+    }
     capturing = status != hipStreamCaptureStatusNone;
     captured = captured || capturing;
 }

@@ -1332,16 +1332,21 @@ namespace {
 // view (256 and 128 columns) 31.9 -> 35.9 and 23.6 -> 25.4.
 constexpr size_t kFewColumns = 2048;
 
+// Whole columns up to which a workgroup takes four views' instead of eight: fewer
+// of them end half empty, but fewer share tap rows.  Eight and four: 256^3 from 60
+// views of 512 x 384 (30720 columns) 1023 and 982 us, from 360 (184320) 5.77 and 5.73
+// ms; 512^3 of 1024 x 768 from 90 (92160) 16.7 and 15.6, from 720 (737280) 102.6 and
+// 107.1.
+constexpr size_t kFewRounds = 262144;
+
 template <int K, bool SPLIT>
 void launch_column_kernel(const JosephSepFpLaunch& p, hipStream_t s)
 {
     const size_t column = size_t(column_pitch(p.vol.nz)) * sizeof(float);
     // the waves' columns in 32 KiB; a longer column has a workgroup to itself
     int waves = column <= 4096 ? kColumnWaves : column <= 8192 ? 4 : column <= 16384 ? 2 : 1;
-    // (whole columns: four views a workgroup leave no half-empty ones at the end of
-    // a call, 256^3 from 60 views of 512 x 384 1023 -> 982 us, of 256 x 192 570 -> 495,
-    // from 360 5.77 -> 5.73 ms)
-    if (!SPLIT || size_t(p.nu) * p.count >= kFewColumns) waves = std::min(waves, 4);
+    const size_t columns = size_t(p.nu) * p.count;
+    if (SPLIT ? columns >= kFewColumns : columns <= kFewRounds) waves = std::min(waves, 4);
     const size_t lds = column * waves + (SPLIT ? size_t(kColumnParts) * 64 * K * sizeof(float) : 0);
     if (waves == 1)
         YK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(joseph_fp_column_kernel<K, SPLIT>),

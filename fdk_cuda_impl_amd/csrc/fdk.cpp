@@ -218,7 +218,13 @@ yk_fdk::yk_fdk(yk_ctx* c, const yk_fdk_desc& d, const yk_view* v, int n, int nu_
     }
     build_tiles();
     const int parts = part_count(n);
-    if (parts > 1) d_parts.resize(size_t(parts) * grid.nx * grid.ny * grid.nz);
+    if (parts > 1) {
+        try {
+            d_parts.resize(size_t(parts) * grid.nx * grid.ny * grid.nz);
+        } catch (const Error&) {
+            (void)hipGetLastError();  // no memory for them: one part
+        }
+    }
     YK_HIP(hipStreamSynchronize(s));
 
     batch = desc.batch_views > 0 ? std::min(desc.batch_views, n) : n;

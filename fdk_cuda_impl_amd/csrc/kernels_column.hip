@@ -17,9 +17,9 @@
 // The columns of a slice and block of rows are found by projecting the block's
 // ends; their parameters are formed 64 at a time, a column a lane, and handed
 // to the wave by lane reads, so a column's candidates differ by lane only in z.
-// Bound: VALU issue, 20 instructions for each column and 64 voxels, with the
-// vector memory pipe (16 cycles of a CU for the same) close behind.  Joseph
-// transpose against the gather over both axes: 256^3 x 360 views of 512 x 384
+// Bound: the vector memory pipe (16 cycles of a CU for each column and 64 voxels;
+// its addressers are 86 % busy, profiles/projectors_counters.txt) and VALU issue (20
+// instructions for the same).  Joseph transpose against the gather over both axes: 256^3 x 360 views of 512 x 384
 // 15.3 -> 5.8 ms, 128^3 x 120 of 256 x 192 870 -> 426 us, 96^3 x 60 237 -> 169.
 #include <hip/hip_runtime.h>
 

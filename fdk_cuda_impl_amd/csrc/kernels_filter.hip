@@ -605,7 +605,7 @@ void launch_length(const FilterLaunch& p, int rows, size_t lds, hipStream_t s)
 template <int STORAGE>
 void launch_storage(const FilterLaunch& p, int rows, size_t lds, hipStream_t s)
 {
-    // bfloat16 rows of 65 to 256 padded values keep the run-time form (90 x 96
+    // bfloat16 rows of up to 256 padded values keep the run-time form (90 x 96
     // rows 23.5 us against 9.4): the compiler contracts other products in the
     // two, the FP32 values differ in the last bit, and a value that then rounds
     // the other way in bfloat16 moves a voxel of few views by up to 2e-3 of the

@@ -30,8 +30,9 @@
 // 0.11 ms.  Untilted views have forms of their own where they are faster
 // (kernels_column.hip, siddon_flat_gather).
 // Bound: VALU issue (Joseph: 324 instructions a voxel pair and view, of which 218
-// weigh its 5.4 rows of 4 candidates; the texture addressers are 63 % busy;
-// Siddon: its six 12-byte loads for 84 instructions keep those busier).
+// weigh its 5.4 rows of 4 candidates; the texture addressers are 67 % busy) or the
+// addressers (Siddon: six 12-byte loads for 84 instructions, 95 % busy; untilted 84
+// %); profiles/projectors_counters.txt.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

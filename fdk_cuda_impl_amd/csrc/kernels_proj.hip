@@ -13,8 +13,8 @@
 // src/FlatFpBp/FP/kernels/YkFPSiddonKernel.cu:19-124); voxel boundaries are
 // recomputed from integer indices instead of accumulated.
 //
-// Transposes are deterministic gathers (no atomics).  The ones here serve the
-// views that kernels_gather.hip and kernels_column.hip leave: for each voxel and
+// Transposes are deterministic (no atomics).  The gathers here serve the views that
+// kernels_gather.hip, kernels_column.hip and kernels_scatter.hip leave: for each voxel and
 // view the candidate rays are the detector pixels inside the projection of the
 // voxel's support, and each is re-evaluated with exactly the arithmetic of the
 // forward kernel (shared functions below, FP contraction off).
@@ -179,12 +179,13 @@ typedef float float4u __attribute__((ext_vector_type(4), aligned(8)));
 // The copy has kJosephGuard zero planes on both sides of both minor axes, and
 // sample positions are clamped to [-2, n], so a position outside (-1, n) reads
 // only zeros and no sample is tested for range.
-// Bound: the vector memory pipe (two rows of the volume a column and slice;
-// without these loads 25 % less) with VALU issue close behind (without loads
-// and LDS reads 47 % less).  Six waves a SIMD hide the slice's chain: with
-// four 5 % slower, with eight the spills cost as much again.  Copies included,
-// with gathers -> here: 256^3 x 360 views of 512 x 384 9.2 -> 5.7 ms, 512^3 x
-// 90 of 1024 x 768 23.7 -> 15.0 ms, 128^3 x 12 of 256 x 192 69 -> 55 us.
+// Bound: the chain of a slice (load, interpolation, LDS, samples), with the vector
+// memory pipe 64 %, the LDS 50 % and the VALU up to 97 % busy
+// (profiles/projectors_counters.txt; without the volume's loads 25 % less time,
+// without loads and LDS reads 47 %).  Six waves a SIMD hide the chain: with four 4 %
+// slower, with eight the spills cost as much again.  Copies included, with gathers
+// -> here: 256^3 x 360 views of 512 x 384 9.2 -> 5.7 ms, 512^3 x 90 of 1024 x 768 23.7
+// -> 15.7 ms, 128^3 x 12 of 256 x 192 69 -> 55 us.
 constexpr int kColumnChunk = 256;  // z a wave loads at a time, four a lane
 // values of a copy's row: whole 16-byte groups
 __host__ __device__ __forceinline__ int column_pitch(int nz) { return (nz + 2 * kJosephGuard + 3) & ~3; }

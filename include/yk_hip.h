@@ -338,7 +338,10 @@ int yk_fdk_complete(const yk_fdk* fdk);
 yk_status yk_fdk_filter(yk_fdk* fdk, const float* d_projection, int first_view,
     int count, void* d_filtered, int storage, float* d_row_scales);
 /* Voxel-driven FDK backprojection of filtered views [first, first+count) into
- * d_volume ([z][y][x]); accumulate = 0 overwrites. */
+ * d_volume ([z][y][x]); accumulate = 0 overwrites.  The plan of a volume too
+ * small to fill the GPU keeps part volumes for it (at most 96 MiB), so the
+ * backprojections of one plan, replays of captured ones among them, run one
+ * after another. */
 yk_status yk_fdk_backproject(yk_fdk* fdk, const void* d_filtered, int storage,
     const float* d_row_scales, int first_view, int count, float* d_volume,
     int accumulate);
@@ -371,7 +374,20 @@ yk_status yk_projector_create(yk_ctx* ctx, const yk_view* views, int n_views,
     int nu, int nv, const yk_volume_grid* volume, float scan_range_rad,
     yk_projector** out);
 yk_status yk_projector_destroy(yk_projector* projector);
-/* d_projection holds views [first, first+count); accumulate = 0 overwrites */
+/* d_projection holds views [first, first+count); accumulate = 0 overwrites.
+ * A ray of yk_project has the same bits whatever range of views the call asks
+ * for (except where no memory is left for the volume copies, or none may be
+ * allocated under a stream capture before a first eager call).
+ *
+ * A projector keeps the scratch that its calls made until it is destroyed:
+ * copies of the volume (Joseph untilted 4, Joseph tilted and Siddon 8 bytes a
+ * voxel for each of the X and Y main axes that the views have; Joseph
+ * transpose of untilted views 4), ray or view tables of at most 1 GiB for each
+ * kind of operator, and at most 1 GiB of the algebraic solvers' arrays.  At
+ * 1024^3 that is 17 GB for a Siddon projection all around.  Where there is no
+ * memory for them a slower form without them serves the call (the Joseph
+ * projection of views along X and Y fails).  Calls of one projector, replays of captured ones among them, run one after another; a
+ * captured call goes on using its scratch when later calls need more. */
 yk_status yk_project(yk_projector* projector, int forward_kind, const float* d_volume,
     float* d_projection, int first_view, int count, int accumulate);
 yk_status yk_backproject(yk_projector* projector, int back_kind, const float* d_projection,
